@@ -1,0 +1,58 @@
+// direct.h -- the cal_w system L x = f by a direct method (k_direct.hip).
+//
+// L has constant coefficients along the periodic x, so the discrete Hartley
+// transform along x (real, its own inverse up to 1/N) makes it one tridiagonal
+// system along z for each of the N frequencies: diagonal
+// cx_j lambda_q + cu_j + cu_{j-1}, lambda_q = 4 sin^2(pi q / N), off-diagonal
+// -cu_j.  Any N and M: the transform is a mixed-radix FFT (8, 4, 2, 3, 5, and
+// a direct sum for any other prime factor).
+#pragma once
+
+#include "vvm_internal.h"
+
+namespace vvmd {
+
+constexpr int kMaxStages = 16;
+
+// The factors of N and the launch shape of the row transforms.
+struct RowPlan {
+    int N = 0, M = 0;
+    int nst = 0, radix[kMaxStages] = {};
+    int threads = 0;      // at least N / 8: a thread holds at most 8 outputs of a stage
+    int tw_lds = 0;       // twiddles staged in LDS (a prime factor above 5)
+};
+
+template <typename T>
+class Direct {
+   public:
+    // cx [M+2], cu [M+1]: level-0 coefficients on the device.  Returns VVM_OK
+    // or VVM_ERR_NOMEM / VVM_ERR_HIP.
+    int init(int N, int M, const double *cx, const double *cu);
+    void destroy();
+    bool ready() const { return spec != nullptr; }
+
+    // x = L^-1 r on rows 1..M of (M+2) x N arrays, or x0 + L^-1 r if x0 is set
+    // (which may be x).
+    void solve(const double *r, const double *x0, double *x, hipStream_t st);
+    // cal_w whole: f = -b / rhow from zetap (f is written, for the residual),
+    // x = L^-1 f, w = x / rhow with its halos.
+    void solve_step(const Grid &G, const double *zetap, const double *rhow, double *f, double *x, double *w,
+                    hipStream_t st);
+
+   private:
+    RowPlan plan;
+    size_t row_lds = 0, col_lds = 0;
+    T *tw = nullptr;    // [N][2]: cos, -sin of 2 pi k / N
+    T *g = nullptr;     // [M][N/2+1] elimination factors
+    T *di = nullptr;    // [M][N/2+1] 1 / (N pivot)
+    T *spec = nullptr;  // [M][N] transformed rows
+    void columns(hipStream_t st);
+};
+
+// ||wD (f - L x)||^2 and ||wD f||^2, one pair of partial sums per workgroup in
+// hres (host-mapped memory, 2 x the returned count of doubles).
+constexpr int kResidualBlocks = 512;
+int launch_residual_norms(int N, int M, const double *f, const double *x, const double *cx, const double *cu,
+                          const double *wD, double *hres, hipStream_t st);
+
+}  // namespace vvmd

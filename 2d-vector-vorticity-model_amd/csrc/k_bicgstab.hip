@@ -191,12 +191,12 @@ SolveResult Poisson::solve_bicgstab(double tol, bool absolute, int max_iter, hip
     double *rh = bcg, *p = bcg + n, *v = bcg + 2 * n, *s = bcg + 3 * n, *t = bcg + 4 * n, *ph = bcg + 5 * n,
            *sh = bcg + 6 * n;
     PCG<double> &P = pcg64;
-    const double *cx = P.mg.lev[0].cx, *cu = P.mg.lev[0].cu;
+    const double *cx = cx0, *cu = cu0;
     const dim3 g = bgrid(N, M), b(BX, BY);
     const int nb = nblocks(g);
     // r = f - A x with the pending guess, ||wD r||^2 and ||b||^2 into hscal;
     // r^ = r, rho_0 = r^.r
-    first_residual(P.r, false, st);
+    first_residual(P.r, st);
     hipLaunchKernelGGL(k_bcg_copy, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, n, P.r, rh);
     hipLaunchKernelGGL(k_bcg_dot, g, b, 0, st, N, M, P.r, P.r, red);
     finalize<1>(red, nb, bsc, RED_STORE, B_RHO0, st);

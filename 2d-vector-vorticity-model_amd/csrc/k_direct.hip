@@ -1,0 +1,617 @@
+// k_direct.hip -- direct solve of the cal_w system (direct.h).
+//
+// Three kernels: the forward row transforms, the tridiagonal systems, the
+// inverse row transforms.  At 2048 x 255 they move 8 + 12 + 8 MB and are
+// bound by latency (four LDS round trips a transform, the elimination's
+// serial chain), not by bandwidth.
+#include <algorithm>
+#include <cmath>
+#include <vector>
+
+#include "direct.h"
+
+namespace vvmd {
+
+namespace {
+
+// ---------------------------------------------------------- row transforms
+//
+// One workgroup transforms two rows at once, as the real and imaginary part
+// of one complex FFT in LDS; the two spectra are separated as they leave.
+// The FFT is Stockham's: each stage reads its inputs N/R apart and writes
+// them in order, all reads before a barrier and all writes after it, so one
+// buffer is enough (8192 columns in FP64 take 135 KB).  Real and imaginary
+// parts lie in separate arrays with one word of padding every 32, which makes
+// the strided writes of the first stages conflict-free.
+
+__device__ inline int pad(int i) { return i + (i >> 5); }
+
+template <typename T>
+struct Cx {
+    T x, y;
+};
+template <typename T>
+__device__ inline Cx<T> operator+(Cx<T> a, Cx<T> b) {
+    return {a.x + b.x, a.y + b.y};
+}
+template <typename T>
+__device__ inline Cx<T> operator-(Cx<T> a, Cx<T> b) {
+    return {a.x - b.x, a.y - b.y};
+}
+template <typename T>
+__device__ inline Cx<T> mul(Cx<T> a, Cx<T> b) {
+    return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
+}
+template <typename T>
+__device__ inline Cx<T> mul_mi(Cx<T> a) {  // -i a
+    return {a.y, -a.x};
+}
+
+// Forward DFTs of R values in place (kernel exp(-2 pi i / R)).
+template <typename T>
+__device__ inline void dft2(Cx<T> &a, Cx<T> &b) {
+    const Cx<T> t = a;
+    a = t + b;
+    b = t - b;
+}
+template <typename T>
+__device__ inline void dft4(Cx<T> &a, Cx<T> &b, Cx<T> &c, Cx<T> &d) {
+    dft2(a, c);
+    dft2(b, d);
+    d = mul_mi(d);
+    dft2(a, b);
+    dft2(c, d);
+    const Cx<T> t = b;  // bit-reversed order back to natural
+    b = c;
+    c = t;
+}
+
+// odd R: cos and sin of 2 pi k / R, k = 1..(R-1)/2
+template <int R>
+struct Roots;
+template <>
+struct Roots<3> {
+    static constexpr double c[1] = {-0.5}, s[1] = {8.66025403784438646764e-01};
+};
+template <>
+struct Roots<5> {
+    static constexpr double c[2] = {3.09016994374947424102e-01, -8.09016994374947424102e-01},
+                            s[2] = {9.51056516295153572116e-01, 5.87785252292473129169e-01};
+};
+template <int R, typename T>
+__device__ inline void dft(Cx<T> (&v)[R]) {
+    if constexpr (R == 2) {
+        dft2(v[0], v[1]);
+    } else if constexpr (R == 4) {
+        dft4(v[0], v[1], v[2], v[3]);
+    } else if constexpr (R == 8) {
+        constexpr T h = T(0.70710678118654752440);
+        dft4(v[0], v[2], v[4], v[6]);
+        dft4(v[1], v[3], v[5], v[7]);
+        // odd part times exp(-2 pi i k / 8)
+        const Cx<T> o0 = v[1], o1{h * (v[3].x + v[3].y), h * (v[3].y - v[3].x)}, o2 = mul_mi(v[5]),
+                    o3{h * (v[7].y - v[7].x), -h * (v[7].x + v[7].y)};
+        const Cx<T> e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6];
+        v[0] = e0 + o0;
+        v[1] = e1 + o1;
+        v[2] = e2 + o2;
+        v[3] = e3 + o3;
+        v[4] = e0 - o0;
+        v[5] = e1 - o1;
+        v[6] = e2 - o2;
+        v[7] = e3 - o3;
+    } else {
+        constexpr int H = (R - 1) / 2;
+        Cx<T> a[H], b[H], out[R];
+        out[0] = v[0];
+#pragma unroll
+        for (int r = 0; r < H; r++) {
+            a[r] = v[r + 1] + v[R - 1 - r];
+            b[r] = v[r + 1] - v[R - 1 - r];
+            out[0] = out[0] + a[r];
+        }
+#pragma unroll
+        for (int k = 1; k <= H; k++) {
+            Cx<T> p = v[0], m{T(0), T(0)};  // sums with cos and with sin
+#pragma unroll
+            for (int r = 1; r <= H; r++) {
+                const int t = (k * r) % R, u = t <= H ? t : R - t;
+                const T c = T(Roots<R>::c[u - 1]), s = t <= H ? T(Roots<R>::s[u - 1]) : -T(Roots<R>::s[u - 1]);
+                p.x += c * a[r - 1].x;
+                p.y += c * a[r - 1].y;
+                m.x += s * b[r - 1].x;
+                m.y += s * b[r - 1].y;
+            }
+            out[k] = {p.x + m.y, p.y - m.x};      // p - i m
+            out[R - k] = {p.x - m.y, p.y + m.x};  // p + i m
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = out[r];
+    }
+}
+
+// One Stockham stage of radix R after stages of product Ns.  NB: butterflies
+// a thread, ceil(8 / R) since threads >= N / 8.
+template <int R, typename T>
+__device__ inline void stage(T *re, T *im, int N, int Ns, const T *__restrict__ tw) {
+    constexpr int NB = (8 + R - 1) / R;
+    const int nb = N / R, tws = N / (Ns * R);
+    Cx<T> v[NB][R];
+    int dst[NB];
+#pragma unroll
+    for (int t = 0; t < NB; t++) {
+        const int j = threadIdx.x + t * blockDim.x;
+        if (j < nb) {
+            const int q = int(unsigned(j) / unsigned(Ns)), k = j - q * Ns;
+            dst[t] = q * Ns * R + k;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int a = pad(j + r * nb);
+                v[t][r] = {re[a], im[a]};
+            }
+            if (Ns > 1) {
+#pragma unroll
+                for (int r = 1; r < R; r++) {
+                    const int a = 2 * r * k * tws;
+                    v[t][r] = mul(v[t][r], Cx<T>{tw[a], tw[a + 1]});
+                }
+            }
+            dft<R>(v[t]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NB; t++) {
+        if (int(threadIdx.x + t * blockDim.x) < nb) {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int a = pad(dst[t] + r * Ns);
+                re[a] = v[t][r].x;
+                im[a] = v[t][r].y;
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// A stage of any other (prime) radix: every thread forms up to 8 outputs as
+// sums over their R inputs.  O(N R) a row, for columns no one picks for speed.
+template <typename T>
+__device__ inline void stage_any(T *re, T *im, int N, int Ns, int R, const T *tw) {
+    const int nb = N / R, m = N / (Ns * R);
+    T ax[8], ay[8];
+    int b[8], dst[8], step[8], idx[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const int e = threadIdx.x + t * blockDim.x, ee = e < N ? e : 0;
+        const int r = ee / nb;
+        b[t] = ee - r * nb;
+        const int q = b[t] / Ns, k = b[t] - q * Ns;
+        dst[t] = q * Ns * R + k + r * Ns;
+        step[t] = k * m + r * nb;  // < N
+        idx[t] = 0;
+        ax[t] = ay[t] = T(0);
+    }
+    for (int s = 0; s < R; s++) {
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            const int a = pad(b[t] + s * nb);
+            const T vx = re[a], vy = im[a], c = tw[2 * idx[t]], d = tw[2 * idx[t] + 1];
+            ax[t] += vx * c - vy * d;
+            ay[t] += vx * d + vy * c;
+            idx[t] += step[t];
+            if (idx[t] >= N) idx[t] -= N;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 8; t++)
+        if (int(threadIdx.x + t * blockDim.x) < N) {
+            const int a = pad(dst[t]);
+            re[a] = ax[t];
+            im[a] = ay[t];
+        }
+    __syncthreads();
+}
+
+template <typename T>
+__device__ inline void fft(const RowPlan &P, T *re, T *im, const T *__restrict__ tw, T *twl) {
+    const int N = P.N;
+    const T *tws = tw;
+    if (P.tw_lds) {
+        for (int t = threadIdx.x; t < 2 * N; t += blockDim.x) twl[t] = tw[t];
+        tws = twl;
+    }
+    __syncthreads();
+    int Ns = 1;
+    for (int s = 0; s < P.nst; s++) {
+        const int R = P.radix[s];
+        switch (R) {
+            case 8: stage<8>(re, im, N, Ns, tw); break;
+            case 4: stage<4>(re, im, N, Ns, tw); break;
+            case 2: stage<2>(re, im, N, Ns, tw); break;
+            case 3: stage<3>(re, im, N, Ns, tw); break;
+            case 5: stage<5>(re, im, N, Ns, tw); break;
+            default: stage_any(re, im, N, Ns, R, tws); break;
+        }
+        Ns *= R;
+    }
+}
+
+// Hartley values (Re - Im) of the two rows at frequency q, from the complex
+// spectrum Z of row a + i row b: A(q) = (Z(q) + Z*(N-q)) / 2,
+// B(q) = (Z(q) - Z*(N-q)) / 2i.
+template <typename T>
+__device__ inline void hartley_pair(const T *re, const T *im, int N, int q, T &ha, T &hb) {
+    const int a = pad(q), c = pad(q == 0 ? 0 : N - q);
+    const T zr = re[a], zi = im[a], cr = re[c], ci = im[c];
+    ha = T(0.5) * ((zr + cr) - (zi - ci));
+    hb = T(0.5) * ((zi + ci) + (zr - cr));
+}
+
+// Forward: rows j, j+1 of r (RHS false), or cal_w's right-hand side
+// f = -b / rhow, b = rhow^2 (zetap[i+1] - zetap[i]) dx
+// (src/PoissonSolver.cpp:444-450), formed from zetap and stored (RHS true).
+template <typename T, bool RHS>
+__global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restrict__ tw, const double *__restrict__ r,
+                                                   T *__restrict__ spec, Grid G, const double *__restrict__ zetap,
+                                                   const double *__restrict__ rhow, double *__restrict__ f) {
+    extern __shared__ unsigned char lds_raw[];
+    const int N = P.N, M = P.M, LN = pad(N - 1) + 1;
+    T *re = reinterpret_cast<T *>(lds_raw), *im = re + LN, *twl = im + LN;
+    const int j = 1 + 2 * blockIdx.x;
+    const bool two = j + 1 <= M;
+    auto value = [&](int row, int i) -> double {
+        if constexpr (!RHS) return r[size_t(row) * N + i];
+        const int k = row + 1;
+        const double rw = rhow[k];
+        double v;
+        {
+#pragma clang fp contract(off)
+            const double b = rw * rw * (zetap[ix(G, i + 2, k)] - zetap[ix(G, i + 1, k)]) * G.dx;
+            v = -b / rw;
+        }
+        f[size_t(row) * N + i] = v;
+        return v;
+    };
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+        re[pad(i)] = T(value(j, i));
+        im[pad(i)] = two ? T(value(j + 1, i)) : T(0);
+    }
+    fft(P, re, im, tw, twl);
+    for (int q = threadIdx.x; q < N; q += blockDim.x) {
+        T ha, hb;
+        hartley_pair(re, im, N, q, ha, hb);
+        spec[size_t(j - 1) * N + q] = ha;
+        if (two) spec[size_t(j) * N + q] = hb;
+    }
+}
+
+// Inverse: x = the transform of rows j, j+1 of spec (ADD: x0 + it); with w also
+// w[i][k] = x / rhow[k] and BoundaryProcess2D_westdown(w)
+// (src/PoissonSolver.cpp:469-476).
+template <typename T, bool ADD, bool W>
+__global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restrict__ tw, const T *__restrict__ spec,
+                                                   const double *x0, double *x, Grid G, double *__restrict__ w,
+                                                   const double *__restrict__ rhow) {
+    extern __shared__ unsigned char lds_raw[];
+    const int N = P.N, M = P.M, LN = pad(N - 1) + 1;
+    T *re = reinterpret_cast<T *>(lds_raw), *im = re + LN, *twl = im + LN;
+    const int j = 1 + 2 * blockIdx.x;
+    const bool two = j + 1 <= M;
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+        re[pad(i)] = spec[size_t(j - 1) * N + i];
+        im[pad(i)] = two ? spec[size_t(j) * N + i] : T(0);
+    }
+    if constexpr (W) {  // the zero rows of w
+        for (int i = threadIdx.x; i < G.nx; i += blockDim.x) {
+            if (blockIdx.x == 0) w[ix(G, i, 0)] = w[ix(G, i, 1)] = 0.;
+            if (blockIdx.x == gridDim.x - 1) w[ix(G, i, G.nz - 1)] = 0.;
+        }
+    }
+    fft(P, re, im, tw, twl);
+    auto put = [&](int row, int i, T e) {
+        const size_t a = size_t(row) * N + i;
+        const double v = ADD ? x0[a] + double(e) : double(e);
+        x[a] = v;
+        if constexpr (W) store_westdown(w, G, i + 1, row + 1, v / rhow[row + 1]);
+    };
+    for (int q = threadIdx.x; q < N; q += blockDim.x) {
+        T ha, hb;
+        hartley_pair(re, im, N, q, ha, hb);
+        put(j, q, ha);
+        if (two) put(j + 1, q, hb);
+    }
+}
+
+// ------------------------------------------------------ tridiagonal systems
+//
+// Row j (1-based) of frequency q: d_j x_j - cu_j x_{j+1} - cu_{j-1} x_{j-1} =
+// F_j.  Eliminated from both ends towards row mid = (M+1)/2 at once, which
+// halves the serial chain:
+//   downwards (j < mid): g_j = cu_j / p_j, y_{j+1} = F_{j+1} + g_j y_j,
+//   upwards   (j > mid): g_j = cu_{j-1} / p_j, y_{j-1} = F_{j-1} + g_j y_j,
+// x_mid = y_mid / p_mid, and back x_j = y_j / p_j + g_j x_{j+-1}.
+// The factors g and 1 / (N p) (the inverse transform's 1/N folded in) are
+// formed once, for q = 0..N/2 (lambda_q = lambda_{N-q}).
+
+template <typename T>
+__global__ void __launch_bounds__(64) k_factor(int N, int M, const double *__restrict__ cx,
+                                               const double *__restrict__ cu, T *__restrict__ g, T *__restrict__ di) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x, Nq = N / 2 + 1;
+    if (q >= Nq) return;
+    const double s = sinpi(double(q) / N), lam = 4. * s * s;
+    const int mid = (M + 1) / 2;
+    auto diag = [&](int j) { return cx[j] * lam + cu[j] + cu[j - 1]; };
+    double top = 0., bot = 0.;  // what the rows above and below take off p_mid
+    for (int j = 1; j < mid; j++) {
+        const double p = diag(j) - top, gj = cu[j] / p;
+        g[size_t(j - 1) * Nq + q] = T(gj);
+        di[size_t(j - 1) * Nq + q] = T(1. / (p * N));
+        top = cu[j] * gj;
+    }
+    for (int j = M; j > mid; j--) {
+        const double p = diag(j) - bot, gj = cu[j - 1] / p;
+        g[size_t(j - 1) * Nq + q] = T(gj);
+        di[size_t(j - 1) * Nq + q] = T(1. / (p * N));
+        bot = cu[j - 1] * gj;
+    }
+    g[size_t(mid - 1) * Nq + q] = T(0);
+    di[size_t(mid - 1) * Nq + q] = T(1. / ((diag(mid) - top - bot) * N));
+}
+
+// Eight columns a workgroup: every thread moves them and their factors to LDS
+// (all loads in flight at once), then 16 lanes run the eliminations, 8
+// columns x 2 directions, chunk by chunk from registers, and every thread
+// moves the result back.
+constexpr int KC = 8, KCHUNK = 8;
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_columns(int N, int M, T *__restrict__ spec, const T *__restrict__ g,
+                                                 const T *__restrict__ di) {
+    extern __shared__ unsigned char lds_raw[];
+    T *F = reinterpret_cast<T *>(lds_raw), *Gs = F + size_t(M) * KC, *Ds = Gs + size_t(M) * KC;
+    const int q0 = blockIdx.x * KC, Nq = N / 2 + 1;
+    for (int t = threadIdx.x; t < M * KC; t += blockDim.x) {
+        const int j = t / KC, q = q0 + t % KC;
+        if (q < N) {
+            const int qq = min(q, N - q);
+            F[t] = spec[size_t(j) * N + q];
+            Gs[t] = g[size_t(j) * Nq + qq];
+            Ds[t] = di[size_t(j) * Nq + qq];
+        } else {
+            F[t] = Gs[t] = Ds[t] = T(0);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 * KC) {
+        const int c = threadIdx.x % KC, up = threadIdx.x / KC;  // up: from the last row
+        const int mid = (M + 1) / 2 - 1;                        // 0-based here
+        const int cnt = up ? M - 1 - mid : mid, cmax = M - 1 - mid > mid ? M - 1 - mid : mid;
+        const int first = (up ? M - 1 : 0) * KC + c, inc = up ? -KC : KC;
+        T y = T(0), gp = T(0);
+        T nf[KCHUNK], ng[KCHUNK], nd[KCHUNK];
+        auto fetch = [&](int s0) {
+#pragma unroll
+            for (int u = 0; u < KCHUNK; u++) {
+                const int a = first + (s0 + u < cnt ? s0 + u : 0) * inc;
+                nf[u] = F[a];
+                ng[u] = Gs[a];
+                nd[u] = Ds[a];
+            }
+        };
+        fetch(0);
+        for (int s0 = 0; s0 < cmax; s0 += KCHUNK) {
+            T vf[KCHUNK], vg[KCHUNK], vd[KCHUNK];
+#pragma unroll
+            for (int u = 0; u < KCHUNK; u++) {
+                vf[u] = nf[u];
+                vg[u] = ng[u];
+                vd[u] = nd[u];
+            }
+            fetch(s0 + KCHUNK);
+#pragma unroll
+            for (int u = 0; u < KCHUNK; u++) {
+                if (s0 + u < cnt) {
+                    y = vf[u] + gp * y;
+                    gp = vg[u];
+                    F[first + (s0 + u) * inc] = y * vd[u];
+                }
+            }
+        }
+        const T off = cnt > 0 ? gp * y : T(0);
+        const T other = __shfl_xor(off, KC, kWave);
+        // the same order of terms in both directions' lanes
+        T x = (F[mid * KC + c] + (up ? other : off) + (up ? off : other)) * Ds[mid * KC + c];
+        if (!up) F[mid * KC + c] = x;
+        // back: steps cnt-1 .. 0
+        auto fetch_back = [&](int s0) {
+#pragma unroll
+            for (int u = 0; u < KCHUNK; u++) {
+                const int s = cnt - 1 - (s0 + u);
+                const int a = first + (s > 0 ? s : 0) * inc;
+                nf[u] = F[a];
+                ng[u] = Gs[a];
+            }
+        };
+        fetch_back(0);
+        for (int s0 = 0; s0 < cmax; s0 += KCHUNK) {
+            T vf[KCHUNK], vg[KCHUNK];
+#pragma unroll
+            for (int u = 0; u < KCHUNK; u++) {
+                vf[u] = nf[u];
+                vg[u] = ng[u];
+            }
+            fetch_back(s0 + KCHUNK);
+#pragma unroll
+            for (int u = 0; u < KCHUNK; u++) {
+                const int s = cnt - 1 - (s0 + u);
+                if (s >= 0) {
+                    x = vf[u] + vg[u] * x;
+                    F[first + s * inc] = x;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < M * KC; t += blockDim.x) {
+        const int j = t / KC, q = q0 + t % KC;
+        if (q < N) spec[size_t(j) * N + q] = F[t];
+    }
+}
+
+// ---------------------------------------------------------------- residual
+
+constexpr int RX = 64, RY = 4;
+
+__global__ void __launch_bounds__(RX *RY) k_residual_norms(int N, int M, const double *__restrict__ f,
+                                                           const double *__restrict__ x,
+                                                           const double *__restrict__ cx,
+                                                           const double *__restrict__ cu,
+                                                           const double *__restrict__ wD, double *hres) {
+    const int tx = (N + RX - 1) / RX, nt = tx * ((M + RY - 1) / RY);
+    double part[2] = {0., 0.};
+    for (int t = blockIdx.x; t < nt; t += gridDim.x) {
+        const int i = (t % tx) * RX + threadIdx.x, j = 1 + (t / tx) * RY + threadIdx.y;
+        if (i < N && j <= M) {
+            const int im = (i == 0) ? N - 1 : i - 1, ip = (i == N - 1) ? 0 : i + 1;
+            const size_t r = size_t(j) * N;
+            const double c = x[r + i], fv = f[r + i];
+            double Lx;
+            {
+#pragma clang fp contract(off)
+                Lx = cx[j] * (2. * c - x[r + im] - x[r + ip]) + cu[j] * (c - x[r + N + i]) +
+                     cu[j - 1] * (c - x[r - N + i]);
+            }
+            const double wr = wD[j] * (fv - Lx), wb = wD[j] * fv;
+            part[0] += wr * wr;
+            part[1] += wb * wb;
+        }
+    }
+    block_sum<2>(part);
+    if (threadIdx.x == 0 && threadIdx.y == 0) {
+        __hip_atomic_store(hres + 2 * blockIdx.x, part[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(hres + 2 * blockIdx.x + 1, part[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+constexpr size_t kLdsMax = 160 * 1024;
+
+template <typename T>
+T *dalloc(size_t n) {
+    void *p = nullptr;
+    if (hipMalloc(&p, n * sizeof(T)) != hipSuccess) return nullptr;
+    return static_cast<T *>(p);
+}
+
+template <typename K>
+bool allow_lds(K kernel, size_t bytes) {
+    return bytes <= 64 * 1024 || hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     int(bytes)) == hipSuccess;
+}
+
+}  // namespace
+
+int launch_residual_norms(int N, int M, const double *f, const double *x, const double *cx, const double *cu,
+                          const double *wD, double *hres, hipStream_t st) {
+    const int tiles = ((N + RX - 1) / RX) * ((M + RY - 1) / RY);
+    const int nb = tiles < kResidualBlocks ? tiles : kResidualBlocks;
+    hipLaunchKernelGGL(k_residual_norms, dim3(nb), dim3(RX, RY), 0, st, N, M, f, x, cx, cu, wD, hres);
+    return nb;
+}
+
+template <typename T>
+int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
+    plan = RowPlan();
+    plan.N = N;
+    plan.M = M;
+    int n = N;
+    for (int r : {8, 4, 2, 3, 5})
+        while (n % r == 0 && plan.nst < kMaxStages) {
+            plan.radix[plan.nst++] = r;
+            n /= r;
+        }
+    bool other = false;
+    for (int r = 7; n > 1 && plan.nst < kMaxStages; r += 2) {
+        if (r * r > n) r = n;
+        while (n % r == 0 && plan.nst < kMaxStages) {
+            plan.radix[plan.nst++] = r;
+            n /= r;
+            other = true;
+        }
+    }
+    if (n != 1 || N > 8192) return VVM_ERR_SIZE;
+    plan.threads = std::min(1024, std::max(64, ((N + 7) / 8 + 63) / 64 * 64));
+    const size_t LN = size_t(N - 1) + size_t((N - 1) >> 5) + 1;
+    row_lds = 2 * LN * sizeof(T);
+    if (other && row_lds + 2 * size_t(N) * sizeof(T) <= kLdsMax) {
+        plan.tw_lds = 1;
+        row_lds += 2 * size_t(N) * sizeof(T);
+    }
+    col_lds = 3 * size_t(M) * KC * sizeof(T);
+    if (row_lds > kLdsMax || col_lds > kLdsMax) return VVM_ERR_SIZE;
+    if (!allow_lds(k_rows_fwd<T, false>, row_lds) || !allow_lds(k_rows_fwd<T, true>, row_lds) ||
+        !allow_lds(k_rows_inv<T, false, false>, row_lds) || !allow_lds(k_rows_inv<T, true, false>, row_lds) ||
+        !allow_lds(k_rows_inv<T, false, true>, row_lds) || !allow_lds(k_columns<T>, col_lds))
+        return VVM_ERR_HIP;
+    const size_t Nq = size_t(N) / 2 + 1;
+    tw = dalloc<T>(2 * size_t(N));
+    g = dalloc<T>(Nq * M);
+    di = dalloc<T>(Nq * M);
+    spec = dalloc<T>(size_t(N) * M);
+    if (!tw || !g || !di || !spec) {
+        destroy();
+        return VVM_ERR_NOMEM;
+    }
+    std::vector<T> t(2 * size_t(N));
+    for (int k = 0; k < N; k++) {
+        const long double a = 2.0L * 3.14159265358979323846264338327950288L * k / N;
+        t[2 * k] = T(std::cos(a));
+        t[2 * k + 1] = T(-std::sin(a));
+    }
+    if (hipMemcpy(tw, t.data(), t.size() * sizeof(T), hipMemcpyHostToDevice) != hipSuccess) return VVM_ERR_HIP;
+    hipLaunchKernelGGL(k_factor<T>, dim3(unsigned((Nq + 63) / 64)), dim3(64), 0, nullptr, N, M, cx, cu, g, di);
+    return hipStreamSynchronize(nullptr) == hipSuccess ? VVM_OK : VVM_ERR_HIP;
+}
+
+template <typename T>
+void Direct<T>::destroy() {
+    for (T *p : {tw, g, di, spec})
+        if (p) (void)hipFree(p);
+    tw = g = di = spec = nullptr;
+}
+
+template <typename T>
+void Direct<T>::columns(hipStream_t st) {
+    hipLaunchKernelGGL(k_columns<T>, dim3((plan.N + KC - 1) / KC), dim3(256), col_lds, st, plan.N, plan.M, spec, g,
+                       di);
+}
+
+template <typename T>
+void Direct<T>::solve(const double *r, const double *x0, double *x, hipStream_t st) {
+    const dim3 gr((plan.M + 1) / 2), b(plan.threads);
+    hipLaunchKernelGGL((k_rows_fwd<T, false>), gr, b, row_lds, st, plan, tw, r, spec, Grid{}, nullptr, nullptr,
+                       nullptr);
+    columns(st);
+    if (x0)
+        hipLaunchKernelGGL((k_rows_inv<T, true, false>), gr, b, row_lds, st, plan, tw, spec, x0, x, Grid{}, nullptr,
+                           nullptr);
+    else
+        hipLaunchKernelGGL((k_rows_inv<T, false, false>), gr, b, row_lds, st, plan, tw, spec, x0, x, Grid{}, nullptr,
+                           nullptr);
+}
+
+template <typename T>
+void Direct<T>::solve_step(const Grid &G, const double *zetap, const double *rhow, double *f, double *x, double *w,
+                           hipStream_t st) {
+    const dim3 gr((plan.M + 1) / 2), b(plan.threads);
+    hipLaunchKernelGGL((k_rows_fwd<T, true>), gr, b, row_lds, st, plan, tw, nullptr, spec, G, zetap, rhow, f);
+    columns(st);
+    hipLaunchKernelGGL((k_rows_inv<T, false, true>), gr, b, row_lds, st, plan, tw, spec, nullptr, x, G, w, rhow);
+}
+
+template class Direct<double>;
+template class Direct<float>;
+
+}  // namespace vvmd

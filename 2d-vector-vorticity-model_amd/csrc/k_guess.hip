@@ -97,20 +97,24 @@ void Poisson::guess_features(float *dst, hipStream_t st) {
     // rows 2-5 of the reduction slots: row 1 may hold the pending ||b||^2
     // partials of the right-hand side
     const RedSlot rf{red.partial + 2 * size_t(red.max_blocks), red.max_blocks};
-    hipLaunchKernelGGL(k_guess_features, g, dim3(GX, GY), 0, st, N, M, f, xprev, xprev2, xprev3, xe_order(), pcg64.mg.lev[0].cx,
-                       pcg64.mg.lev[0].cu, pcg64.wD, gfeat, rf);
+    hipLaunchKernelGGL(k_guess_features, g, dim3(GX, GY), 0, st, N, M, f, xprev, xprev2, xprev3, xe_order(), cx0,
+                       cu0, pcg64.wD, gfeat, rf);
     finalize<4>(rf, nblocks(g), gsc, RED_STORE, 0, st);
     hipLaunchKernelGGL(k_guess_normalize, dim3(unsigned((3 * plane + 255) / 256)), dim3(256), 0, st, plane,
                        double(plane), gsc, gfeat, dst);
 }
 
-bool Poisson::learned_guess(hipStream_t st) {
+bool Poisson::net_due() {
     if (!net || nsolves < 2) return false;
     if (net_skip > 0) {
         net_skip--;
         guess_skipped++;
         return false;
     }
+    return true;
+}
+
+bool Poisson::learned_guess(hipStream_t st) {
     const size_t plane = size_t(M) * N;
     if (!gfeat) {
         hipMalloc(reinterpret_cast<void **>(&gfeat), sizeof(float) * 3 * plane);
@@ -123,8 +127,8 @@ bool Poisson::learned_guess(hipStream_t st) {
     // rows 2-5 of the reduction slots: row 1 may hold the pending ||b||^2
     // partials of the right-hand side
     const RedSlot rf{red.partial + 2 * size_t(red.max_blocks), red.max_blocks};
-    hipLaunchKernelGGL(k_guess_features, g, dim3(GX, GY), 0, st, N, M, f, xprev, xprev2, xprev3, xe_order(), pcg64.mg.lev[0].cx,
-                       pcg64.mg.lev[0].cu, pcg64.wD, gfeat, rf);
+    hipLaunchKernelGGL(k_guess_features, g, dim3(GX, GY), 0, st, N, M, f, xprev, xprev2, xprev3, xe_order(), cx0,
+                       cu0, pcg64.wD, gfeat, rf);
     // the extrapolated guess's residual norm goes to the host as well: the
     // solve keeps the network's guess only if it starts lower
     finalize<4>(rf, nblocks(g), gsc, RED_STORE, 0, st, -1, hscal_dev + H_GUESS);

@@ -570,14 +570,9 @@ int mg_vcycle(MGHier<T> &H, const T *r, T *&zA, T *&zB, const RedSlot &rs, doubl
 }
 
 template int mg_plan<double>(MGHier<double> &, size_t);
-template int mg_plan<float>(MGHier<float> &, size_t);
 template int mg_vcycle<double>(MGHier<double> &, const double *, double *&, double *&, const RedSlot &, double *,
                                bool, hipStream_t, bool, double *);
-template int mg_vcycle<float>(MGHier<float> &, const float *, float *&, float *&, const RedSlot &, double *, bool,
-                              hipStream_t, bool, float *);
 template bool mg_cg_fusable<double>(const MGHier<double> &, int);
-template bool mg_cg_fusable<float>(const MGHier<float> &, int);
 template int mg_down0_cg<double>(MGHier<double> &, double *, const CGFuse<double> &, int, hipStream_t);
-template int mg_down0_cg<float>(MGHier<float> &, float *, const CGFuse<float> &, int, hipStream_t);
 
 }  // namespace vvmd

@@ -1,7 +1,8 @@
 // k_poisson.hip -- the elliptic part of a VVM timestep on the device:
-// PoissonSolver::cal_w (src/PoissonSolver.cpp:439-477) as multigrid-
-// preconditioned CG in FP64, or FP32 MG-PCG inside FP64 iterative
-// refinement, and PoissonSolver::cal_u (src/PoissonSolver.cpp:580-653).
+// PoissonSolver::cal_w (src/PoissonSolver.cpp:439-477) by the direct solver
+// (k_direct.hip) with FP64 iterative refinement, or as multigrid-
+// preconditioned CG in FP64, and PoissonSolver::cal_u
+// (src/PoissonSolver.cpp:580-653).
 //
 // Multigrid: geometric, vertex coarsening (N -> N/2 periodic columns,
 // M -> (M-1)/2 Dirichlet rows), operators rediscretised with harmonic-mean
@@ -98,28 +99,22 @@ __global__ void __launch_bounds__(LX *LY) k_pcg_update(int N, int M, T *x, T *r,
     block_partials<1>(part, rs);
 }
 
-// The solve's first residual with the guess or the refinement correction
-// folded in.  XF_EXTRAP: x = the extrapolation of order ord (2 x1 - x2, or
-// 3 (x1 - x2) + x3), XF_ZERO:
-// x = 0, XF_CORR: x = xin + e32 (the FP32 correction; written to another
-// buffer, since neighbouring workgroups read xin), XF_NONE: x as it is.
-// Every value of x the stencil needs is formed on the fly with the same
-// arithmetic the separate kernels used, so r and x are bit for bit what they
-// gave.  With r32 the FP32 right-hand side of the next correction (r as
-// float, x32 = 0) is written too.
-enum { XF_NONE = 0, XF_EXTRAP, XF_ZERO, XF_CORR };
+// The solve's first residual with the guess folded in.  XF_EXTRAP: x = the
+// extrapolation of order ord (2 x1 - x2, or 3 (x1 - x2) + x3), XF_ZERO:
+// x = 0, XF_NONE: x as it is.  Every value of x the stencil needs is formed
+// on the fly with the same arithmetic the separate kernels used, so r and x
+// are bit for bit what they gave.
+enum { XF_NONE = 0, XF_EXTRAP, XF_ZERO };
 template <int XF>
-__global__ void __launch_bounds__(LX *LY) k_residual_x(int N, int M, const double *f, const double *xin,
-                                                       double *xout, const double *x1, const double *x2,
-                                                       const double *x3, int ord, const float *e32, double *r, const double *cx,
-                                                       const double *cu, const double *wD, RedSlot rs, float *r32,
-                                                       float *x32) {
+__global__ void __launch_bounds__(LX *LY) k_residual_x(int N, int M, const double *f, double *x, const double *x1,
+                                                       const double *x2, const double *x3, int ord, double *r,
+                                                       const double *cx, const double *cu, const double *wD,
+                                                       RedSlot rs) {
     const int i = blockIdx.x * LX + threadIdx.x, j = 1 + blockIdx.y * LY + threadIdx.y;
     auto xv = [&](size_t a) -> double {
         if (XF == XF_EXTRAP) return extrap_at(x1, x2, x3, ord, a);
         if (XF == XF_ZERO) return 0.;
-        if (XF == XF_CORR) return xin[a] + double(e32[a]);
-        return xin[a];
+        return x[a];
     };
     double part[1] = {0.};
     if (i < N && j <= M) {
@@ -132,15 +127,9 @@ __global__ void __launch_bounds__(LX *LY) k_residual_x(int N, int M, const doubl
         const double rv = f[c] - Lx;
         r[c] = rv;
         if (XF != XF_NONE) {
-            xout[c] = xc;
-            // the boundary rows: XF_EXTRAP and XF_ZERO form them as the
-            // separate kernels did, XF_CORR carries them over
-            if (j == 1) xout[i] = (XF == XF_CORR) ? xin[i] : xv(i);
-            if (j == M) xout[rw + N + i] = (XF == XF_CORR) ? xin[rw + N + i] : xv(rw + N + i);
-        }
-        if (r32) {
-            r32[c] = float(rv);
-            x32[c] = 0.f;
+            x[c] = xc;
+            if (j == 1) x[i] = xv(i);
+            if (j == M) x[rw + N + i] = xv(rw + N + i);
         }
         const double wr = wD[j] * rv;
         part[0] = wr * wr;
@@ -355,13 +344,6 @@ __global__ void __launch_bounds__(UW *UC) k_calu_cols(Grid G, StepPtrs S) {
     }
 }
 
-// LDS budget of the one-workgroup coarse kernel for an FP64-sized budget:
-// the FP32 hierarchy takes the levels the FP64 one takes.
-template <typename T>
-size_t coarse_budget(size_t fp64_bytes) {
-    return fp64_bytes * sizeof(T) / sizeof(double);
-}
-
 template <typename T>
 T *dalloc(size_t n) {
     void *p = nullptr;
@@ -465,11 +447,9 @@ bool build_hier(MGHier<T> &H, int N, int M, const std::vector<double> &cx0, cons
             }
         }
     }
-    // the one-workgroup kernel takes every level that fits in 64 KiB of LDS
-    // in FP64 (the same levels in FP32: one more level there, 4x the
-    // points, made the one-CU kernel 50% slower than the tiled launch it
-    // saves); the finest levels run as tiled down/up kernels
-    return mg_plan(H, coarse_budget<T>(size_t(64) * 1024)) == 0;
+    // the one-workgroup kernel takes every level that fits in 64 KiB of LDS;
+    // the finest levels run as tiled down/up kernels
+    return mg_plan(H, size_t(64) * 1024) == 0;
 }
 
 template <typename T>
@@ -602,63 +582,41 @@ int pcg_loop(PCG<T> &P, double target, int max_iter, bool stall_stop, const RedS
 
 }  // namespace
 
-int Poisson::init(const Grid &G, const double *rhou, const double *rhow, const RedSlot &rs, bool with_fp32) {
+int Poisson::init(const Grid &G, const double *rhou, const double *rhow, const RedSlot &rs, bool with_direct,
+                  bool with_fp32, bool with_pcg) {
     N = G.nx - 2;
     M = G.nz - 3;
     red = rs;
+    have_pcg = with_pcg;
     std::vector<double> cx(M + 2, 0.), cu(M + 1, 0.);
     for (int j = 1; j <= M; j++) cx[j] = 1. / rhow[j + 1];
     for (int j = 0; j <= M; j++) cu[j] = 1. / rhou[j + 1];
     const size_t n = size_t(M + 2) * N;
     std::vector<double> wd(M + 2, 0.);
     for (int j = 1; j <= M; j++) wd[j] = rhow[j + 1];
-    {
-        PCG<double> &P = pcg64;
-        P.N = N;
-        P.M = M;
+    cx0 = dalloc<double>(M + 2);
+    cu0 = dalloc<double>(M + 1);
+    if (!cx0 || !cu0) return VVM_ERR_NOMEM;
+    hipMemcpy(cx0, cx.data(), sizeof(double) * (M + 2), hipMemcpyHostToDevice);
+    hipMemcpy(cu0, cu.data(), sizeof(double) * (M + 1), hipMemcpyHostToDevice);
+    PCG<double> &P = pcg64;
+    P.N = N;
+    P.M = M;
+    P.x = dalloc<double>(n);
+    P.r = dalloc<double>(n);
+    P.wD = dalloc<double>(M + 2);
+    P.sc = dalloc<double>(NPSCAL);
+    if (!P.x || !P.r || !P.wD || !P.sc) return VVM_ERR_NOMEM;
+    hipMemcpy(P.wD, wd.data(), sizeof(double) * (M + 2), hipMemcpyHostToDevice);
+    if (with_pcg) {
         if (!build_hier(P.mg, N, M, cx, cu)) return VVM_ERR_NOMEM;
-        P.x = dalloc<double>(n);
-        P.r = dalloc<double>(n);
-        P.rB = dalloc<double>(n);
-        P.zA = dalloc<double>(n);
-        P.zB = dalloc<double>(n);
-        P.pA = dalloc<double>(n);
-        P.pB = dalloc<double>(n);
-        P.q = dalloc<double>(n);
-        P.qB = dalloc<double>(n);
-        P.w = dalloc<double>(n);
-        P.wD = dalloc<double>(M + 2);
-        P.sc = dalloc<double>(NPSCAL);
-        if (!P.x || !P.r || !P.rB || !P.zA || !P.zB || !P.pA || !P.pB || !P.q || !P.qB || !P.w || !P.wD || !P.sc)
-            return VVM_ERR_NOMEM;
-        hipMemcpy(P.wD, wd.data(), sizeof(double) * (M + 2), hipMemcpyHostToDevice);
+        for (double **v : {&P.rB, &P.zA, &P.zB, &P.pA, &P.pB, &P.q, &P.qB, &P.w})
+            if (!(*v = dalloc<double>(n))) return VVM_ERR_NOMEM;
     }
-    have32 = with_fp32;
-    if (with_fp32) {
-        PCG<float> &P = pcg32;
-        P.N = N;
-        P.M = M;
-        if (!build_hier(P.mg, N, M, cx, cu)) return VVM_ERR_NOMEM;
-        P.x = dalloc<float>(n);
-        P.r = dalloc<float>(n);
-        P.rB = dalloc<float>(n);
-        P.zA = dalloc<float>(n);
-        P.zB = dalloc<float>(n);
-        P.pA = dalloc<float>(n);
-        P.pB = dalloc<float>(n);
-        P.q = dalloc<float>(n);
-        P.qB = dalloc<float>(n);
-        P.w = dalloc<float>(n);
-        P.wD = dalloc<float>(M + 2);
-        P.sc = dalloc<double>(NPSCAL);
-        if (!P.x || !P.r || !P.rB || !P.zA || !P.zB || !P.pA || !P.pB || !P.q || !P.qB || !P.w || !P.wD || !P.sc)
-            return VVM_ERR_NOMEM;
-        std::vector<float> wf(wd.begin(), wd.end());
-        hipMemcpy(P.wD, wf.data(), sizeof(float) * (M + 2), hipMemcpyHostToDevice);
-        r64 = dalloc<double>(n);
-        x32B = dalloc<float>(n);
-        if (!r64 || !x32B) return VVM_ERR_NOMEM;
-    }
+    if (with_direct)
+        if (const int rc = direct64.init(N, M, cx0, cu0)) return rc;
+    if (with_fp32)
+        if (const int rc = direct32.init(N, M, cx0, cu0)) return rc;
     f = dalloc<double>(n);
     xprev = dalloc<double>(n);
     xprev2 = dalloc<double>(n);
@@ -671,6 +629,10 @@ int Poisson::init(const Grid &G, const double *rhou, const double *rhow, const R
                       hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
         return VVM_ERR_NOMEM;
     if (hipHostGetDevicePointer(reinterpret_cast<void **>(&hscal_dev), hscal, 0) != hipSuccess) return VVM_ERR_HIP;
+    if (hipHostMalloc(reinterpret_cast<void **>(&hres), 2 * kResidualBlocks * sizeof(double),
+                      hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+        return VVM_ERR_NOMEM;
+    if (hipHostGetDevicePointer(reinterpret_cast<void **>(&hres_dev), hres, 0) != hipSuccess) return VVM_ERR_HIP;
     // per-workgroup residual norms of the fused CG update, read by the host
     if (hipHostMalloc(reinterpret_cast<void **>(&hpart), sizeof(double) * size_t(rs.max_blocks),
                       hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
@@ -692,16 +654,18 @@ static void free_pcg(PCG<T> &P) {
 
 void Poisson::destroy() {
     free_pcg(pcg64);
-    if (have32) free_pcg(pcg32);
-    for (void *p : {(void *)f, (void *)xprev, (void *)xprev2, (void *)xprev3, (void *)x64B, (void *)x32B, (void *)bcg, (void *)bsc,
-                    (void *)r64, (void *)gfeat,
-                    (void *)gsc, (void *)samples})
+    have_pcg = false;
+    direct64.destroy();
+    direct32.destroy();
+    for (void *p : {(void *)f, (void *)xprev, (void *)xprev2, (void *)xprev3, (void *)x64B, (void *)bcg, (void *)bsc,
+                    (void *)cx0, (void *)cu0, (void *)gfeat, (void *)gsc, (void *)samples})
         if (p) hipFree(p);
-    f = xprev = xprev2 = xprev3 = r64 = x64B = bcg = bsc = nullptr;
-    gfeat = samples = x32B = nullptr;
+    f = xprev = xprev2 = xprev3 = x64B = bcg = bsc = cx0 = cu0 = nullptr;
+    gfeat = samples = nullptr;
     bn_pending = 0;
     x_pending = 0;
-    corr_pending = false;
+    if (hres) hipHostFree(hres);
+    hres = hres_dev = nullptr;
     gsc = nullptr;
     gscratch.release();
     sample_cap = sample_count = 0;
@@ -719,8 +683,7 @@ void Poisson::destroy() {
 
 int Poisson::replan(size_t budget) {
     if (budget > size_t(64) * 1024) return VVM_ERR_ARG;
-    if (mg_plan(pcg64.mg, coarse_budget<double>(budget)) != 0) return VVM_ERR_NOMEM;
-    if (have32 && mg_plan(pcg32.mg, coarse_budget<float>(budget)) != 0) return VVM_ERR_NOMEM;
+    if (have_pcg && mg_plan(pcg64.mg, budget) != 0) return VVM_ERR_NOMEM;
     lds_budget = budget;
     return VVM_OK;
 }
@@ -755,31 +718,19 @@ void Poisson::flush_pending(hipStream_t st) {
     x_pending = XF_NONE;
 }
 
-void Poisson::first_residual(double *r, bool fp32_rhs, hipStream_t st) {
+void Poisson::first_residual(double *r, hipStream_t st) {
     const dim3 g = lgrid(N, M), b(LX, LY);
     PCG<double> &D = pcg64;
-    const float *e32 = have32 ? pcg32.x : nullptr;
-    const int xf = corr_pending ? int(XF_CORR) : x_pending;
-    double *xo = (xf == XF_CORR) ? x64B : D.x;
-    // the FP32 copy of r, and the FP32 x zeroed for the next correction; the
-    // correction being applied is read from pcg32.x, so the zeros then go to
-    // the other FP32 buffer
-    float *r32 = fp32_rhs ? pcg32.r : nullptr;
-    float *x32 = fp32_rhs ? ((xf == XF_CORR) ? x32B : pcg32.x) : nullptr;
-#define VVM_RESIDUAL_X(XF)                                                                                        \
-    hipLaunchKernelGGL((k_residual_x<XF>), g, b, 0, st, N, M, f, D.x, xo, xprev, xprev2, xprev3, x_pending_ord, e32, r, D.mg.lev[0].cx, \
-                       D.mg.lev[0].cu, D.wD, red, r32, x32)
-    switch (xf) {
+#define VVM_RESIDUAL_X(XF)                                                                                         \
+    hipLaunchKernelGGL((k_residual_x<XF>), g, b, 0, st, N, M, f, D.x, xprev, xprev2, xprev3, x_pending_ord, r, cx0, \
+                       cu0, D.wD, red)
+    switch (x_pending) {
         case XF_EXTRAP: VVM_RESIDUAL_X(XF_EXTRAP); break;
         case XF_ZERO: VVM_RESIDUAL_X(XF_ZERO); break;
-        case XF_CORR: VVM_RESIDUAL_X(XF_CORR); break;
         default: VVM_RESIDUAL_X(XF_NONE); break;
     }
 #undef VVM_RESIDUAL_X
-    if (xf == XF_CORR) std::swap(D.x, x64B);
-    if (fp32_rhs && xf == XF_CORR) std::swap(pcg32.x, x32B);
     x_pending = XF_NONE;
-    corr_pending = false;
     // the norms land in mapped host memory (hscal) directly: no copy in the stream
     if (bn_pending) {
         // rows 0 (r) and 1 (b), same grid: sc[P_RNORM2], sc[P_BNORM2]
@@ -833,30 +784,32 @@ void Poisson::remember_solution(hipStream_t st) {
     nsolves++;
 }
 
-template <typename T>
-void Poisson::start_solve(double *r, bool fp32_rhs, PCG<T> *pre_vcycle, int *n_rz_pre, double *bn2, double *rn2,
-                          hipStream_t st) {
+// Whether the solve keeps the network's guess, whose residual is rn2.
+bool Poisson::keep_guess(double rn2) {
+    if (std::isfinite(rn2) && rn2 <= hscal[H_GUESS + 3]) {
+        net_backoff = 0;
+        return true;
+    }
+    net_backoff = std::min(std::max(1, 4 * net_backoff), kMaxNetSkip);
+    net_skip = net_backoff;
+    guess_fallbacks++;
+    return false;
+}
+
+void Poisson::start_solve(double *r, int *n_rz_pre, double *bn2, double *rn2, hipStream_t st) {
     const bool judge = guess_from_net;
     guess_from_net = false;
     for (int attempt = 0;; attempt++) {
-        first_residual(r, fp32_rhs, st);
+        first_residual(r, st);
         hipEventRecord(ev_res, st);
-        if (pre_vcycle) *n_rz_pre = pcg_first_vcycle(*pre_vcycle, red, hpart_dev, st);
+        *n_rz_pre = pcg_first_vcycle(pcg64, red, hpart_dev, st);
         hipEventSynchronize(ev_res);
         *bn2 = hscal[P_BNORM2];
         *rn2 = hscal[P_RNORM2];
-        if (!judge || attempt > 0) return;
-        const double rn2_xe = hscal[H_GUESS + 3];
-        if (std::isfinite(*rn2) && *rn2 <= rn2_xe) {
-            net_backoff = 0;
-            return;
-        }
-        net_backoff = std::min(std::max(1, 4 * net_backoff), kMaxNetSkip);
-        net_skip = net_backoff;
+        if (!judge || attempt > 0 || keep_guess(*rn2)) return;
         // the network's guess starts worse than the extrapolation it corrects
         // (or is not finite): start from the extrapolation instead; the first
         // V-cycle queued on the rejected residual is simply overwritten
-        guess_fallbacks++;
         x_pending = XF_EXTRAP;
         x_pending_ord = xe_order();
     }
@@ -869,7 +822,7 @@ SolveResult Poisson::solve_fp64(double tol, int max_iter, hipStream_t st) {
     // that already meets the stop rule wastes it, which is rare)
     int n_rz_pre = 0;
     double bn2 = 0., rn2 = 0.;
-    start_solve(P.r, false, &P, &n_rz_pre, &bn2, &rn2, st);
+    start_solve(P.r, &n_rz_pre, &bn2, &rn2, st);
     if (!std::isfinite(bn2) || !std::isfinite(rn2)) {  // a non-finite right-hand side or guess
         R.rel0 = R.rel = std::sqrt(rn2 / bn2);
         return R;
@@ -880,7 +833,6 @@ SolveResult Poisson::solve_fp64(double tol, int max_iter, hipStream_t st) {
         return R;
     }
     R.rel0 = std::sqrt(rn2 / bn2);
-    (void)P;
     const bool parity = (tol <= 0.);
     const double target = parity ? 1e-30 * bn2 : tol * tol * bn2;
     if (!(rn2 > target)) {
@@ -897,59 +849,103 @@ SolveResult Poisson::solve_fp64(double tol, int max_iter, hipStream_t st) {
     return R;
 }
 
-// smallest relative residual reduction asked of one FP32 inner solve
-constexpr double kInnerFloor = 1e-6;
+// Relative residual below which one that no longer decreases counts as FP64's
+// round-off.  A direct solve leaves 1e-16 to 1e-14 on the model's right-hand
+// sides; the bound is the condition number's worth above that.
+constexpr double kRoundOff = 1e-12;
 
-SolveResult Poisson::solve_mixed(double tol, int max_outer, int max_inner, double inner_tol, hipStream_t st) {
+// Each sweep: the FP64 residual, then x += L^-1 r by a direct solve, formed in
+// another buffer so that the first one can be queued before the host has read
+// the residual of the guess (which may already meet the stop rule).
+template <typename T>
+SolveResult Poisson::refine(Direct<T> &D, double tol, bool to_floor, int max_sweeps, hipStream_t st) {
     SolveResult R;
-    if (!have32) return solve_fp64(tol, max_inner * max_outer, st);
-    PCG<double> &D = pcg64;
-    PCG<float> &F = pcg32;
-    double bn2 = -1.;
-    for (int outer = 0; outer <= max_outer; outer++) {
-        // r64, and its FP32 copy for the correction solve (unused if converged);
-        // on the first sweep the inner solve's first V-cycle goes in before
-        // the host reads the residual (the guess almost never meets the stop
-        // rule); on later sweeps the residual is usually the final check
-        int n_rz_pre = -1;
-        double rn2 = 0.;
-        start_solve(r64, true, outer == 0 ? &F : static_cast<PCG<float> *>(nullptr), &n_rz_pre, &bn2, &rn2, st);
-        if (!std::isfinite(bn2) || !std::isfinite(rn2)) {  // a non-finite right-hand side, guess or correction
-            R.rel = std::sqrt(rn2 / bn2);
-            if (outer == 0) R.rel0 = R.rel;
-            return R;
-        }
-        if (bn2 == 0.) {
-            hipMemsetAsync(D.x, 0, size_t(M + 2) * N * sizeof(double), st);
+    double prev = -1.;
+    for (int sweep = 0;; sweep++) {
+        first_residual(pcg64.r, st);
+        hipEventRecord(ev_res, st);
+        if (sweep == 0) D.solve(pcg64.r, pcg64.x, x64B, st);
+        hipEventSynchronize(ev_res);
+        const double bn2 = hscal[P_BNORM2], rn2 = hscal[P_RNORM2];
+        const bool finite = std::isfinite(bn2) && std::isfinite(rn2);  // else: a bad right-hand side or guess
+        if (finite && bn2 == 0.) {
+            hipMemsetAsync(pcg64.x, 0, size_t(M + 2) * N * sizeof(double), st);
             R.converged = true;
             return R;
         }
-        const double rel = std::sqrt(rn2 / bn2);
-        if (outer == 0) R.rel0 = rel;
-        R.rel = rel;
-        if (rel <= tol) {
-            R.converged = true;
-            return R;
-        }
-        if (outer == max_outer) break;
-        R.refine++;
-        // The inner solve reduces its residual just enough to meet tol (with
-        // a margin for the FP64 residual after the correction), by no more
-        // than FP32 resolves and by at least inner_tol: one refinement when
-        // the guess is good, instead of a fixed 1e-4 per refinement that
-        // overshoots the target.  Its starting norm is the FP64 residual's
-        // (the FP32 copy differs in the 8th digit), so no read-back is needed.
-        const double need = 0.3 * tol / rel;
-        const double itol = std::min(inner_tol, std::max(need, kInnerFloor));
-        const double r0 = rn2;
-        double last = r0;
-        bool conv = false;
-        R.iters += pcg_loop(F, itol * itol * r0, max_inner, false, red, hscal + 8, hscal_dev + 8, hpart, hpart_dev, ev, st, r0, &last,
-                            &conv, n_rz_pre);
-        corr_pending = true;  // x += e, in the next sweep's residual kernel
+        R.rel = std::sqrt(rn2 / bn2);
+        if (sweep == 0) R.rel0 = R.rel;
+        R.iters = R.refine = sweep;
+        if (!finite) return R;
+        const bool stalled = prev >= 0. && R.rel > 0.5 * prev;
+        R.converged = R.rel <= tol || (to_floor && stalled && R.rel <= kRoundOff);
+        if (R.converged || stalled || sweep == max_sweeps) return R;
+        prev = R.rel;
+        if (sweep > 0) D.solve(pcg64.r, pcg64.x, x64B, st);
+        std::swap(pcg64.x, x64B);
     }
-    (void)D;
+}
+
+SolveResult Poisson::solve_direct(double tol, bool to_floor, int max_sweeps, hipStream_t st) {
+    SolveResult R = refine(direct64, tol, to_floor, max_sweeps, st);
+    R.refine = 0;
     return R;
+}
+
+SolveResult Poisson::solve_mixed(double tol, int max_sweeps, hipStream_t st) {
+    return refine(direct32, tol, false, max_sweeps, st);
+}
+
+void Poisson::queue_step(const Grid &G, const double *zetap, const double *rhow_dev, double *w, bool f_ready,
+                         hipStream_t st) {
+    x_pending = XF_NONE;
+    if (guess_from_net) {
+        guess_from_net = false;
+        first_residual(pcg64.r, st);
+        hipEventRecord(ev_res, st);
+        hipEventSynchronize(ev_res);
+        if (keep_guess(hscal[P_RNORM2])) {
+            direct64.solve(pcg64.r, pcg64.x, x64B, st);
+            std::swap(pcg64.x, x64B);
+        } else {
+            direct64.solve(f, nullptr, pcg64.x, st);
+        }
+        back_to_w(G, w, rhow_dev, st);
+    } else if (f_ready) {
+        direct64.solve(f, nullptr, pcg64.x, st);
+        back_to_w(G, w, rhow_dev, st);
+    } else {
+        direct64.solve_step(G, zetap, rhow_dev, f, pcg64.x, w, st);
+    }
+    bn_pending = 0;
+    res_blocks = launch_residual_norms(N, M, f, pcg64.x, cx0, cu0, pcg64.wD, hres_dev, st);
+    hipEventRecord(ev_res, st);
+}
+
+SolveResult Poisson::finish_step(const Grid &G, double *w, const double *rhow_dev, double tol, bool to_floor,
+                                 int max_sweeps, bool *redo, hipStream_t st) {
+    SolveResult R;
+    *redo = false;
+    hipEventSynchronize(ev_res);
+    double rn2 = 0., bn2 = 0.;
+    const volatile double *p = hres;
+    for (int b = 0; b < res_blocks; b++) {  // fixed order: deterministic
+        rn2 += p[2 * b];
+        bn2 += p[2 * b + 1];
+    }
+    R.iters = 1;
+    R.rel0 = 1.;
+    R.rel = bn2 > 0. ? std::sqrt(rn2 / bn2) : std::sqrt(rn2);
+    R.converged = std::isfinite(bn2) && R.rel <= tol;
+    if (R.converged || !std::isfinite(R.rel) || max_sweeps <= 1) return R;
+    // beyond what one solve gives: corrected further
+    hscal[P_BNORM2] = bn2;
+    SolveResult C = refine(direct64, tol, to_floor, max_sweeps - 1, st);
+    C.iters++;
+    C.rel0 = 1.;
+    back_to_w(G, w, rhow_dev, st);
+    *redo = true;
+    return C;
 }
 
 // ---------------------------------------------------------------- cal_u

@@ -10,8 +10,15 @@
 //
 // Unknown arrays are (M+2) rows x N columns, x-contiguous, rows 0 and M+1
 // held at zero (the Dirichlet rows); N = nx-2, M = nz-3.
+//
+// Three solvers.  The direct one (direct.h) needs no guess and is what a step
+// and an isolated solve take.  MG-PCG runs where the FP64 solver is asked to
+// start from a guess (guess_mode other than zero): there the iteration count,
+// which tells one guess from another, is part of what the caller asked for.
+// BiCGSTAB is a comparison mode.
 #pragma once
 
+#include "direct.h"
 #include "mg.h"
 #include "net.h"
 
@@ -41,7 +48,10 @@ struct SolveResult {
 class Poisson {
    public:
     // rhou/rhow are the host profiles (nz long).  Allocates with hipMalloc.
-    int init(const Grid &G, const double *rhou, const double *rhow, const RedSlot &rs, bool with_fp32);
+    // with_direct: the FP64 direct solver (and with_fp32 its FP32 form, for
+    // solve_mixed); with_pcg: the multigrid hierarchy and the CG vectors.
+    int init(const Grid &G, const double *rhou, const double *rhow, const RedSlot &rs, bool with_direct,
+             bool with_fp32, bool with_pcg);
     void destroy();
 
     // cal_w right-hand side: f from zetap, and ||b||^2.
@@ -68,10 +78,25 @@ class Poisson {
     // order of the extrapolation the learned guess corrects and the
     // recorded samples use: quadratic once three solutions exist
     int xe_order() const { return nsolves >= 3 ? 2 : 1; }
-    // Plain FP64 MG-PCG.  tol: relative true residual ||b-Ax||/||b||.
+    // FP64 MG-PCG.  tol: relative true residual ||b-Ax||/||b||; 0: until the
+    // residual no longer decreases.
     SolveResult solve_fp64(double tol, int max_iter, hipStream_t st);
-    // FP32 MG-PCG inside FP64 iterative refinement.
-    SolveResult solve_mixed(double tol, int max_outer, int max_inner, double inner_tol, hipStream_t st);
+    // x as the guess, corrected by direct solves of the FP64 residual's system
+    // until ||b-Ax||/||b|| <= tol: by FP64 ones (solve_direct) or FP32 ones
+    // (solve_mixed).  to_floor: also done when the residual has stopped
+    // decreasing at FP64's round-off (kRoundOff).
+    SolveResult solve_direct(double tol, bool to_floor, int max_sweeps, hipStream_t st);
+    SolveResult solve_mixed(double tol, int max_sweeps, hipStream_t st);
+    // The step's cal_w in two halves.  queue_step: right-hand side (formed
+    // already if f_ready), solve, w and the residual's norms, nothing waited
+    // for; the network's guess (if learned_guess wrote one) is judged here,
+    // which does wait.  finish_step: waits for the norms and, if they miss the
+    // stop rule, corrects x further; *redo says that x and w have changed
+    // since queue_step, so what was queued behind it has to run again.
+    void queue_step(const Grid &G, const double *zetap, const double *rhow_dev, double *w, bool f_ready,
+                    hipStream_t st);
+    SolveResult finish_step(const Grid &G, double *w, const double *rhow_dev, double tol, bool to_floor,
+                            int max_sweeps, bool *redo, hipStream_t st);
     // The reference GPU back-end's solver (k_bicgstab.hip): BiCGSTAB with a
     // red-black ILU0 preconditioner; stops at ||b - A x||_2 <= tol
     // (absolute) or <= tol ||b||_2.  Needs an even column count.
@@ -89,13 +114,15 @@ class Poisson {
 
     // Learned initial guess (k_guess.hip).  With a network attached and two
     // previous solutions, x = xe + s_d * net(features), xe the extrapolation
-    // of order xe_order(); returns false (nothing written) otherwise.
+    // of order xe_order(); false (nothing written) if it failed to run.
     GuessNet *net = nullptr;
+    // net_due: whether this solve runs it (and counts the solves it sits out)
+    bool net_due();
     bool learned_guess(hipStream_t st);
     // The network's guess was written for the next solve.  That solve keeps
     // it only if its initial residual is finite and below the extrapolated
-    // guess's (which the feature pass measured); otherwise it restarts from
-    // the extrapolation, so a poor or broken network never costs iterations
+    // guess's (which the feature pass measured); otherwise it starts as it
+    // would without the network, so a poor or broken network never costs iterations
     // or accuracy.  guess_fallbacks counts the restarts.
     bool guess_from_net = false;
     int guess_fallbacks = 0;
@@ -116,16 +143,20 @@ class Poisson {
     int sample_ord = 1;                     // extrapolation order of the open sample
 
    private:
-    void vcycle64(hipStream_t st, bool first_done, double **zcur);
-    SolveResult pcg_run64(double tol, int max_iter, hipStream_t st);
-    PCG<double> pcg64;
-    PCG<float> pcg32;
-    bool have32 = false;
+    PCG<double> pcg64;  // x and r for every solver; the rest for MG-PCG only
+    bool have_pcg = false;
+    Direct<double> direct64;
+    Direct<float> direct32;
+    double *cx0 = nullptr, *cu0 = nullptr;  // coefficients of L
+    double *hres = nullptr, *hres_dev = nullptr;  // launch_residual_norms (mapped host memory)
+    int res_blocks = 0;
+    template <typename T>
+    SolveResult refine(Direct<T> &D, double tol, bool to_floor, int max_sweeps, hipStream_t st);
+    bool keep_guess(double rn2);
     double *f = nullptr;       // rhs of L x = f, (M+2)*N
     double *xprev = nullptr;   // previous solution (for extrapolation)
     double *xprev2 = nullptr;
     double *xprev3 = nullptr;
-    double *r64 = nullptr;     // FP64 residual of the refinement loop
     // pinned host copy of scalars: [P_RNORM2], [P_BNORM2] of the first
     // residual, [8..] the CG loop's, [H_GUESS..H_GUESS+3] the feature pass's
     // sums (H_GUESS + 3: ||wD r||^2 of the extrapolated guess)
@@ -142,29 +173,23 @@ class Poisson {
     hipEvent_t ev_res = nullptr;  // after the first residual: the host waits on it, not on the whole stream
     // Work folded into the next solve's first residual kernel (one launch
     // instead of two each): the ||b||^2 partials the right-hand-side kernel
-    // left in row 1 of red (their block count, 0 for none), the guess
-    // (GuessMode below) and, between refinement sweeps, the FP32
-    // correction.  flush_pending runs the first two on their own, for
-    // callers that use red or x before the solve.
+    // left in row 1 of red (their block count, 0 for none) and the guess
+    // (GuessMode below).  flush_pending runs them on their own, for callers
+    // that use red or x before the solve.
     int bn_pending = 0;
     int x_pending = 0;
     int x_pending_ord = 1;   // extrapolation order of a pending XF_EXTRAP guess
-    bool corr_pending = false;
-    double *x64B = nullptr;  // the other FP64 solution buffer (the correction writes it)
+    double *x64B = nullptr;  // the other solution buffer (a refinement sweep writes it)
     double *bcg = nullptr, *bsc = nullptr;  // BiCGSTAB vectors and scalars (allocated on first use)
-    float *x32B = nullptr;   // the other FP32 solution buffer (zeroed while the correction reads x)
     void flush_pending(hipStream_t st);
-    // r = f - L x (x with the pending guess or correction applied, and
-    // written), ||w r||^2 (and ||b||^2 if pending) into sc and hscal; with
-    // fp32_rhs also the FP32 copy of r and a zero FP32 x.
-    void first_residual(double *r, bool fp32_rhs, hipStream_t st);
-    // The first residual of a solve, with its first V-cycle queued before the
-    // host reads the norms (pre_vcycle: that V-cycle's partial count into
-    // *n_rz_pre), and the learned guess judged against the extrapolation.
-    // Returns ||b||^2 and ||w r||^2 as the host read them.
-    template <typename T>
-    void start_solve(double *r, bool fp32_rhs, PCG<T> *pre_vcycle, int *n_rz_pre, double *bn2, double *rn2,
-                     hipStream_t st);
+    // r = f - L x (x with the pending guess applied, and written), ||w r||^2
+    // (and ||b||^2 if pending) into sc and hscal.
+    void first_residual(double *r, hipStream_t st);
+    // The first residual of a PCG solve, with its first V-cycle queued before
+    // the host reads the norms (its partial count into *n_rz_pre), and the
+    // learned guess judged against the extrapolation.  Returns ||b||^2 and
+    // ||w r||^2 as the host read them.
+    void start_solve(double *r, int *n_rz_pre, double *bn2, double *rn2, hipStream_t st);
 };
 
 // cal_u on the device (src/PoissonSolver.cpp:580-653): top-row potential

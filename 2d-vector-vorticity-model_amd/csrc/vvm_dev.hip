@@ -243,13 +243,30 @@ int upload_level_constants(vvm_dev *h, const vvm_host_view *v) {
     return VVM_OK;
 }
 
+// FP64 from a guess: MG-PCG, whose iteration count tells what the guess is
+// worth.  Everything else but BiCGSTAB is solved directly, which takes no
+// guess.  A step's cal_w and cal_u at 2048 x 256: 95 us, against 870 us with
+// FP64 MG-PCG from zero and 480 us with FP32 MG-PCG in FP64 refinement from
+// the quadratic extrapolation; columns that cannot be halved (317 x 61): 0.1
+// against 13 ms.
+bool uses_pcg(const vvm_dev_config &c) {
+    return c.solver_mode == VVM_SOLVER_FP64 && c.guess_mode != VVM_GUESS_ZERO;
+}
+bool uses_direct(const vvm_dev_config &c) { return c.solver_mode != VVM_SOLVER_BICGSTAB && !uses_pcg(c); }
+constexpr double kParityTol = 1e-13;  // VVM_STOP_PARITY where the residual is formed anew each sweep
+constexpr int kMaxSweeps = 8;
+double stop_tol(const vvm_dev_config &c) { return c.stop_mode == VVM_STOP_PARITY ? kParityTol : c.tol_rel; }
+int max_iterations(const vvm_dev_config &c) { return c.max_iter > 0 ? c.max_iter : 200; }
+
 int ensure_poisson(vvm_dev *h, const double *rhou, const double *rhow) {
     const int nz = h->cfg.nz;
     std::vector<double> ru(rhou, rhou + nz), rw(rhow, rhow + nz);
     if (h->pois_ready && ru == h->h_rhou && rw == h->h_rhow) return VVM_OK;
     if (h->pois_ready) h->pois.destroy();
     h->pois_ready = false;
-    const int rc = h->pois.init(h->G, rhou, rhow, h->red.solver, true);
+    const vvm_dev_config &c = h->cfg;
+    const int rc = h->pois.init(h->G, rhou, rhow, h->red.solver, c.solver_mode != VVM_SOLVER_BICGSTAB,
+                                c.solver_mode == VVM_SOLVER_MIXED, uses_pcg(c));
     if (rc != VVM_OK) return fail(h, rc, "Poisson solver allocation failed");
     h->pois_ready = true;
     h->h_rhou = ru;
@@ -257,44 +274,64 @@ int ensure_poisson(vvm_dev *h, const double *rhou, const double *rhow) {
     return VVM_OK;
 }
 
-// cal_w's right-hand side and the initial guess, on stream st.
-void prepare_guess(vvm_dev *h, const StepPtrs &S, hipStream_t st) {
-    const vvm_dev_config &c = h->cfg;
+// cal_w's right-hand side and, if run_net, the learned guess, on stream st.
+void prepare_guess(vvm_dev *h, const StepPtrs &S, bool run_net, hipStream_t st) {
     h->pois.rhs_from_zetap(h->G, S.fut[F_ZETA], h->P.rhow, st);
     h->pois.collect_features(st);  // no-op unless recording samples
-    h->pois.net = h->guess_net;
-    const bool learned = (c.guess_mode == VVM_GUESS_LEARNED) && h->pois.learned_guess(st);
+    if (run_net && h->pois.learned_guess(st)) return;
     // without a network (or before two solutions exist) the learned mode
     // starts from the extrapolation the network would correct
-    if (!learned) h->pois.set_guess(c.guess_mode == VVM_GUESS_LEARNED ? VVM_GUESS_EXTRAP2 : c.guess_mode, st);
+    const int mode = h->cfg.guess_mode;
+    h->pois.set_guess(mode == VVM_GUESS_LEARNED ? VVM_GUESS_EXTRAP2 : mode, st);
 }
 
-// prepared: prepare_guess has already run (on the second stream, which the
-// main stream has waited for)
-int solve_w(vvm_dev *h, const StepPtrs &S, vvm_solve_stats *ss, bool prepared = false) {
+bool net_due(vvm_dev *h) {
+    h->pois.net = h->guess_net;
+    return h->cfg.guess_mode == VVM_GUESS_LEARNED && h->pois.net_due();
+}
+
+void report(vvm_solve_stats *ss, const SolveResult &R) {
+    if (!ss) return;
+    ss->iters = R.iters;
+    ss->refine = R.refine;
+    ss->rel_residual = R.rel;
+    ss->rel_residual0 = R.rel0;
+}
+
+// cal_w by an iterative solver (MG-PCG or BiCGSTAB).  prepared: prepare_guess
+// has already run (on the second stream, which the main stream has waited for)
+int solve_w_iter(vvm_dev *h, const StepPtrs &S, vvm_solve_stats *ss, bool run_net, bool prepared) {
     const vvm_dev_config &c = h->cfg;
-    if (!prepared) prepare_guess(h, S, h->st);
-    SolveResult R;
-    const int maxit = c.max_iter > 0 ? c.max_iter : 200;
-    if (c.solver_mode == VVM_SOLVER_BICGSTAB) {
-        const double tol = (c.stop_mode == VVM_STOP_PARITY) ? 1e-13 : c.tol_rel;
-        R = h->pois.solve_bicgstab(tol, c.stop_mode == VVM_STOP_ABS, maxit, h->st);
-    } else if (c.solver_mode == VVM_SOLVER_MIXED) {
-        const double tol = (c.stop_mode == VVM_STOP_PARITY) ? 1e-13 : c.tol_rel;
-        R = h->pois.solve_mixed(tol, 8, maxit, 1e-4, h->st);
-    } else {
-        const double tol = (c.stop_mode == VVM_STOP_PARITY) ? 0. : c.tol_rel;
-        R = h->pois.solve_fp64(tol, maxit, h->st);
-    }
+    if (!prepared) prepare_guess(h, S, run_net, h->st);
+    const int maxit = max_iterations(c);
+    const SolveResult R =
+        c.solver_mode == VVM_SOLVER_BICGSTAB
+            ? h->pois.solve_bicgstab(stop_tol(c), c.stop_mode == VVM_STOP_ABS, maxit, h->st)
+            : h->pois.solve_fp64(c.stop_mode == VVM_STOP_PARITY ? 0. : c.tol_rel, maxit, h->st);
     h->pois.collect_target(h->st);  // before x_{t-1}, x_{t-2} move on
     h->pois.back_to_w(h->G, S.w, h->P.rhow, h->st);
     h->pois.remember_solution(h->st);  // x becomes x_{t-1} (buffer rotation)
-    if (ss) {
-        ss->iters = R.iters;
-        ss->refine = R.refine;
-        ss->rel_residual = R.rel;
-        ss->rel_residual0 = R.rel0;
-    }
+    report(ss, R);
+    return R.converged ? VVM_OK : VVM_WARN_NOT_CONVERGED;
+}
+
+// cal_w by the direct solver: queued first, so that what follows it can be
+// queued behind it, then finished, which waits for the residual's norms.
+// redo: w has changed since, and what was queued behind it has to run again.
+void queue_w(vvm_dev *h, const StepPtrs &S, bool run_net, bool prepared) {
+    const bool first = prepared || run_net || h->pois.sample_cap > 0;
+    if (first && !prepared) prepare_guess(h, S, run_net, h->st);
+    h->pois.queue_step(h->G, S.fut[F_ZETA], h->P.rhow, S.w, first, h->st);
+}
+int finish_w(vvm_dev *h, const StepPtrs &S, vvm_solve_stats *ss, bool *redo) {
+    const vvm_dev_config &c = h->cfg;
+    const bool fp64 = c.solver_mode == VVM_SOLVER_FP64;
+    SolveResult R = h->pois.finish_step(h->G, S.w, h->P.rhow, stop_tol(c), fp64,
+                                        std::min(kMaxSweeps, max_iterations(c)), redo, h->st);
+    if (!fp64) R.refine = R.iters;
+    h->pois.collect_target(h->st);
+    h->pois.remember_solution(h->st);
+    report(ss, R);
     return R.converged ? VVM_OK : VVM_WARN_NOT_CONVERGED;
 }
 
@@ -712,8 +749,8 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
         const bool overlap = h->overlap_c && !h->mp_fn;
         // the learned guess's network is the longest serial chain before the
         // solve; it needs only pzeta's zetap and the past solutions
-        const bool early_guess = overlap && c.guess_mode == VVM_GUESS_LEARNED && h->guess_net &&
-                                 h->pois.sample_cap == 0;
+        const bool run_net = net_due(h);
+        const bool early_guess = overlap && run_net && h->pois.sample_cap == 0;
         rec(0, h->st);
         // A: advection, buoyancy, forcing, halos (src/Iteration.cpp:263-285)
         {
@@ -723,7 +760,7 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
         if (early_guess) {
             hipEventRecord(h->ev_fork0, h->st);
             hipStreamWaitEvent(h->side, h->ev_fork0, 0);
-            prepare_guess(h, S, h->side);
+            prepare_guess(h, S, true, h->side);
             hipEventRecord(h->ev_guess, h->side);
         }
         {
@@ -764,10 +801,21 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
         launch_pubartop(G, S, h->step, h->st);
         vvm_solve_stats ss{};
         int rc;
+        const bool direct = uses_direct(c);
         {
             KTimer t(h, VVM_KT_SOLVE);
             if (early_guess) hipStreamWaitEvent(h->st, h->ev_guess, 0);
-            rc = solve_w(h, S, &ss, early_guess);
+            if (direct) queue_w(h, S, run_net, early_guess);
+            else rc = solve_w_iter(h, S, &ss, run_net, early_guess);
+        }
+        {
+            KTimer t(h, VVM_KT_CALU);
+            launch_cal_u(G, S, h->st);
+        }
+        if (direct) {
+            bool redo = false;
+            rc = finish_w(h, S, &ss, &redo);
+            if (redo) launch_cal_u(G, S, h->st);
         }
         if (rc == VVM_WARN_NOT_CONVERGED) {
             warn = rc;
@@ -779,10 +827,6 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
         acc.solve_iters_last = ss.iters;
         acc.refine_last = ss.refine;
         acc.rel_residual_last = ss.rel_residual;
-        {
-            KTimer t(h, VVM_KT_CALU);
-            launch_cal_u(G, S, h->st);
-        }
         rec(2, h->st);
         if (overlap) hipStreamWaitEvent(h->st, h->ev_join, 0);
         if (h->mp_fn) {
@@ -890,7 +934,13 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
         case VVM_OP_CAL_W: {
             vvm_dev_config saved = h->cfg;
             h->cfg.guess_mode = VVM_GUESS_ZERO;
-            rc = solve_w(h, S, nullptr);
+            if (uses_direct(h->cfg)) {
+                bool redo = false;
+                queue_w(h, S, false, false);
+                rc = finish_w(h, S, nullptr, &redo);
+            } else {
+                rc = solve_w_iter(h, S, nullptr, false, false);
+            }
             h->cfg = saved;
             break;
         }
@@ -1021,15 +1071,15 @@ static int poisson_common(vvm_dev *h, const double *d_b, double *d_x, vvm_solve_
     h->pois.x_from_ref(d_x, h->st);
     hipEventRecord(h->ev[6], h->st);
     SolveResult R;
-    const int maxit = c.max_iter > 0 ? c.max_iter : 200;
-    if (c.solver_mode == VVM_SOLVER_BICGSTAB) {
-        R = h->pois.solve_bicgstab(c.stop_mode == VVM_STOP_PARITY ? 1e-13 : c.tol_rel, c.stop_mode == VVM_STOP_ABS,
-                                   maxit, h->st);
-    } else if (c.solver_mode == VVM_SOLVER_MIXED) {
-        R = h->pois.solve_mixed(c.stop_mode == VVM_STOP_PARITY ? 1e-13 : c.tol_rel, 8, maxit, 1e-4, h->st);
-    } else {
+    const int maxit = max_iterations(c), sweeps = std::min(kMaxSweeps, maxit);
+    if (c.solver_mode == VVM_SOLVER_BICGSTAB)
+        R = h->pois.solve_bicgstab(stop_tol(c), c.stop_mode == VVM_STOP_ABS, maxit, h->st);
+    else if (c.solver_mode == VVM_SOLVER_MIXED)
+        R = h->pois.solve_mixed(stop_tol(c), sweeps, h->st);
+    else if (uses_pcg(c))
         R = h->pois.solve_fp64(c.stop_mode == VVM_STOP_PARITY ? 0. : c.tol_rel, maxit, h->st);
-    }
+    else
+        R = h->pois.solve_direct(stop_tol(c), true, sweeps, h->st);
     hipEventRecord(h->ev[7], h->st);
     h->pois.x_to_ref(d_x, h->st);
     HIPCHK(h, hipStreamSynchronize(h->st));

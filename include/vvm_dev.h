@@ -41,8 +41,14 @@ extern "C" {
 #define VVM_ERR_NOMEM (-5)
 
 /* Poisson back-ends (north of the reference's single Eigen path). */
-#define VVM_SOLVER_FP64 0   /* FP64 multigrid-preconditioned CG            */
-#define VVM_SOLVER_MIXED 1  /* FP32 MG-PCG inside FP64 iterative refinement */
+/* FP64: a direct solve (Fourier along the periodic x, tridiagonal along z)
+ * with FP64 refinement until the stop rule holds; with a guess_mode other than
+ * zero, multigrid-preconditioned CG from that guess. */
+#define VVM_SOLVER_FP64 0
+/* FP32 direct solves inside FP64 iterative refinement (vvm_dev_poisson); a
+ * step takes the FP64 direct solve, which needs no refinement, and runs a
+ * guess only where a network is attached (VVM_GUESS_LEARNED). */
+#define VVM_SOLVER_MIXED 1
 /* The reference GPU back-end's solver (src/PoissonSolver_GPU_mpi.cpp:41:
  * AMGX BiCGSTAB + ILU0, tolerance 1e-12, 10000 iterations): BiCGSTAB with a
  * red-black ILU0 preconditioner, for comparison runs; with VVM_STOP_ABS and
@@ -78,7 +84,8 @@ typedef struct vvm_dev_config {
     int32_t solver_mode;     /* VVM_SOLVER_*                                 */
     int32_t guess_mode;      /* VVM_GUESS_*                                  */
     int32_t stop_mode;       /* VVM_STOP_*                                   */
-    int32_t max_iter;        /* cap on PCG iterations per solve              */
+    int32_t max_iter;        /* cap on PCG iterations, or direct solves (at
+                                most 8), per solve                           */
     double tol_rel;          /* used by VVM_STOP_REL                         */
 } vvm_dev_config;
 
@@ -116,15 +123,16 @@ typedef struct vvm_host_view {
  * (src/Declare.hpp:695-699, filled at src/Iteration.cpp:286,297,405,418,435). */
 typedef struct vvm_step_stats {
     int32_t steps;             /* steps taken by this call                   */
-    int32_t solve_iters_total; /* PCG iterations summed over the steps      */
-    int32_t solve_iters_last;  /* PCG iterations of the last step           */
+    int32_t solve_iters_total; /* direct solves, or PCG iterations, summed over
+                                  the steps                                 */
+    int32_t solve_iters_last;  /* the same, of the last step                */
     int32_t refine_last;       /* outer refinement sweeps of the last step  */
     int32_t not_converged;     /* solves that hit max_iter                   */
     double rel_residual_last;  /* ||b-Ax||/||b|| of the last solve          */
     double t_advection, t_poisson, t_microphysics, t_diffusion, t_all; /* s */
     int32_t guess_fallbacks;   /* solves whose learned guess started worse
                                   than the extrapolation (or not finite) and
-                                  were restarted from the extrapolation    */
+                                  were dropped                             */
     int32_t guess_skipped;     /* solves that did not run the network: after
                                   a restart it sits out 1, 4, 16, then 64
                                   solves (while its guesses keep losing;
@@ -132,7 +140,7 @@ typedef struct vvm_step_stats {
 } vvm_step_stats;
 
 typedef struct vvm_solve_stats {
-    int32_t iters;          /* PCG iterations (inner, summed)               */
+    int32_t iters;          /* direct solves, or PCG iterations              */
     int32_t refine;         /* outer FP64 refinement sweeps (mixed only)    */
     double rel_residual;    /* ||b - A x||_2 / ||b||_2                      */
     double rel_residual0;   /* same, for the initial guess                  */
