@@ -7,10 +7,17 @@
 // where a, d hold the diffusion coefficients and c the old centre, east and
 // upper values; ghost cells are never updated during the sweep.
 //
-// Two kernels.  k_diff_coeffs forms a, c, d for every point of the five
-// fields in parallel over the whole GPU (a and d of Hparam depend only on
-// RKH and are shared by th, qv, qc, qr).  k_diff_sweep then does only the
-// sequential part: row k is a first-order linear recurrence in i once row
+// The weights a and d are diffusion numbers, K dt / dx^2 and K dt / dz^2, of
+// order 1e-3 to 1e-2 in the model's flows, so what a value owes to values m
+// columns or rows away falls as (a + d)^m and is below FP64's rounding after a
+// few.  Where that holds (diffusion_halo), k_diff_tiles cuts the fields into
+// independent tiles, each of which starts that many columns and rows early.
+//
+// Otherwise the sweep runs in order, in two kernels.  k_diff_coeffs forms
+// a, c, d for every point of the five fields in parallel over the whole GPU (a
+// and d of Hparam depend only on RKH and are shared by th, qv, qc, qr).
+// k_diff_sweep then does only the sequential part: row k is a first-order
+// linear recurrence in i once row
 // k-1 is final.  One workgroup per field; wavefront w owns a strip of 64*E
 // consecutive columns and walks the rows in order.  In each row a wave
 // composes its lanes' affine maps y -> a y + e (e = c + d y_below) with a
@@ -26,6 +33,7 @@
 #pragma clang fp contract(off)
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <vector>
 
@@ -533,6 +541,164 @@ __global__ void __launch_bounds__((CW + 1) * kWave) k_diff_strips(Grid G, StepPt
 }
 
 
+// ---------------------------------------------------------------------------
+// Independent tiles, out of place (S.fut -> S.dcoef[DC_C0 + field], ghost cells
+// copied).  A wavefront walks the rows of one field's tile; lane l holds the
+// columns c and c + 1, c = c0 + 2 l.  The first H columns and the first H rows
+// only warm up: the row below the first is taken from the old field, and along
+// a row H/2 sweeps over the lanes (y_c = a_c y_{c-1} + e_c, then y_{c+1}) start
+// from the old field too, so what reaches the columns and rows that are stored
+// is wrong by less than (a + d)^H |new - old|.  Lane 63 only supplies the east
+// neighbour.  Rows come in blocks of eight, loaded one block ahead; every old
+// value is loaded once a tile, and neighbours in x come by DPP.  The four
+// wavefronts of a workgroup take the four scalars of one tile (whose K they
+// share) or four tiles of zeta.
+//
+// Two columns a lane halve the lane moves of one (0.7 us a row for the four
+// scalars in one wavefront, which the instruction count bound) and leave twice
+// the wavefronts of four.
+//
+// 2048 x 256, FP64: 20 us (H = 8) against 122 us for k_diff_coeffs and
+// k_diff_strips, whose time is 256 rows one after another.
+constexpr int TROWS = 8;
+constexpr int TWAVES = 4;
+__host__ __device__ constexpr int tile_cols(int H) { return 2 * (kWave - 1) - H; }
+
+// wave_shr:1 / wave_shl:1: the value of the lane on the left / right (0 for the
+// first / last lane, which only warm up or supply a neighbour).
+template <int CTRL>
+__device__ inline double lane_move(double v) {
+    const long long x = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, int(x & 0xffffffffll), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, int(x >> 32), CTRL, 0xF, 0xF, true);
+    return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
+}
+__device__ inline double from_left(double v) { return lane_move<0x138>(v); }
+__device__ inline double from_right(double v) { return lane_move<0x130>(v); }
+
+// Per-row values of a workgroup's rows, read from LDS: a load or a division in
+// the row loop would add its latency to every row.
+struct RowConst {
+    double ct, cb, bk;  // densities above and below, dt / dz^2 over the density
+    double rate, thbi;  // nudging
+};
+
+template <int H, bool MOM>
+__device__ inline void diff_tile(const Grid &G, const double *__restrict__ f, const double *__restrict__ K,
+                                 double *__restrict__ out, bool is_theta, bool nudged, const RowConst *rc, int kl, int ks,
+                                 int ke) {
+    const int lane = threadIdx.x % kWave, n = G.nx - 2, nz = G.nz;
+    const int c = int(blockIdx.x) * tile_cols(H) - H + 2 * lane;  // even: the pairs are 16-byte aligned
+    const int cl = min(max(c, 0), G.pitch - 2);
+    const double A = G.rdx2 * G.dt;
+    // columns 0..n+1 are stored, the two ghost columns with their old value
+    const bool st0 = 2 * lane >= H && lane < kWave - 1 && c <= n + 1, st1 = st0 && c + 1 <= n + 1;
+    const bool gh0 = c == 0 || c == n + 1, gh1 = c + 1 == n + 1;
+    const bool in0 = c >= 1, in1 = c + 1 >= 1;  // west of column 1 nothing changes
+    const int k0 = max(1, ks - H);              // first row worked on (exact if it is row 1)
+    auto load = [&](const double *a, int k) { return *reinterpret_cast<const double2 *>(a + ix(G, cl, k)); };
+    auto put = [&](int k, double v0, double v1) {
+        double *o = out + ix(G, c, k);
+        if (st1) *reinterpret_cast<double2 *>(o) = make_double2(v0, v1);
+        else if (st0) *o = v0;
+    };
+    double2 pK = load(K, k0 - 1), cK = load(K, k0), cf = load(f, k0), y = load(f, k0 - 1);
+    double2 nK[TROWS], nf[TROWS];  // rows k+1 .. k+TROWS
+    auto fetch = [&](int k) {
+#pragma unroll
+        for (int r = 0; r < TROWS; r++) {
+            nK[r] = load(K, min(k + r, nz - 1));
+            nf[r] = load(f, min(k + r, nz - 1));
+        }
+    };
+    fetch(k0 + 1);
+    if (ks == 1) put(0, y.x, y.y);
+    for (int kb = k0; kb <= ke; kb += TROWS) {
+        double2 bK[TROWS], bf[TROWS];
+#pragma unroll
+        for (int r = 0; r < TROWS; r++) {
+            bK[r] = nK[r];
+            bf[r] = nf[r];
+        }
+        fetch(kb + TROWS + 1);
+#pragma unroll
+        for (int r = 0; r < TROWS; r++) {
+            const int k = kb + r;
+            if (k > ke) break;
+            const RowConst R = rc[k - kl];
+            const double2 tK = bK[r], tf = bf[r];
+            double Ke0, Ke1, Kw0, Ct0, Ct1, Cb0, Cb1;  // Kw1 = Ke0
+            if (MOM) {
+                const double wK = from_left(cK.y), wpK = from_left(pK.y);
+                Ke0 = 0.5 * (cK.x + pK.x);
+                Ke1 = 0.5 * (cK.y + pK.y);
+                Kw0 = 0.5 * (wK + wpK);
+                Ct0 = R.ct * 0.5 * (cK.x + wK);
+                Ct1 = R.ct * 0.5 * (cK.y + cK.x);
+                Cb0 = R.cb * 0.5 * (pK.x + wpK);
+                Cb1 = R.cb * 0.5 * (pK.y + pK.x);
+            } else {
+                Ke0 = 0.5 * (cK.y + cK.x);
+                Ke1 = 0.5 * (from_right(cK.x) + cK.y);
+                Kw0 = 0.5 * (cK.x + from_left(cK.y));
+                Ct0 = R.ct * 0.5 * (tK.x + cK.x);
+                Ct1 = R.ct * 0.5 * (tK.y + cK.y);
+                Cb0 = R.cb * 0.5 * (cK.x + pK.x);
+                Cb1 = R.cb * 0.5 * (cK.y + pK.y);
+            }
+            const double a0 = in0 ? A * Kw0 : 0., a1 = in1 ? A * Ke0 : 0.;
+            const double east = from_right(cf.x);
+            const double c0 = cf.x + A * (Ke0 * (cf.y - cf.x) - Kw0 * cf.x) + R.bk * (Ct0 * (tf.x - cf.x) - Cb0 * cf.x);
+            const double c1 = cf.y + A * (Ke1 * (east - cf.y) - Ke0 * cf.y) + R.bk * (Ct1 * (tf.y - cf.y) - Cb1 * cf.y);
+            const double e0 = in0 ? c0 + R.bk * Cb0 * y.x : cf.x, e1 = in1 ? c1 + R.bk * Cb1 * y.y : cf.y;
+            y = cf;
+#pragma unroll
+            for (int s = 0; s < H / 2; s++) {
+                y.x = __builtin_fma(a0, from_left(y.y), e0);
+                y.y = __builtin_fma(a1, y.x, e1);
+            }
+            if (k >= ks) {
+                double o0 = y.x, o1 = y.y;
+                if (nudged && R.rate != 0.) {
+                    o0 = o0 - R.rate * (is_theta ? o0 - R.thbi : o0);
+                    o1 = o1 - R.rate * (is_theta ? o1 - R.thbi : o1);
+                }
+                put(k, gh0 ? cf.x : o0, gh1 ? cf.y : o1);
+                if (k == nz - 2) put(nz - 1, tf.x, tf.y);
+            }
+            pK = cK;
+            cK = tK;
+            cf = tf;
+        }
+    }
+}
+
+// blockIdx.z 0: the four scalars, a row chunk a workgroup; 1: zeta, four.
+template <int H>
+__global__ void __launch_bounds__(TWAVES *kWave) k_diff_tiles(Grid G, StepPtrs S, int nudge, int rows) {
+    extern __shared__ RowConst rc[];  // rows kl .. of this workgroup
+    const bool mom = blockIdx.z == 1;
+    const int chunks = mom ? TWAVES : 1;
+    const int kb = 1 + blockIdx.y * chunks * rows, kl = max(1, kb - H), kh = min(kb + chunks * rows - 1, G.nz - 2);
+    if (kb > G.nz - 2) return;
+    for (int k = kl + threadIdx.x; k <= kh; k += blockDim.x) {
+        RowConst r;
+        r.ct = mom ? S.P.rhou[k] : S.P.rhow[k + 1];
+        r.cb = mom ? S.P.rhou[k - 1] : S.P.rhow[k];
+        r.bk = G.rdz2 * G.dt / (mom ? S.P.rhow[k] : S.P.rhou[k]);
+        // the nudging of this wavefront's field: zeta, or th (wavefront 0)
+        r.rate = mom ? ((nudge & 2) ? S.P.rate_z[k] : 0.) : ((nudge & 1) ? S.P.rate_th[k] : 0.);
+        r.thbi = S.P.thb_init[k];
+        rc[k - kl] = r;
+    }
+    __syncthreads();
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int ks = kb + (mom ? w : 0) * rows, ke = min(ks + rows - 1, G.nz - 2);
+    if (ks > G.nz - 2) return;
+    if (mom) diff_tile<H, true>(G, S.fut[F_ZETA], S.RKM, S.dcoef[DC_C0 + F_ZETA], false, true, rc, kl, ks, ke);
+    else diff_tile<H, false>(G, S.fut[F_TH + w], S.RKH, S.dcoef[DC_C0 + F_TH + w], w == 0, w == 0, rc, kl, ks, ke);
+}
+
 template <int E>
 void launch_e(const Grid &G, const StepPtrs &S, int nudge, int fbase, int nfld, hipStream_t st) {
     const int n = G.nx - 2;
@@ -590,6 +756,31 @@ void diffusion_slots_release(unsigned long long *p) {
     std::lock_guard<std::mutex> lk(g_slot_mu);
     for (SlotRegion &r : g_slots)
         if (r.p == p) r.busy = false;
+}
+
+// Smallest warm-up H the tiles may take at the largest weight sum
+// rho = max(a + d): rho^H <= 2^-53.  0: none, the sweep runs in order (also for
+// a rho that is not a number).
+int diffusion_halo(double rho) {
+    for (int H : {8, 16, 32})
+        if (rho <= std::exp2(-53. / H)) return H;
+    return 0;
+}
+
+// Rows a wavefront stores: 8 to 24 (but not fewer than it warms up on), the
+// fewest that give no more than a workgroup a CU.  Measured with 8 / 16 / 24 /
+// 32 rows (H = 8, launch included): 128 x 64 11.6 / 14.3 / 17.0 / 20.0 us,
+// 1024 x 128 13.3 / 15.8 / 18.3 / 21.1, 2048 x 256 25.8 / 23.2 / 21.3 / 23.2,
+// 4096 x 256 43.9 / 36.2 / 32.9 / 35.4.
+void launch_diffusion_tiles(const Grid &G, const StepPtrs &S, int nudge, int H, hipStream_t st) {
+    const int out = tile_cols(H), windows = (G.nx + out - 1) / out;
+    int rows = H;
+    while (rows < 24 && windows * ((G.nz - 2 + rows - 1) / rows) > 256) rows += 8;
+    const size_t lds = size_t(TWAVES * rows + H) * sizeof(RowConst);
+    const dim3 g((G.nx + out - 1) / out, (G.nz - 2 + rows - 1) / rows, 2), b(TWAVES * kWave);
+    if (H == 8) hipLaunchKernelGGL(k_diff_tiles<8>, g, b, lds, st, G, S, nudge, rows);
+    else if (H == 16) hipLaunchKernelGGL(k_diff_tiles<16>, g, b, lds, st, G, S, nudge, rows);
+    else hipLaunchKernelGGL(k_diff_tiles<32>, g, b, lds, st, G, S, nudge, rows);
 }
 
 void launch_diffusion(const Grid &G, const StepPtrs &S, int nudge, hipStream_t st, int only_field) {

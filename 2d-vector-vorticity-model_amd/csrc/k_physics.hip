@@ -18,6 +18,7 @@ namespace {
 
 constexpr int BX = 64, BY = 4;
 
+__device__ inline double max_or_nan(double a, double b) { return (a != a || a > b) ? a : b; }
 __device__ inline double maxs(double a, double b) { return (a < b) ? b : a; }
 __device__ inline double mins(double a, double b) { return (b < a) ? b : a; }
 
@@ -132,10 +133,8 @@ __global__ void __launch_bounds__(BX *BY) k_negval_scale(Grid G, double *a, cons
 }
 
 // Turbulence::RKM_RKH coefficient part (Turbulent.cpp:13-45), with the
-// center halos of RKM and RKH.
-__global__ void __launch_bounds__(BX *BY) k_turb_coeffs(Grid G, StepPtrs S) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
-    if (i < 1 || i > G.nx - 2 || k < 1 || k > G.nz - 2) return;
+// center halos of RKM and RKH.  Returns the larger of the two.
+__device__ inline double turb_point(const Grid &G, const StepPtrs &S, int i, int k) {
     const double *u = S.u, *w = S.w, *thp = S.fut[F_TH];
     const double Rz =
         0.5 * ((w[ix(G, i + 1, k + 1)] + w[ix(G, i + 1, k)]) - (w[ix(G, i - 1, k + 1)] + w[ix(G, i - 1, k)])) * G.r2dx +
@@ -163,7 +162,35 @@ __global__ void __launch_bounds__(BX *BY) k_turb_coeffs(Grid G, StepPtrs S) {
     kh = mins(kh, kmax);
     store_center(S.RKM, G, i, k, km);
     store_center(S.RKH, G, i, k, kh);
+    return max_or_nan(km, kh);
 }
+
+// At most kTurbBlocks workgroups walk the tiles; each leaves the largest
+// coefficient it formed in kmax, from which the host chooses the diffusion
+// sweep.  A NaN (unstable stratification at rest: Ri = -inf) stays one.
+__global__ void __launch_bounds__(BX *BY) k_turb_coeffs(Grid G, StepPtrs S, double *kmax) {
+    const int tx = (G.nx + BX - 1) / BX, nt = tx * ((G.nz + BY - 1) / BY);
+    double m = 0.;
+    for (int t = blockIdx.x; t < nt; t += gridDim.x) {
+        const int i = (t % tx) * BX + threadIdx.x, k = (t / tx) * BY + threadIdx.y;
+        if (i < 1 || i > G.nx - 2 || k < 1 || k > G.nz - 2) continue;
+        const double v = turb_point(G, S, i, k);
+        m = max_or_nan(m, v);
+    }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        const double o = __shfl_xor(m, off, kWave);
+        m = max_or_nan(m, o);
+    }
+    __shared__ double sh[BY];
+    if (threadIdx.x == 0) sh[threadIdx.y] = m;
+    __syncthreads();
+    if (threadIdx.x == 0 && threadIdx.y == 0) {
+        for (int w = 1; w < BY; w++) m = max_or_nan(m, sh[w]);
+        __hip_atomic_store(kmax + blockIdx.x, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 
 // NumericalProcess::Nudge_qv (NumericalProcess.cpp:86-95), all points.
 __global__ void __launch_bounds__(BX *BY) k_nudge_qv(Grid G, StepPtrs S, double tau) {
@@ -236,8 +263,10 @@ void launch_negative_value(const Grid &G, const StepPtrs &S, double *a, const Re
     finalize<2>(rs, nblocks(grid2d(G)), S.s, RED_NEGVAL, S_NEG_RATIO, st);
     hipLaunchKernelGGL(k_negval_scale, grid2d(G), dim3(BX, BY), 0, st, G, a, S.s + S_NEG_RATIO);
 }
-void launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, hipStream_t st) {
-    hipLaunchKernelGGL(k_turb_coeffs, grid2d(G), dim3(BX, BY), 0, st, G, S);
+int launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, double *kmax, hipStream_t st) {
+    const int nt = nblocks(grid2d(G)), nb = nt < kTurbBlocks ? nt : kTurbBlocks;
+    hipLaunchKernelGGL(k_turb_coeffs, dim3(nb), dim3(BX, BY), 0, st, G, S, kmax);
+    return nb;
 }
 
 // Nudge_theta and Nudge_zeta alone (NumericalProcess.cpp:60-84), pointwise;

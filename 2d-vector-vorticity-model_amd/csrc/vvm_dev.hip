@@ -35,6 +35,14 @@ struct vvm_dev {
     double *dcoef[DC_N] = {};
     unsigned long long *dslots = nullptr;
     int dstrip_cw = 0;              // diffusion strip width in wavefronts (0: default)
+    // The diffusion sweep's warm-up (diffusion_halo; 0: in order), guessed from
+    // the last step's coefficients and checked against this step's, which
+    // k_turb_coeffs leaves in kmax (host-mapped) before ev_turb.
+    int diff_halo = 0;
+    double *kmax = nullptr, *kmax_dev = nullptr;
+    int kmax_blocks = 0;
+    double rho_per_k = 0.;          // largest a + d of the sweep per unit of K
+    hipEvent_t ev_turb = nullptr;
     GuessNet *guess_net = nullptr;  // attached learned guess (not owned)
     int guess_net_device = -1;
     Profiles P{};
@@ -177,6 +185,49 @@ StepPtrs ptrs(vvm_dev *h) {
     S.dslots = h->dslots;
     S.dstrip_cw = h->dstrip_cw;
     return S;
+}
+
+// Turbulence coefficients, and the largest of them on its way to the host.
+void queue_turbulence(vvm_dev *h, const StepPtrs &S) {
+    h->kmax_blocks = launch_turbulence_coeffs(h->G, S, h->kmax_dev, h->st);
+    hipEventRecord(h->ev_turb, h->st);
+}
+
+// The sweep's largest weight sum, once ev_turb has passed.
+double diffusion_rho(vvm_dev *h) {
+    hipEventSynchronize(h->ev_turb);
+    const volatile double *p = h->kmax;
+    double m = 0.;
+    for (int b = 0; b < h->kmax_blocks; b++) {
+        const double v = p[b];
+        if (!(v <= m)) m = v;
+        if (v != v) break;  // a NaN stays one
+    }
+    return m * h->rho_per_k;
+}
+
+// The tiled sweep has written the p fields to the planes of c: swap the two.
+void take_tiles(vvm_dev *h, StepPtrs &S) {
+    for (int f = 0; f < NPROG; f++) {
+        std::swap(h->prog[f][h->idx_fut], h->dcoef[DC_C0 + f]);
+        S.fut[f] = h->prog[f][h->idx_fut];
+        S.dcoef[DC_C0 + f] = h->dcoef[DC_C0 + f];
+    }
+}
+
+// Mparam and Hparam of the five fields.  queued: the halo of the tiled sweep
+// that is in the stream already (0: none); it is redone where the
+// coefficients ask for a longer one.
+void finish_diffusion(vvm_dev *h, StepPtrs &S, int nudge, int queued) {
+    const double rho = diffusion_rho(h);
+    const int need = diffusion_halo(rho);
+    h->diff_halo = diffusion_halo(1.25 * rho);
+    if (need == 0) {
+        launch_diffusion(h->G, S, nudge, h->st);
+        return;
+    }
+    if (need > queued) launch_diffusion_tiles(h->G, S, nudge, need, h->st);
+    take_tiles(h, S);
 }
 
 // m <- now <- p by rotation (src/Iteration.cpp:158-203 copies).
@@ -425,6 +476,11 @@ int vvm_dev_create(const vvm_dev_config *cfg, int device, vvm_dev_t **out) {
         rs->max_blocks = maxb;
         rs->partial = A(size_t(8) * maxb);
     }
+    ok = ok &&
+         hipHostMalloc(reinterpret_cast<void **>(&h->kmax), kTurbBlocks * sizeof(double),
+                       hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess &&
+         hipHostGetDevicePointer(reinterpret_cast<void **>(&h->kmax_dev), h->kmax, 0) == hipSuccess &&
+         hipEventCreateWithFlags(&h->ev_turb, hipEventDisableTiming) == hipSuccess;
     for (auto &e : h->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
     for (auto &e : h->ev_mp) ok = ok && hipEventCreate(&e) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&h->ev_fork0, hipEventDisableTiming) == hipSuccess &&
@@ -452,11 +508,12 @@ void vvm_dev_destroy(vvm_dev_t *h) {
     if (h->pois_ready) h->pois.destroy();
     for (void *p : h->allocs) hipFree(p);
     if (h->pinned) hipHostFree(h->pinned);
+    if (h->kmax) hipHostFree(h->kmax);
     for (auto &e : h->ev)
         if (e) hipEventDestroy(e);
     for (auto &e : h->kt_ev)
         if (e) hipEventDestroy(e);
-    for (hipEvent_t e : {h->ev_fork0, h->ev_guess, h->ev_fork, h->ev_join, h->ev_mp[0], h->ev_mp[1]})
+    for (hipEvent_t e : {h->ev_turb, h->ev_fork0, h->ev_guess, h->ev_fork, h->ev_join, h->ev_mp[0], h->ev_mp[1]})
         if (e) hipEventDestroy(e);
     for (hipEvent_t e : h->tev)
         if (e) hipEventDestroy(e);
@@ -550,6 +607,14 @@ int vvm_dev_upload(vvm_dev_t *h, const vvm_host_view *v) {
     sc[S_DUBAR0] = v->dubarTop_advect[0];
     sc[S_DUBAR1] = v->dubarTop_advect[1];
     HIPCHK(h, hipMemcpy(h->s, sc, S_NEG_RATIO * sizeof(double), hipMemcpyHostToDevice));
+    // a + d of the diffusion sweep (k_diffusion.hip): K dt / dx^2 from the west,
+    // K dt / dz^2 times a density ratio from below
+    double ratio = 0.;
+    for (int k = 1; k <= nz - 2; k++)
+        for (double r : {v->rhou[k - 1] / v->rhow[k], v->rhow[k] / v->rhou[k]})
+            if (!(r <= ratio)) ratio = r;
+    h->rho_per_k = h->cfg.dt * (h->G.rdx2 + h->G.rdz2 * ratio);
+    h->diff_halo = diffusion_halo(20. * h->rho_per_k);  // twice the smallest K the closure gives
     int rc = upload_level_constants(h, v);
     if (rc) return rc;
     rc = ensure_poisson(h, v->rhou, v->rhow);
@@ -812,21 +877,20 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
             KTimer t(h, VVM_KT_CALU);
             launch_cal_u(G, S, h->st);
         }
-        if (direct) {
+        // The direct solve is finished (its residual read) as late as what
+        // follows can still be run again: with the tiled diffusion sweep, which
+        // leaves its inputs alone, after that is queued, so that the GPU has
+        // work while the host waits.
+        const int halo = h->diff_halo;
+        bool solved = !direct;
+        auto finish_solve = [&]() -> bool {
             bool redo = false;
-            rc = finish_w(h, S, &ss, &redo);
+            if (!solved) rc = finish_w(h, S, &ss, &redo);
+            solved = true;
             if (redo) launch_cal_u(G, S, h->st);
-        }
-        if (rc == VVM_WARN_NOT_CONVERGED) {
-            warn = rc;
-            acc.not_converged++;
-        }
-        acc.solve_iters_total += ss.iters;
-        acc.guess_fallbacks = h->pois.guess_fallbacks - fallbacks0;
-        acc.guess_skipped = h->pois.guess_skipped - skipped0;
-        acc.solve_iters_last = ss.iters;
-        acc.refine_last = ss.refine;
-        acc.rel_residual_last = ss.rel_residual;
+            return redo;
+        };
+        if (h->mp_fn || halo == 0) finish_solve();
         rec(2, h->st);
         if (overlap) hipStreamWaitEvent(h->st, h->ev_join, 0);
         if (h->mp_fn) {
@@ -838,14 +902,30 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
         rec(3, h->st);
         // D: RKM_RKH with Mparam/Hparam, nudging (:408-417); the first
         // updateMean (:408) is overwritten by nextTimeStep's before any read.
+        const int nudge = 1 | (c.CASE != 2 ? 2 : 0);
         {
             KTimer t(h, VVM_KT_TURB);
-            launch_turbulence_coeffs(G, S, h->st);
+            queue_turbulence(h, S);
         }
         {
             KTimer t(h, VVM_KT_DIFFUSION);
-            launch_diffusion(G, S, 1 | (c.CASE != 2 ? 2 : 0), h->st);
+            if (halo) launch_diffusion_tiles(G, S, nudge, halo, h->st);
+            if (finish_solve()) {
+                queue_turbulence(h, S);
+                if (halo) launch_diffusion_tiles(G, S, nudge, halo, h->st);
+            }
+            finish_diffusion(h, S, nudge, halo);
         }
+        if (rc == VVM_WARN_NOT_CONVERGED) {
+            warn = rc;
+            acc.not_converged++;
+        }
+        acc.solve_iters_total += ss.iters;
+        acc.guess_fallbacks = h->pois.guess_fallbacks - fallbacks0;
+        acc.guess_skipped = h->pois.guess_skipped - skipped0;
+        acc.solve_iters_last = ss.iters;
+        acc.refine_last = ss.refine;
+        acc.rel_residual_last = ss.rel_residual;
         if (c.moisture_nudge_time != 0) launch_nudge_qv(G, S, c.moisture_nudge_time, h->st);
         rec(4, h->st);
         // E: nextTimeStep (:153-204)
@@ -953,8 +1033,8 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             launch_bc_all_prog(G, S, h->st);
             break;
         case VVM_OP_TURBULENCE:
-            launch_turbulence_coeffs(G, S, h->st);
-            launch_diffusion(G, S, 0, h->st);
+            queue_turbulence(h, S);
+            finish_diffusion(h, S, 0, 0);
             break;
         case VVM_OP_NUDGE:
             launch_nudge(G, S, 1 | (c.CASE != 2 ? 2 : 0), h->st);

@@ -53,7 +53,8 @@ struct StepPtrs {
     Profiles P;
     // diffusion-sweep coefficients (new = a yW + c + d yB), formed in
     // parallel before the sequential sweep: a, d of Mparam (zeta) and of
-    // Hparam (shared by th, qv, qc, qr), and c of each field.
+    // Hparam (shared by th, qv, qc, qr), and c of each field.  The tiled sweep
+    // writes the new fields to the planes of c instead.
     double *dcoef[DC_N];
     // carry slots of the multi-workgroup diffusion sweep (uncached device
     // memory, [field][strip][k]); nullptr: the one-workgroup sweep runs
@@ -94,11 +95,17 @@ void launch_negative_value(const Grid &G, const StepPtrs &S, double *a, const Re
 
 // Physics (k_physics.hip)
 void launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipStream_t st);
-void launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, hipStream_t st);
+// kmax (host-mapped, kTurbBlocks doubles): the largest RKM or RKH each
+// workgroup formed; returns their count.
+constexpr int kTurbBlocks = 512;
+int launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, double *kmax, hipStream_t st);
 bool diffusion_supported(const Grid &G);  // nx - 2 <= 8192
 // nudge bit 0 fuses Nudge_theta, bit 1 Nudge_zeta into the sweep's store;
 // only_field >= 0 sweeps that one field (Mparam or one Hparam) alone.
 void launch_diffusion(const Grid &G, const StepPtrs &S, int nudge, hipStream_t st, int only_field = -1);
+// The sweep as independent tiles, out of place into S.dcoef[DC_C0 + field].
+int diffusion_halo(double rho);
+void launch_diffusion_tiles(const Grid &G, const StepPtrs &S, int nudge, int H, hipStream_t st);
 // Carry slots for the multi-workgroup sweep on `device` (allocated once per
 // process and device, never freed); nullptr when unavailable.
 unsigned long long *diffusion_slots(const Grid &G, int device);
