@@ -42,7 +42,7 @@ class Direct {
    private:
     RowPlan plan;
     size_t row_lds = 0, col_lds = 0;
-    T *tw = nullptr;    // [N][2]: cos, -sin of 2 pi k / N
+    T *tw = nullptr;    // [N][2]: cos, -sin of 2 pi k / N; then the stages' twiddles, [N-1][2]
     T *g = nullptr;     // [M][N/2+1] elimination factors
     T *di = nullptr;    // [M][N/2+1] 1 / (N pivot)
     T *spec = nullptr;  // [M][N] transformed rows

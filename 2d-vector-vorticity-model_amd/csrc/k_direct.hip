@@ -131,11 +131,12 @@ __device__ inline void dft(Cx<T> (&v)[R]) {
 }
 
 // One Stockham stage of radix R after stages of product Ns.  NB: butterflies
-// a thread, ceil(8 / R) since threads >= N / 8.
+// a thread, ceil(8 / R) since threads >= N / 8.  tw: exp(-2 pi i r k / (Ns R))
+// at (r - 1) Ns + k, so that neighbouring threads read neighbouring values.
 template <int R, typename T>
 __device__ inline void stage(T *re, T *im, int N, int Ns, const T *__restrict__ tw) {
     constexpr int NB = (8 + R - 1) / R;
-    const int nb = N / R, tws = N / (Ns * R);
+    const int nb = N / R;
     Cx<T> v[NB][R];
     int dst[NB];
 #pragma unroll
@@ -152,7 +153,7 @@ __device__ inline void stage(T *re, T *im, int N, int Ns, const T *__restrict__ 
             if (Ns > 1) {
 #pragma unroll
                 for (int r = 1; r < R; r++) {
-                    const int a = 2 * r * k * tws;
+                    const int a = 2 * ((r - 1) * Ns + k);
                     v[t][r] = mul(v[t][r], Cx<T>{tw[a], tw[a + 1]});
                 }
             }
@@ -226,12 +227,15 @@ __device__ inline void fft(const RowPlan &P, T *re, T *im, const T *__restrict__
     int Ns = 1;
     for (int s = 0; s < P.nst; s++) {
         const int R = P.radix[s];
+        // the stages' tables follow the table of all N roots; those before
+        // hold sum (R - 1) Ns = Ns - 1 values
+        const T *ts = tw + 2 * (N + Ns - 1);
         switch (R) {
-            case 8: stage<8>(re, im, N, Ns, tw); break;
-            case 4: stage<4>(re, im, N, Ns, tw); break;
-            case 2: stage<2>(re, im, N, Ns, tw); break;
-            case 3: stage<3>(re, im, N, Ns, tw); break;
-            case 5: stage<5>(re, im, N, Ns, tw); break;
+            case 8: stage<8>(re, im, N, Ns, ts); break;
+            case 4: stage<4>(re, im, N, Ns, ts); break;
+            case 2: stage<2>(re, im, N, Ns, ts); break;
+            case 3: stage<3>(re, im, N, Ns, ts); break;
+            case 5: stage<5>(re, im, N, Ns, ts); break;
             default: stage_any(re, im, N, Ns, R, tws); break;
         }
         Ns *= R;
@@ -274,16 +278,24 @@ __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restric
         f[size_t(row) * N + i] = v;
         return v;
     };
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        re[pad(i)] = T(value(j, i));
-        im[pad(i)] = two ? T(value(j + 1, i)) : T(0);
+#pragma unroll
+    for (int t = 0; t < 8; t++) {  // threads >= N / 8; unrolled, all loads in flight at once
+        const int i = threadIdx.x + t * blockDim.x;
+        if (i < N) {
+            re[pad(i)] = T(value(j, i));
+            im[pad(i)] = two ? T(value(j + 1, i)) : T(0);
+        }
     }
     fft(P, re, im, tw, twl);
-    for (int q = threadIdx.x; q < N; q += blockDim.x) {
-        T ha, hb;
-        hartley_pair(re, im, N, q, ha, hb);
-        spec[size_t(j - 1) * N + q] = ha;
-        if (two) spec[size_t(j) * N + q] = hb;
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const int q = threadIdx.x + t * blockDim.x;
+        if (q < N) {
+            T ha, hb;
+            hartley_pair(re, im, N, q, ha, hb);
+            spec[size_t(j - 1) * N + q] = ha;
+            if (two) spec[size_t(j) * N + q] = hb;
+        }
     }
 }
 
@@ -299,9 +311,13 @@ __global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restric
     T *re = reinterpret_cast<T *>(lds_raw), *im = re + LN, *twl = im + LN;
     const int j = 1 + 2 * blockIdx.x;
     const bool two = j + 1 <= M;
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        re[pad(i)] = spec[size_t(j - 1) * N + i];
-        im[pad(i)] = two ? spec[size_t(j) * N + i] : T(0);
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const int i = threadIdx.x + t * blockDim.x;
+        if (i < N) {
+            re[pad(i)] = spec[size_t(j - 1) * N + i];
+            im[pad(i)] = two ? spec[size_t(j) * N + i] : T(0);
+        }
     }
     if constexpr (W) {  // the zero rows of w
         for (int i = threadIdx.x; i < G.nx; i += blockDim.x) {
@@ -316,11 +332,15 @@ __global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restric
         x[a] = v;
         if constexpr (W) store_westdown(w, G, i + 1, row + 1, v / rhow[row + 1]);
     };
-    for (int q = threadIdx.x; q < N; q += blockDim.x) {
-        T ha, hb;
-        hartley_pair(re, im, N, q, ha, hb);
-        put(j, q, ha);
-        if (two) put(j + 1, q, hb);
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const int q = threadIdx.x + t * blockDim.x;
+        if (q < N) {
+            T ha, hb;
+            hartley_pair(re, im, N, q, ha, hb);
+            put(j, q, ha);
+            if (two) put(j + 1, q, hb);
+        }
     }
 }
 
@@ -360,104 +380,145 @@ __global__ void __launch_bounds__(64) k_factor(int N, int M, const double *__res
     di[size_t(mid - 1) * Nq + q] = T(1. / ((diag(mid) - top - bot) * N));
 }
 
-// Eight columns a workgroup: every thread moves them and their factors to LDS
-// (all loads in flight at once), then 16 lanes run the eliminations, 8
-// columns x 2 directions, chunk by chunk from registers, and every thread
-// moves the result back.
-constexpr int KC = 8, KCHUNK = 8;
+// Eight columns a workgroup.  Every thread moves them and their factors to LDS
+// in the order of the elimination's steps (all loads in flight at once): slot s
+// of a direction holds its s-th row, after enough empty slots to make the
+// number of steps a multiple of eight.  Then 16 lanes, 8 columns x 2
+// directions, run all steps without a branch, the next eight steps' values in
+// registers; an empty slot leaves y = 0 and x is not read after it.
+// At 2048 x 255: 15 us; with the rows in place and the two directions'
+// last steps under a mask 27 us.
+constexpr int KC = 8, KSTEP = 8, KL = 2 * KC;
+struct ColSteps {
+    int mid, steps, pad_dn, pad_up;
+};
+__host__ __device__ inline ColSteps col_steps(int M) {
+    ColSteps c;
+    c.mid = (M + 1) / 2 - 1;  // 0-based
+    const int dn = c.mid, up = M - 1 - c.mid;
+    c.steps = ((dn > up ? dn : up) + KSTEP - 1) / KSTEP * KSTEP;
+    c.pad_dn = c.steps - dn;
+    c.pad_up = c.steps - up;
+    return c;
+}
+// LDS elements: [steps][F, g, 1/p][KL], then the middle row's F and 1/p
+inline size_t col_lds_elems(int M) { return size_t(col_steps(M).steps) * 3 * KL + 2 * KC; }
 
 template <typename T>
 __global__ void __launch_bounds__(256) k_columns(int N, int M, T *__restrict__ spec, const T *__restrict__ g,
                                                  const T *__restrict__ di) {
     extern __shared__ unsigned char lds_raw[];
-    T *F = reinterpret_cast<T *>(lds_raw), *Gs = F + size_t(M) * KC, *Ds = Gs + size_t(M) * KC;
-    const int q0 = blockIdx.x * KC, Nq = N / 2 + 1;
-    for (int t = threadIdx.x; t < M * KC; t += blockDim.x) {
-        const int j = t / KC, q = q0 + t % KC;
-        if (q < N) {
-            const int qq = min(q, N - q);
-            F[t] = spec[size_t(j) * N + q];
-            Gs[t] = g[size_t(j) * Nq + qq];
-            Ds[t] = di[size_t(j) * Nq + qq];
-        } else {
-            F[t] = Gs[t] = Ds[t] = T(0);
+    T *L = reinterpret_cast<T *>(lds_raw);
+    const ColSteps cs = col_steps(M);
+    T *Mid = L + size_t(cs.steps) * 3 * KL;
+    const int Nq = N / 2 + 1;
+    // columns past the last repeat it (never stored)
+    const int c = threadIdx.x % KC, q = min(int(blockIdx.x) * KC + c, N - 1), qq = min(q, N - q);
+    const int rstep = blockDim.x / KC;
+    // element of row j (0-based, not mid) in L
+    auto slot = [&](int j) {
+        return j < cs.mid ? (cs.pad_dn + j) * 3 * KL + c : (cs.pad_up + M - 1 - j) * 3 * KL + KC + c;
+    };
+    for (int j0 = threadIdx.x / KC; j0 < M; j0 += 8 * rstep) {
+        T vf[8], vg[8], vd[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int j = min(j0 + u * rstep, M - 1);
+            vf[u] = spec[size_t(j) * N + q];
+            vg[u] = g[size_t(j) * Nq + qq];
+            vd[u] = di[size_t(j) * Nq + qq];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int j = j0 + u * rstep;
+            if (j < M && j != cs.mid) {
+                T *p = L + slot(j);
+                p[0] = vf[u];
+                p[KL] = vg[u];
+                p[2 * KL] = vd[u];
+            } else if (j == cs.mid) {
+                Mid[c] = vf[u];
+                Mid[KC + c] = vd[u];
+            }
         }
     }
+    for (int t = threadIdx.x; t < cs.pad_dn * 3 * KL; t += blockDim.x)
+        if (t % KL < KC) L[t] = T(0);
+    for (int t = threadIdx.x; t < cs.pad_up * 3 * KL; t += blockDim.x)
+        if (t % KL >= KC) L[t] = T(0);
     __syncthreads();
-    if (threadIdx.x < 2 * KC) {
-        const int c = threadIdx.x % KC, up = threadIdx.x / KC;  // up: from the last row
-        const int mid = (M + 1) / 2 - 1;                        // 0-based here
-        const int cnt = up ? M - 1 - mid : mid, cmax = M - 1 - mid > mid ? M - 1 - mid : mid;
-        const int first = (up ? M - 1 : 0) * KC + c, inc = up ? -KC : KC;
+    if (threadIdx.x < KL) {
+        T *p = L + threadIdx.x;
         T y = T(0), gp = T(0);
-        T nf[KCHUNK], ng[KCHUNK], nd[KCHUNK];
-        auto fetch = [&](int s0) {
+        T nf[KSTEP], ng[KSTEP], nd[KSTEP];
 #pragma unroll
-            for (int u = 0; u < KCHUNK; u++) {
-                const int a = first + (s0 + u < cnt ? s0 + u : 0) * inc;
-                nf[u] = F[a];
-                ng[u] = Gs[a];
-                nd[u] = Ds[a];
-            }
-        };
-        fetch(0);
-        for (int s0 = 0; s0 < cmax; s0 += KCHUNK) {
-            T vf[KCHUNK], vg[KCHUNK], vd[KCHUNK];
+        for (int u = 0; u < KSTEP; u++) {
+            nf[u] = p[u * 3 * KL];
+            ng[u] = p[u * 3 * KL + KL];
+            nd[u] = p[u * 3 * KL + 2 * KL];
+        }
+        for (int s = 0; s < cs.steps; s += KSTEP, p += KSTEP * 3 * KL) {
+            T vf[KSTEP], vg[KSTEP], vd[KSTEP];
 #pragma unroll
-            for (int u = 0; u < KCHUNK; u++) {
+            for (int u = 0; u < KSTEP; u++) {
                 vf[u] = nf[u];
                 vg[u] = ng[u];
                 vd[u] = nd[u];
             }
-            fetch(s0 + KCHUNK);
+            // past the last step this reads the same eight again
+            const T *nx = s + KSTEP < cs.steps ? p + KSTEP * 3 * KL : p;
 #pragma unroll
-            for (int u = 0; u < KCHUNK; u++) {
-                if (s0 + u < cnt) {
-                    y = vf[u] + gp * y;
-                    gp = vg[u];
-                    F[first + (s0 + u) * inc] = y * vd[u];
-                }
+            for (int u = 0; u < KSTEP; u++) {
+                nf[u] = nx[u * 3 * KL];
+                ng[u] = nx[u * 3 * KL + KL];
+                nd[u] = nx[u * 3 * KL + 2 * KL];
             }
+#pragma unroll
+            for (int u = 0; u < KSTEP; u++) {
+                y = vf[u] + gp * y;
+                gp = vg[u];
+                vf[u] = y * vd[u];
+            }
+#pragma unroll
+            for (int u = 0; u < KSTEP; u++) p[u * 3 * KL] = vf[u];
         }
-        const T off = cnt > 0 ? gp * y : T(0);
-        const T other = __shfl_xor(off, KC, kWave);
+        const int col = threadIdx.x % KC;
+        const bool up = threadIdx.x >= KC;
+        const T off = gp * y, other = __shfl_xor(off, KC, kWave);
         // the same order of terms in both directions' lanes
-        T x = (F[mid * KC + c] + (up ? other : off) + (up ? off : other)) * Ds[mid * KC + c];
-        if (!up) F[mid * KC + c] = x;
-        // back: steps cnt-1 .. 0
-        auto fetch_back = [&](int s0) {
+        T x = (Mid[col] + (up ? other : off) + (up ? off : other)) * Mid[KC + col];
+        if (!up) Mid[col] = x;
+        p -= KSTEP * 3 * KL;
 #pragma unroll
-            for (int u = 0; u < KCHUNK; u++) {
-                const int s = cnt - 1 - (s0 + u);
-                const int a = first + (s > 0 ? s : 0) * inc;
-                nf[u] = F[a];
-                ng[u] = Gs[a];
-            }
-        };
-        fetch_back(0);
-        for (int s0 = 0; s0 < cmax; s0 += KCHUNK) {
-            T vf[KCHUNK], vg[KCHUNK];
+        for (int u = 0; u < KSTEP; u++) {
+            nf[u] = p[u * 3 * KL];
+            ng[u] = p[u * 3 * KL + KL];
+        }
+        for (int s = cs.steps; s > 0; s -= KSTEP, p -= KSTEP * 3 * KL) {
+            T vf[KSTEP], vg[KSTEP];
 #pragma unroll
-            for (int u = 0; u < KCHUNK; u++) {
+            for (int u = 0; u < KSTEP; u++) {
                 vf[u] = nf[u];
                 vg[u] = ng[u];
             }
-            fetch_back(s0 + KCHUNK);
+            const T *nx = s > KSTEP ? p - KSTEP * 3 * KL : p;
 #pragma unroll
-            for (int u = 0; u < KCHUNK; u++) {
-                const int s = cnt - 1 - (s0 + u);
-                if (s >= 0) {
-                    x = vf[u] + vg[u] * x;
-                    F[first + s * inc] = x;
-                }
+            for (int u = 0; u < KSTEP; u++) {
+                nf[u] = nx[u * 3 * KL];
+                ng[u] = nx[u * 3 * KL + KL];
             }
+#pragma unroll
+            for (int u = KSTEP - 1; u >= 0; u--) {
+                x = vf[u] + vg[u] * x;
+                vf[u] = x;
+            }
+#pragma unroll
+            for (int u = 0; u < KSTEP; u++) p[u * 3 * KL] = vf[u];
         }
     }
     __syncthreads();
-    for (int t = threadIdx.x; t < M * KC; t += blockDim.x) {
-        const int j = t / KC, q = q0 + t % KC;
-        if (q < N) spec[size_t(j) * N + q] = F[t];
-    }
+    if (int(blockIdx.x) * KC + c >= N) return;
+    for (int j = threadIdx.x / KC; j < M; j += rstep) spec[size_t(j) * N + q] = j == cs.mid ? Mid[c] : L[slot(j)];
 }
 
 // ---------------------------------------------------------------- residual
@@ -549,14 +610,14 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
         plan.tw_lds = 1;
         row_lds += 2 * size_t(N) * sizeof(T);
     }
-    col_lds = 3 * size_t(M) * KC * sizeof(T);
+    col_lds = col_lds_elems(M) * sizeof(T);
     if (row_lds > kLdsMax || col_lds > kLdsMax) return VVM_ERR_SIZE;
     if (!allow_lds(k_rows_fwd<T, false>, row_lds) || !allow_lds(k_rows_fwd<T, true>, row_lds) ||
         !allow_lds(k_rows_inv<T, false, false>, row_lds) || !allow_lds(k_rows_inv<T, true, false>, row_lds) ||
         !allow_lds(k_rows_inv<T, false, true>, row_lds) || !allow_lds(k_columns<T>, col_lds))
         return VVM_ERR_HIP;
     const size_t Nq = size_t(N) / 2 + 1;
-    tw = dalloc<T>(2 * size_t(N));
+    tw = dalloc<T>(4 * size_t(N));
     g = dalloc<T>(Nq * M);
     di = dalloc<T>(Nq * M);
     spec = dalloc<T>(size_t(N) * M);
@@ -564,11 +625,21 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
         destroy();
         return VVM_ERR_NOMEM;
     }
-    std::vector<T> t(2 * size_t(N));
+    std::vector<T> t(4 * size_t(N), T(0));
     for (int k = 0; k < N; k++) {
         const long double a = 2.0L * 3.14159265358979323846264338327950288L * k / N;
         t[2 * k] = T(std::cos(a));
         t[2 * k + 1] = T(-std::sin(a));
+    }
+    // the stages' twiddles, picked from those (r k < Ns R, so r k N / (Ns R) < N)
+    for (int s = 0, Ns = 1; s < plan.nst; Ns *= plan.radix[s++]) {
+        const int R = plan.radix[s], m = N / (Ns * R);
+        for (int r = 1; r < R; r++)
+            for (int k = 0; k < Ns; k++) {
+                const size_t a = 2 * (size_t(N) + Ns - 1 + size_t(r - 1) * Ns + k), b = 2 * size_t(r) * k * m;
+                t[a] = t[b];
+                t[a + 1] = t[b + 1];
+            }
     }
     if (hipMemcpy(tw, t.data(), t.size() * sizeof(T), hipMemcpyHostToDevice) != hipSuccess) return VVM_ERR_HIP;
     hipLaunchKernelGGL(k_factor<T>, dim3(unsigned((Nq + 63) / 64)), dim3(64), 0, nullptr, N, M, cx, cu, g, di);
