@@ -640,7 +640,8 @@ int Poisson::init(const Grid &G, const double *rhou, const double *rhow, const R
     if (hipHostGetDevicePointer(reinterpret_cast<void **>(&hpart_dev), hpart, 0) != hipSuccess) return VVM_ERR_HIP;
     if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return VVM_ERR_HIP;
     if (hipEventCreateWithFlags(&ev_res, hipEventDisableTiming) != hipSuccess) return VVM_ERR_HIP;
-    return VVM_OK;
+    // the zeroing of the allocations, before anything on the caller's stream
+    return hipStreamSynchronize(nullptr) == hipSuccess ? VVM_OK : VVM_ERR_HIP;
 }
 
 template <typename T>

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "poisson.h"
+#include "transfer.h"
 #include "vvm_internal.h"
 
 using namespace vvmd;
@@ -25,6 +26,7 @@ struct vvm_dev {
     std::string err;
 
     std::vector<void *> allocs;
+    HostLink link;  // host arrays <-> device planes
     double *prog[NPROG][3] = {};
     int idx_now = 0, idx_past = 1, idx_fut = 2;
     double *hist[NHIST][2] = {};
@@ -63,8 +65,6 @@ struct vvm_dev {
     bool p_alias_now = false;
     std::vector<double> h_thb_zeta;  // as uploaded (the step does not read it)
 
-    double *pinned = nullptr;  // nx*nz staging for the random kick
-    size_t pinned_n = 0;
     hipEvent_t ev[8] = {};
     // phase C (Kessler and its negative-value pass) runs on its own stream,
     // overlapping phase B (the elliptic solve): C reads and writes only th,
@@ -239,36 +239,28 @@ void rotate(vvm_dev *h) {
     h->p_alias_now = true;
 }
 
-// Host [i][k] (k fastest) -> device [k][i] with pitch, and back.
-void to_dev_layout(const Grid &G, const double *src, std::vector<double> &dst, int stride = 1, int off = 0) {
-    dst.assign(size_t(G.nz) * G.pitch, 0.);
-    for (int i = 0; i < G.nx; i++)
-        for (int k = 0; k < G.nz; k++) dst[size_t(k) * G.pitch + i] = src[(size_t(i) * G.nz + k) * stride + off];
+// Moves what has been listed in h->link.
+int send(vvm_dev *h) {
+    const int rc = h->link.upload(h->G, h->device, h->st);
+    return rc ? fail(h, rc, "copy to the device failed") : VVM_OK;
 }
-void from_dev_layout(const Grid &G, const std::vector<double> &src, double *dst, int stride = 1, int off = 0) {
-    for (int i = 0; i < G.nx; i++)
-        for (int k = 0; k < G.nz; k++) dst[(size_t(i) * G.nz + k) * stride + off] = src[size_t(k) * G.pitch + i];
-}
-
-int put2d(vvm_dev *h, double *d, const double *src, int stride = 1, int off = 0) {
-    std::vector<double> tmp;
-    to_dev_layout(h->G, src, tmp, stride, off);
-    HIPCHK(h, hipMemcpy(d, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice));
-    return VVM_OK;
-}
-int get2d(vvm_dev *h, const double *d, double *dst, int stride = 1, int off = 0) {
-    std::vector<double> tmp(size_t(h->G.nz) * h->G.pitch);
-    HIPCHK(h, hipMemcpy(tmp.data(), d, tmp.size() * sizeof(double), hipMemcpyDeviceToHost));
-    from_dev_layout(h->G, tmp, dst, stride, off);
-    return VVM_OK;
+int receive(vvm_dev *h) {
+    const int rc = h->link.download(h->G, h->device, h->st);
+    return rc ? fail(h, rc, "copy to the host failed") : VVM_OK;
 }
 
 // Per-level constants the kernels read instead of re-evaluating pow()
 // (host C library, the reference's own rounding).
-int upload_level_constants(vvm_dev *h, const vvm_host_view *v) {
+struct LevelConstants {
+    std::vector<double> vtfac, pcoef, rth, rz;
+    double precip_fac;
+};
+LevelConstants level_constants(vvm_dev *h, const vvm_host_view *v) {
     const vvm_dev_config &c = h->cfg;
     const int nz = c.nz;
-    std::vector<double> vtfac(nz, 0.), pcoef(nz, 0.), rth(nz, 0.), rz(nz, 0.);
+    const std::vector<double> zero(nz, 0.);
+    LevelConstants L{zero, zero, zero, zero, std::pow(v->rhou[1] / v->rhow[1], -0.5)};
+    auto &[vtfac, pcoef, rth, rz, precip_fac] = L;
     for (int k = 0; k < nz; k++) {
         vtfac[k] = std::pow(v->rhow[k] / v->rhow[1], -0.5);
         pcoef[k] = 380. / (std::pow(v->pib[k], c.Cp / c.Rd) * c.P0);
@@ -285,13 +277,7 @@ int upload_level_constants(vvm_dev *h, const vvm_host_view *v) {
             rz[k] = (c.CASE != 2) ? c.dt * cgz : 0.;
         }
     }
-    HIPCHK(h, hipMemcpy(h->P.vtfac, vtfac.data(), nz * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemcpy(h->P.pcoef, pcoef.data(), nz * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemcpy(h->P.rate_th, rth.data(), nz * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemcpy(h->P.rate_z, rz.data(), nz * sizeof(double), hipMemcpyHostToDevice));
-    const double pf = std::pow(v->rhou[1] / v->rhow[1], -0.5);
-    HIPCHK(h, hipMemcpy(h->s + S_PRECIP_FAC, &pf, sizeof(double), hipMemcpyHostToDevice));
-    return VVM_OK;
+    return L;
 }
 
 // FP64 from a guess: MG-PCG, whose iteration count tells what the guess is
@@ -491,6 +477,8 @@ int vvm_dev_create(const vvm_dev_config *cfg, int device, vvm_dev_t **out) {
     // streams to its few hardware queues in creation order, and a stream
     // created here but never used (ensemble members) would leave the members'
     // main streams on every other queue
+    // the zeroing of the allocations, before anything on the handle's own stream
+    ok = ok && hipStreamSynchronize(nullptr) == hipSuccess;
     if (!ok) {
         vvm_dev_destroy(h);
         return VVM_ERR_NOMEM;
@@ -507,7 +495,6 @@ void vvm_dev_destroy(vvm_dev_t *h) {
     diffusion_slots_release(h->dslots);
     if (h->pois_ready) h->pois.destroy();
     for (void *p : h->allocs) hipFree(p);
-    if (h->pinned) hipHostFree(h->pinned);
     if (h->kmax) hipHostFree(h->kmax);
     for (auto &e : h->ev)
         if (e) hipEventDestroy(e);
@@ -545,22 +532,19 @@ int vvm_dev_upload(vvm_dev_t *h, const vvm_host_view *v) {
     h->idx_now = 0;
     h->idx_past = 1;
     h->idx_fut = 2;
+    h->link.clear();
     const double *trip[NPROG][3] = {{v->zeta, v->zetam, v->zetap}, {v->th, v->thm, v->thp}, {v->qv, v->qvm, v->qvp},
                                     {v->qc, v->qcm, v->qcp},       {v->qr, v->qrm, v->qrp}};
     for (int f = 0; f < NPROG; f++)
         for (int s = 0; s < 3; s++) {
             if (!trip[f][s]) return fail(h, VVM_ERR_ARG, "upload: prognostic field missing");
-            int rc = put2d(h, h->prog[f][s], trip[f][s]);
-            if (rc) return rc;
+            h->link.field(trip[f][s], h->prog[f][s]);
         }
     const double *hv[NHIST] = {v->dth_advect, v->dth_buoyancy, v->dzeta_advect, v->dqv_advect,
                                v->dqc_advect, v->dqr_advect,   v->dqr_VT};
     for (int q = 0; q < NHIST; q++) {
         if (!hv[q]) return fail(h, VVM_ERR_ARG, "upload: AB2 history missing");
-        for (int s = 0; s < 2; s++) {
-            int rc = put2d(h, h->hist[q][s], hv[q], 2, s);
-            if (rc) return rc;
-        }
+        h->link.pair(hv[q], h->hist[q][0], h->hist[q][1]);
     }
     struct {
         const double *src;
@@ -575,8 +559,7 @@ int vvm_dev_upload(vvm_dev_t *h, const vvm_host_view *v) {
             if (e.required) return fail(h, VVM_ERR_ARG, "upload: u/w/RKM/RKH missing");
             continue;
         }
-        int rc = put2d(h, e.dst, e.src);
-        if (rc) return rc;
+        h->link.field(e.src, e.dst);
     }
     const int nx = h->G.nx, nz = h->G.nz;
     struct {
@@ -597,7 +580,7 @@ int vvm_dev_upload(vvm_dev_t *h, const vvm_host_view *v) {
                 continue;
             return fail(h, VVM_ERR_ARG, "upload: profile missing");
         }
-        HIPCHK(h, hipMemcpy(e.dst, e.src, e.n * sizeof(double), hipMemcpyHostToDevice));
+        h->link.line(e.src, e.dst, e.n);
     }
     if (v->thb_zeta) h->h_thb_zeta.assign(v->thb_zeta, v->thb_zeta + nz);
     double sc[NSCALAR] = {0.};
@@ -606,7 +589,13 @@ int vvm_dev_upload(vvm_dev_t *h, const vvm_host_view *v) {
     sc[S_UBARTOPM] = v->ubarTopm;
     sc[S_DUBAR0] = v->dubarTop_advect[0];
     sc[S_DUBAR1] = v->dubarTop_advect[1];
-    HIPCHK(h, hipMemcpy(h->s, sc, S_NEG_RATIO * sizeof(double), hipMemcpyHostToDevice));
+    h->link.line(sc, h->s, S_NEG_RATIO);
+    const LevelConstants lc = level_constants(h, v);
+    h->link.line(lc.vtfac.data(), h->P.vtfac, nz);
+    h->link.line(lc.pcoef.data(), h->P.pcoef, nz);
+    h->link.line(lc.rth.data(), h->P.rate_th, nz);
+    h->link.line(lc.rz.data(), h->P.rate_z, nz);
+    h->link.line(&lc.precip_fac, h->s + S_PRECIP_FAC, 1);
     // a + d of the diffusion sweep (k_diffusion.hip): K dt / dx^2 from the west,
     // K dt / dz^2 times a density ratio from below
     double ratio = 0.;
@@ -615,7 +604,7 @@ int vvm_dev_upload(vvm_dev_t *h, const vvm_host_view *v) {
             if (!(r <= ratio)) ratio = r;
     h->rho_per_k = h->cfg.dt * (h->G.rdx2 + h->G.rdz2 * ratio);
     h->diff_halo = diffusion_halo(20. * h->rho_per_k);  // twice the smallest K the closure gives
-    int rc = upload_level_constants(h, v);
+    int rc = send(h);
     if (rc) return rc;
     rc = ensure_poisson(h, v->rhou, v->rhow);
     if (rc) return rc;
@@ -632,39 +621,27 @@ int vvm_dev_download(vvm_dev_t *h, vvm_host_view *v) {
     if (!h || !v) return VVM_ERR_ARG;
     if (!h->uploaded) return fail(h, VVM_ERR_STATE, "download before upload");
     HIPCHK(h, hipSetDevice(h->device));
-    HIPCHK(h, hipStreamSynchronize(h->st));
+    h->link.clear();
     double *trip[NPROG][3] = {{v->zeta, v->zetam, v->zetap}, {v->th, v->thm, v->thp}, {v->qv, v->qvm, v->qvp},
                               {v->qc, v->qcm, v->qcp},       {v->qr, v->qrm, v->qrp}};
     const int order[3] = {h->idx_now, h->idx_past, h->p_alias_now ? h->idx_now : h->idx_fut};
     for (int f = 0; f < NPROG; f++)
         for (int s = 0; s < 3; s++)
-            if (trip[f][s]) {
-                int rc = get2d(h, h->prog[f][order[s]], trip[f][s]);
-                if (rc) return rc;
-            }
+            if (trip[f][s]) h->link.field(trip[f][s], h->prog[f][order[s]]);
     double *hv[NHIST] = {v->dth_advect, v->dth_buoyancy, v->dzeta_advect, v->dqv_advect,
                          v->dqc_advect, v->dqr_advect,   v->dqr_VT};
     for (int q = 0; q < NHIST; q++)
-        if (hv[q])
-            for (int s = 0; s < 2; s++) {
-                int rc = get2d(h, h->hist[q][s], hv[q], 2, s);
-                if (rc) return rc;
-            }
+        if (hv[q]) h->link.pair(hv[q], h->hist[q][0], h->hist[q][1]);
     struct {
-        double *dst;
-        const double *src;
+        double *dst, *src;
     } f2[] = {{v->u, h->u},           {v->w, h->w},           {v->RKM, h->RKM},         {v->RKH, h->RKH},
               {v->init_th_forcing, h->forcing}, {v->evaporation, h->evap}, {v->accretion, h->accr},
               {v->autoconversion, h->autoc}, {v->condensation, h->cond}};
     for (auto &e : f2)
-        if (e.dst) {
-            int rc = get2d(h, e.src, e.dst);
-            if (rc) return rc;
-        }
+        if (e.dst) h->link.field(e.dst, e.src);
     const int nx = h->G.nx, nz = h->G.nz;
     struct {
-        double *dst;
-        const double *src;
+        double *dst, *src;
         int n;
     } f1[] = {{v->precip, h->precip, nx}, {v->xi, h->xi, nx},          {v->uxi, h->uxi, nx},
               {v->rhou, h->P.rhou, nz},   {v->rhow, h->P.rhow, nz},    {v->pib, h->P.pib, nz},
@@ -674,7 +651,10 @@ int vvm_dev_download(vvm_dev_t *h, vvm_host_view *v) {
               {v->z, h->P.z, nz},         {v->z_zeta, h->P.z_zeta, nz}, {v->lambda2, h->P.lambda2, nz},
               {v->Q1LS, h->P.Q1LS, nz},   {v->Q2LS, h->P.Q2LS, nz}};
     for (auto &e : f1)
-        if (e.dst) HIPCHK(h, hipMemcpy(e.dst, e.src, e.n * sizeof(double), hipMemcpyDeviceToHost));
+        if (e.dst) h->link.line(e.dst, e.src, e.n);
+    double sc[S_NEG_RATIO];
+    h->link.line(sc, h->s, S_NEG_RATIO);
+    if (const int rc = receive(h)) return rc;
     if (v->thb_zeta) {
         if (h->stepped && v->thb) {
             // updateMean's thb_zeta (src/Iteration.cpp:80-84), not read by the step
@@ -685,8 +665,6 @@ int vvm_dev_download(vvm_dev_t *h, vvm_host_view *v) {
             std::copy(h->h_thb_zeta.begin(), h->h_thb_zeta.end(), v->thb_zeta);
         }
     }
-    double sc[S_NEG_RATIO];
-    HIPCHK(h, hipMemcpy(sc, h->s, sizeof(sc), hipMemcpyDeviceToHost));
     v->ubarTop = sc[S_UBARTOP];
     v->ubarTopp = sc[S_UBARTOPP];
     v->ubarTopm = sc[S_UBARTOPM];
@@ -723,30 +701,25 @@ static int host_microphysics(vvm_dev *h, const StepPtrs &S) {
                           &v.thvbm, &v.qvb, &v.qvb0, &v.qvsb, &v.z, &v.z_zeta, &v.lambda2, &v.Q1LS, &v.Q2LS};
         for (double **p : f1z) *p = take(G.nz);
     }
-    HIPCHK(h, hipStreamSynchronize(h->st));
+    h->link.clear();
     double *trip[NPROG][3] = {{v.zeta, v.zetam, v.zetap}, {v.th, v.thm, v.thp}, {v.qv, v.qvm, v.qvp},
                               {v.qc, v.qcm, v.qcp},       {v.qr, v.qrm, v.qrp}};
     for (int f = 0; f < NPROG; f++) {
-        const double *src[3] = {S.now[f], S.past[f], S.fut[f]};
-        for (int s = 0; s < 3; s++) {
-            int rc = get2d(h, src[s], trip[f][s]);
-            if (rc) return rc;
-        }
+        double *src[3] = {S.now[f], S.past[f], S.fut[f]};
+        for (int s = 0; s < 3; s++) h->link.field(trip[f][s], src[s]);
     }
-    const double *d2[] = {S.u, S.w, S.RKM, S.RKH, S.forcing, S.evap, S.accr, S.autoc, S.cond};
+    double *d2[] = {S.u, S.w, S.RKM, S.RKH, S.forcing, S.evap, S.accr, S.autoc, S.cond};
     double *h2[] = {v.u, v.w, v.RKM, v.RKH, v.init_th_forcing, v.evaporation, v.accretion, v.autoconversion,
                     v.condensation};
-    for (int q = 0; q < 9; q++) {
-        int rc = get2d(h, d2[q], h2[q]);
-        if (rc) return rc;
-    }
-    HIPCHK(h, hipMemcpy(v.precip, S.precip, G.nx * sizeof(double), hipMemcpyDeviceToHost));
-    const double *p1[] = {h->P.rhou, h->P.rhow, h->P.pib, h->P.pb, h->P.thb, h->P.thbm, h->P.thb_init,
+    for (int q = 0; q < 9; q++) h->link.field(h2[q], d2[q]);
+    h->link.line(v.precip, S.precip, G.nx);
+    double *p1[] = {h->P.rhou, h->P.rhow, h->P.pib, h->P.pb, h->P.thb, h->P.thbm, h->P.thb_init,
                           h->P.thb_zeta, h->P.thvb, h->P.thvbm, h->P.qvb, h->P.qvb0, h->P.qvsb, h->P.z,
                           h->P.z_zeta, h->P.lambda2, h->P.Q1LS, h->P.Q2LS};
     double *h1[] = {v.rhou, v.rhow, v.pib, v.pb, v.thb, v.thbm, v.thb_init, v.thb_zeta, v.thvb,
                     v.thvbm, v.qvb, v.qvb0, v.qvsb, v.z, v.z_zeta, v.lambda2, v.Q1LS, v.Q2LS};
-    for (int q = 0; q < 18; q++) HIPCHK(h, hipMemcpy(h1[q], p1[q], G.nz * sizeof(double), hipMemcpyDeviceToHost));
+    for (int q = 0; q < 18; q++) h->link.line(h1[q], p1[q], G.nz);
+    if (const int rc = receive(h)) return rc;
     v.step = h->step;
     v.status_for_adding_forcing = h->status_for_adding_forcing;
     const int urc = h->mp_fn(h->mp_user, &v);
@@ -754,10 +727,9 @@ static int host_microphysics(vvm_dev *h, const StepPtrs &S) {
     const double *back[] = {v.thp, v.qvp, v.qcp, v.qrp, v.evaporation, v.accretion, v.autoconversion,
                             v.condensation};
     double *dst[] = {S.fut[F_TH], S.fut[F_QV], S.fut[F_QC], S.fut[F_QR], S.evap, S.accr, S.autoc, S.cond};
-    for (int q = 0; q < 8; q++) {
-        int rc = put2d(h, dst[q], back[q]);
-        if (rc) return rc;
-    }
+    h->link.clear();
+    for (int q = 0; q < 8; q++) h->link.field(back[q], dst[q]);
+    if (const int rc = send(h)) return rc;
     launch_bc_all_prog(G, S, h->st);
     return VVM_OK;
 }
@@ -776,11 +748,9 @@ static int upload_random_kick(vvm_dev *h) {
     v.init_th_forcing = host.data();
     int rc = vvm_random_perturbation(&h->cfg, &v, h->step + 0, -0.001, 0.001, 1.);
     if (rc) return fail(h, rc, "random perturbation failed");
-    std::vector<double> tmp;
-    to_dev_layout(h->G, host.data(), tmp);
-    HIPCHK(h, hipMemcpyAsync(h->forcing, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice, h->st));
-    HIPCHK(h, hipStreamSynchronize(h->st));
-    return VVM_OK;
+    h->link.clear();
+    h->link.field(host.data(), h->forcing);
+    return send(h);
 }
 
 int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
@@ -1254,9 +1224,11 @@ int vvm_dev_set_radiation(vvm_dev_t *h, const double *heating_rate, int cooling)
         if (!h->rad) {
             h->rad = dev_alloc(h, size_t(h->G.nz) * h->G.pitch);
             if (!h->rad) return fail(h, VVM_ERR_NOMEM, "radiation rate");
+            HIPCHK(h, hipStreamSynchronize(nullptr));  // its zeroing
         }
-        const int rc = put2d(h, h->rad, heating_rate);
-        if (rc) return rc;
+        h->link.clear();
+        h->link.field(heating_rate, h->rad);
+        if (const int rc = send(h)) return rc;
     }
     h->rad_on = heating_rate != nullptr;
     h->radcool = cooling;
