@@ -21,7 +21,7 @@
 // Weight-gradient kernel (k_conv_wgrad): one wavefront per tap; the GEMM
 // runs over pixels (K) with the input tile and the output gradient staged
 // channel-major in LDS; partial sums per workgroup are reduced by
-// k_wgrad_reduce.
+// k_wgrad_reduce.  All layers in one launch of each, after the data gradients.
 #include <algorithm>
 #include <mutex>
 #include <cstdint>
@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(256) k_conv(NetGeo g, const __bf16 *__restrict
     double sc[3];
     if (IN == 1) {
 #pragma unroll
-        for (int c = 0; c < 3; c++) sc[c] = inv_rms(fin.sumsq[c], fin.npts);
+        for (int c = 0; c < 3; c++) sc[c] = fin.sumsq ? inv_rms(fin.sumsq[c], fin.npts) : 1.;
     }
     const long hw = long(g.h) * g.w;
     bf16x8 pf[IN == 0 ? NPF : 1];     // IN 0: prefetched chunks
@@ -341,81 +341,145 @@ __global__ void __launch_bounds__(256) k_conv_pair(NetGeo g, const __bf16 *__res
     }
 }
 
-// Weight gradient of one layer: dW[co][ci][t] = sum_p dZ[p][co] X[p + off_t][ci]
-// and db[co] = sum_p dZ[p][co].  Workgroup = 9 wavefronts (one per tap),
-// grid-stride over 64 x 2 tiles; per-workgroup partials [blk][9][32 ci][32 co]
-// then 32 bias sums.
-__global__ void __launch_bounds__(576) k_conv_wgrad(NetGeo g, const __bf16 *__restrict__ x,
-                                                    const __bf16 *__restrict__ dz, float *__restrict__ partial) {
-    __shared__ __attribute__((aligned(16))) __bf16 xt[NET_C][HH * HW + 8];  // channel-major haloed input
-    __shared__ __attribute__((aligned(16))) __bf16 dzt[NET_C][TH * TW];     // channel-major output gradient
-    const int lane = threadIdx.x & 63, t = threadIdx.x >> 6;
+// Weight gradients of all layers: dW[co][ci][t] = sum_p dZ[p][co] X[p + off_t][ci]
+// and db[co] = sum_p dZ[p][co].  Workgroup (k, l): 9 wavefronts (one per tap),
+// every gridDim.x-th 64 x 2 tile of layer l; per-workgroup partials
+// [l][k][9][32 ci][32 co] then 32 bias sums.
+//
+// The GEMM runs over pixels, so both operands need eight consecutive pixels of
+// one channel a lane, and tensors are pixel-major.  A thread fetches eight
+// pixels x eight channels (eight 16-byte loads, one tile ahead), transposes
+// them in registers and writes eight 16-byte runs to channel-major LDS tiles
+// (an odd number of 16-byte units a channel: no bank conflicts).  The input
+// tile starts at column x0 - 1, so the taps' runs start 0, 1 or 2 pixels
+// after a 16-byte boundary: one 16-byte and one 4-byte read, shifted in
+// registers.  Staging element by element and reading shifted runs as eight
+// 2-byte reads bound the kernel: 16 x 64 x 64 pixels, 52 us a layer, 300 us
+// the six; now 46 us for the six in one launch.
+constexpr int WP = TW + 8;                        // input tile row: 66 pixels in runs of 8
+constexpr int WXS = HH * WP + 8, WDS = TH * TW + 8;  // LDS elements a channel
+constexpr int WXB = HH * (WP / 8) * 4, WDB = TH * (TW / 8) * 4;  // 8 x 8 blocks to stage, one a thread
+
+__global__ void __launch_bounds__(576) k_conv_wgrad(NetGeo g, NetWgrad L, float *__restrict__ partial) {
+    __shared__ __attribute__((aligned(16))) __bf16 xt[NET_C * WXS];
+    __shared__ __attribute__((aligned(16))) __bf16 dzt[NET_C * WDS];
+    const __bf16 *__restrict__ x = L.x[blockIdx.y], *__restrict__ dz = L.dz[blockIdx.y];
+    const int lane = threadIdx.x & 63, t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int dy = t / 3 - 1, dx = t % 3 - 1;
     const int gk = lane >> 5, ch = lane & 31;
     const int tx_n = (g.w + TW - 1) / TW, ty_n = (g.h + TH - 1) / TH;
     const long ntile = long(tx_n) * ty_n * g.nb;
+    // this thread's block of the staging: of the input, of the gradient, or none
+    const bool is_x = threadIdx.x < WXB, is_d = !is_x && threadIdx.x < WXB + WDB;
+    const int id = is_x ? threadIdx.x : threadIdx.x - WXB, part = id & 3;
+    const int runs = is_x ? WP / 8 : TW / 8, row = (id >> 2) / runs, run = (id >> 2) % runs;
+    bf16x8 v[8];
+    auto fetch = [&](long tile) {
+        const int b = int(tile / (long(tx_n) * ty_n)), rem = int(tile % (long(tx_n) * ty_n));
+        const int y0 = (rem / tx_n) * TH, x0 = (rem % tx_n) * TW;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            v[e] = bf16x8{};
+            const int c = run * 8 + e;
+            if (is_x) {
+                const long src = c < HW ? halo_src(g, b, y0, x0, row, c) : -1;
+                if (src >= 0) v[e] = *reinterpret_cast<const bf16x8 *>(x + src * NET_C + part * 8);
+            } else if (is_d && y0 + row < g.h && x0 + c < g.w) {
+                const long src = (long(b) * g.h + y0 + row) * g.w + x0 + c;
+                v[e] = *reinterpret_cast<const bf16x8 *>(dz + src * NET_C + part * 8);
+            }
+        }
+    };
+    __bf16 *dst0 = is_x ? xt + part * 8 * WXS + row * WP + run * 8 : dzt + part * 8 * WDS + row * TW + run * 8;
+    const int dst_ch = is_x ? WXS : WDS;
     f32x16 acc = {};
     float bsum = 0.f;
-    for (long tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
-        const int b = int(tile / (long(tx_n) * ty_n));
-        const int rem = int(tile % (long(tx_n) * ty_n));
-        const int y0 = (rem / tx_n) * TH, x0 = (rem % tx_n) * TW;
+    long tile = blockIdx.x;
+    if (tile < ntile) fetch(tile);
+    for (; tile < ntile; tile += gridDim.x) {
         __syncthreads();  // the previous tile's reads are done
-        for (int c = threadIdx.x; c < HH * HW * NET_C; c += blockDim.x) {
-            const int px = c / NET_C, ci = c % NET_C;
-            const long src = halo_src(g, b, y0, x0, px / HW, px % HW);
-            xt[ci][px] = (src >= 0) ? x[src * NET_C + ci] : to_bf16(0.f);
-        }
-        for (int c = threadIdx.x; c < TH * TW * NET_C; c += blockDim.x) {
-            const int px = c / NET_C, co = c % NET_C;
-            const int yy = y0 + px / TW, xx = x0 + px % TW;
-            __bf16 v = to_bf16(0.f);
-            if (yy < g.h && xx < g.w) v = dz[((long(b) * g.h + yy) * g.w + xx) * NET_C + co];
-            dzt[co][px] = v;
+        if (is_x || is_d) {
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                bf16x8 o;
+#pragma unroll
+                for (int e = 0; e < 8; e++) o[e] = v[e][c];
+                *reinterpret_cast<bf16x8 *>(dst0 + c * dst_ch) = o;
+            }
         }
         __syncthreads();
+        if (tile + gridDim.x < ntile) fetch(tile + gridDim.x);
 #pragma unroll
         for (int kk = 0; kk < TH * TW / 16; kk++) {
             const int ty = kk / (TW / 16), c0 = (kk % (TW / 16)) * 16 + 8 * gk;
-            bf16x8 a, bb;
-            const int base = (ty + 1 + dy) * HW + c0 + 1 + dx;
+            const __bf16 *src = xt + ch * WXS + (ty + 1 + dy) * WP + c0;
+            union {
+                bf16x8 v;
+                unsigned u[4];
+            } q, a;
+            q.v = *reinterpret_cast<const bf16x8 *>(src);
+            const unsigned r = *reinterpret_cast<const unsigned *>(src + 8);
+            if (dx < 0) {
+                a.v = q.v;
+            } else if (dx == 0) {
+                a.u[0] = __builtin_amdgcn_alignbit(q.u[1], q.u[0], 16);
+                a.u[1] = __builtin_amdgcn_alignbit(q.u[2], q.u[1], 16);
+                a.u[2] = __builtin_amdgcn_alignbit(q.u[3], q.u[2], 16);
+                a.u[3] = __builtin_amdgcn_alignbit(r, q.u[3], 16);
+            } else {
+                a.u[0] = q.u[1];
+                a.u[1] = q.u[2];
+                a.u[2] = q.u[3];
+                a.u[3] = r;
+            }
+            const bf16x8 bb = *reinterpret_cast<const bf16x8 *>(dzt + ch * WDS + ty * TW + c0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, bb, acc, 0, 0, 0);
+            if (t == 0) {
 #pragma unroll
-            for (int e = 0; e < 8; e++) a[e] = xt[ch][base + e];
-            bb = *reinterpret_cast<const bf16x8 *>(&dzt[ch][ty * TW + c0]);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bb, acc, 0, 0, 0);
+                for (int e = 0; e < 8; e++) bsum += from_bf16(bb[e]);
+            }
         }
-        if (t == 0 && lane < NET_C)
-            for (int px = 0; px < TH * TW; px++) bsum += from_bf16(dzt[lane][px]);
     }
     // D[m][n]: m = ci, n = co
-    float *dst = partial + size_t(blockIdx.x) * NET_WGRAD_PARTIAL;
+    float *dst = partial + (size_t(blockIdx.y) * gridDim.x + blockIdx.x) * NET_WGRAD_PARTIAL;
 #pragma unroll
     for (int r = 0; r < 16; r++) {
         const int ci = 8 * (r >> 2) + 4 * gk + (r & 3), co = lane & 31;
         dst[(t * NET_C + ci) * NET_C + co] = acc[r];
     }
-    if (t == 0 && lane < NET_C) dst[NET_T * NET_C * NET_C + lane] = bsum;
+    if (t == 0) {
+        bsum += __shfl_xor(bsum, 32, 64);
+        if (lane < NET_C) dst[NET_T * NET_C * NET_C + lane] = bsum;
+    }
 }
 
-// grad[co][ci][t] and grad bias from nblk partials; masked entries (frozen
-// weights) stay zero.
-__global__ void k_wgrad_reduce(const float *__restrict__ partial, int nblk, float *__restrict__ grad, int layer) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= NET_LAYER_PARAMS) return;
-    int src;
-    bool live;
-    if (e < NET_C * NET_C * NET_T) {
-        const int co = e / (NET_C * NET_T), ci = (e / NET_T) % NET_C, t = e % NET_T;
-        src = (t * NET_C + ci) * NET_C + co;
-        live = !(layer == 0 && ci >= NET_CIN) && !(layer == NET_L - 1 && co >= 1);
-    } else {
-        const int co = e - NET_C * NET_C * NET_T;
-        src = NET_T * NET_C * NET_C + co;
-        live = !(layer == NET_L - 1 && co >= 1);
-    }
+// grad[l][co][ci][t] and grad bias from nblk partials; masked entries (frozen
+// weights) stay zero.  A thread adds every fourth partial of one value, in the
+// partials' order, so that neighbouring threads read neighbouring values (one
+// thread a parameter, in the parameters' order, took 44 us a layer).  hgrad: a
+// copy in host-mapped memory, if set.
+__global__ void __launch_bounds__(256) k_wgrad_reduce(const float *__restrict__ partial, int nblk,
+                                                      float *__restrict__ grad, float *__restrict__ hgrad) {
+    __shared__ double sh[4][64];
+    const int lane = threadIdx.x & 63, part = threadIdx.x >> 6, layer = blockIdx.y;
+    const int src = blockIdx.x * 64 + lane;
     double s = 0.;
-    for (int k = 0; k < nblk; k++) s += partial[size_t(k) * NET_WGRAD_PARTIAL + src];
-    grad[size_t(layer) * NET_LAYER_PARAMS + e] = live ? float(s) : 0.f;
+    if (src < NET_WGRAD_PARTIAL) {
+        const float *p = partial + size_t(layer) * nblk * NET_WGRAD_PARTIAL + src;
+#pragma unroll 8
+        for (int k = part; k < nblk; k += 4) s += p[size_t(k) * NET_WGRAD_PARTIAL];
+    }
+    sh[part][lane] = s;
+    __syncthreads();
+    if (part != 0 || src >= NET_WGRAD_PARTIAL) return;
+    s = sh[0][lane] + sh[1][lane] + sh[2][lane] + sh[3][lane];
+    const bool bias = src >= NET_T * NET_C * NET_C;
+    const int co = src % NET_C, ci = (src / NET_C) % NET_C, t = src / (NET_C * NET_C);
+    const int e = bias ? NET_C * NET_C * NET_T + co : (co * NET_C + ci) * NET_T + t;
+    const bool live = !(layer == 0 && !bias && ci >= NET_CIN) && !(layer == NET_L - 1 && co >= 1);
+    const float v = live ? float(s) : 0.f;
+    grad[size_t(layer) * NET_LAYER_PARAMS + e] = v;
+    if (hgrad) hgrad[size_t(layer) * NET_LAYER_PARAMS + e] = v;
 }
 
 // Pack bf16 weights in the lane order of the MFMA B operand.
@@ -622,11 +686,11 @@ void net_conv_bwd(const NetGeo &g, const __bf16 *dz, const __bf16 *wpk_bwd, cons
     conv<2>(g, dz, wpk_bwd, nullptr, dzbelow, nullptr, nullptr, zbelow, NetFeatIn{}, NetApply{}, st);
 }
 
-void net_wgrad(const NetGeo &g, const __bf16 *x, const __bf16 *dz, float *partial, int nblk, float *grad, int layer,
+void net_wgrad(const NetGeo &g, const NetWgrad &L, float *partial, int nblk, float *grad, float *hgrad,
                hipStream_t st) {
-    hipLaunchKernelGGL(k_conv_wgrad, dim3(nblk), dim3(576), 0, st, g, x, dz, partial);
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3((NET_LAYER_PARAMS + 255) / 256), dim3(256), 0, st, partial, nblk, grad,
-                       layer);
+    hipLaunchKernelGGL(k_conv_wgrad, dim3(nblk, NET_L), dim3(576), 0, st, g, L, partial);
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3((NET_WGRAD_PARTIAL + 63) / 64, NET_L), dim3(256), 0, st, partial, nblk,
+                       grad, hgrad);
 }
 
 void net_loss(long n, const float *out, const float *target, const float *mask, float inv_msum, __bf16 *dz,

@@ -41,7 +41,7 @@ void net_gather(int nb, int ch, int cw, int margin, const CropDesc *d, float *fe
                 hipStream_t st);
 // Inference ends of the network fused with the guess: the first layer
 // reads the three raw FP32 feature planes and scales feature c by
-// 1/RMS = 1/sqrt(sumsq[c]/npts); the last layer writes the guess
+// 1/RMS = 1/sqrt(sumsq[c]/npts) (by 1 without sumsq); the last layer writes the guess
 // x = xe + sqrt(sumsq[1]/npts) * out straight into the solver's unknown
 // (row y of the network is row y+1 of x, N columns), xe the extrapolation
 // of the previous solutions (extrap_at).
@@ -83,7 +83,13 @@ void net_conv_bwd(const NetGeo &g, const __bf16 *dz, const __bf16 *wpk_bwd, cons
 // two hidden layers in one pass (inference only: no pre-activations kept)
 void net_conv_pair(const NetGeo &g, const __bf16 *in, const __bf16 *wa, const float *ba, const __bf16 *wb,
                    const float *bb, __bf16 *out, hipStream_t st);
-void net_wgrad(const NetGeo &g, const __bf16 *x, const __bf16 *dz, float *partial, int nblk, float *grad, int layer,
+// each layer's input and pre-activation gradient
+struct NetWgrad {
+    const __bf16 *x[NET_L], *dz[NET_L];
+};
+// grad of every layer (and a copy in hgrad, host-mapped, if set); partial:
+// NET_L * nblk * NET_WGRAD_PARTIAL floats
+void net_wgrad(const NetGeo &g, const NetWgrad &L, float *partial, int nblk, float *grad, float *hgrad,
                hipStream_t st);
 void net_loss(long n, const float *out, const float *target, const float *mask, float inv_msum, __bf16 *dz,
               double *lpart, hipStream_t st);
@@ -114,9 +120,10 @@ class GuessNet {
     // out[nb][h][w] (device fp32) from feat[nb][3][h][w] (device fp32), on
     // stream s (the network's own stream when null)
     int forward(const NetGeo &g, const float *feat, float *out, bool keep, hipStream_t s = nullptr);
-    // loss and parameter gradient (into grad) for the last forward with keep
+    // loss and parameter gradient (into grad, and to hgrad on the host if set)
+    // for the last forward with keep; waits only where loss or hgrad is set
     int backward(const NetGeo &g, const float *out, const float *target, const float *mask, double msum,
-                 double *loss);
+                 double *loss, float *hgrad = nullptr);
     void adam_step(float lr, float b1 = 0.9f, float b2 = 0.999f, float eps = 1e-8f);
     void repack();  // bf16 copies after the fp32 parameters changed
     void reset_adam();
@@ -131,10 +138,13 @@ class GuessNet {
     bool cap_train = false;
     __bf16 *act[NET_L] = {};   // X0 (input), A1..A5
     __bf16 *zpre[NET_L] = {};  // Z1..Z5 (training)
-    __bf16 *dz[2] = {};        // pre-activation gradients (ping-pong)
+    __bf16 *dz[NET_L] = {};    // pre-activation gradients (training)
     float *partial = nullptr;  // weight-gradient partials
     double *lpart = nullptr;   // loss partials
-    double *hloss = nullptr;   // pinned
+    // mapped pinned memory: the loss kernel's partials and the gradient go there
+    // directly where the host wants them
+    double *hloss = nullptr, *hloss_dev = nullptr;
+    float *hgrad_buf = nullptr, *hgrad_dev = nullptr;
     int nblk_wgrad = 128;
 };
 

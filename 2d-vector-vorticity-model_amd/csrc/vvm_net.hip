@@ -32,10 +32,15 @@ int GuessNet::init(int device, hipStream_t stream) {
     v = dmalloc<float>(NET_PARAMS);
     wf = dmalloc<__bf16>(size_t(NET_L) * NET_PACK);
     wb = dmalloc<__bf16>(size_t(NET_L) * NET_PACK);
-    partial = dmalloc<float>(size_t(nblk_wgrad) * NET_WGRAD_PARTIAL);
+    partial = dmalloc<float>(size_t(NET_L) * nblk_wgrad * NET_WGRAD_PARTIAL);
     if (!params || !grad || !m || !v || !wf || !wb || !partial) return VVM_ERR_NOMEM;
-    if (hipHostMalloc(reinterpret_cast<void **>(&hloss), sizeof(double) * 4096, hipHostMallocDefault) != hipSuccess)
+    const unsigned mapped = hipHostMallocMapped | hipHostMallocCoherent;
+    if (hipHostMalloc(reinterpret_cast<void **>(&hloss), sizeof(double) * 4096, mapped) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&hgrad_buf), sizeof(float) * NET_PARAMS, mapped) != hipSuccess)
         return VVM_ERR_NOMEM;
+    if (hipHostGetDevicePointer(reinterpret_cast<void **>(&hloss_dev), hloss, 0) != hipSuccess ||
+        hipHostGetDevicePointer(reinterpret_cast<void **>(&hgrad_dev), hgrad_buf, 0) != hipSuccess)
+        return VVM_ERR_HIP;
     hipMemsetAsync(params, 0, sizeof(float) * NET_PARAMS, st);
     hipMemsetAsync(grad, 0, sizeof(float) * NET_PARAMS, st);
     reset_adam();
@@ -51,10 +56,11 @@ void GuessNet::reset_adam() {
 void GuessNet::destroy() {
     if (st) hipStreamSynchronize(st);
     void *ps[] = {params, grad, m, v, wf, wb, partial, lpart, act[0], act[1], act[2], act[3], act[4], act[5],
-                  zpre[0], zpre[1], zpre[2], zpre[3], zpre[4], zpre[5], dz[0], dz[1]};
+                  zpre[0], zpre[1], zpre[2], zpre[3], zpre[4], zpre[5], dz[0], dz[1], dz[2], dz[3], dz[4], dz[5]};
     for (void *p : ps)
         if (p) hipFree(p);
     if (hloss) hipHostFree(hloss);
+    if (hgrad_buf) hipHostFree(hgrad_buf);
     *this = GuessNet();
 }
 
@@ -163,17 +169,19 @@ int GuessNet::forward(const NetGeo &g, const float *feat, float *out, bool keep,
     int rc = reserve(npx, keep);
     if (rc) return rc;
     const hipStream_t st = s ? s : this->st;
-    net_pack_input(g, feat, act[0], st);
     if (!keep) {  // inference: activations alternate between act[0] and act[1]
-        int cur = 0;
-        for (int l = 0; l < NET_L - 1;) {
-            l += hidden_step(g, l, act[cur], act[cur ^ 1], st, l > 0);
+        // the first layer takes the feature planes as they are
+        int cur = 1;
+        net_conv_first_features(g, NetFeatIn{feat, nullptr, 1.}, wf, params + NET_C * NET_C * NET_T, act[1], st);
+        for (int l = 1; l < NET_L - 1;) {
+            l += hidden_step(g, l, act[cur], act[cur ^ 1], st);
             cur ^= 1;
         }
         net_conv_last(g, act[cur], wf + size_t(NET_L - 1) * NET_PACK,
                       params + size_t(NET_L - 1) * NET_LAYER_PARAMS + NET_C * NET_C * NET_T, out, st);
         return hipGetLastError() == hipSuccess ? VVM_OK : VVM_ERR_HIP;
     }
+    net_pack_input(g, feat, act[0], st);
     for (int l = 0; l < NET_L; l++) {
         const __bf16 *wl = wf + size_t(l) * NET_PACK;
         const float *bl = params + size_t(l) * NET_LAYER_PARAMS + NET_C * NET_C * NET_T;
@@ -186,23 +194,24 @@ int GuessNet::forward(const NetGeo &g, const float *feat, float *out, bool keep,
 }
 
 int GuessNet::backward(const NetGeo &g, const float *out, const float *target, const float *mask, double msum,
-                       double *loss) {
+                       double *loss, float *hgrad) {
     const long npx = long(g.nb) * g.h * g.w;
     if (!cap_train || npx > cap) return VVM_ERR_STATE;
     const int nlb = int((npx + 255) / 256);
-    net_loss(npx, out, target, mask, float(1.0 / msum), dz[0], lpart, st);
-    int cur = 0;
-    for (int l = NET_L - 1; l >= 0; l--) {
-        // layer l+1 of the network: input act[l], pre-activation gradient dz[cur]
-        net_wgrad(g, act[l], dz[cur], partial, nblk_wgrad, grad, l, st);
-        if (l == 0) break;
-        net_conv_bwd(g, dz[cur], wb + size_t(l) * NET_PACK, zpre[l], dz[cur ^ 1], st);
-        cur ^= 1;
+    if (loss && nlb > 4096) return VVM_ERR_SIZE;
+    // dz[l]: the gradient of the pre-activation that layer l+1 of the network
+    // (input act[l]) forms
+    net_loss(npx, out, target, mask, float(1.0 / msum), dz[NET_L - 1], loss ? hloss_dev : lpart, st);
+    for (int l = NET_L - 1; l > 0; l--) net_conv_bwd(g, dz[l], wb + size_t(l) * NET_PACK, zpre[l], dz[l - 1], st);
+    NetWgrad L;
+    for (int l = 0; l < NET_L; l++) {
+        L.x[l] = act[l];
+        L.dz[l] = dz[l];
     }
+    net_wgrad(g, L, partial, nblk_wgrad, grad, hgrad ? hgrad_dev : nullptr, st);
+    if ((loss || hgrad) && hipStreamSynchronize(st) != hipSuccess) return VVM_ERR_HIP;
+    if (hgrad) std::memcpy(hgrad, hgrad_buf, sizeof(float) * NET_PARAMS);
     if (loss) {
-        if (nlb > 4096) return VVM_ERR_SIZE;
-        hipMemcpyAsync(hloss, lpart, sizeof(double) * nlb, hipMemcpyDeviceToHost, st);
-        if (hipStreamSynchronize(st) != hipSuccess) return VVM_ERR_HIP;
         double s = 0.;
         for (int i = 0; i < nlb; i++) s += hloss[i];
         *loss = s / msum;
@@ -367,20 +376,22 @@ int vvm_net_grad_host(vvm_net_t *n, int nb, int h, int w, int periodic, const fl
     const long npx = long(nb) * h * w;
     int rc = stage(n, npx);
     if (rc) return rc;
-    double msum = 0.;
-    for (long i = 0; i < npx; i++) msum += mask[i];
-    if (msum <= 0.) msum = 1.;
     hipMemcpyAsync(n->dfeat, input, sizeof(float) * 3 * npx, hipMemcpyHostToDevice, n->st);
-    hipMemcpyAsync(n->dtgt, target, sizeof(float) * npx, hipMemcpyHostToDevice, n->st);
-    hipMemcpyAsync(n->dmask, mask, sizeof(float) * npx, hipMemcpyHostToDevice, n->st);
     const NetGeo g{nb, h, w, periodic};
     rc = n->net.forward(g, n->dfeat, n->dout, true);
     if (rc) return nfail(n, rc, "forward failed");
+    // the mask's sum (four chains: one is bound by the latency of its additions)
+    // and the other copies while the forward pass runs
+    double ms[4] = {0., 0., 0., 0.};
+    for (long i = 0; i < npx; i++) ms[i & 3] += mask[i];
+    double msum = (ms[0] + ms[1]) + (ms[2] + ms[3]);
+    if (msum <= 0.) msum = 1.;
+    hipMemcpyAsync(n->dtgt, target, sizeof(float) * npx, hipMemcpyHostToDevice, n->st);
+    hipMemcpyAsync(n->dmask, mask, sizeof(float) * npx, hipMemcpyHostToDevice, n->st);
     double l = 0.;
-    rc = n->net.backward(g, n->dout, n->dtgt, n->dmask, msum, &l);
+    rc = n->net.backward(g, n->dout, n->dtgt, n->dmask, msum, &l, grad);
     if (rc) return nfail(n, rc, "backward failed");
     if (loss) *loss = l;
-    if (grad) return vvm_net_get_grad(n, grad);
     return VVM_OK;
 }
 

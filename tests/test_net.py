@@ -274,3 +274,24 @@ def test_learned_guess_gain():
           f"{s_le.guess_skipped}, of 48", flush=True)
     assert s_le.solve_iters_total < s_ex.solve_iters_total, (s_le.solve_iters_total, s_ex.solve_iters_total)
     assert s_le.solve_iters_total <= s_q.solve_iters_total, (s_le.solve_iters_total, s_q.solve_iters_total)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,periodic", [((1, 1, 1), True), ((2, 3, 5), True), ((1, 5, 63), False),
+                                            ((3, 2, 64), True), ((2, 7, 65), False), ((1, 2, 130), True),
+                                            ((20, 16, 48), False)])
+def test_device_gradient_tile_edges(oracle, shape, periodic):
+    """The weight-gradient kernel's 64 x 2 tiles cut at any width and height,
+    fewer tiles than workgroups and more, every layer against the oracle at
+    the bar of bf16 operands summed in another order (all parameters at once:
+    a layer's gradient on a handful of pixels has no norm to speak of)."""
+    nb, h, w = shape
+    p = random_params(50 + h + w)
+    inp, tgt, mask = sample(51 + w, nb, h, w)
+    lw, gw = oracle.net_grad(p, inp, tgt, mask, periodic)
+    print(f"net gradient {shape} periodic={periodic}", flush=True)
+    with V.Net() as net:
+        net.set_params(p)
+        lg, gg = net.grad(inp, tgt, mask, periodic)
+    assert abs(lg - lw) <= 1e-2 * abs(lw)
+    assert rel(gg, gw) <= GRAD_TOL, rel(gg, gw)
