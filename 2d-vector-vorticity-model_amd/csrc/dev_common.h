@@ -22,24 +22,40 @@ struct Grid {
 
 __host__ __device__ inline size_t ix(const Grid &G, int i, int k) { return size_t(k) * G.pitch + i; }
 
+// Element (i,k) of a field, addressed as a row pointer plus a 32-bit byte
+// offset.  Where k is the same for a whole wavefront (uniform), the row pointer
+// stays in scalar registers and one vector register holds the offset for every
+// field; with a 64-bit index per access half of a stencil kernel's vector
+// instructions were address arithmetic.
+__device__ inline double &at(double *a, const Grid &G, int i, int k) {
+    return *reinterpret_cast<double *>(reinterpret_cast<char *>(a + size_t(k) * G.pitch) + unsigned(i) * 8u);
+}
+__device__ inline const double &at(const double *a, const Grid &G, int i, int k) {
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a + size_t(k) * G.pitch) +
+                                             unsigned(i) * 8u);
+}
+// A value that is the same in every lane, as a scalar: threadIdx.y where
+// blockDim.x is a wavefront.
+__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // Stores v at interior point (i,k) and at every ghost cell that
 // BoundaryProcess2D_center (src/Boundary.cpp:9-19) fills from it: the
 // periodic column image for k in 1..nz-2, the zero-gradient row image at
 // k = 1 / nz-2, and the corner that takes both.
 __device__ inline void store_center(double *a, const Grid &G, int i, int k, double v) {
-    a[ix(G, i, k)] = v;
+    at(a, G, i, k) = v;
     const bool west_img = (i == G.nx - 2), east_img = (i == 1);
-    if (west_img) a[ix(G, 0, k)] = v;
-    if (east_img) a[ix(G, G.nx - 1, k)] = v;
+    if (west_img) at(a, G, 0, k) = v;
+    if (east_img) at(a, G, G.nx - 1, k) = v;
     if (k == 1) {
-        a[ix(G, i, 0)] = v;
-        if (west_img) a[ix(G, 0, 0)] = v;
-        if (east_img) a[ix(G, G.nx - 1, 0)] = v;
+        at(a, G, i, 0) = v;
+        if (west_img) at(a, G, 0, 0) = v;
+        if (east_img) at(a, G, G.nx - 1, 0) = v;
     }
     if (k == G.nz - 2) {
-        a[ix(G, i, G.nz - 1)] = v;
-        if (west_img) a[ix(G, 0, G.nz - 1)] = v;
-        if (east_img) a[ix(G, G.nx - 1, G.nz - 1)] = v;
+        at(a, G, i, G.nz - 1) = v;
+        if (west_img) at(a, G, 0, G.nz - 1) = v;
+        if (east_img) at(a, G, G.nx - 1, G.nz - 1) = v;
     }
 }
 
@@ -47,9 +63,9 @@ __device__ inline void store_center(double *a, const Grid &G, int i, int k, doub
 // BoundaryProcess2D_westdown (src/Boundary.cpp:21-31) does; rows 0, 1 and
 // nz-1 are zero and are written by the caller.
 __device__ inline void store_westdown(double *a, const Grid &G, int i, int k, double v) {
-    a[ix(G, i, k)] = v;
-    if (i == G.nx - 2) a[ix(G, 0, k)] = v;
-    if (i == 1) a[ix(G, G.nx - 1, k)] = v;
+    at(a, G, i, k) = v;
+    if (i == G.nx - 2) at(a, G, 0, k) = v;
+    if (i == 1) at(a, G, G.nx - 1, k) = v;
 }
 
 // ---------------------------------------------------------------- sums
@@ -101,14 +117,29 @@ struct RedSlot {
 };
 
 template <int NV>
-__device__ inline void block_partials(double (&v)[NV], const RedSlot &rs) {
+__device__ inline void block_partials(double (&v)[NV], const RedSlot &rs, int bid) {
     const int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-    const int bid = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
     block_sum<NV>(v);
     if (tid == 0) {
 #pragma unroll
         for (int j = 0; j < NV; j++) rs.partial[size_t(j) * rs.max_blocks + bid] = v[j];
     }
+}
+template <int NV>
+__device__ inline void block_partials(double (&v)[NV], const RedSlot &rs) {
+    block_partials<NV>(v, rs, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+}
+
+// Workgroups go round the 8 XCDs in turn, each with an L2 of its own.  Stencil
+// kernels whose tiles share halos map them so that an XCD works one contiguous
+// run of the n tiles (a band of rows): workgroup b of xcd_grid(n) takes tile
+// xcd_tile(n), none if that is >= n.
+constexpr int kXcds = 8;
+__host__ __device__ inline int xcd_run(int n) { return (n + kXcds - 1) / kXcds; }
+inline dim3 xcd_grid(int n) { return dim3(unsigned(kXcds * xcd_run(n))); }
+__device__ inline int xcd_tile(int n) {
+    const int b = blockIdx.x, run = xcd_run(n), t = (b % kXcds) * run + b / kXcds;
+    return t;
 }
 
 // Scalars of the preconditioned CG (doubles in its scalar block).
@@ -125,18 +156,35 @@ enum RedMode {
     RED_RZ_INIT      // CG: sc[P_RZ] = rz
 };
 
+// NegativeValueProcess's ratio from the sums of the positives and negatives
+// (MicroPhysics.cpp:129-131): no rescale when nothing is positive or the
+// negatives outweigh the positives (marked by a ratio < 0).
+__device__ inline double negval_ratio(double P, double N) {
+    return (P == 0. || fabs(N) > P) ? -1. : 1. - fabs(N / P);
+}
+
+// The totals of nblk workgroups' partials, in every thread of a workgroup.
+// The partials are added by a fixed 256 threads in a fixed order, so that all
+// callers agree bit for bit; blockDim is 256.
+template <int NV>
+__device__ inline void sum_partials(const RedSlot &rs, int nblk, double (&acc)[NV]) {
+    const int tid = threadIdx.x + blockDim.x * threadIdx.y;
+#pragma unroll
+    for (int j = 0; j < NV; j++) acc[j] = 0.;
+#pragma unroll 4
+    for (int b = tid; b < nblk; b += 256) {
+#pragma unroll
+        for (int j = 0; j < NV; j++) acc[j] += rs.partial[size_t(j) * rs.max_blocks + b];
+    }
+    block_sum<NV>(acc);
+}
+
 namespace {
 template <int NV>
 __global__ void __launch_bounds__(256) k_finalize(RedSlot rs, int nblk, double *sc, int mode, int dst, int dst2,
                                                   double *hout) {
     double acc[NV];
-#pragma unroll
-    for (int j = 0; j < NV; j++) acc[j] = 0.;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-#pragma unroll
-        for (int j = 0; j < NV; j++) acc[j] += rs.partial[size_t(j) * rs.max_blocks + b];
-    }
-    block_sum<NV>(acc);
+    sum_partials<NV>(rs, nblk, acc);
     if (threadIdx.x != 0) return;
     switch (mode) {
         case RED_STORE:
@@ -149,12 +197,7 @@ __global__ void __launch_bounds__(256) k_finalize(RedSlot rs, int nblk, double *
             }
             break;
         case RED_NEGVAL:
-            // MicroPhysics.cpp:129-131: no rescale when nothing is positive or
-            // the negatives outweigh the positives (marked by a ratio < 0).
-            for (int q = 0; q < NV / 2; q++) {
-                const double P = acc[2 * q], N = acc[2 * q + 1];
-                sc[dst + q] = (P == 0. || fabs(N) > P) ? -1. : 1. - fabs(N / P);
-            }
+            for (int q = 0; q < NV / 2; q++) sc[dst + q] = negval_ratio(acc[2 * q], acc[2 * q + 1]);
             break;
         case RED_RZ_INIT:
             sc[P_RZ] = acc[0];

@@ -35,9 +35,9 @@ class Direct {
     // (which may be x).
     void solve(const double *r, const double *x0, double *x, hipStream_t st);
     // cal_w whole: f = -b / rhow from zetap (f is written, for the residual),
-    // x = L^-1 f, w = x / rhow with its halos.
-    void solve_step(const Grid &G, const double *zetap, const double *rhow, double *f, double *x, double *w,
-                    hipStream_t st);
+    // x = L^-1 f, w = x / rhow with its halos; pubarTop_pt beside the first
+    // kernel's row transforms (step < 0: not).
+    void solve_step(const Grid &G, const StepPtrs &S, int step, double *f, double *x, hipStream_t st);
 
    private:
     RowPlan plan;
@@ -48,11 +48,5 @@ class Direct {
     T *spec = nullptr;  // [M][N] transformed rows
     void columns(hipStream_t st);
 };
-
-// ||wD (f - L x)||^2 and ||wD f||^2, one pair of partial sums per workgroup in
-// hres (host-mapped memory, 2 x the returned count of doubles).
-constexpr int kResidualBlocks = 512;
-int launch_residual_norms(int N, int M, const double *f, const double *x, const double *cx, const double *cu,
-                          const double *wD, double *hres, hipStream_t st);
 
 }  // namespace vvmd

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "direct.h"
+#include "pubartop.h"
 
 namespace vvmd {
 
@@ -256,11 +257,18 @@ __device__ inline void hartley_pair(const T *re, const T *im, int N, int q, T &h
 // Forward: rows j, j+1 of r (RHS false), or cal_w's right-hand side
 // f = -b / rhow, b = rhow^2 (zetap[i+1] - zetap[i]) dx
 // (src/PoissonSolver.cpp:444-450), formed from zetap and stored (RHS true).
+// With RHS and a step the last workgroup does pubarTop_pt instead: it reads u, w and K as
+// the solve finds them, and alone it was a launch of 5 to 8 us.
 template <typename T, bool RHS>
 __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restrict__ tw, const double *__restrict__ r,
-                                                   T *__restrict__ spec, Grid G, const double *__restrict__ zetap,
-                                                   const double *__restrict__ rhow, double *__restrict__ f) {
+                                                   T *__restrict__ spec, Grid G, StepPtrs S, int step,
+                                                   double *__restrict__ f) {
     extern __shared__ unsigned char lds_raw[];
+    if (RHS && step >= 0 && blockIdx.x == gridDim.x - 1) {
+        pubartop_block(G, S, step);
+        return;
+    }
+    const double *zetap = S.fut[F_ZETA], *rhow = S.P.rhow;
     const int N = P.N, M = P.M, LN = pad(N - 1) + 1;
     T *re = reinterpret_cast<T *>(lds_raw), *im = re + LN, *twl = im + LN;
     const int j = 1 + 2 * blockIdx.x;
@@ -521,41 +529,6 @@ __global__ void __launch_bounds__(256) k_columns(int N, int M, T *__restrict__ s
     for (int j = threadIdx.x / KC; j < M; j += rstep) spec[size_t(j) * N + q] = j == cs.mid ? Mid[c] : L[slot(j)];
 }
 
-// ---------------------------------------------------------------- residual
-
-constexpr int RX = 64, RY = 4;
-
-__global__ void __launch_bounds__(RX *RY) k_residual_norms(int N, int M, const double *__restrict__ f,
-                                                           const double *__restrict__ x,
-                                                           const double *__restrict__ cx,
-                                                           const double *__restrict__ cu,
-                                                           const double *__restrict__ wD, double *hres) {
-    const int tx = (N + RX - 1) / RX, nt = tx * ((M + RY - 1) / RY);
-    double part[2] = {0., 0.};
-    for (int t = blockIdx.x; t < nt; t += gridDim.x) {
-        const int i = (t % tx) * RX + threadIdx.x, j = 1 + (t / tx) * RY + threadIdx.y;
-        if (i < N && j <= M) {
-            const int im = (i == 0) ? N - 1 : i - 1, ip = (i == N - 1) ? 0 : i + 1;
-            const size_t r = size_t(j) * N;
-            const double c = x[r + i], fv = f[r + i];
-            double Lx;
-            {
-#pragma clang fp contract(off)
-                Lx = cx[j] * (2. * c - x[r + im] - x[r + ip]) + cu[j] * (c - x[r + N + i]) +
-                     cu[j - 1] * (c - x[r - N + i]);
-            }
-            const double wr = wD[j] * (fv - Lx), wb = wD[j] * fv;
-            part[0] += wr * wr;
-            part[1] += wb * wb;
-        }
-    }
-    block_sum<2>(part);
-    if (threadIdx.x == 0 && threadIdx.y == 0) {
-        __hip_atomic_store(hres + 2 * blockIdx.x, part[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(hres + 2 * blockIdx.x + 1, part[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-}
-
 constexpr size_t kLdsMax = 160 * 1024;
 
 template <typename T>
@@ -573,14 +546,6 @@ bool allow_lds(K kernel, size_t bytes) {
 }
 
 }  // namespace
-
-int launch_residual_norms(int N, int M, const double *f, const double *x, const double *cx, const double *cu,
-                          const double *wD, double *hres, hipStream_t st) {
-    const int tiles = ((N + RX - 1) / RX) * ((M + RY - 1) / RY);
-    const int nb = tiles < kResidualBlocks ? tiles : kResidualBlocks;
-    hipLaunchKernelGGL(k_residual_norms, dim3(nb), dim3(RX, RY), 0, st, N, M, f, x, cx, cu, wD, hres);
-    return nb;
-}
 
 template <typename T>
 int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
@@ -662,7 +627,7 @@ void Direct<T>::columns(hipStream_t st) {
 template <typename T>
 void Direct<T>::solve(const double *r, const double *x0, double *x, hipStream_t st) {
     const dim3 gr((plan.M + 1) / 2), b(plan.threads);
-    hipLaunchKernelGGL((k_rows_fwd<T, false>), gr, b, row_lds, st, plan, tw, r, spec, Grid{}, nullptr, nullptr,
+    hipLaunchKernelGGL((k_rows_fwd<T, false>), gr, b, row_lds, st, plan, tw, r, spec, Grid{}, StepPtrs{}, 0,
                        nullptr);
     columns(st);
     if (x0)
@@ -674,12 +639,12 @@ void Direct<T>::solve(const double *r, const double *x0, double *x, hipStream_t 
 }
 
 template <typename T>
-void Direct<T>::solve_step(const Grid &G, const double *zetap, const double *rhow, double *f, double *x, double *w,
-                           hipStream_t st) {
+void Direct<T>::solve_step(const Grid &G, const StepPtrs &S, int step, double *f, double *x, hipStream_t st) {
     const dim3 gr((plan.M + 1) / 2), b(plan.threads);
-    hipLaunchKernelGGL((k_rows_fwd<T, true>), gr, b, row_lds, st, plan, tw, nullptr, spec, G, zetap, rhow, f);
+    hipLaunchKernelGGL((k_rows_fwd<T, true>), dim3(gr.x + (step >= 0 ? 1 : 0)), b, row_lds, st, plan, tw, nullptr, spec, G, S, step, f);
     columns(st);
-    hipLaunchKernelGGL((k_rows_inv<T, false, true>), gr, b, row_lds, st, plan, tw, spec, nullptr, x, G, w, rhow);
+    hipLaunchKernelGGL((k_rows_inv<T, false, true>), gr, b, row_lds, st, plan, tw, spec, nullptr, x, G, S.w,
+                       S.P.rhow);
 }
 
 template class Direct<double>;

@@ -9,6 +9,7 @@
 // pow/sqrt/exp do).
 #pragma clang fp contract(off)
 
+#include "pubartop.h"
 #include "vvm_internal.h"
 
 namespace vvmd {
@@ -38,80 +39,80 @@ __device__ inline bool corr_window(const Grid &G, int i, int k) {
 // Scalar x-face flux at (i,k) (between i-1 and i), Advection.cpp:36,40-44.
 __device__ inline double sflux_x(const Grid &G, const double *__restrict__ f, const double *__restrict__ u,
                                  const double *__restrict__ rhou, int i, int k) {
-    const double r = rhou[k], ui = u[ix(G, i, k)];
-    const double f0 = f[ix(G, i, k)], fm1 = f[ix(G, i - 1, k)];
+    const double r = rhou[k], ui = at(u, G, i, k);
+    const double f0 = at(f, G, i, k), fm1 = at(f, G, i - 1, k);
     double fl = r * ui * (f0 + fm1);
     if (corr_window(G, i, k))
-        fl += upwind3(r, ui, r, u[ix(G, i - 1, k)], r, u[ix(G, i + 1, k)], f[ix(G, i - 2, k)], fm1, f0,
-                      f[ix(G, i + 1, k)]);
+        fl += upwind3(r, ui, r, at(u, G, i - 1, k), r, at(u, G, i + 1, k), at(f, G, i - 2, k), fm1, f0,
+                      at(f, G, i + 1, k));
     return fl;
 }
 
 // Scalar z-face flux at (i,k) (between k-1 and k), Advection.cpp:37,46-50.
 __device__ inline double sflux_z(const Grid &G, const double *__restrict__ f, const double *__restrict__ w,
                                  const double *__restrict__ rhow, int i, int k) {
-    const double r = rhow[k], wk = w[ix(G, i, k)];
-    const double f0 = f[ix(G, i, k)], fm1 = f[ix(G, i, k - 1)];
+    const double r = rhow[k], wk = at(w, G, i, k);
+    const double f0 = at(f, G, i, k), fm1 = at(f, G, i, k - 1);
     double fl = r * wk * (f0 + fm1);
     if (corr_window(G, i, k))
-        fl += upwind3(r, wk, rhow[k - 1], w[ix(G, i, k - 1)], rhow[k + 1], w[ix(G, i, k + 1)], f[ix(G, i, k - 2)],
-                      fm1, f0, f[ix(G, i, k + 1)]);
+        fl += upwind3(r, wk, rhow[k - 1], at(w, G, i, k - 1), rhow[k + 1], at(w, G, i, k + 1), at(f, G, i, k - 2),
+                      fm1, f0, at(f, G, i, k + 1));
     return fl;
 }
 
 // Corner velocities of Advection_zeta, Advection.cpp:90-91.
 __device__ inline double Uw(const Grid &G, const double *u, const double *rhou, int i, int k) {
-    return 0.25 * (rhou[k] * (u[ix(G, i + 1, k)] + u[ix(G, i, k)]) +
-                   rhou[k - 1] * (u[ix(G, i + 1, k - 1)] + u[ix(G, i, k - 1)]));
+    return 0.25 * (rhou[k] * (at(u, G, i + 1, k) + at(u, G, i, k)) +
+                   rhou[k - 1] * (at(u, G, i + 1, k - 1) + at(u, G, i, k - 1)));
 }
 __device__ inline double Wu(const Grid &G, const double *w, const double *rhow, int i, int k) {
-    return 0.25 * (rhow[k + 1] * (w[ix(G, i, k + 1)] + w[ix(G, i - 1, k + 1)]) +
-                   rhow[k] * (w[ix(G, i, k)] + w[ix(G, i - 1, k)]));
+    return 0.25 * (rhow[k + 1] * (at(w, G, i, k + 1) + at(w, G, i - 1, k + 1)) +
+                   rhow[k] * (at(w, G, i, k) + at(w, G, i - 1, k)));
 }
 
 // Vorticity fluxes, Advection.cpp:107-118 (the density already sits in U_w/W_u).
 __device__ inline double zflux_x(const Grid &G, const double *z, const double *u, const double *rhou, int i, int k) {
     const double U = Uw(G, u, rhou, i, k);
-    const double z0 = z[ix(G, i, k)], z1 = z[ix(G, i + 1, k)];
+    const double z0 = at(z, G, i, k), z1 = at(z, G, i + 1, k);
     double fl = U * (z1 + z0);
     if (corr_window(G, i, k)) {
         const double Pu = plus_(U), Pum = plus_(Uw(G, u, rhou, i - 1, k));
         const double Mu = minu_(U), Mup = minu_(Uw(G, u, rhou, i + 1, k));
         fl += -1. / 3. *
-              (Pu * (z1 - z0) - sqrt(Pu * Pum) * (z0 - z[ix(G, i - 1, k)]) - Mu * (z1 - z0) -
-               sqrt(fabs(Mu * Mup)) * (z[ix(G, i + 2, k)] - z1));
+              (Pu * (z1 - z0) - sqrt(Pu * Pum) * (z0 - at(z, G, i - 1, k)) - Mu * (z1 - z0) -
+               sqrt(fabs(Mu * Mup)) * (at(z, G, i + 2, k) - z1));
     }
     return fl;
 }
 __device__ inline double zflux_z(const Grid &G, const double *z, const double *w, const double *rhow, int i, int k) {
     const double W = Wu(G, w, rhow, i, k);
-    const double z0 = z[ix(G, i, k)], z1 = z[ix(G, i, k + 1)];
+    const double z0 = at(z, G, i, k), z1 = at(z, G, i, k + 1);
     double fl = W * (z1 + z0);
     if (corr_window(G, i, k)) {
         const double Pw = plus_(W), Pwm = plus_(Wu(G, w, rhow, i, k - 1));
         const double Mw = minu_(W), Mwp = minu_(Wu(G, w, rhow, i, k + 1));
         fl += -1. / 3. *
-              (Pw * (z1 - z0) - sqrt(Pw * Pwm) * (z0 - z[ix(G, i, k - 1)]) - Mw * (z1 - z0) -
-               sqrt(fabs(Mw * Mwp)) * (z[ix(G, i, k + 2)] - z1));
+              (Pw * (z1 - z0) - sqrt(Pw * Pwm) * (z0 - at(z, G, i, k - 1)) - Mw * (z1 - z0) -
+               sqrt(fabs(Mw * Mwp)) * (at(z, G, i, k + 2) - z1));
     }
     return fl;
 }
 
 __device__ inline double thv(const Grid &G, const double *th, const double *qv, int i, int k) {
-    return th[ix(G, i, k)] * (1 + 0.608 * qv[ix(G, i, k)]);
+    return at(th, G, i, k) * (1 + 0.608 * at(qv, G, i, k));
 }
 
 // AB2 update of one history slot: writes d to slot sn (and to slot 0 on the
 // reference's step-0 start, Advection.cpp:70) and returns the old slot.
-__device__ inline double ab2_hist(double *const (&h)[2], size_t p, int step, double d) {
+__device__ inline double ab2_hist(double *const (&h)[2], const Grid &G, int i, int k, int step, double d) {
     // the slot pointers are picked by selects, not by a run-time index into
     // the kernel-argument array (which would read them through generic
     // memory accesses)
     const bool odd = (step & 1) != 0;
     double *const hn = odd ? h[0] : h[1], *const ho = odd ? h[1] : h[0];
-    hn[p] = d;
-    if (step == 0) h[0][p] = d;
-    return ho[p];
+    at(hn, G, i, k) = d;
+    if (step == 0) at(h[0], G, i, k) = d;
+    return at(ho, G, i, k);
 }
 
 // ------------------------------------------------------------------ zeta
@@ -122,7 +123,10 @@ __device__ inline double ab2_hist(double *const (&h)[2], size_t p, int step, dou
 // the flux on its own east and upper faces, the first two waves the faces on
 // the tile's west and lower edges, and after a barrier each point takes the
 // differences.
+// The tiles start at the first point that the advection changes (k = 2).
 constexpr int PZX = 64, PZY = 8;
+__host__ __device__ inline int pz_tiles_x(const Grid &G) { return (G.nx - 2 + PZX - 1) / PZX; }
+__host__ __device__ inline int pz_tiles_z(const Grid &G) { return (G.nz - 3 + PZY - 1) / PZY; }
 
 // PARTS: PZ_ADV Advection_zeta, PZ_BUOY Bouyancy; both (the timestep) also
 // apply BoundaryProcess2D_westdown.  Alone each writes what the reference
@@ -134,32 +138,42 @@ template <int PARTS>
 __global__ void __launch_bounds__(PZX *PZY) k_pzeta(Grid G, StepPtrs S, int step) {
     __shared__ double Fx[PZY][PZX + 1];  // slot c: x-flux east of column i0 + c - 1
     __shared__ double Fz[PZY + 1][PZX];  // slot r: z-flux above row k0 + r - 1
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    const int i0 = blockIdx.x * PZX, k0 = blockIdx.y * PZY;
+    const int tx = threadIdx.x, ty = uniform(threadIdx.y);  // PZX = T4X = 64: one row a wavefront
+    const int tiles_x = pz_tiles_x(G), tiles_z = pz_tiles_z(G), tile = xcd_tile(tiles_x * tiles_z);
+    if (tile >= tiles_x * tiles_z) return;
+    const int i0 = 1 + (tile % tiles_x) * PZX, k0 = 2 + (tile / tiles_x) * PZY;
     const int i = i0 + tx, k = k0 + ty;
     const int nx = G.nx, nz = G.nz;
     const double *z = S.now[F_ZETA], *u = S.u, *w = S.w, *rhou = S.P.rhou, *rhow = S.P.rhow;
     if constexpr ((PARTS & PZ_ADV) != 0) {
-        // flux_u at i-1 = 0 is the periodic image of nx-2 (BoundaryProcess2D_center
-        // on flux_u): the ghost column 0 holds it for column 1
-        if (k >= 2 && k <= nz - 2 && i <= nx - 2) Fx[ty][tx + 1] = zflux_x(G, z, u, rhou, (i == 0) ? nx - 2 : i, k);
-        if (k >= 1 && k <= nz - 2 && i >= 1 && i <= nx - 2) Fz[ty + 1][tx] = zflux_z(G, z, w, rhow, i, k);
+        if (k <= nz - 2 && i <= nx - 2) {
+            Fx[ty][tx + 1] = zflux_x(G, z, u, rhou, i, k);
+            Fz[ty + 1][tx] = zflux_z(G, z, w, rhow, i, k);
+        }
         if (ty == 0 && tx < PZY) {  // west edge: the face east of column i0 - 1
             const int kr = k0 + tx;
-            if (i0 >= 1 && i0 <= nx - 2 && kr >= 2 && kr <= nz - 2) Fx[tx][0] = zflux_x(G, z, u, rhou, i0 - 1, kr);
+            // east of column 0: the periodic image of nx-2
+            // (BoundaryProcess2D_center on flux_u)
+            if (kr <= nz - 2) Fx[tx][0] = zflux_x(G, z, u, rhou, (i0 == 1) ? nx - 2 : i0 - 1, kr);
         } else if (ty == 1) {  // lower edge: the face above row k0 - 1
-            if (k0 >= 2 && k0 <= nz - 2 && i >= 1 && i <= nx - 2) Fz[0][tx] = zflux_z(G, z, w, rhow, i, k0 - 1);
+            if (i <= nx - 2) Fz[0][tx] = zflux_z(G, z, w, rhow, i, k0 - 1);
         }
         __syncthreads();
     }
-    if (i >= nx || k >= nz) return;
     double *zp = S.fut[F_ZETA];
-    if (k == 0 || k == 1 || k == nz - 1) {
-        if (PARTS == PZ_BOTH) zp[ix(G, i, k)] = 0.;
-        return;
+    if (PARTS == PZ_BOTH && (ty == 0 || ty == 1) && i <= nx - 2) {
+        // the zero rows 0, 1 (first tiles) and nz-1 (last tiles), ghosts included
+        const bool first = k0 == 2, last = k0 + PZY > nz - 2;
+        const int kz = (ty == 0) ? 0 : 1;
+        auto clear = [&](int kc) {
+            at(zp, G, i, kc) = 0.;
+            if (i == 1) at(zp, G, 0, kc) = 0.;
+            if (i == nx - 2) at(zp, G, nx - 1, kc) = 0.;
+        };
+        if (first) clear(kz);
+        if (last && ty == 0) clear(nz - 1);
     }
-    if (i < 1 || i > nx - 2) return;
-    const size_t p = ix(G, i, k);
+    if (i > nx - 2 || k > nz - 2) return;
     double zeta_new;
     if constexpr ((PARTS & PZ_ADV) != 0) {
         const double fu0 = Fx[ty][tx + 1], fum = Fx[ty][tx];
@@ -167,14 +181,14 @@ __global__ void __launch_bounds__(PZX *PZY) k_pzeta(Grid G, StepPtrs S, int step
         const double px = (fu0 - fum) * G.r2dx / rhow[k];
         const double pz = (fw0 - fwm) * G.r2dz / rhow[k];
         const double dadv = -px - pz;
-        const double dold = ab2_hist(S.hist[H_ZETA_ADV], p, step, dadv);
-        zeta_new = z[p] + 1.5 * G.dt * dadv - 0.5 * G.dt * dold;
+        const double dold = ab2_hist(S.hist[H_ZETA_ADV], G, i, k, step, dadv);
+        zeta_new = at(z, G, i, k) + 1.5 * G.dt * dadv - 0.5 * G.dt * dold;
         if constexpr (PARTS == PZ_ADV) {
-            zp[p] = zeta_new;
+            at(zp, G, i, k) = zeta_new;
             return;
         }
     } else {
-        zeta_new = zp[p];
+        zeta_new = at(zp, G, i, k);
     }
 
     const double *th = S.now[F_TH], *qv = S.now[F_QV], *qc = S.now[F_QC], *qr = S.now[F_QR], *thvb = S.P.thvb;
@@ -183,17 +197,17 @@ __global__ void __launch_bounds__(PZX *PZY) k_pzeta(Grid G, StepPtrs S, int step
                         (thv(G, th, qv, i, k - 1) - thv(G, th, qv, i - 1, k - 1)) / thvb[k - 1]) *
                        G.rdx;
     const double gqc = G.GRAVITY / rhow[k] *
-                       (0.5 * (qc[ix(G, i, k)] + qc[ix(G, i, k - 1)]) - 0.5 * (qc[ix(G, i - 1, k)] + qc[ix(G, i - 1, k - 1)])) *
+                       (0.5 * (at(qc, G, i, k) + at(qc, G, i, k - 1)) - 0.5 * (at(qc, G, i - 1, k) + at(qc, G, i - 1, k - 1))) *
                        G.rdx;
     const double gqr = G.GRAVITY / rhow[k] *
-                       (0.5 * (qr[ix(G, i, k)] + qr[ix(G, i, k - 1)]) - 0.5 * (qr[ix(G, i - 1, k)] + qr[ix(G, i - 1, k - 1)])) *
+                       (0.5 * (at(qr, G, i, k) + at(qr, G, i, k - 1)) - 0.5 * (at(qr, G, i - 1, k) + at(qr, G, i - 1, k - 1))) *
                        G.rdx;
     double db = gth;
     db += -gqc - gqr;
-    const double bold = ab2_hist(S.hist[H_TH_BUOY], p, step, db);
+    const double bold = ab2_hist(S.hist[H_TH_BUOY], G, i, k, step, db);
     zeta_new += (1.5 * G.dt * db) - (0.5 * G.dt * bold);
     if constexpr (PARTS == PZ_BOTH) store_westdown(zp, G, i, k, zeta_new);
-    else zp[p] = zeta_new;
+    else at(zp, G, i, k) = zeta_new;
 }
 
 // ----------------------------------------------------------- scalars
@@ -214,27 +228,28 @@ __device__ inline double thermo_tend(const Grid &G, const double *f, const doubl
 // velocity), formed once and applied to every field advected across it.
 // flux(f) rounds exactly as sflux_x / sflux_z do: the same products in the
 // same order (upwind3's rho0 p0 (f0 - fm1) is (rho0 p0) (f0 - fm1), and so on).
+template <bool X>  // an x face (between i-1 and i) or a z face (between k-1 and k)
 struct FaceFlux {
     double rv;          // r v of the centred term
     double a, b, c, d;  // rho0 p0, sqrt(rho0 p0 rhom pm), rho0 m0, sqrt(|rho0 m0 rhop mp|)
     bool corr;          // inside the third-order correction window
-    size_t s;           // index step across the face (1 for x faces, the row pitch for z faces)
-    __device__ double flux(const double *__restrict__ f, size_t p) const {
-        const double f0 = f[p], fm1 = f[p - s];
+    __device__ double flux(const Grid &G, const double *__restrict__ f, int i, int k) const {
+        auto across = [&](int s) { return X ? at(f, G, i + s, k) : at(f, G, i, k + s); };
+        const double f0 = across(0), fm1 = across(-1);
         double fl = rv * (f0 + fm1);
         if (corr) {
-            const double fm2 = f[p - 2 * s], fp1 = f[p + s];
+            const double fm2 = across(-2), fp1 = across(1);
             fl += -1. / 3. * (a * (f0 - fm1) - b * (fm1 - fm2) - c * (f0 - fm1) - d * (fp1 - f0));
         }
         return fl;
     }
 };
-__device__ inline FaceFlux face_coeffs(double rho0, double v0, double rhom, double vm, double rhop, double vp,
-                                       bool corr, size_t s) {
-    FaceFlux F;
+template <bool X>
+__device__ inline FaceFlux<X> face_coeffs(double rho0, double v0, double rhom, double vm, double rhop, double vp,
+                                          bool corr) {
+    FaceFlux<X> F;
     F.rv = rho0 * v0;
     F.corr = corr;
-    F.s = s;
     F.a = F.b = F.c = F.d = 0.;
     if (corr) {
         const double p0 = plus_(v0), pm = plus_(vm), m0 = minu_(v0), mp = minu_(vp);
@@ -246,22 +261,22 @@ __device__ inline FaceFlux face_coeffs(double rho0, double v0, double rhom, doub
     return F;
 }
 // x face between i-1 and i / z face between k-1 and k, as sflux_x / sflux_z
-__device__ inline FaceFlux face_x(const Grid &G, const double *u, const double *rhou, int i, int k) {
+__device__ inline FaceFlux<true> face_x(const Grid &G, const double *u, const double *rhou, int i, int k) {
     const bool corr = corr_window(G, i, k);
     const double r = rhou[k];
-    return face_coeffs(r, u[ix(G, i, k)], r, corr ? u[ix(G, i - 1, k)] : 0., r, corr ? u[ix(G, i + 1, k)] : 0., corr,
-                       1);
+    return face_coeffs<true>(r, at(u, G, i, k), r, corr ? at(u, G, i - 1, k) : 0., r, corr ? at(u, G, i + 1, k) : 0., corr);
 }
-__device__ inline FaceFlux face_z(const Grid &G, const double *w, const double *rhow, int i, int k) {
+__device__ inline FaceFlux<false> face_z(const Grid &G, const double *w, const double *rhow, int i, int k) {
     const bool corr = corr_window(G, i, k);
-    return face_coeffs(rhow[k], w[ix(G, i, k)], corr ? rhow[k - 1] : 0., corr ? w[ix(G, i, k - 1)] : 0.,
-                       corr ? rhow[k + 1] : 0., corr ? w[ix(G, i, k + 1)] : 0., corr, G.pitch);
+    return face_coeffs<false>(rhow[k], at(w, G, i, k), corr ? rhow[k - 1] : 0., corr ? at(w, G, i, k - 1) : 0.,
+                       corr ? rhow[k + 1] : 0., corr ? at(w, G, i, k + 1) : 0., corr);
 }
 
 // Rain sedimentation flux of Advection_qrVT (Advection.cpp:165-166) at (i,k).
 __device__ inline double vt_flux(const Grid &G, const double *qr, const double *rhow, const double *vtfac, int i,
                                  int k) {
-    const double s = qr[ix(G, i, k)] + qr[ix(G, i, k - 1)];
+    const double s = at(qr, G, i, k) + at(qr, G, i, k - 1);
+    if (s == 0.) return s;  // no rain, over most of a domain: VT is zero, and pow is a third of the kernel
     const double VT = 1E-2 * (3634 * pow(1E-3 * rhow[k] * 0.5 * s, 0.1346) * vtfac[k]);
     return rhow[k] * VT * s;
 }
@@ -279,15 +294,22 @@ __device__ inline double vt_flux(const Grid &G, const double *qr, const double *
 // and top edges; after a barrier each point takes the differences.  (Forming
 // both faces of every point would evaluate each flux, with its square roots
 // and powers, twice.)
+// The tiles start at the first interior point: 2048 x 256 are 1024 of them, one
+// round at four workgroups a CU.  (From the ghost cells on they were 1089, and
+// the last 65 took a round of their own.)
 constexpr int T4X = 64, T4Y = 8;
+__host__ __device__ inline int t4_tiles_x(const Grid &G) { return (G.nx - 2 + T4X - 1) / T4X; }
+__host__ __device__ inline int t4_tiles_z(const Grid &G) { return (G.nz - 2 + T4Y - 1) / T4Y; }
 
 // Four workgroups a CU (the LDS allows four), so that 1024 of them cover
 // 2048 x 256 in one round: eight waves a SIMD, at most 64 VGPRs.
 __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8))) k_thermo4(Grid G, StepPtrs S, int step, RedSlot rs) {
     __shared__ double Fx[4][T4Y][T4X + 1];  // x-face flux at faces i0 .. i0+T4X (west faces)
     __shared__ double Fz[5][T4Y + 1][T4X];  // z-face flux (4 fields, rain fall) at faces k0 .. k0+T4Y
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    const int i0 = blockIdx.x * T4X, k0 = blockIdx.y * T4Y;
+    const int tx = threadIdx.x, ty = uniform(threadIdx.y);  // PZX = T4X = 64: one row a wavefront
+    const int tiles_x = t4_tiles_x(G), ntiles = tiles_x * t4_tiles_z(G), tile = xcd_tile(ntiles);
+    if (tile >= ntiles) return;
+    const int i0 = 1 + (tile % tiles_x) * T4X, k0 = 1 + (tile / tiles_x) * T4Y;
     const int i = i0 + tx, k = k0 + ty;
     const int nx = G.nx, nz = G.nz;
     const double *u = S.u, *w = S.w, *rhou = S.P.rhou, *rhow = S.P.rhow;
@@ -299,16 +321,14 @@ __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8
     // fields (sflux_x / sflux_z per field would repeat its square roots)
     if (row_in && i >= 1 && i <= nx - 1) {
         const int ii = (i == nx - 1) ? 1 : i;
-        const FaceFlux F = face_x(G, u, rhou, ii, k);
-        const size_t p = ix(G, ii, k);
+        const FaceFlux<true> F = face_x(G, u, rhou, ii, k);
 #pragma unroll
-        for (int q = 0; q < 4; q++) Fx[q][ty][tx] = F.flux(fl[q], p);
+        for (int q = 0; q < 4; q++) Fx[q][ty][tx] = F.flux(G, fl[q], ii, k);
     }
     if (inside) {
-        const FaceFlux F = face_z(G, w, rhow, i, k);
-        const size_t p = ix(G, i, k);
+        const FaceFlux<false> F = face_z(G, w, rhow, i, k);
 #pragma unroll
-        for (int q = 0; q < 4; q++) Fz[q][ty][tx] = F.flux(fl[q], p);
+        for (int q = 0; q < 4; q++) Fz[q][ty][tx] = F.flux(G, fl[q], i, k);
         Fz[4][ty][tx] = vt_flux(G, fl[3], rhow, S.P.vtfac, i, k);
     }
     // edge faces: waves 0-1 the top faces (four fields each), wave 2 the
@@ -317,10 +337,9 @@ __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8
         const int kt = k0 + T4Y, ie = i0 + T4X;
         if (ty == 0) {
             if (i >= 1 && i <= nx - 2 && kt <= nz - 2) {
-                const FaceFlux F = face_z(G, w, rhow, i, kt);
-                const size_t p = ix(G, i, kt);
+                const FaceFlux<false> F = face_z(G, w, rhow, i, kt);
 #pragma unroll
-                for (int q = 0; q < 4; q++) Fz[q][T4Y][tx] = F.flux(fl[q], p);
+                for (int q = 0; q < 4; q++) Fz[q][T4Y][tx] = F.flux(G, fl[q], i, kt);
             }
         } else if (ty == 2) {
             if (i >= 1 && i <= nx - 2 && kt <= nz - 2) Fz[4][T4Y][tx] = vt_flux(G, fl[3], rhow, S.P.vtfac, i, kt);
@@ -329,17 +348,15 @@ __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8
             // the face east of column nx-2 is the periodic image of face 1
             if (ie - 1 <= nx - 2 && kr >= 1 && kr <= nz - 2) {
                 const int ii = (ie == nx - 1) ? 1 : ie;
-                const FaceFlux F = face_x(G, u, rhou, ii, kr);
-                const size_t p = ix(G, ii, kr);
+                const FaceFlux<true> F = face_x(G, u, rhou, ii, kr);
 #pragma unroll
-                for (int q = 0; q < 4; q++) Fx[q][tx][T4X] = F.flux(fl[q], p);
+                for (int q = 0; q < 4; q++) Fx[q][tx][T4X] = F.flux(G, fl[q], ii, kr);
             }
         }
     }
     __syncthreads();
     double part[6] = {0., 0., 0., 0., 0., 0.};
     if (inside) {
-        const size_t p = ix(G, i, k);
         const int hid[4] = {H_TH_ADV, H_QV_ADV, H_QC_ADV, H_QR_ADV};
         const bool top = (k + 1 == nz - 1);
 #pragma unroll
@@ -351,17 +368,17 @@ __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8
             const double px = (fu1 - fu0) * G.r2dx / rhou[k];
             const double pz = (fw1 - fw0) * G.r2dz / rhou[k];
             const double d = -px - pz;
-            const double dold = ab2_hist(S.hist[hid[q]], p, step, d);
-            double v = fl[q][p] + 1.5 * G.dt * d - 0.5 * G.dt * dold;
+            const double dold = ab2_hist(S.hist[hid[q]], G, i, k, step, d);
+            double v = at(fl[q], G, i, k) + 1.5 * G.dt * d - 0.5 * G.dt * dold;
             if (q == 0) {
-                S.fut[F_TH][p] = v;
+                at(S.fut[F_TH], G, i, k) = v;
                 continue;
             }
             if (q == 3) {
                 const double f1 = top ? 0. : Fz[4][ty + 1][tx];
                 const double f0 = Fz[4][ty][tx];
                 const double dvt = (f1 - f0) * G.r2dz / rhou[k];
-                const double vold = ab2_hist(S.hist[H_QR_VT], p, step, dvt);
+                const double vold = ab2_hist(S.hist[H_QR_VT], G, i, k, step, dvt);
                 v += 1.5 * G.dt * dvt - 0.5 * G.dt * vold;
             }
             if (v >= 0.) part[2 * (q - 1)] += v;
@@ -369,50 +386,61 @@ __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8
                 part[2 * (q - 1) + 1] += v;
                 v = 0.;
             }
-            S.fut[F_QV + q - 1][p] = v;
+            at(S.fut[F_QV + q - 1], G, i, k) = v;
         }
         if (k == 1) {
             // surface precipitation, src/Iteration.cpp:114-119 (now-qr, last w)
             const double r1 = rhou[1];
-            const double q1 = S.now[F_QR][ix(G, i, 1)];
+            const double q1 = at(S.now[F_QR], G, i, 1);
             const double VT = 1E-2 * (3634 * pow(1E-3 * r1 * q1, 0.1346) * S.s[S_PRECIP_FAC]);
-            const double rain = -r1 * (0.5 * (w[ix(G, i, 2)] + 0.) - VT) * q1;
+            const double rain = -r1 * (0.5 * (at(w, G, i, 2) + 0.) - VT) * q1;
             S.precip[i] = (rain < 0) ? 0. : rain;
         }
     }
-    block_partials<6>(part, rs);
+    block_partials<6>(part, rs, tile);
 }
 
 // Second pass of NegativeValueProcess for qv, qc, qr (MicroPhysics.cpp:
 // 129-137), AddForcing (AddForcing.cpp:6-28: Q1LS/Q2LS and the random
 // theta kick) when `forcing`, and the center halos of thp, qvp, qcp, qrp.
 // halos == 0 is AddForcing alone (ratios < 0): interior thp and qvp only.
+// nblk > 0: the ratios from the producing kernel's nblk partials in rs, formed
+// by every workgroup; otherwise from the scalars k_finalize left.
 __global__ void __launch_bounds__(BX *BY) k_scale_forcing(Grid G, StepPtrs S, int forcing, int tropical,
-                                                          int random_kick, int halos) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+                                                          int random_kick, int halos, RedSlot rs, int nblk) {
+    const int i = 1 + blockIdx.x * BX + threadIdx.x, k = 1 + blockIdx.y * BY + uniform(threadIdx.y);
+    double ratios[3];
+    if (nblk > 0) {
+        double acc[6];
+        sum_partials<6>(rs, nblk, acc);
+#pragma unroll
+        for (int q = 0; q < 3; q++) ratios[q] = negval_ratio(acc[2 * q], acc[2 * q + 1]);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 3; q++) ratios[q] = S.s[S_NEG_RATIO + q];
+    }
     if (i < 1 || i > G.nx - 2 || k < 1 || k > G.nz - 2) return;
-    const size_t p = ix(G, i, k);
 #pragma unroll
     for (int q = 0; q < 3; q++) {
         const int f = F_QV + q;
-        double v = S.fut[f][p];
-        const double ratio = S.s[S_NEG_RATIO + q];
+        double v = at(S.fut[f], G, i, k);
+        const double ratio = ratios[q];
         if (ratio >= 0. && v > 0) v = v * ratio;
         if (forcing && tropical && f == F_QV) v += G.dt * S.P.Q2LS[k];
         if (halos) store_center(S.fut[f], G, i, k, v);
-        else if (f == F_QV) S.fut[f][p] = v;
+        else if (f == F_QV) at(S.fut[f], G, i, k) = v;
     }
-    double th = S.fut[F_TH][p];
+    double th = at(S.fut[F_TH], G, i, k);
     if (forcing) {
         // AddForcing's order (AddForcing.cpp:15-25): large-scale forcing,
         // radiation heating [K/day], RADIATIONCOOLING, the random kick
         if (tropical) th += G.dt * S.P.Q1LS[k];
-        if (S.rad) th += G.dt * S.rad[p] / 86400.;
+        if (S.rad) th += G.dt * at(S.rad, G, i, k) / 86400.;
         if (S.radcool) th += G.dt * (-2. / 86400.);
-        if (random_kick) th += G.dt * S.forcing[p];
+        if (random_kick) th += G.dt * at(S.forcing, G, i, k);
     }
     if (halos) store_center(S.fut[F_TH], G, i, k, th);
-    else S.fut[F_TH][p] = th;
+    else at(S.fut[F_TH], G, i, k) = th;
 }
 
 // Halo value of BoundaryProcess2D_center at a perimeter cell.
@@ -424,16 +452,16 @@ __device__ inline size_t center_src(const Grid &G, int i, int k) {
 
 // BoundaryProcess2D_center / _westdown on the perimeter of a field.
 __device__ inline void bc_center_cell(double *a, const Grid &G, int i, int k) {
-    if (i == 0 || i == G.nx - 1 || k == 0 || k == G.nz - 1) a[ix(G, i, k)] = a[center_src(G, i, k)];
+    if (i == 0 || i == G.nx - 1 || k == 0 || k == G.nz - 1) at(a, G, i, k) = a[center_src(G, i, k)];
 }
 __device__ inline void bc_westdown_cell(double *a, const Grid &G, int i, int k) {
-    if (k == 0 || k == 1 || k == G.nz - 1) a[ix(G, i, k)] = 0.;
-    else if (i == 0) a[ix(G, i, k)] = a[ix(G, G.nx - 2, k)];
-    else if (i == G.nx - 1) a[ix(G, i, k)] = a[ix(G, 1, k)];
+    if (k == 0 || k == 1 || k == G.nz - 1) at(a, G, i, k) = 0.;
+    else if (i == 0) at(a, G, i, k) = at(a, G, G.nx - 2, k);
+    else if (i == G.nx - 1) at(a, G, i, k) = at(a, G, 1, k);
 }
 
 __global__ void __launch_bounds__(BX *BY) k_bc_uw(Grid G, StepPtrs S) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + uniform(threadIdx.y);
     if (i >= G.nx || k >= G.nz) return;
     bc_center_cell(S.u, G, i, k);
     bc_westdown_cell(S.w, G, i, k);
@@ -441,7 +469,7 @@ __global__ void __launch_bounds__(BX *BY) k_bc_uw(Grid G, StepPtrs S) {
 
 // BoundaryProcess2D_all (src/Boundary.cpp:33-52), Kessler build.
 __global__ void __launch_bounds__(BX *BY) k_bc_all(Grid G, StepPtrs S) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + uniform(threadIdx.y);
     if (i >= G.nx || k >= G.nz) return;
     bc_westdown_cell(S.fut[F_ZETA], G, i, k);
     bc_center_cell(S.fut[F_TH], G, i, k);
@@ -459,93 +487,65 @@ __global__ void __launch_bounds__(BX *BY) k_bc_all(Grid G, StepPtrs S) {
 // Advection_thermo (Advection.cpp:25-81) of field q (F_TH..F_QR): the
 // interior of its p-field and its AB2 history.
 __global__ void __launch_bounds__(BX *BY) k_adv_scalar(Grid G, StepPtrs S, int step, int q) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + uniform(threadIdx.y);
     if (i < 1 || i > G.nx - 2 || k < 1 || k > G.nz - 2) return;
     const int hid[NPROG] = {H_ZETA_ADV, H_TH_ADV, H_QV_ADV, H_QC_ADV, H_QR_ADV};
     const double *f = S.now[q];
-    const size_t p = ix(G, i, k);
     const double d = thermo_tend(G, f, S.u, S.w, S.P.rhou, S.P.rhow, i, k);
-    const double dold = ab2_hist(S.hist[hid[q]], p, step, d);
-    S.fut[q][p] = f[p] + 1.5 * G.dt * d - 0.5 * G.dt * dold;
+    const double dold = ab2_hist(S.hist[hid[q]], G, i, k, step, d);
+    at(S.fut[q], G, i, k) = at(f, G, i, k) + 1.5 * G.dt * d - 0.5 * G.dt * dold;
 }
 
 // Advection_qrVT (Advection.cpp:153-192): the rain fall added to the
 // interior of qrp, and its AB2 history.
 __global__ void __launch_bounds__(BX *BY) k_qrvt(Grid G, StepPtrs S, int step) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + uniform(threadIdx.y);
     if (i < 1 || i > G.nx - 2 || k < 1 || k > G.nz - 2) return;
     const double *qr = S.now[F_QR], *rhow = S.P.rhow;
-    const size_t p = ix(G, i, k);
     const double f1 = (k + 1 == G.nz - 1) ? 0. : vt_flux(G, qr, rhow, S.P.vtfac, i, k + 1);
     const double f0 = vt_flux(G, qr, rhow, S.P.vtfac, i, k);
     const double dvt = (f1 - f0) * G.r2dz / S.P.rhou[k];
-    const double vold = ab2_hist(S.hist[H_QR_VT], p, step, dvt);
-    S.fut[F_QR][p] += 1.5 * G.dt * dvt - 0.5 * G.dt * vold;
+    const double vold = ab2_hist(S.hist[H_QR_VT], G, i, k, step, dvt);
+    at(S.fut[F_QR], G, i, k) += 1.5 * G.dt * dvt - 0.5 * G.dt * vold;
 }
 
 // Surface precipitation of pqr_pt (src/Iteration.cpp:114-119).
 __global__ void k_precip(Grid G, StepPtrs S) {
     const int i = 1 + blockIdx.x * blockDim.x + threadIdx.x;
     if (i > G.nx - 2) return;
-    const double r1 = S.P.rhou[1], q1 = S.now[F_QR][ix(G, i, 1)];
+    const double r1 = S.P.rhou[1], q1 = at(S.now[F_QR], G, i, 1);
     const double VT = 1E-2 * (3634 * pow(1E-3 * r1 * q1, 0.1346) * S.s[S_PRECIP_FAC]);
-    const double rain = -r1 * (0.5 * (S.w[ix(G, i, 2)] + 0.) - VT) * q1;
+    const double rain = -r1 * (0.5 * (at(S.w, G, i, 2) + 0.) - VT) * q1;
     S.precip[i] = (rain < 0) ? 0. : rain;
 }
 
 // BoundaryProcess2D_center (westdown = 0) or _westdown on one field.
 __global__ void __launch_bounds__(BX *BY) k_bc_one(Grid G, double *a, int westdown) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + uniform(threadIdx.y);
     if (i >= G.nx || k >= G.nz) return;
     if (westdown) bc_westdown_cell(a, G, i, k);
     else bc_center_cell(a, G, i, k);
 }
 
-// PoissonSolver::pubarTop_pt (src/PoissonSolver.cpp:655-676): domain-mean
-// vertical momentum flux and K_M shear at the top, AB2 for ubarTopp.
-__global__ void __launch_bounds__(1024) k_pubartop(Grid G, StepPtrs S, int step) {
-    const int nx = G.nx, nz = G.nz;
-    const double *u = S.u, *w = S.w, *K = S.RKM, *rhou = S.P.rhou, *rhow = S.P.rhow;
-    double acc[3] = {0., 0., 0.};
-    for (int i = 1 + threadIdx.x; i < nx - 1; i += blockDim.x) {
-        acc[0] += 0.25 * (rhou[nz - 2] * u[ix(G, i, nz - 2)] + rhou[nz - 3] * u[ix(G, i, nz - 3)]) *
-                  (w[ix(G, i, nz - 2)] + w[ix(G, i - 1, nz - 2)]);
-        acc[1] += rhow[nz - 1] * 0.25 *
-                  (K[ix(G, i, nz - 1)] + K[ix(G, i, nz - 2)] + K[ix(G, i - 1, nz - 1)] + K[ix(G, i - 1, nz - 2)]) *
-                  (G.rdz * (u[ix(G, i, nz - 1)] - u[ix(G, i, nz - 2)]));
-        acc[2] += rhow[nz - 2] * 0.25 *
-                  (K[ix(G, i, nz - 2)] + K[ix(G, i, nz - 3)] + K[ix(G, i - 1, nz - 2)] + K[ix(G, i - 1, nz - 3)]) *
-                  (G.rdx * (w[ix(G, i, nz - 2)] - w[ix(G, i - 1, nz - 2)]) +
-                   G.rdz * (u[ix(G, i, nz - 2)] - u[ix(G, i, nz - 3)]));
-    }
-    block_sum<3>(acc);
-    if (threadIdx.x == 0) {
-        const double n = (double)(nx - 2.);
-        const double down = acc[0] / n, kup = acc[1] / n, kdown = acc[2] / n;
-        const double p1 = (-down) * G.rdz / rhou[nz - 2];
-        const double p2 = (kup - kdown) * G.rdz / rhou[nz - 2];
-        const int sn = (step + 1) % 2, so = step % 2;
-        double *dub = S.s + S_DUBAR0;
-        dub[sn] = -p1 + p2;
-        if (step == 0) dub[0] = dub[1];
-        S.s[S_UBARTOPP] = S.s[S_UBARTOP] + 1.5 * G.dt * dub[sn] - 0.5 * G.dt * dub[so];
-    }
-}
+__global__ void __launch_bounds__(1024) k_pubartop(Grid G, StepPtrs S, int step) { pubartop_block(G, S, step); }
 
 inline dim3 grid2d(const Grid &G) { return dim3((G.nx + BX - 1) / BX, (G.nz + BY - 1) / BY); }
+// tiles from the first interior point on (2048 x 256: 2048 of them, one round
+// at eight workgroups a CU; from the ghost cells on, 2145)
+inline dim3 interior_grid(const Grid &G) { return dim3((G.nx - 2 + BX - 1) / BX, (G.nz - 2 + BY - 1) / BY); }
 
 }  // namespace
 
 void launch_pzeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st) {
-    const dim3 g((G.nx + PZX - 1) / PZX, (G.nz + PZY - 1) / PZY);
+    const dim3 g = xcd_grid(pz_tiles_x(G) * pz_tiles_z(G));
     hipLaunchKernelGGL(k_pzeta<PZ_BOTH>, g, dim3(PZX, PZY), 0, st, G, S, step);
 }
 void launch_advection_zeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st) {
-    const dim3 g((G.nx + PZX - 1) / PZX, (G.nz + PZY - 1) / PZY);
+    const dim3 g = xcd_grid(pz_tiles_x(G) * pz_tiles_z(G));
     hipLaunchKernelGGL(k_pzeta<PZ_ADV>, g, dim3(PZX, PZY), 0, st, G, S, step);
 }
 void launch_buoyancy(const Grid &G, const StepPtrs &S, int step, hipStream_t st) {
-    const dim3 g((G.nx + PZX - 1) / PZX, (G.nz + PZY - 1) / PZY);
+    const dim3 g = xcd_grid(pz_tiles_x(G) * pz_tiles_z(G));
     hipLaunchKernelGGL(k_pzeta<PZ_BUOY>, g, dim3(PZX, PZY), 0, st, G, S, step);
 }
 void launch_advection_scalar(const Grid &G, const StepPtrs &S, int step, int field, hipStream_t st) {
@@ -560,15 +560,26 @@ void launch_precip(const Grid &G, const StepPtrs &S, hipStream_t st) {
 void launch_bc_one(const Grid &G, double *a, bool westdown, hipStream_t st) {
     hipLaunchKernelGGL(k_bc_one, grid2d(G), dim3(BX, BY), 0, st, G, a, int(westdown));
 }
-void launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
-    const dim3 g((G.nx + T4X - 1) / T4X, (G.nz + T4Y - 1) / T4Y);
-    hipLaunchKernelGGL(k_thermo4, g, dim3(T4X, T4Y), 0, st, G, S, step, rs);
-    finalize<6>(rs, nblocks(g), S.s, RED_NEGVAL, S_NEG_RATIO, st);
+int launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
+    const int n = t4_tiles_x(G) * t4_tiles_z(G);
+    hipLaunchKernelGGL(k_thermo4, xcd_grid(n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
+    return negval_partials(S, rs, n, st);
+}
+// The ratios of NegativeValueProcess from nblk workgroups' partials: by
+// k_finalize (returns 0), or, up to kFoldBlocks, by the workgroups of
+// k_scale_forcing themselves (returns nblk).  The launch costs 4 to 5 us
+// whatever it does; every workgroup's own sum costs the traffic of all partials
+// for each of them, which at 2048 x 256 (1089 and 2145 partials) is no gain.
+int negval_partials(const StepPtrs &S, const RedSlot &rs, int nblk, hipStream_t st) {
+    constexpr int kFoldBlocks = 640;
+    if (nblk <= kFoldBlocks) return nblk;
+    finalize<6>(rs, nblk, S.s, RED_NEGVAL, S_NEG_RATIO, st);
+    return 0;
 }
 void launch_scale_forcing(const Grid &G, const StepPtrs &S, bool forcing, bool tropical, bool random_kick,
-                          hipStream_t st, bool halos) {
-    hipLaunchKernelGGL(k_scale_forcing, grid2d(G), dim3(BX, BY), 0, st, G, S, int(forcing), int(tropical),
-                       int(random_kick), int(halos));
+                          hipStream_t st, const RedSlot &rs, int nblk, bool halos) {
+    hipLaunchKernelGGL(k_scale_forcing, interior_grid(G), dim3(BX, BY), 0, st, G, S, int(forcing), int(tropical),
+                       int(random_kick), int(halos), rs, nblk);
 }
 void launch_bc_uw(const Grid &G, const StepPtrs &S, hipStream_t st) {
     hipLaunchKernelGGL(k_bc_uw, grid2d(G), dim3(BX, BY), 0, st, G, S);

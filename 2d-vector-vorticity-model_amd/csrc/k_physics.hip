@@ -23,6 +23,9 @@ __device__ inline double maxs(double a, double b) { return (a < b) ? b : a; }
 __device__ inline double mins(double a, double b) { return (b < a) ? b : a; }
 
 inline dim3 grid2d(const Grid &G) { return dim3((G.nx + BX - 1) / BX, (G.nz + BY - 1) / BY); }
+// from the first interior point on: one tile less where the grid's columns and
+// rows are multiples of the tile, and with it the last, nearly empty round
+inline dim3 interior_grid(const Grid &G) { return dim3((G.nx - 2 + BX - 1) / BX, (G.nz - 2 + BY - 1) / BY); }
 
 // MicroPhysics::autoconversion, accretion, evaporation, condensation
 // (MicroPhysics.cpp:29-51, 54-77, 80-114, 7-26).  Each is pointwise, so
@@ -36,13 +39,12 @@ enum { KP_AUTO = 1, KP_ACCR = 2, KP_EVAP = 4, KP_COND = 8, KP_NEG = 16, KP_ALL =
 
 template <int PROC>
 __global__ void __launch_bounds__(BX *BY) k_kessler(Grid G, StepPtrs S, RedSlot rs) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+    const int i = 1 + blockIdx.x * BX + threadIdx.x, k = 1 + blockIdx.y * BY + uniform(threadIdx.y);
     const bool inside = (i >= 1 && i <= G.nx - 2 && k >= 1 && k <= G.nz - 2);
     double part[6] = {0., 0., 0., 0., 0., 0.};
     if (inside) {
-        const size_t p = ix(G, i, k);
         const double dt = G.dt, pib = S.P.pib[k], rhou = S.P.rhou[k], pb = S.P.pb[k], pc = S.P.pcoef[k];
-        double qc = S.fut[F_QC][p], qr = S.fut[F_QR][p], qv = S.fut[F_QV][p], th = S.fut[F_TH][p];
+        double qc = at(S.fut[F_QC], G, i, k), qr = at(S.fut[F_QR], G, i, k), qv = at(S.fut[F_QV], G, i, k), th = at(S.fut[F_TH], G, i, k);
         if constexpr ((PROC & KP_AUTO) != 0) {  // autoconversion
             const double qcplus = maxs(0., qc);
             double ar = 0.001 * (qcplus - 0.001);
@@ -50,28 +52,32 @@ __global__ void __launch_bounds__(BX *BY) k_kessler(Grid G, StepPtrs S, RedSlot 
             const double arcrdt = mins(ar * dt, qcplus);
             qc = qc - arcrdt;
             qr = qr + arcrdt;
-            S.autoc[p] = arcrdt;
+            at(S.autoc, G, i, k) = arcrdt;
         }
         if constexpr ((PROC & KP_ACCR) != 0) {  // accretion
             const double qcplus = maxs(0., qc), qrplus = maxs(0., qr);
-            const double cr = 2.2 * qcplus * (pow(qrplus, 0.875));
+            // no rain, over most of a domain: the power is zero
+            const double cr = 2.2 * qcplus * (qrplus == 0. ? 0. : pow(qrplus, 0.875));
             const double arcrdt = mins(cr * dt, qcplus);
             qc = qc - arcrdt;
             qr = qr + arcrdt;
-            S.accr[p] = arcrdt;
+            at(S.accr, G, i, k) = arcrdt;
         }
         if constexpr ((PROC & KP_EVAP) != 0) {  // rain evaporation
             const double qrplus = maxs(0., qr), qvplus = maxs(0., qv);
-            const double qvs = pc * exp(17.27 * (pib * th - 273.) / (pib * th - 36.));
-            const double deficit = maxs((1. - qvplus / qvs), 0.);
-            const double coef = 1.6 + 124.9 * pow((1E-3 * rhou * qrplus), 0.2046);
-            const double er = coef * deficit * (pow(1E-3 * rhou * qrplus, 0.525)) /
-                              ((5.4E5 + 2.55E6 / (1E-2 * pb * qvs)) * 1E-3 * rhou);
-            const double erdt = mins(qrplus, maxs(0., er * dt));
+            double erdt = 0.;
+            if (qrplus != 0.) {  // otherwise nothing evaporates: erdt = min(0, ..)
+                const double qvs = pc * exp(17.27 * (pib * th - 273.) / (pib * th - 36.));
+                const double deficit = maxs((1. - qvplus / qvs), 0.);
+                const double coef = 1.6 + 124.9 * pow((1E-3 * rhou * qrplus), 0.2046);
+                const double er = coef * deficit * (pow(1E-3 * rhou * qrplus, 0.525)) /
+                                  ((5.4E5 + 2.55E6 / (1E-2 * pb * qvs)) * 1E-3 * rhou);
+                erdt = mins(qrplus, maxs(0., er * dt));
+            }
             qr = qr - erdt;
             qv = qv + erdt;
             th = th - G.Lv * erdt / (G.Cp * pib);
-            S.evap[p] = erdt;
+            at(S.evap, G, i, k) = erdt;
         }
         if constexpr ((PROC & KP_COND) != 0) {  // saturation adjustment
             const double qvs = pc * exp(17.27 * (pib * th - 273.) / (pib * th - 36.));
@@ -82,7 +88,7 @@ __global__ void __launch_bounds__(BX *BY) k_kessler(Grid G, StepPtrs S, RedSlot 
             qv = qv - C;
             qc = qc + C;
             th = th + G.Lv / (G.Cp * pib) * C;
-            S.cond[p] = C;
+            at(S.cond, G, i, k) = C;
         }
         double q3[3] = {qv, qc, qr};
         if constexpr ((PROC & KP_NEG) != 0) {
@@ -99,10 +105,10 @@ __global__ void __launch_bounds__(BX *BY) k_kessler(Grid G, StepPtrs S, RedSlot 
         constexpr bool wc = (PROC & (KP_AUTO | KP_ACCR | KP_COND | KP_NEG)) != 0;
         constexpr bool wr = (PROC & (KP_AUTO | KP_ACCR | KP_EVAP | KP_NEG)) != 0;
         constexpr bool wt = (PROC & (KP_EVAP | KP_COND)) != 0;
-        if (wv) S.fut[F_QV][p] = q3[0];
-        if (wc) S.fut[F_QC][p] = q3[1];
-        if (wr) S.fut[F_QR][p] = q3[2];
-        if (wt) S.fut[F_TH][p] = th;
+        if (wv) at(S.fut[F_QV], G, i, k) = q3[0];
+        if (wc) at(S.fut[F_QC], G, i, k) = q3[1];
+        if (wr) at(S.fut[F_QR], G, i, k) = q3[2];
+        if (wt) at(S.fut[F_TH], G, i, k) = th;
     }
     if constexpr ((PROC & KP_NEG) != 0) block_partials<6>(part, rs);
 }
@@ -111,25 +117,23 @@ __global__ void __launch_bounds__(BX *BY) k_kessler(Grid G, StepPtrs S, RedSlot 
 // field: the first pass zeroes the negatives and sums positives and
 // negatives (k_finalize forms the ratio), the second rescales.
 __global__ void __launch_bounds__(BX *BY) k_negval_sums(Grid G, double *a, RedSlot rs) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + uniform(threadIdx.y);
     double part[2] = {0., 0.};
     if (i >= 1 && i <= G.nx - 2 && k >= 1 && k <= G.nz - 2) {
-        const size_t p = ix(G, i, k);
-        const double v = a[p];
+        const double v = at(a, G, i, k);
         if (v >= 0.) part[0] += v;
         else {
             part[1] += v;
-            a[p] = 0.;
+            at(a, G, i, k) = 0.;
         }
     }
     block_partials<2>(part, rs);
 }
 __global__ void __launch_bounds__(BX *BY) k_negval_scale(Grid G, double *a, const double *ratio) {
-    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + threadIdx.y;
+    const int i = blockIdx.x * BX + threadIdx.x, k = blockIdx.y * BY + uniform(threadIdx.y);
     if (i < 1 || i > G.nx - 2 || k < 1 || k > G.nz - 2) return;
     const double r = *ratio;
-    const size_t p = ix(G, i, k);
-    if (r >= 0. && a[p] > 0) a[p] = a[p] * r;
+    if (r >= 0. && at(a, G, i, k) > 0) at(a, G, i, k) = at(a, G, i, k) * r;
 }
 
 // Turbulence::RKM_RKH coefficient part (Turbulent.cpp:13-45), with the
@@ -137,11 +141,11 @@ __global__ void __launch_bounds__(BX *BY) k_negval_scale(Grid G, double *a, cons
 __device__ inline double turb_point(const Grid &G, const StepPtrs &S, int i, int k) {
     const double *u = S.u, *w = S.w, *thp = S.fut[F_TH];
     const double Rz =
-        0.5 * ((w[ix(G, i + 1, k + 1)] + w[ix(G, i + 1, k)]) - (w[ix(G, i - 1, k + 1)] + w[ix(G, i - 1, k)])) * G.r2dx +
-        0.5 * ((u[ix(G, i + 1, k + 1)] + u[ix(G, i, k + 1)]) - (u[ix(G, i + 1, k - 1)] + u[ix(G, i, k - 1)])) * G.r2dz;
-    const double dv = (u[ix(G, i + 1, k)] - u[ix(G, i, k)]) * G.rdx + (w[ix(G, i, k + 1)] - w[ix(G, i, k)]) * G.rdz;
+        0.5 * ((at(w, G, i + 1, k + 1) + at(w, G, i + 1, k)) - (at(w, G, i - 1, k + 1) + at(w, G, i - 1, k))) * G.r2dx +
+        0.5 * ((at(u, G, i + 1, k + 1) + at(u, G, i, k + 1)) - (at(u, G, i + 1, k - 1) + at(u, G, i, k - 1))) * G.r2dz;
+    const double dv = (at(u, G, i + 1, k) - at(u, G, i, k)) * G.rdx + (at(w, G, i, k + 1) - at(w, G, i, k)) * G.rdz;
     const double Ro = dv * dv;
-    const double Ri = (G.GRAVITY / thp[ix(G, i, k)] * (thp[ix(G, i, k + 1)] - thp[ix(G, i, k - 1)]) * G.r2dz) /
+    const double Ri = (G.GRAVITY / at(thp, G, i, k) * (at(thp, G, i, k + 1) - at(thp, G, i, k - 1)) * G.r2dz) /
                       (Rz * Rz + 2. * Ro);
     const double l2 = S.P.lambda2[k];
     double km, kh;
@@ -165,14 +169,16 @@ __device__ inline double turb_point(const Grid &G, const StepPtrs &S, int i, int
     return max_or_nan(km, kh);
 }
 
-// At most kTurbBlocks workgroups walk the tiles; each leaves the largest
+constexpr int TBY = 16;
+// At most kTurbBlocks workgroups walk the tiles (few and large: every one ends
+// with a store to host memory, and 1089 of them made the kernel 2 us longer); each leaves the largest
 // coefficient it formed in kmax, from which the host chooses the diffusion
 // sweep.  A NaN (unstable stratification at rest: Ri = -inf) stays one.
-__global__ void __launch_bounds__(BX *BY) k_turb_coeffs(Grid G, StepPtrs S, double *kmax) {
-    const int tx = (G.nx + BX - 1) / BX, nt = tx * ((G.nz + BY - 1) / BY);
+__global__ void __launch_bounds__(BX *TBY) k_turb_coeffs(Grid G, StepPtrs S, double *kmax) {
+    const int tx = (G.nx - 2 + BX - 1) / BX, nt = tx * ((G.nz - 2 + TBY - 1) / TBY);
     double m = 0.;
     for (int t = blockIdx.x; t < nt; t += gridDim.x) {
-        const int i = (t % tx) * BX + threadIdx.x, k = (t / tx) * BY + threadIdx.y;
+        const int i = 1 + (t % tx) * BX + threadIdx.x, k = 1 + (t / tx) * TBY + uniform(threadIdx.y);
         if (i < 1 || i > G.nx - 2 || k < 1 || k > G.nz - 2) continue;
         const double v = turb_point(G, S, i, k);
         m = max_or_nan(m, v);
@@ -182,11 +188,11 @@ __global__ void __launch_bounds__(BX *BY) k_turb_coeffs(Grid G, StepPtrs S, doub
         const double o = __shfl_xor(m, off, kWave);
         m = max_or_nan(m, o);
     }
-    __shared__ double sh[BY];
+    __shared__ double sh[TBY];
     if (threadIdx.x == 0) sh[threadIdx.y] = m;
     __syncthreads();
     if (threadIdx.x == 0 && threadIdx.y == 0) {
-        for (int w = 1; w < BY; w++) m = max_or_nan(m, sh[w]);
+        for (int w = 1; w < TBY; w++) m = max_or_nan(m, sh[w]);
         __hip_atomic_store(kmax + blockIdx.x, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
@@ -245,17 +251,17 @@ __global__ void __launch_bounds__(256) k_update_mean(Grid G, StepPtrs S, int shi
 
 }  // namespace
 
-void launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipStream_t st) {
-    hipLaunchKernelGGL(k_kessler<KP_ALL>, grid2d(G), dim3(BX, BY), 0, st, G, S, rs);
-    finalize<6>(rs, nblocks(grid2d(G)), S.s, RED_NEGVAL, S_NEG_RATIO, st);
+int launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipStream_t st) {
+    hipLaunchKernelGGL(k_kessler<KP_ALL>, interior_grid(G), dim3(BX, BY), 0, st, G, S, rs);
+    return negval_partials(S, rs, nblocks(interior_grid(G)), st);
 }
 void launch_kessler_process(const Grid &G, const StepPtrs &S, int process, hipStream_t st) {
     const RedSlot none{nullptr, 0};
     switch (process) {
-        case 0: hipLaunchKernelGGL(k_kessler<KP_AUTO>, grid2d(G), dim3(BX, BY), 0, st, G, S, none); break;
-        case 1: hipLaunchKernelGGL(k_kessler<KP_ACCR>, grid2d(G), dim3(BX, BY), 0, st, G, S, none); break;
-        case 2: hipLaunchKernelGGL(k_kessler<KP_EVAP>, grid2d(G), dim3(BX, BY), 0, st, G, S, none); break;
-        default: hipLaunchKernelGGL(k_kessler<KP_COND>, grid2d(G), dim3(BX, BY), 0, st, G, S, none); break;
+        case 0: hipLaunchKernelGGL(k_kessler<KP_AUTO>, interior_grid(G), dim3(BX, BY), 0, st, G, S, none); break;
+        case 1: hipLaunchKernelGGL(k_kessler<KP_ACCR>, interior_grid(G), dim3(BX, BY), 0, st, G, S, none); break;
+        case 2: hipLaunchKernelGGL(k_kessler<KP_EVAP>, interior_grid(G), dim3(BX, BY), 0, st, G, S, none); break;
+        default: hipLaunchKernelGGL(k_kessler<KP_COND>, interior_grid(G), dim3(BX, BY), 0, st, G, S, none); break;
     }
 }
 void launch_negative_value(const Grid &G, const StepPtrs &S, double *a, const RedSlot &rs, hipStream_t st) {
@@ -264,8 +270,9 @@ void launch_negative_value(const Grid &G, const StepPtrs &S, double *a, const Re
     hipLaunchKernelGGL(k_negval_scale, grid2d(G), dim3(BX, BY), 0, st, G, a, S.s + S_NEG_RATIO);
 }
 int launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, double *kmax, hipStream_t st) {
-    const int nt = nblocks(grid2d(G)), nb = nt < kTurbBlocks ? nt : kTurbBlocks;
-    hipLaunchKernelGGL(k_turb_coeffs, dim3(nb), dim3(BX, BY), 0, st, G, S, kmax);
+    const int nt = ((G.nx - 2 + BX - 1) / BX) * ((G.nz - 2 + TBY - 1) / TBY), turns = (nt + kTurbBlocks - 1) / kTurbBlocks,
+              nb = (nt + turns - 1) / turns;
+    hipLaunchKernelGGL(k_turb_coeffs, dim3(nb), dim3(BX, TBY), 0, st, G, S, kmax);
     return nb;
 }
 

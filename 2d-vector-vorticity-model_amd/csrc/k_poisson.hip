@@ -219,127 +219,127 @@ __device__ inline double block_excl_sum(double v, double *total) {
     return (lane == 0) ? wpre : wpre + below;
 }
 
-// Top row: h (mean removed), the periodic 1-D problem G y = h solved in
-// closed form through its first differences D_r = y_r - y_{r-1}:
+// The residual's norms, one pair of partial sums per workgroup: block of nblk
+// 1024-thread workgroups, each walking 64 x 16 tiles.
+__device__ inline void residual_norms(const Residual &R, int block, int nblk) {
+    constexpr int RX = 64, RY = 16;
+    const int N = R.N, M = R.M, tx = (N + RX - 1) / RX, nt = tx * ((M + RY - 1) / RY);
+    double part[2] = {0., 0.};
+    for (int t = block; t < nt; t += nblk) {
+        const int i = (t % tx) * RX + threadIdx.x % RX, j = 1 + (t / tx) * RY + threadIdx.x / RX;
+        if (i < N && j <= M) {
+            const double fv = R.f[size_t(j) * N + i];
+            const double wr = R.wD[j] * (fv - applyL(R.x, N, i, j, R.cx[j], R.cu[j], R.cu[j - 1])), wb = R.wD[j] * fv;
+            part[0] += wr * wr;
+            part[1] += wb * wb;
+        }
+    }
+    block_sum<2>(part);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(R.hres + 2 * block, part[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(R.hres + 2 * block + 1, part[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// cal_u.  Top row: h (mean removed), the periodic 1-D problem G y = h solved
+// in closed form through its first differences D_r = y_r - y_{r-1}:
 // D_{r+1} - D_r = h_r and sum_r D_r = 0, so D_r = S_r - mean(S) with S the
 // exclusive prefix sum of h.  uxi = D rdx (mean removed as in the
-// reference), u[i][nz-2] = uxi + ubarTopp, and xi = the mean-free y.
-__global__ void __launch_bounds__(1024) k_calu_top(Grid G, StepPtrs S) {
-    extern __shared__ double sh[];  // N doubles
-    const int N = G.nx - 2, nz = G.nz;
-    const int E = (N + blockDim.x - 1) / blockDim.x;
-    const int r0 = threadIdx.x * E;
-    const double *w = S.w, *rhow = S.P.rhow, *rhou = S.P.rhou;
-    // h and its mean (src/PoissonSolver.cpp:585-594)
+// reference), u[i][nz-2] = uxi + ubarTopp, and xi = the mean-free y.  With P
+// the prefix sum of h as it is, S_r = P_r - r mean(h).
+//
+// Then the downward integration u[i][k] = u[i][nz-2] - dz sum_{k'=k}^{nz-3}
+// ((w[i][k'+1]-w[i-1][k'+1]) rdx - rhow[k'+1] zetap[i][k'+1]) (:643-650):
+// UW columns x UC vertical chunks per block (narrow blocks, so that there are
+// enough workgroups for every CU), chunk sums scanned in LDS.
+//
+// Every workgroup forms the whole top row's prefix sums for its own 16
+// columns, three block scans of about half a microsecond: cheaper than a
+// kernel of one workgroup before this one (13 us at 2048 columns, 11 at 128).
+// The workgroups from ncol on form the residual norms of the solve that left
+// w, which would be a launch of 4 to 5 us.
+constexpr int UW = 16, UC = 64;
+__global__ void __launch_bounds__(UW *UC) k_calu(Grid G, StepPtrs S, int ncol, Residual R) {
+    extern __shared__ double sh[];  // N doubles: P
+    __shared__ double cs[UC][UW], top[UW];
+    if (int(blockIdx.x) >= ncol) {
+        residual_norms(R, blockIdx.x - ncol, gridDim.x - ncol);
+        return;
+    }
+    const int N = G.nx - 2, nz = G.nz, tid = threadIdx.x;
+    const double *w = S.w, *zp = S.fut[F_ZETA], *rhow = S.P.rhow, *rhou = S.P.rhou;
+    const int i = 1 + blockIdx.x * UW + tid % UW, c = tid / UW;
+    const int K = nz - 3;  // levels nz-3 .. 1
+    const int C = (K + UC - 1) / UC;
+    const bool col = (i <= N);
+    auto term = [&](int k) {  // level k's part of the integral
+        return ((w[ix(G, i, k + 1)] - w[ix(G, i - 1, k + 1)]) * G.rdx - rhow[k + 1] * zp[ix(G, i, k + 1)]) * -G.dz;
+    };
     double loc = 0.;
-    for (int e = 0; e < E; e++) {
-        const int r = r0 + e;
-        if (r >= N) break;
+    if (col)
+        for (int kk = c * C; kk < min((c + 1) * C, K); kk++) loc += term(nz - 3 - kk);
+    cs[c][tid % UW] = loc;
+
+    const int E = (N + UW * UC - 1) / (UW * UC), r0 = tid * E, r1 = min(r0 + E, N);
+    loc = 0.;
+    for (int r = r0; r < r1; r++) {  // src/PoissonSolver.cpp:585-594
         const double h = -(0. - rhow[nz - 2] * w[ix(G, r + 1, nz - 2)]) / rhou[nz - 2] * G.dx;
         sh[r] = h;
         loc += h;
     }
     double tot;
-    block_excl_sum(loc, &tot);
-    const double hm = tot / (N);
-    loc = 0.;
-    for (int e = 0; e < E; e++) {
-        const int r = r0 + e;
-        if (r >= N) break;
-        sh[r] = sh[r] - hm;
-        loc += sh[r];
-    }
-    // exclusive prefix S_r of h, written over h
-    double pre = block_excl_sum(loc, &tot);
-    double sloc = 0.;
-    for (int e = 0; e < E; e++) {
-        const int r = r0 + e;
-        if (r >= N) break;
+    double p = block_excl_sum(loc, &tot);
+    const double hm = tot / N;
+    double sp = 0.;
+    for (int r = r0; r < r1; r++) {
         const double h = sh[r];
-        sh[r] = pre;
-        sloc += pre;
-        pre += h;
+        sh[r] = p;
+        sp += p;
+        p += h;
     }
-    block_excl_sum(sloc, &tot);
-    const double D0 = -tot / N;
-    // uxi = D rdx, then its mean removed (:621-634)
-    double usum = 0.;
-    for (int e = 0; e < E; e++) {
-        const int r = r0 + e;
-        if (r >= N) break;
-        const double D = D0 + sh[r];
-        sh[r] = D;
-        usum += D * G.rdx;
-    }
-    block_excl_sum(usum, &tot);
-    const double um = tot / (N);
+    block_excl_sum(sp, &tot);
+    const double sm = tot / N - hm * (0.5 * (N - 1));
+    auto D = [&](int r) { return sh[r] - r * hm - sm; };
+    double sd = 0.;
+    for (int r = r0; r < r1; r++) sd += D(r);
+    double y = block_excl_sum(sd, &tot);
+    const double um = tot * G.rdx / N;  // :621-634
     const double ubp = S.s[S_UBARTOPP];
-    for (int e = 0; e < E; e++) {
-        const int r = r0 + e;
-        if (r >= N) break;
-        const double uxi = sh[r] * G.rdx - um;
+    const int b0 = blockIdx.x * UW;
+    for (int r = max(r0, b0); r < min(r1, b0 + UW); r++) {
+        const double uxi = D(r) * G.rdx - um;
         S.uxi[r + 1] = uxi;
         if (r + 1 == N) S.uxi[0] = uxi;
         if (r == 0) S.uxi[N + 1] = uxi;
+        top[r - b0] = uxi + ubp;
         store_center(S.u, G, r + 1, nz - 2, uxi + ubp);
     }
-    // xi: y_r = sum_{j<=r} D_j minus its mean (min-norm solution)
-    double dl = 0.;
-    for (int e = 0; e < E; e++) {
-        const int r = r0 + e;
-        if (r >= N) break;
-        dl += (r == 0) ? 0. : sh[r];
-    }
-    double ypre = block_excl_sum(dl, &tot);
-    double ysum = 0.;
-    for (int e = 0; e < E; e++) {
-        const int r = r0 + e;
-        if (r >= N) break;
-        ypre += (r == 0) ? 0. : sh[r];
-        ysum += ypre;
-    }
-    block_excl_sum(ysum, &tot);
-    const double ym = tot / N;
-    ypre = block_excl_sum(dl, &tot);
-    for (int e = 0; e < E; e++) {
-        const int r = r0 + e;
-        if (r >= N) break;
-        ypre += (r == 0) ? 0. : sh[r];
-        const double xi = ypre - ym;
-        S.xi[r + 1] = xi;
-        if (r + 1 == N) S.xi[0] = xi;
-        if (r == 0) S.xi[N + 1] = xi;
-    }
-}
-
-// Downward integration u[i][k] = u[i][nz-2] - dz sum_{k'=k}^{nz-3}
-// ((w[i][k'+1]-w[i-1][k'+1]) rdx - rhow[k'+1] zetap[i][k'+1]) (:643-650):
-// UW columns x UC vertical chunks per block (narrow blocks, so that the
-// 2-D grid has enough workgroups for every CU), chunk sums scanned in LDS.
-constexpr int UW = 16, UC = 64;
-__global__ void __launch_bounds__(UW *UC) k_calu_cols(Grid G, StepPtrs S) {
-    __shared__ double cs[UC][UW];
-    const int i = 1 + blockIdx.x * UW + threadIdx.x, c = threadIdx.y;
-    const int K = G.nz - 3;  // levels nz-3 .. 1
-    const int C = (K + UC - 1) / UC;
-    const bool col = (i <= G.nx - 2);
-    const double *w = S.w, *zp = S.fut[F_ZETA], *rhow = S.P.rhow;
-    double loc = 0.;
-    if (col) {
-        for (int kk = c * C; kk < min((c + 1) * C, K); kk++) {
-            const int k = G.nz - 3 - kk;
-            loc += ((w[ix(G, i, k + 1)] - w[ix(G, i - 1, k + 1)]) * G.rdx - rhow[k + 1] * zp[ix(G, i, k + 1)]) * -G.dz;
+    if (blockIdx.x == 0) {
+        // xi: y_r = sum_{j<=r} D_j minus its mean (min-norm solution)
+        double sy = 0., yr = y;
+        for (int r = r0; r < r1; r++) {
+            yr += D(r);
+            sy += yr;
+        }
+        block_excl_sum(sy, &tot);
+        const double ym = tot / N;
+        yr = y;
+        for (int r = r0; r < r1; r++) {
+            yr += D(r);
+            const double xi = yr - ym;
+            S.xi[r + 1] = xi;
+            if (r + 1 == N) S.xi[0] = xi;
+            if (r == 0) S.xi[N + 1] = xi;
         }
     }
-    cs[c][threadIdx.x] = loc;
-    __syncthreads();
+    __syncthreads();  // top
     if (!col) return;
     double area = 0.;
-    for (int c2 = 0; c2 < c; c2++) area += cs[c2][threadIdx.x];
-    const double utop = S.u[ix(G, i, G.nz - 2)];
+    for (int c2 = 0; c2 < c; c2++) area += cs[c2][tid % UW];
+    const double utop = top[tid % UW];
     for (int kk = c * C; kk < min((c + 1) * C, K); kk++) {
-        const int k = G.nz - 3 - kk;
-        area += ((w[ix(G, i, k + 1)] - w[ix(G, i - 1, k + 1)]) * G.rdx - rhow[k + 1] * zp[ix(G, i, k + 1)]) * -G.dz;
+        const int k = nz - 3 - kk;
+        area += term(k);
         store_center(S.u, G, i, k, area + utop);
     }
 }
@@ -897,9 +897,11 @@ SolveResult Poisson::solve_mixed(double tol, int max_sweeps, hipStream_t st) {
     return refine(direct32, tol, false, max_sweeps, st);
 }
 
-void Poisson::queue_step(const Grid &G, const double *zetap, const double *rhow_dev, double *w, bool f_ready,
-                         hipStream_t st) {
+void Poisson::queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, hipStream_t st) {
+    double *w = S.w;
+    const double *rhow_dev = S.P.rhow;
     x_pending = XF_NONE;
+    if (step >= 0 && (guess_from_net || f_ready)) launch_pubartop(G, S, step, st);
     if (guess_from_net) {
         guess_from_net = false;
         first_residual(pcg64.r, st);
@@ -916,11 +918,9 @@ void Poisson::queue_step(const Grid &G, const double *zetap, const double *rhow_
         direct64.solve(f, nullptr, pcg64.x, st);
         back_to_w(G, w, rhow_dev, st);
     } else {
-        direct64.solve_step(G, zetap, rhow_dev, f, pcg64.x, w, st);
+        direct64.solve_step(G, S, step, f, pcg64.x, st);
     }
     bn_pending = 0;
-    res_blocks = launch_residual_norms(N, M, f, pcg64.x, cx0, cu0, pcg64.wD, hres_dev, st);
-    hipEventRecord(ev_res, st);
 }
 
 SolveResult Poisson::finish_step(const Grid &G, double *w, const double *rhow_dev, double tol, bool to_floor,
@@ -954,9 +954,23 @@ SolveResult Poisson::finish_step(const Grid &G, double *w, const double *rhow_de
 bool cal_u_supported(const Grid &G) { return G.nx - 2 <= 8192; }
 
 void launch_cal_u(const Grid &G, const StepPtrs &S, hipStream_t st) {
-    const int N = G.nx - 2;
-    hipLaunchKernelGGL(k_calu_top, dim3(1), dim3(1024), size_t(N) * sizeof(double), st, G, S);
-    hipLaunchKernelGGL(k_calu_cols, dim3((N + UW - 1) / UW), dim3(UW, UC), 0, st, G, S);
+    const int N = G.nx - 2, ncol = (N + UW - 1) / UW;
+    hipLaunchKernelGGL(k_calu, dim3(ncol), dim3(UW * UC), size_t(N) * sizeof(double), st, G, S, ncol, Residual{});
+}
+
+void Poisson::queue_cal_u(const Grid &G, const StepPtrs &S, hipStream_t st) {
+    const int ncol = (N + UW - 1) / UW;
+    queue_residual(G, S, ncol, st);
+}
+
+void Poisson::queue_check(hipStream_t st) { queue_residual(Grid{}, StepPtrs{}, 0, st); }
+
+// k_calu's residual workgroups, behind ncol workgroups of cal_u
+void Poisson::queue_residual(const Grid &G, const StepPtrs &S, int ncol, hipStream_t st) {
+    res_blocks = std::min(kResidualBlocks, ((N + 63) / 64) * ((M + 15) / 16));
+    hipLaunchKernelGGL(k_calu, dim3(ncol + res_blocks), dim3(UW * UC), ncol ? size_t(N) * sizeof(double) : 0, st, G,
+                       S, ncol, Residual{N, M, f, pcg64.x, cx0, cu0, pcg64.wD, hres_dev});
+    hipEventRecord(ev_res, st);
 }
 
 }  // namespace vvmd

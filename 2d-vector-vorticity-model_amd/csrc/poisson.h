@@ -45,6 +45,15 @@ struct SolveResult {
     bool converged = false;
 };
 
+// ||wD (f - L x)||^2 and ||wD f||^2: a pair of partial sums per workgroup into
+// hres (host-mapped memory, at most kResidualBlocks pairs).
+constexpr int kResidualBlocks = 512;
+struct Residual {
+    int N, M;
+    const double *f, *x, *cx, *cu, *wD;
+    double *hres;
+};
+
 class Poisson {
    public:
     // rhou/rhow are the host profiles (nz long).  Allocates with hipMalloc.
@@ -87,14 +96,17 @@ class Poisson {
     // decreasing at FP64's round-off (kRoundOff).
     SolveResult solve_direct(double tol, bool to_floor, int max_sweeps, hipStream_t st);
     SolveResult solve_mixed(double tol, int max_sweeps, hipStream_t st);
-    // The step's cal_w in two halves.  queue_step: right-hand side (formed
-    // already if f_ready), solve, w and the residual's norms, nothing waited
-    // for; the network's guess (if learned_guess wrote one) is judged here,
-    // which does wait.  finish_step: waits for the norms and, if they miss the
-    // stop rule, corrects x further; *redo says that x and w have changed
-    // since queue_step, so what was queued behind it has to run again.
-    void queue_step(const Grid &G, const double *zetap, const double *rhow_dev, double *w, bool f_ready,
-                    hipStream_t st);
+    // The step's pubarTop_pt (not if step < 0), cal_w and cal_u in two halves.
+    // queue_step: mean flow at the top, right-hand side (formed already if f_ready), solve and
+    // w; queue_cal_u: u, and the residual's norms on their way to the host
+    // (queue_check: the norms alone).  Nothing is waited for, but the network's
+    // guess (if learned_guess wrote one) is judged in queue_step.  finish_step:
+    // waits for the norms and, if they miss the stop rule, corrects x further;
+    // *redo says that x and w have changed since queue_step, so cal_u and what
+    // was queued behind it have to run again.
+    void queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, hipStream_t st);
+    void queue_cal_u(const Grid &G, const StepPtrs &S, hipStream_t st);
+    void queue_check(hipStream_t st);
     SolveResult finish_step(const Grid &G, double *w, const double *rhow_dev, double tol, bool to_floor,
                             int max_sweeps, bool *redo, hipStream_t st);
     // The reference GPU back-end's solver (k_bicgstab.hip): BiCGSTAB with a
@@ -148,7 +160,8 @@ class Poisson {
     Direct<double> direct64;
     Direct<float> direct32;
     double *cx0 = nullptr, *cu0 = nullptr;  // coefficients of L
-    double *hres = nullptr, *hres_dev = nullptr;  // launch_residual_norms (mapped host memory)
+    double *hres = nullptr, *hres_dev = nullptr;  // k_calu's residual norms (mapped host memory)
+    void queue_residual(const Grid &G, const StepPtrs &S, int ncol, hipStream_t st);
     int res_blocks = 0;
     template <typename T>
     SolveResult refine(Direct<T> &D, double tol, bool to_floor, int max_sweeps, hipStream_t st);

@@ -352,13 +352,13 @@ int solve_w_iter(vvm_dev *h, const StepPtrs &S, vvm_solve_stats *ss, bool run_ne
     return R.converged ? VVM_OK : VVM_WARN_NOT_CONVERGED;
 }
 
-// cal_w by the direct solver: queued first, so that what follows it can be
+// pubarTop_pt (not if step < 0) and cal_w by the direct solver: queued first, so that what follows it can be
 // queued behind it, then finished, which waits for the residual's norms.
 // redo: w has changed since, and what was queued behind it has to run again.
-void queue_w(vvm_dev *h, const StepPtrs &S, bool run_net, bool prepared) {
+void queue_w(vvm_dev *h, const StepPtrs &S, int step, bool run_net, bool prepared) {
     const bool first = prepared || run_net || h->pois.sample_cap > 0;
     if (first && !prepared) prepare_guess(h, S, run_net, h->st);
-    h->pois.queue_step(h->G, S.fut[F_ZETA], h->P.rhow, S.w, first, h->st);
+    h->pois.queue_step(h->G, S, step, first, h->st);
 }
 int finish_w(vvm_dev *h, const StepPtrs &S, vvm_solve_stats *ss, bool *redo) {
     const vvm_dev_config &c = h->cfg;
@@ -798,13 +798,15 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
             prepare_guess(h, S, true, h->side);
             hipEventRecord(h->ev_guess, h->side);
         }
+        int negval;
         {
             KTimer t(h, VVM_KT_THERMO4);
-            launch_thermo4(G, S, h->step, h->red.negval, h->st);
+            negval = launch_thermo4(G, S, h->step, h->red.negval, h->st);
         }
         {
             KTimer t(h, VVM_KT_SCALE);
-            launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st);
+            launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st,
+                                 h->red.negval, negval);
         }
         if (h->ghosts_dirty) {
             launch_bc_uw(G, S, h->st);
@@ -823,29 +825,30 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
             rec(6, cs);
             {
                 KTimer t(h, VVM_KT_KESSLER, cs);
-                launch_kessler(G, S, h->red.negval, cs);
+                negval = launch_kessler(G, S, h->red.negval, cs);
             }
             {
                 KTimer t(h, VVM_KT_SCALE, cs);
-                launch_scale_forcing(G, S, false, false, false, cs);
+                launch_scale_forcing(G, S, false, false, false, cs, h->red.negval, negval);
             }
             rec(7, cs);
         }
         if (overlap) hipEventRecord(h->ev_join, h->side);
         // B: pubarTop_pt, cal_w, cal_u (:292-296)
-        launch_pubartop(G, S, h->step, h->st);
         vvm_solve_stats ss{};
         int rc;
         const bool direct = uses_direct(c);
+        if (!direct) launch_pubartop(G, S, h->step, h->st);
         {
             KTimer t(h, VVM_KT_SOLVE);
             if (early_guess) hipStreamWaitEvent(h->st, h->ev_guess, 0);
-            if (direct) queue_w(h, S, run_net, early_guess);
+            if (direct) queue_w(h, S, h->step, run_net, early_guess);
             else rc = solve_w_iter(h, S, &ss, run_net, early_guess);
         }
         {
             KTimer t(h, VVM_KT_CALU);
-            launch_cal_u(G, S, h->st);
+            if (direct) h->pois.queue_cal_u(G, S, h->st);
+            else launch_cal_u(G, S, h->st);
         }
         // The direct solve is finished (its residual read) as late as what
         // follows can still be run again: with the tiled diffusion sweep, which
@@ -968,13 +971,14 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             launch_pzeta(G, S, h->step, h->st);
             break;
         case VVM_OP_PSCALARS:
-            launch_thermo4(G, S, h->step, h->red.negval, h->st);
-            launch_scale_forcing(G, S, false, false, false, h->st);
+            launch_scale_forcing(G, S, false, false, false, h->st, h->red.negval,
+                                 launch_thermo4(G, S, h->step, h->red.negval, h->st));
             break;
         case VVM_OP_FORCING_BC: {
             const double none[3] = {-1., -1., -1.};
             HIPCHK(h, hipMemcpyAsync(h->s + S_NEG_RATIO, none, sizeof(none), hipMemcpyHostToDevice, h->st));
-            launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st);
+            launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st,
+                                 h->red.negval, 0);
             launch_bc_all_prog(G, S, h->st);
             break;
         }
@@ -986,7 +990,8 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             h->cfg.guess_mode = VVM_GUESS_ZERO;
             if (uses_direct(h->cfg)) {
                 bool redo = false;
-                queue_w(h, S, false, false);
+                queue_w(h, S, -1, false, false);
+                h->pois.queue_check(h->st);
                 rc = finish_w(h, S, nullptr, &redo);
             } else {
                 rc = solve_w_iter(h, S, nullptr, false, false);
@@ -998,8 +1003,8 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             launch_cal_u(G, S, h->st);
             break;
         case VVM_OP_MICROPHYSICS:
-            launch_kessler(G, S, h->red.negval, h->st);
-            launch_scale_forcing(G, S, false, false, false, h->st);
+            launch_scale_forcing(G, S, false, false, false, h->st, h->red.negval,
+                                 launch_kessler(G, S, h->red.negval, h->st));
             launch_bc_all_prog(G, S, h->st);
             break;
         case VVM_OP_TURBULENCE:
@@ -1101,7 +1106,7 @@ int vvm_dev_op_field(vvm_dev_t *h, int op, int field) {
             const double none[3] = {-1., -1., -1.};
             HIPCHK(h, hipMemcpyAsync(h->s + S_NEG_RATIO, none, sizeof(none), hipMemcpyHostToDevice, h->st));
             launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st,
-                                 false);
+                                 h->red.negval, 0, false);
             break;
         }
         default: return fail(h, VVM_ERR_ARG, "unknown op");

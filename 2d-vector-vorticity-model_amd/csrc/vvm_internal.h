@@ -71,9 +71,13 @@ struct Reductions {
 // ------------------------------------------------------------ launchers
 // Dynamics (k_dynamics.hip)
 void launch_pzeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st);
-void launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);
+// launch_thermo4 and launch_kessler leave NegativeValueProcess's first pass;
+// what they return (negval_partials) goes to the launch_scale_forcing behind
+// them, with rs.
+int launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);
+int negval_partials(const StepPtrs &S, const RedSlot &rs, int nblk, hipStream_t st);
 void launch_scale_forcing(const Grid &G, const StepPtrs &S, bool forcing, bool tropical, bool random_kick,
-                          hipStream_t st, bool halos = true);
+                          hipStream_t st, const RedSlot &rs, int nblk, bool halos = true);
 void launch_bc_uw(const Grid &G, const StepPtrs &S, hipStream_t st);
 void launch_bc_all_prog(const Grid &G, const StepPtrs &S, hipStream_t st);
 // Whether a handle runs the microphysics phase on its second stream beside
@@ -94,10 +98,10 @@ void launch_kessler_process(const Grid &G, const StepPtrs &S, int process, hipSt
 void launch_negative_value(const Grid &G, const StepPtrs &S, double *a, const RedSlot &rs, hipStream_t st);
 
 // Physics (k_physics.hip)
-void launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipStream_t st);
+int launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipStream_t st);
 // kmax (host-mapped, kTurbBlocks doubles): the largest RKM or RKH each
 // workgroup formed; returns their count.
-constexpr int kTurbBlocks = 512;
+constexpr int kTurbBlocks = 640;
 int launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, double *kmax, hipStream_t st);
 bool diffusion_supported(const Grid &G);  // nx - 2 <= 8192
 // nudge bit 0 fuses Nudge_theta, bit 1 Nudge_zeta into the sweep's store;
