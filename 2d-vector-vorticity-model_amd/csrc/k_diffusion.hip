@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(kMaxWaves *kWave) k_diff_sweep(Grid G, StepPtr
     const bool mpar = (fld == F_ZETA);
     const double *rate = mpar ? ((nudge & 2) ? S.P.rate_z : nullptr) : ((fld == F_TH && (nudge & 1)) ? S.P.rate_th : nullptr);
     sweep<E>(G, S.fut[fld], S.dcoef[mpar ? DC_AM : DC_AH], S.dcoef[DC_C0 + fld], S.dcoef[mpar ? DC_DM : DC_DH], rate,
-             fld == F_TH, S.P.thb_init, carry, S.s + S_DIFF_ERR);
+             fld == F_TH, S.P.thb_init, carry, S.sweep_err);
 }
 
 // ---------------------------------------------------------------------------
@@ -370,7 +370,7 @@ __global__ void __launch_bounds__((CW + 1) * kWave) k_diff_strips(Grid G, StepPt
     const unsigned long long *in = (s > 0) ? S.dslots + (size_t(fld) * nstrip + (s - 1)) * nz : nullptr;
     unsigned long long *out = (s + 1 < nstrip) ? S.dslots + (size_t(fld) * nstrip + s) * nz : nullptr;
     if (w == cw) {
-        courier(in, out, cin, carry + size_t(cw - 1) * nz, nz, S.s + S_DIFF_ERR);
+        courier(in, out, cin, carry + size_t(cw - 1) * nz, nz, S.sweep_err);
         return;
     }
     const bool mpar = (fld == F_ZETA);
@@ -491,7 +491,7 @@ __global__ void __launch_bounds__((CW + 1) * kWave) k_diff_strips(Grid G, StepPt
             int spins = 0;
             while (bits == kEmpty && !gave_up) {
                 if (++spins > kSpinLimit) {
-                    S.s[S_DIFF_ERR] = 1.;
+                    *S.sweep_err = 1.;
                     gave_up = true;
                 }
                 bits = lds_load(src + k);

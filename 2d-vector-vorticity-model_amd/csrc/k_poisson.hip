@@ -927,7 +927,6 @@ SolveResult Poisson::finish_step(const Grid &G, double *w, const double *rhow_de
                                  int max_sweeps, bool *redo, hipStream_t st) {
     SolveResult R;
     *redo = false;
-    hipEventSynchronize(ev_res);
     double rn2 = 0., bn2 = 0.;
     const volatile double *p = hres;
     for (int b = 0; b < res_blocks; b++) {  // fixed order: deterministic
@@ -970,7 +969,6 @@ void Poisson::queue_residual(const Grid &G, const StepPtrs &S, int ncol, hipStre
     res_blocks = std::min(kResidualBlocks, ((N + 63) / 64) * ((M + 15) / 16));
     hipLaunchKernelGGL(k_calu, dim3(ncol + res_blocks), dim3(UW * UC), ncol ? size_t(N) * sizeof(double) : 0, st, G,
                        S, ncol, Residual{N, M, f, pcg64.x, cx0, cu0, pcg64.wD, hres_dev});
-    hipEventRecord(ev_res, st);
 }
 
 }  // namespace vvmd

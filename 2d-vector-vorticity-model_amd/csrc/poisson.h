@@ -100,9 +100,9 @@ class Poisson {
     // queue_step: mean flow at the top, right-hand side (formed already if f_ready), solve and
     // w; queue_cal_u: u, and the residual's norms on their way to the host
     // (queue_check: the norms alone).  Nothing is waited for, but the network's
-    // guess (if learned_guess wrote one) is judged in queue_step.  finish_step:
-    // waits for the norms and, if they miss the stop rule, corrects x further;
-    // *redo says that x and w have changed since queue_step, so cal_u and what
+    // guess (if learned_guess wrote one) is judged in queue_step.  finish_step
+    // (the caller has waited for queue_cal_u's or queue_check's work): if the
+    // norms miss the stop rule, corrects x further; *redo says that x and w have changed since queue_step, so cal_u and what
     // was queued behind it have to run again.
     void queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, hipStream_t st);
     void queue_cal_u(const Grid &G, const StepPtrs &S, hipStream_t st);

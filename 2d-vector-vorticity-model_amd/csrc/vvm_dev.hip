@@ -41,7 +41,7 @@ struct vvm_dev {
     // the last step's coefficients and checked against this step's, which
     // k_turb_coeffs leaves in kmax (host-mapped) before ev_turb.
     int diff_halo = 0;
-    double *kmax = nullptr, *kmax_dev = nullptr;
+    double *kmax = nullptr, *kmax_dev = nullptr;  // [kTurbBlocks], then the sweep's error flag
     int kmax_blocks = 0;
     double rho_per_k = 0.;          // largest a + d of the sweep per unit of K
     hipEvent_t ev_turb = nullptr;
@@ -92,6 +92,16 @@ struct vvm_dev {
     // stream beside the scalar advection: forked after pzeta, joined before
     // the solve
     hipEvent_t ev_fork0 = nullptr, ev_guess = nullptr;
+
+    // the step that is under way (step_begin .. step_finish)
+    struct Run {
+        StepPtrs S{};
+        vvm_solve_stats ss{};
+        int rc = VVM_OK, halo = 0;
+        bool solved = true;
+        int timer = -1;     // its row of tev (-1: not timed per step)
+        bool last = false;  // its phase boundaries go to ev and ev_mp
+    } run;
 
     // per-kernel event timer (vvm_dev_kernel_timer)
     static constexpr int kKtMax = 256;
@@ -184,6 +194,7 @@ StepPtrs ptrs(vvm_dev *h) {
     for (int q = 0; q < DC_N; q++) S.dcoef[q] = h->dcoef[q];
     S.dslots = h->dslots;
     S.dstrip_cw = h->dstrip_cw;
+    S.sweep_err = h->kmax_dev + kTurbBlocks;
     return S;
 }
 
@@ -229,6 +240,8 @@ void finish_diffusion(vvm_dev *h, StepPtrs &S, int nudge, int queued) {
     if (need > queued) launch_diffusion_tiles(h->G, S, nudge, need, h->st);
     take_tiles(h, S);
 }
+
+int step_nudge(const vvm_dev_config &c) { return 1 | (c.CASE != 2 ? 2 : 0); }
 
 // m <- now <- p by rotation (src/Iteration.cpp:158-203 copies).
 void rotate(vvm_dev *h) {
@@ -372,6 +385,12 @@ int finish_w(vvm_dev *h, const StepPtrs &S, vvm_solve_stats *ss, bool *redo) {
     return R.converged ? VVM_OK : VVM_WARN_NOT_CONVERGED;
 }
 
+// after a synchronisation
+int check_sweep(vvm_dev *h) {
+    if (*static_cast<volatile double *>(h->kmax + kTurbBlocks) == 0.) return VVM_OK;
+    return fail(h, VVM_ERR_STATE, "diffusion sweep: a wavefront gave up waiting for its carry");
+}
+
 int check_launch(vvm_dev *h) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(h, VVM_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
@@ -463,10 +482,11 @@ int vvm_dev_create(const vvm_dev_config *cfg, int device, vvm_dev_t **out) {
         rs->partial = A(size_t(8) * maxb);
     }
     ok = ok &&
-         hipHostMalloc(reinterpret_cast<void **>(&h->kmax), kTurbBlocks * sizeof(double),
+         hipHostMalloc(reinterpret_cast<void **>(&h->kmax), (kTurbBlocks + 1) * sizeof(double),
                        hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess &&
          hipHostGetDevicePointer(reinterpret_cast<void **>(&h->kmax_dev), h->kmax, 0) == hipSuccess &&
          hipEventCreateWithFlags(&h->ev_turb, hipEventDisableTiming) == hipSuccess;
+    if (h->kmax) h->kmax[kTurbBlocks] = 0.;
     for (auto &e : h->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
     for (auto &e : h->ev_mp) ok = ok && hipEventCreate(&e) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&h->ev_fork0, hipEventDisableTiming) == hipSuccess &&
@@ -753,171 +773,199 @@ static int upload_random_kick(vvm_dev *h) {
     return send(h);
 }
 
+}  // extern "C": the step's two halves
+
+namespace {
+
+// Phase boundary `slot` (0-5: ev, 6-7: ev_mp) of the step, on stream s.
+void mark(vvm_dev *h, int slot, hipStream_t s) {
+    const vvm_dev::Run &r = h->run;
+    if (r.timer >= 0) hipEventRecord(h->tev[size_t(r.timer) * 8 + slot], s);
+    if (r.last) hipEventRecord(slot < 6 ? h->ev[slot] : h->ev_mp[slot - 6], s);
+}
+
+// Reads the direct solve's residual (wait: which may not have arrived yet) and
+// corrects the solve if it has to; true if w and u have changed.
+bool finish_solve(vvm_dev *h, bool wait) {
+    vvm_dev::Run &r = h->run;
+    bool redo = false;
+    if (!r.solved) {
+        if (wait) hipStreamSynchronize(h->st);
+        r.rc = finish_w(h, r.S, &r.ss, &redo);
+    }
+    r.solved = true;
+    if (redo) launch_cal_u(h->G, r.S, h->st);
+    return redo;
+}
+
+// Queues the loop body of TimeMarching up to the diffusion sweep.  The direct
+// solve's residual is read as late as what follows can still be run again:
+// with the tiled sweep, which leaves its inputs alone, that is after the sweep
+// is queued (step_finish), so that the GPU has work while the host waits, or,
+// in an ensemble, queues other members' steps.
+int step_begin(vvm_dev *h, int timer, bool last) {
+    const Grid &G = h->G;
+    const vvm_dev_config &c = h->cfg;
+    h->step++;
+    h->status_for_adding_forcing = (h->step * c.dt <= c.addforcingtime) ? 1 : 0;
+    if (h->status_for_adding_forcing) {
+        int rc = upload_random_kick(h);
+        if (rc) return rc;
+    }
+    vvm_dev::Run &r = h->run;
+    r = vvm_dev::Run();
+    r.S = ptrs(h);
+    r.timer = timer;
+    r.last = last;
+    const StepPtrs &S = r.S;
+    if (h->overlap_c && !h->mp_fn && !h->side)
+        HIPCHK(h, hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking));
+    const bool overlap = h->overlap_c && !h->mp_fn;
+    // the learned guess's network is the longest serial chain before the
+    // solve; it needs only pzeta's zetap and the past solutions
+    const bool run_net = net_due(h);
+    const bool early_guess = overlap && run_net && h->pois.sample_cap == 0;
+    mark(h, 0, h->st);
+    // A: advection, buoyancy, forcing, halos (src/Iteration.cpp:263-285)
+    {
+        KTimer t(h, VVM_KT_PZETA);
+        launch_pzeta(G, S, h->step, h->st);
+    }
+    if (early_guess) {
+        hipEventRecord(h->ev_fork0, h->st);
+        hipStreamWaitEvent(h->side, h->ev_fork0, 0);
+        prepare_guess(h, S, true, h->side);
+        hipEventRecord(h->ev_guess, h->side);
+    }
+    int negval;
+    {
+        KTimer t(h, VVM_KT_THERMO4);
+        negval = launch_thermo4(G, S, h->step, h->red.negval, h->st);
+    }
+    {
+        KTimer t(h, VVM_KT_SCALE);
+        launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st,
+                             h->red.negval, negval);
+    }
+    if (h->ghosts_dirty) {
+        launch_bc_uw(G, S, h->st);
+        h->ghosts_dirty = false;
+    }
+    mark(h, 1, h->st);
+    // C: Kessler + NegativeValueProcess x3 + halos (:303-311, 404), on
+    // the side stream while B runs; the main stream waits for it before D
+    // (with host microphysics, C runs after B on the host instead)
+    hipStream_t cs = overlap ? h->side : h->st;
+    if (overlap) {
+        hipEventRecord(h->ev_fork, h->st);
+        hipStreamWaitEvent(h->side, h->ev_fork, 0);
+    }
+    if (!h->mp_fn) {
+        mark(h, 6, cs);
+        {
+            KTimer t(h, VVM_KT_KESSLER, cs);
+            negval = launch_kessler(G, S, h->red.negval, cs);
+        }
+        {
+            KTimer t(h, VVM_KT_SCALE, cs);
+            launch_scale_forcing(G, S, false, false, false, cs, h->red.negval, negval);
+        }
+        mark(h, 7, cs);
+    }
+    if (overlap) hipEventRecord(h->ev_join, h->side);
+    // B: pubarTop_pt, cal_w, cal_u (:292-296)
+    const bool direct = uses_direct(c);
+    if (!direct) launch_pubartop(G, S, h->step, h->st);
+    {
+        KTimer t(h, VVM_KT_SOLVE);
+        if (early_guess) hipStreamWaitEvent(h->st, h->ev_guess, 0);
+        if (direct) queue_w(h, S, h->step, run_net, early_guess);
+        else r.rc = solve_w_iter(h, S, &r.ss, run_net, early_guess);
+    }
+    {
+        KTimer t(h, VVM_KT_CALU);
+        if (direct) h->pois.queue_cal_u(G, S, h->st);
+        else launch_cal_u(G, S, h->st);
+    }
+    r.halo = h->diff_halo;
+    r.solved = !direct;
+    if (h->mp_fn || r.halo == 0) finish_solve(h, true);
+    mark(h, 2, h->st);
+    if (overlap) hipStreamWaitEvent(h->st, h->ev_join, 0);
+    if (h->mp_fn) {
+        mark(h, 6, h->st);
+        const int mrc = host_microphysics(h, S);
+        if (mrc) return mrc;
+        mark(h, 7, h->st);
+    }
+    mark(h, 3, h->st);
+    // D: RKM_RKH with Mparam/Hparam, nudging (:408-417); the first
+    // updateMean (:408) is overwritten by nextTimeStep's before any read.
+    {
+        KTimer t(h, VVM_KT_TURB);
+        queue_turbulence(h, S);
+    }
+    if (r.halo) {
+        KTimer t(h, VVM_KT_DIFFUSION);
+        launch_diffusion_tiles(G, S, step_nudge(c), r.halo, h->st);
+    }
+    return check_launch(h);
+}
+
+// The rest of the step: the checks, updateMean, the rotation of the levels.
+// Adds the solve to acc.
+int step_finish(vvm_dev *h, vvm_step_stats *acc) {
+    const Grid &G = h->G;
+    const vvm_dev_config &c = h->cfg;
+    vvm_dev::Run &r = h->run;
+    StepPtrs &S = r.S;
+    hipEventSynchronize(h->ev_turb);  // the residual's norms and the coefficients' maximum are in
+    if (finish_solve(h, false)) {
+        queue_turbulence(h, S);
+        if (r.halo) launch_diffusion_tiles(G, S, step_nudge(c), r.halo, h->st);
+    }
+    finish_diffusion(h, S, step_nudge(c), r.halo);
+    if (r.rc == VVM_WARN_NOT_CONVERGED) acc->not_converged++;
+    acc->solve_iters_total += r.ss.iters;
+    acc->solve_iters_last = r.ss.iters;
+    acc->refine_last = r.ss.refine;
+    acc->rel_residual_last = r.ss.rel_residual;
+    if (c.moisture_nudge_time != 0) launch_nudge_qv(G, S, c.moisture_nudge_time, h->st);
+    mark(h, 4, h->st);
+    // E: nextTimeStep (:153-204)
+    {
+        KTimer t(h, VVM_KT_MEAN);
+        launch_update_mean(G, S, true, h->st);
+    }
+    rotate(h);
+    mark(h, 5, h->st);
+    h->stepped = true;
+    return check_launch(h);
+}
+
+}  // namespace
+
+extern "C" {
+
 int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
     if (!h || nsteps < 0) return VVM_ERR_ARG;
     if (!h->uploaded) return fail(h, VVM_ERR_STATE, "step before upload");
     HIPCHK(h, hipSetDevice(h->device));
-    const Grid &G = h->G;
-    const vvm_dev_config &c = h->cfg;
     vvm_step_stats acc{};
     const int fallbacks0 = h->pois.guess_fallbacks, skipped0 = h->pois.guess_skipped;
-    int warn = 0;
-    const bool timing = (stats != nullptr);
     auto t0 = std::chrono::steady_clock::now();
     for (int n = 0; n < nsteps; n++) {
-        h->step++;
-        h->status_for_adding_forcing = (h->step * c.dt <= c.addforcingtime) ? 1 : 0;
-        if (h->status_for_adding_forcing) {
-            int rc = upload_random_kick(h);
-            if (rc) return rc;
-        }
-        StepPtrs S = ptrs(h);
-        const bool last = (n == nsteps - 1) && timing;
-        const bool per_step = n < h->tcap;
-        // phase boundary `slot` (0-5: ev, 6-7: ev_mp) of this step, on stream s
-        auto rec = [&](int slot, hipStream_t s) {
-            if (per_step) hipEventRecord(h->tev[size_t(n) * 8 + slot], s);
-            if (last) hipEventRecord(slot < 6 ? h->ev[slot] : h->ev_mp[slot - 6], s);
-        };
-        if (h->overlap_c && !h->mp_fn && !h->side)
-            HIPCHK(h, hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking));
-        const bool overlap = h->overlap_c && !h->mp_fn;
-        // the learned guess's network is the longest serial chain before the
-        // solve; it needs only pzeta's zetap and the past solutions
-        const bool run_net = net_due(h);
-        const bool early_guess = overlap && run_net && h->pois.sample_cap == 0;
-        rec(0, h->st);
-        // A: advection, buoyancy, forcing, halos (src/Iteration.cpp:263-285)
-        {
-            KTimer t(h, VVM_KT_PZETA);
-            launch_pzeta(G, S, h->step, h->st);
-        }
-        if (early_guess) {
-            hipEventRecord(h->ev_fork0, h->st);
-            hipStreamWaitEvent(h->side, h->ev_fork0, 0);
-            prepare_guess(h, S, true, h->side);
-            hipEventRecord(h->ev_guess, h->side);
-        }
-        int negval;
-        {
-            KTimer t(h, VVM_KT_THERMO4);
-            negval = launch_thermo4(G, S, h->step, h->red.negval, h->st);
-        }
-        {
-            KTimer t(h, VVM_KT_SCALE);
-            launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st,
-                                 h->red.negval, negval);
-        }
-        if (h->ghosts_dirty) {
-            launch_bc_uw(G, S, h->st);
-            h->ghosts_dirty = false;
-        }
-        rec(1, h->st);
-        // C: Kessler + NegativeValueProcess x3 + halos (:303-311, 404), on
-        // the side stream while B runs; the main stream waits for it before D
-        // (with host microphysics, C runs after B on the host instead)
-        hipStream_t cs = overlap ? h->side : h->st;
-        if (overlap) {
-            hipEventRecord(h->ev_fork, h->st);
-            hipStreamWaitEvent(h->side, h->ev_fork, 0);
-        }
-        if (!h->mp_fn) {
-            rec(6, cs);
-            {
-                KTimer t(h, VVM_KT_KESSLER, cs);
-                negval = launch_kessler(G, S, h->red.negval, cs);
-            }
-            {
-                KTimer t(h, VVM_KT_SCALE, cs);
-                launch_scale_forcing(G, S, false, false, false, cs, h->red.negval, negval);
-            }
-            rec(7, cs);
-        }
-        if (overlap) hipEventRecord(h->ev_join, h->side);
-        // B: pubarTop_pt, cal_w, cal_u (:292-296)
-        vvm_solve_stats ss{};
-        int rc;
-        const bool direct = uses_direct(c);
-        if (!direct) launch_pubartop(G, S, h->step, h->st);
-        {
-            KTimer t(h, VVM_KT_SOLVE);
-            if (early_guess) hipStreamWaitEvent(h->st, h->ev_guess, 0);
-            if (direct) queue_w(h, S, h->step, run_net, early_guess);
-            else rc = solve_w_iter(h, S, &ss, run_net, early_guess);
-        }
-        {
-            KTimer t(h, VVM_KT_CALU);
-            if (direct) h->pois.queue_cal_u(G, S, h->st);
-            else launch_cal_u(G, S, h->st);
-        }
-        // The direct solve is finished (its residual read) as late as what
-        // follows can still be run again: with the tiled diffusion sweep, which
-        // leaves its inputs alone, after that is queued, so that the GPU has
-        // work while the host waits.
-        const int halo = h->diff_halo;
-        bool solved = !direct;
-        auto finish_solve = [&]() -> bool {
-            bool redo = false;
-            if (!solved) rc = finish_w(h, S, &ss, &redo);
-            solved = true;
-            if (redo) launch_cal_u(G, S, h->st);
-            return redo;
-        };
-        if (h->mp_fn || halo == 0) finish_solve();
-        rec(2, h->st);
-        if (overlap) hipStreamWaitEvent(h->st, h->ev_join, 0);
-        if (h->mp_fn) {
-            rec(6, h->st);
-            const int mrc = host_microphysics(h, S);
-            if (mrc) return mrc;
-            rec(7, h->st);
-        }
-        rec(3, h->st);
-        // D: RKM_RKH with Mparam/Hparam, nudging (:408-417); the first
-        // updateMean (:408) is overwritten by nextTimeStep's before any read.
-        const int nudge = 1 | (c.CASE != 2 ? 2 : 0);
-        {
-            KTimer t(h, VVM_KT_TURB);
-            queue_turbulence(h, S);
-        }
-        {
-            KTimer t(h, VVM_KT_DIFFUSION);
-            if (halo) launch_diffusion_tiles(G, S, nudge, halo, h->st);
-            if (finish_solve()) {
-                queue_turbulence(h, S);
-                if (halo) launch_diffusion_tiles(G, S, nudge, halo, h->st);
-            }
-            finish_diffusion(h, S, nudge, halo);
-        }
-        if (rc == VVM_WARN_NOT_CONVERGED) {
-            warn = rc;
-            acc.not_converged++;
-        }
-        acc.solve_iters_total += ss.iters;
-        acc.guess_fallbacks = h->pois.guess_fallbacks - fallbacks0;
-        acc.guess_skipped = h->pois.guess_skipped - skipped0;
-        acc.solve_iters_last = ss.iters;
-        acc.refine_last = ss.refine;
-        acc.rel_residual_last = ss.rel_residual;
-        if (c.moisture_nudge_time != 0) launch_nudge_qv(G, S, c.moisture_nudge_time, h->st);
-        rec(4, h->st);
-        // E: nextTimeStep (:153-204)
-        {
-            KTimer t(h, VVM_KT_MEAN);
-            launch_update_mean(G, S, true, h->st);
-        }
-        rotate(h);
-        rec(5, h->st);
-        int lrc = check_launch(h);
-        if (lrc) return lrc;
-        h->stepped = true;
+        int rc = step_begin(h, n < h->tcap ? n : -1, n == nsteps - 1 && stats);
+        if (rc == VVM_OK) rc = step_finish(h, &acc);
+        if (rc) return rc;
     }
+    acc.guess_fallbacks = h->pois.guess_fallbacks - fallbacks0;
+    acc.guess_skipped = h->pois.guess_skipped - skipped0;
+    const int warn = acc.not_converged ? VVM_WARN_NOT_CONVERGED : VVM_OK;
     HIPCHK(h, hipStreamSynchronize(h->st));
     const double wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     kt_collect(h);
-    double derr = 0.;
-    HIPCHK(h, hipMemcpy(&derr, h->s + S_DIFF_ERR, sizeof(double), hipMemcpyDeviceToHost));
-    if (derr != 0.) return fail(h, VVM_ERR_STATE, "diffusion sweep: a wavefront gave up waiting for its carry");
+    if (const int erc = check_sweep(h)) return erc;
     // per-step phase times, as the reference fills t_*[step] every step
     for (int n = 0; n < std::min(nsteps, h->tcap); n++) {
         const hipEvent_t *E = &h->tev[size_t(n) * 8];
@@ -992,6 +1040,7 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
                 bool redo = false;
                 queue_w(h, S, -1, false, false);
                 h->pois.queue_check(h->st);
+                HIPCHK(h, hipStreamSynchronize(h->st));
                 rc = finish_w(h, S, nullptr, &redo);
             } else {
                 rc = solve_w_iter(h, S, nullptr, false, false);
@@ -1114,9 +1163,7 @@ int vvm_dev_op_field(vvm_dev_t *h, int op, int field) {
     int lrc = check_launch(h);
     if (lrc) return lrc;
     HIPCHK(h, hipStreamSynchronize(h->st));
-    double derr = 0.;
-    HIPCHK(h, hipMemcpy(&derr, h->s + S_DIFF_ERR, sizeof(double), hipMemcpyDeviceToHost));
-    if (derr != 0.) return fail(h, VVM_ERR_STATE, "diffusion sweep: a wavefront gave up waiting for its carry");
+    if (const int erc = check_sweep(h)) return erc;
     return VVM_OK;
 }
 
@@ -1369,6 +1416,16 @@ int vvm_dev_tune(vvm_dev_t *h, int steps, vvm_tune_result *out) {
 namespace vvmd {
 void dev_set_phase_overlap(vvm_dev_t *h, bool on) {
     if (h) h->overlap_c = on;
+}
+int dev_step_begin(vvm_dev_t *h) {
+    if (!h->uploaded) return fail(h, VVM_ERR_STATE, "step before upload");
+    HIPCHK(h, hipSetDevice(h->device));
+    return step_begin(h, -1, false);
+}
+int dev_step_finish(vvm_dev_t *h, vvm_step_stats *acc) { return step_finish(h, acc); }
+int dev_steps_end(vvm_dev_t *h) {
+    HIPCHK(h, hipStreamSynchronize(h->st));
+    return check_sweep(h);
 }
 }  // namespace vvmd
 

@@ -13,6 +13,10 @@
 namespace vvmd {
 // (vvm_dev.hip) members run their microphysics phase on their main stream
 void dev_set_phase_overlap(vvm_dev_t *h, bool on);
+// a step in two halves, and the wait for the last of them
+int dev_step_begin(vvm_dev_t *h);
+int dev_step_finish(vvm_dev_t *h, vvm_step_stats *acc);
+int dev_steps_end(vvm_dev_t *h);
 }  // namespace vvmd
 
 struct vvm_ens {
@@ -139,23 +143,35 @@ int vvm_ens_step(vvm_ens_t *e, int nsteps, vvm_ens_stats *stats) {
     std::mutex emu;
     auto t0 = std::chrono::steady_clock::now();
     auto worker = [&](int w) {
-        // the worker's members advance in lock step, so that every member's
-        // stream has work queued while another member waits on its solver
-        for (int s = 0; s < nsteps && first_err.load() == 0; s++)
-            for (int i : e->work[w]) {
-                vvm_step_stats st{};
-                const int rc = vvm_dev_step(e->dev[i], 1, &st);
-                if (rc < 0) {
-                    std::lock_guard<std::mutex> lk(emu);
-                    if (first_err.load() == 0) {
-                        first_err = rc;
-                        e->err = "member " + std::to_string(i) + ": " + vvm_dev_last_error(e->dev[i]);
-                    }
-                    return;
-                }
-                iters += st.solve_iters_total;
-                notconv += st.not_converged;
+        auto failed = [&](int i, int rc) {
+            if (rc >= 0) return false;
+            std::lock_guard<std::mutex> lk(emu);
+            if (first_err.load() == 0) {
+                first_err = rc;
+                e->err = "member " + std::to_string(i) + ": " + vvm_dev_last_error(e->dev[i]);
             }
+            return true;
+        };
+        // the worker's members advance in lock step: every one's step is queued
+        // before the first one's checks are waited for, so all their streams
+        // have work meanwhile
+        vvm_step_stats st{};
+        bool ok = true;
+        for (int s = 0; s < nsteps && ok && first_err.load() == 0; s++) {
+            size_t begun = 0;
+            for (int i : e->work[w]) {
+                if (failed(i, vvmd::dev_step_begin(e->dev[i]))) break;
+                begun++;
+            }
+            ok = begun == e->work[w].size();
+            for (size_t k = 0; k < begun; k++) {
+                const int i = e->work[w][k];
+                if (failed(i, vvmd::dev_step_finish(e->dev[i], &st))) ok = false;
+            }
+        }
+        for (int i : e->work[w]) failed(i, vvmd::dev_steps_end(e->dev[i]));
+        iters += st.solve_iters_total;
+        notconv += st.not_converged;
     };
     std::vector<std::thread> pool;
     for (int w = 1; w < e->threads; w++) pool.emplace_back(worker, w);

@@ -31,7 +31,6 @@ enum {
     S_DUBAR1,
     S_NEG_RATIO,       // 3 slots
     S_PRECIP_FAC = 9,  // pow(rhou[1]/rhow[1], -0.5)
-    S_DIFF_ERR = 10,   // set to 1 if a diffusion wave gave up waiting
     NSCALAR = 16
 };
 
@@ -60,6 +59,7 @@ struct StepPtrs {
     // memory, [field][strip][k]); nullptr: the one-workgroup sweep runs
     unsigned long long *dslots;
     int dstrip_cw;  // compute wavefronts per strip of that sweep (0: default)
+    double *sweep_err;  // host-mapped: set to 1 if one of its waves gave up waiting
 };
 
 struct Reductions {
@@ -85,6 +85,12 @@ void launch_bc_all_prog(const Grid &G, const StepPtrs &S, hipStream_t st);
 // stream pair per member on a few hardware queues, the cross-stream waits
 // block other members' work queued behind them.
 void dev_set_phase_overlap(vvm_dev_t *h, bool on);
+// A step in two halves, for callers that drive several handles: dev_step_begin
+// queues it, dev_step_finish waits for its checks (and adds the solve to acc)
+// and queues its end, dev_steps_end waits for all of it.  No phase times.
+int dev_step_begin(vvm_dev_t *h);
+int dev_step_finish(vvm_dev_t *h, vvm_step_stats *acc);
+int dev_steps_end(vvm_dev_t *h);
 void launch_pubartop(const Grid &G, const StepPtrs &S, int step, hipStream_t st);
 // The reference operators one at a time (vvm_dev_op_field).
 void launch_advection_zeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st);

@@ -65,6 +65,9 @@ class VvmHostView(C.Structure):
                    ("status_for_adding_forcing", C.c_int32)])
 
 
+# place of each array among the view's pointers, its first fields
+_VIEW_SLOT = {n: k for k, n in enumerate(FIELDS2D + HISTS + ROWS + PROFILES)}
+
 # int fn(void *user, vvm_host_view *view): a host microphysics scheme
 HOST_MP_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.POINTER(VvmHostView))
 
@@ -279,9 +282,13 @@ class HostState:
 
     def view(self) -> VvmHostView:
         v = VvmHostView()
+        # the pointer fields as one array of addresses (a pointer object for each
+        # field made a view cost 75 us); the view keeps the arrays alive
+        ptr = (C.c_void_p * len(_VIEW_SLOT)).from_buffer(v)
         for n, arr in self.a.items():
             assert arr.flags.c_contiguous and arr.dtype == np.float64
-            setattr(v, n, arr.ctypes.data_as(PTR))
+            ptr[_VIEW_SLOT[n]] = arr.ctypes.data
+        v.arrays = list(self.a.values())
         for n in SCALARS:
             setattr(v, n, self.s[n])
         v.dubarTop_advect[0], v.dubarTop_advect[1] = self.dubarTop_advect
