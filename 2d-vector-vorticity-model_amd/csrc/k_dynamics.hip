@@ -10,6 +10,7 @@
 #pragma clang fp contract(off)
 
 #include "pubartop.h"
+#include "scale_forcing.h"
 #include "vvm_internal.h"
 
 namespace vvmd {
@@ -401,44 +402,23 @@ __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8
 }
 
 // Second pass of NegativeValueProcess for qv, qc, qr (MicroPhysics.cpp:
-// 129-137), AddForcing (AddForcing.cpp:6-28: Q1LS/Q2LS and the random
-// theta kick) when `forcing`, and the center halos of thp, qvp, qcp, qrp.
+// 129-137), AddForcing (F.on), and the center halos of thp, qvp, qcp, qrp.
 // halos == 0 is AddForcing alone (ratios < 0): interior thp and qvp only.
-// nblk > 0: the ratios from the producing kernel's nblk partials in rs, formed
-// by every workgroup; otherwise from the scalars k_finalize left.
-__global__ void __launch_bounds__(BX *BY) k_scale_forcing(Grid G, StepPtrs S, int forcing, int tropical,
-                                                          int random_kick, int halos, RedSlot rs, int nblk) {
+__global__ void __launch_bounds__(BX *BY) k_scale_forcing(Grid G, StepPtrs S, Negval nv, Forcing F, int halos) {
     const int i = 1 + blockIdx.x * BX + threadIdx.x, k = 1 + blockIdx.y * BY + uniform(threadIdx.y);
     double ratios[3];
-    if (nblk > 0) {
-        double acc[6];
-        sum_partials<6>(rs, nblk, acc);
-#pragma unroll
-        for (int q = 0; q < 3; q++) ratios[q] = negval_ratio(acc[2 * q], acc[2 * q + 1]);
-    } else {
-#pragma unroll
-        for (int q = 0; q < 3; q++) ratios[q] = S.s[S_NEG_RATIO + q];
-    }
-    if (i < 1 || i > G.nx - 2 || k < 1 || k > G.nz - 2) return;
+    negval_ratios(S, nv.rs, nv.nblk, ratios);
+    if (i > G.nx - 2 || k > G.nz - 2) return;
 #pragma unroll
     for (int q = 0; q < 3; q++) {
         const int f = F_QV + q;
-        double v = at(S.fut[f], G, i, k);
-        const double ratio = ratios[q];
-        if (ratio >= 0. && v > 0) v = v * ratio;
-        if (forcing && tropical && f == F_QV) v += G.dt * S.P.Q2LS[k];
+        double v = rescaled(at(S.fut[f], G, i, k), ratios[q]);
+        if (F.on && f == F_QV) v = forced_qv(G, S, F, k, v);
         if (halos) store_center(S.fut[f], G, i, k, v);
         else if (f == F_QV) at(S.fut[f], G, i, k) = v;
     }
     double th = at(S.fut[F_TH], G, i, k);
-    if (forcing) {
-        // AddForcing's order (AddForcing.cpp:15-25): large-scale forcing,
-        // radiation heating [K/day], RADIATIONCOOLING, the random kick
-        if (tropical) th += G.dt * S.P.Q1LS[k];
-        if (S.rad) th += G.dt * at(S.rad, G, i, k) / 86400.;
-        if (S.radcool) th += G.dt * (-2. / 86400.);
-        if (random_kick) th += G.dt * at(S.forcing, G, i, k);
-    }
+    if (F.on) th = forced_th(G, S, F, i, k, th);
     if (halos) store_center(S.fut[F_TH], G, i, k, th);
     else at(S.fut[F_TH], G, i, k) = th;
 }
@@ -560,26 +540,25 @@ void launch_precip(const Grid &G, const StepPtrs &S, hipStream_t st) {
 void launch_bc_one(const Grid &G, double *a, bool westdown, hipStream_t st) {
     hipLaunchKernelGGL(k_bc_one, grid2d(G), dim3(BX, BY), 0, st, G, a, int(westdown));
 }
-int launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
+Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
     const int n = t4_tiles_x(G) * t4_tiles_z(G);
     hipLaunchKernelGGL(k_thermo4, xcd_grid(n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
     return negval_partials(S, rs, n, st);
 }
 // The ratios of NegativeValueProcess from nblk workgroups' partials: by
-// k_finalize (returns 0), or, up to kFoldBlocks, by the workgroups of
-// k_scale_forcing themselves (returns nblk).  The launch costs 4 to 5 us
+// k_finalize (nblk 0 is returned), or, up to kFoldBlocks, by the workgroups of
+// the second pass themselves (nblk).  The launch costs 4 to 5 us
 // whatever it does; every workgroup's own sum costs the traffic of all partials
 // for each of them, which at 2048 x 256 (1089 and 2145 partials) is no gain.
-int negval_partials(const StepPtrs &S, const RedSlot &rs, int nblk, hipStream_t st) {
+Negval negval_partials(const StepPtrs &S, const RedSlot &rs, int nblk, hipStream_t st) {
     constexpr int kFoldBlocks = 640;
-    if (nblk <= kFoldBlocks) return nblk;
+    if (nblk <= kFoldBlocks) return {rs, nblk};
     finalize<6>(rs, nblk, S.s, RED_NEGVAL, S_NEG_RATIO, st);
-    return 0;
+    return {rs, 0};
 }
-void launch_scale_forcing(const Grid &G, const StepPtrs &S, bool forcing, bool tropical, bool random_kick,
-                          hipStream_t st, const RedSlot &rs, int nblk, bool halos) {
-    hipLaunchKernelGGL(k_scale_forcing, interior_grid(G), dim3(BX, BY), 0, st, G, S, int(forcing), int(tropical),
-                       int(random_kick), int(halos), rs, nblk);
+void launch_scale_forcing(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, hipStream_t st,
+                          bool halos) {
+    hipLaunchKernelGGL(k_scale_forcing, interior_grid(G), dim3(BX, BY), 0, st, G, S, nv, F, int(halos));
 }
 void launch_bc_uw(const Grid &G, const StepPtrs &S, hipStream_t st) {
     hipLaunchKernelGGL(k_bc_uw, grid2d(G), dim3(BX, BY), 0, st, G, S);

@@ -825,6 +825,8 @@ int step_begin(vvm_dev *h, int timer, bool last) {
     // solve; it needs only pzeta's zetap and the past solutions
     const bool run_net = net_due(h);
     const bool early_guess = overlap && run_net && h->pois.sample_cap == 0;
+    const Forcing F{1, c.tropical_forcing != 0, h->status_for_adding_forcing != 0};
+    const bool direct = uses_direct(c);
     mark(h, 0, h->st);
     // A: advection, buoyancy, forcing, halos (src/Iteration.cpp:263-285)
     {
@@ -837,24 +839,25 @@ int step_begin(vvm_dev *h, int timer, bool last) {
         prepare_guess(h, S, true, h->side);
         hipEventRecord(h->ev_guess, h->side);
     }
-    int negval;
+    Negval nv;
     {
         KTimer t(h, VVM_KT_THERMO4);
-        negval = launch_thermo4(G, S, h->step, h->red.negval, h->st);
+        nv = launch_thermo4(G, S, h->step, h->red.negval, h->st);
     }
-    {
+    if (h->mp_fn) {
         KTimer t(h, VVM_KT_SCALE);
-        launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st,
-                             h->red.negval, negval);
+        launch_scale_forcing(G, S, nv, F, h->st);
     }
     if (h->ghosts_dirty) {
         launch_bc_uw(G, S, h->st);
         h->ghosts_dirty = false;
     }
     mark(h, 1, h->st);
-    // C: Kessler + NegativeValueProcess x3 + halos (:303-311, 404), on
-    // the side stream while B runs; the main stream waits for it before D
-    // (with host microphysics, C runs after B on the host instead)
+    // C: Kessler (with the scalars' negative-value rescale and forcing) and its
+    // NegativeValueProcess x3 + halos (:303-311, 404), on the side stream while
+    // B runs; the main stream waits for it before D (with host microphysics, C
+    // runs after B on the host instead).  Its partial sums go to another slot
+    // than thermo4's, which it may still be reading.
     hipStream_t cs = overlap ? h->side : h->st;
     if (overlap) {
         hipEventRecord(h->ev_fork, h->st);
@@ -864,17 +867,16 @@ int step_begin(vvm_dev *h, int timer, bool last) {
         mark(h, 6, cs);
         {
             KTimer t(h, VVM_KT_KESSLER, cs);
-            negval = launch_kessler(G, S, h->red.negval, cs);
+            nv = launch_kessler(G, S, nv, F, h->red.misc, cs);
         }
         {
             KTimer t(h, VVM_KT_SCALE, cs);
-            launch_scale_forcing(G, S, false, false, false, cs, h->red.negval, negval);
+            launch_scale_forcing(G, S, nv, Forcing{}, cs);
         }
         mark(h, 7, cs);
     }
     if (overlap) hipEventRecord(h->ev_join, h->side);
     // B: pubarTop_pt, cal_w, cal_u (:292-296)
-    const bool direct = uses_direct(c);
     if (!direct) launch_pubartop(G, S, h->step, h->st);
     {
         KTimer t(h, VVM_KT_SOLVE);
@@ -1019,14 +1021,13 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             launch_pzeta(G, S, h->step, h->st);
             break;
         case VVM_OP_PSCALARS:
-            launch_scale_forcing(G, S, false, false, false, h->st, h->red.negval,
-                                 launch_thermo4(G, S, h->step, h->red.negval, h->st));
+            launch_scale_forcing(G, S, launch_thermo4(G, S, h->step, h->red.negval, h->st), Forcing{}, h->st);
             break;
         case VVM_OP_FORCING_BC: {
             const double none[3] = {-1., -1., -1.};
             HIPCHK(h, hipMemcpyAsync(h->s + S_NEG_RATIO, none, sizeof(none), hipMemcpyHostToDevice, h->st));
-            launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st,
-                                 h->red.negval, 0);
+            launch_scale_forcing(G, S, Negval{h->red.negval, 0},
+                                 Forcing{1, c.tropical_forcing != 0, h->status_for_adding_forcing != 0}, h->st);
             launch_bc_all_prog(G, S, h->st);
             break;
         }
@@ -1052,8 +1053,7 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             launch_cal_u(G, S, h->st);
             break;
         case VVM_OP_MICROPHYSICS:
-            launch_scale_forcing(G, S, false, false, false, h->st, h->red.negval,
-                                 launch_kessler(G, S, h->red.negval, h->st));
+            launch_scale_forcing(G, S, launch_kessler(G, S, h->red.negval, h->st), Forcing{}, h->st);
             launch_bc_all_prog(G, S, h->st);
             break;
         case VVM_OP_TURBULENCE:
@@ -1154,8 +1154,8 @@ int vvm_dev_op_field(vvm_dev_t *h, int op, int field) {
         case VVM_OP_ADD_FORCING: {
             const double none[3] = {-1., -1., -1.};
             HIPCHK(h, hipMemcpyAsync(h->s + S_NEG_RATIO, none, sizeof(none), hipMemcpyHostToDevice, h->st));
-            launch_scale_forcing(G, S, true, c.tropical_forcing != 0, h->status_for_adding_forcing != 0, h->st,
-                                 h->red.negval, 0, false);
+            launch_scale_forcing(G, S, Negval{h->red.negval, 0},
+                                 Forcing{1, c.tropical_forcing != 0, h->status_for_adding_forcing != 0}, h->st, false);
             break;
         }
         default: return fail(h, VVM_ERR_ARG, "unknown op");

@@ -71,13 +71,20 @@ struct Reductions {
 // ------------------------------------------------------------ launchers
 // Dynamics (k_dynamics.hip)
 void launch_pzeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st);
-// launch_thermo4 and launch_kessler leave NegativeValueProcess's first pass;
-// what they return (negval_partials) goes to the launch_scale_forcing behind
-// them, with rs.
-int launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);
-int negval_partials(const StepPtrs &S, const RedSlot &rs, int nblk, hipStream_t st);
-void launch_scale_forcing(const Grid &G, const StepPtrs &S, bool forcing, bool tropical, bool random_kick,
-                          hipStream_t st, const RedSlot &rs, int nblk, bool halos = true);
+// launch_thermo4 and launch_kessler leave NegativeValueProcess's first pass in
+// rs; what they return (negval_partials) goes, with rs, to the second pass:
+// launch_scale_forcing, or the launch_kessler behind launch_thermo4.
+struct Negval {
+    RedSlot rs;
+    int nblk;
+};
+struct Forcing {
+    int on, tropical, random_kick;
+};
+Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);
+Negval negval_partials(const StepPtrs &S, const RedSlot &rs, int nblk, hipStream_t st);
+void launch_scale_forcing(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, hipStream_t st,
+                          bool halos = true);
 void launch_bc_uw(const Grid &G, const StepPtrs &S, hipStream_t st);
 void launch_bc_all_prog(const Grid &G, const StepPtrs &S, hipStream_t st);
 // Whether a handle runs the microphysics phase on its second stream beside
@@ -104,7 +111,10 @@ void launch_kessler_process(const Grid &G, const StepPtrs &S, int process, hipSt
 void launch_negative_value(const Grid &G, const StepPtrs &S, double *a, const RedSlot &rs, hipStream_t st);
 
 // Physics (k_physics.hip)
-int launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipStream_t st);
+// with nv and F (the timestep): thermo4's second pass and AddForcing first
+Negval launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipStream_t st);
+Negval launch_kessler(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, const RedSlot &rs,
+                      hipStream_t st);
 // kmax (host-mapped, kTurbBlocks doubles): the largest RKM or RKH each
 // workgroup formed; returns their count.
 constexpr int kTurbBlocks = 640;
