@@ -100,7 +100,7 @@ struct vvm_dev {
         int rc = VVM_OK, halo = 0;
         bool solved = true;
         int timer = -1;     // its row of tev (-1: not timed per step)
-        bool last = false;  // its phase boundaries go to ev and ev_mp
+        bool last = false;  // else its phase boundaries go to ev and ev_mp
     } run;
 
     // per-kernel event timer (vvm_dev_kernel_timer)
@@ -781,7 +781,7 @@ namespace {
 void mark(vvm_dev *h, int slot, hipStream_t s) {
     const vvm_dev::Run &r = h->run;
     if (r.timer >= 0) hipEventRecord(h->tev[size_t(r.timer) * 8 + slot], s);
-    if (r.last) hipEventRecord(slot < 6 ? h->ev[slot] : h->ev_mp[slot - 6], s);
+    else if (r.last) hipEventRecord(slot < 6 ? h->ev[slot] : h->ev_mp[slot - 6], s);
 }
 
 // Reads the direct solve's residual (wait: which may not have arrived yet) and
@@ -969,12 +969,12 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
     kt_collect(h);
     if (const int erc = check_sweep(h)) return erc;
     // per-step phase times, as the reference fills t_*[step] every step
+    auto span = [&](hipEvent_t a, hipEvent_t b) {
+        float ms = 0.f;
+        return hipEventElapsedTime(&ms, a, b) == hipSuccess ? double(ms) * 1e-3 : 0.;
+    };
     for (int n = 0; n < std::min(nsteps, h->tcap); n++) {
         const hipEvent_t *E = &h->tev[size_t(n) * 8];
-        auto span = [&](hipEvent_t a, hipEvent_t b) {
-            float ms = 0.f;
-            return hipEventElapsedTime(&ms, a, b) == hipSuccess ? double(ms) * 1e-3 : 0.;
-        };
         double *o = h->tout + size_t(n) * 5;
         o[0] = span(E[0], E[1]);  // advection (phase A)
         o[1] = span(E[1], E[2]);  // poisson (phase B)
@@ -986,15 +986,14 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
         *stats = acc;
         stats->steps = nsteps;
         if (nsteps > 0) {
-            float ms[5];
-            for (int e = 0; e < 5; e++) hipEventElapsedTime(&ms[e], h->ev[e], h->ev[e + 1]);
-            stats->t_advection = ms[0] * 1e-3;
-            stats->t_poisson = ms[1] * 1e-3;
-            // phase C ran on the side stream (ev[2] -> ev[3] is only the wait for it)
-            float mp = 0.f;
-            hipEventElapsedTime(&mp, h->ev_mp[0], h->ev_mp[1]);
-            stats->t_microphysics = mp * 1e-3;
-            stats->t_diffusion = ms[3] * 1e-3;
+            // the last step's boundaries: its timer row's, if it has one
+            const bool row = nsteps <= h->tcap;
+            const hipEvent_t *E = row ? &h->tev[size_t(nsteps - 1) * 8] : h->ev, *mp = row ? E + 6 : h->ev_mp;
+            stats->t_advection = span(E[0], E[1]);
+            stats->t_poisson = span(E[1], E[2]);
+            // phase C ran on the side stream (E[2] -> E[3] is only the wait for it)
+            stats->t_microphysics = span(mp[0], mp[1]);
+            stats->t_diffusion = span(E[3], E[4]);
             stats->t_all = wall / nsteps;
         }
     }
