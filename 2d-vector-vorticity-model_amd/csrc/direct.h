@@ -19,7 +19,10 @@ struct RowPlan {
     int N = 0, M = 0;
     int nst = 0, radix[kMaxStages] = {};
     int threads = 0;      // at least N / 8: a thread holds at most 8 outputs of a stage
-    int tw_lds = 0;       // twiddles staged in LDS (a prime factor above 5)
+    // in LDS: nothing, the table of all roots (a prime factor above 5 reads it),
+    // or the stages' twiddles; nothing where that would pass the LDS size
+    enum { TW_GLOBAL, TW_ROOTS, TW_STAGES };
+    int tw = TW_GLOBAL;
 };
 
 template <typename T>
@@ -43,8 +46,8 @@ class Direct {
     RowPlan plan;
     size_t row_lds = 0, col_lds = 0;
     T *tw = nullptr;    // [N][2]: cos, -sin of 2 pi k / N; then the stages' twiddles, [N-1][2]
-    T *g = nullptr;     // [M][N/2+1] elimination factors
-    T *di = nullptr;    // [M][N/2+1] 1 / (N pivot)
+    T *di = nullptr;    // [M][N/2+1] 1 / pivot
+    const double *cu_dev = nullptr;
     T *spec = nullptr;  // [M][N] transformed rows
     void columns(hipStream_t st);
 };

@@ -1,9 +1,10 @@
 // k_direct.hip -- direct solve of the cal_w system (direct.h).
 //
 // Three kernels: the forward row transforms, the tridiagonal systems, the
-// inverse row transforms.  At 2048 x 255 they move 8 + 12 + 8 MB and are
-// bound by latency (four LDS round trips a transform, the elimination's
-// serial chain), not by bandwidth.
+// inverse row transforms.  At 2048 x 255 they move 8 + 10 + 12 MB in 12.7, 12.7
+// and 11.6 us and are bound by latency: the rows' and the twiddles' first load
+// (2 to 3 us; 5.5 where each was waited for in a branch of its own, 15 us a
+// kernel), four LDS round trips of 1 us, the elimination's serial chain.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -134,37 +135,41 @@ __device__ inline void dft(Cx<T> (&v)[R]) {
 // One Stockham stage of radix R after stages of product Ns.  NB: butterflies
 // a thread, ceil(8 / R) since threads >= N / 8.  tw: exp(-2 pi i r k / (Ns R))
 // at (r - 1) Ns + k, so that neighbouring threads read neighbouring values.
+// A thread without a butterfly repeats the last one and stores nothing: reads
+// under a branch would each be waited for before the next butterfly's are
+// issued (the odd radices keep the branch, as two butterflies at once spill).
 template <int R, typename T>
 __device__ inline void stage(T *re, T *im, int N, int Ns, const T *__restrict__ tw) {
     constexpr int NB = (8 + R - 1) / R;
     const int nb = N / R;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // addresses formed here, not for every radix ahead of all stages (they spill)
     Cx<T> v[NB][R];
     int dst[NB];
 #pragma unroll
     for (int t = 0; t < NB; t++) {
-        const int j = threadIdx.x + t * blockDim.x;
-        if (j < nb) {
-            const int q = int(unsigned(j) / unsigned(Ns)), k = j - q * Ns;
-            dst[t] = q * Ns * R + k;
+        const int jt = tid + t * blockDim.x, j = min(jt, nb - 1);
+        if (R % 2 && jt >= nb) continue;
+        const int q = int(unsigned(j) / unsigned(Ns)), k = j - q * Ns;
+        dst[t] = q * Ns * R + k;
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const int a = pad(j + r * nb);
-                v[t][r] = {re[a], im[a]};
-            }
-            if (Ns > 1) {
-#pragma unroll
-                for (int r = 1; r < R; r++) {
-                    const int a = 2 * ((r - 1) * Ns + k);
-                    v[t][r] = mul(v[t][r], Cx<T>{tw[a], tw[a + 1]});
-                }
-            }
-            dft<R>(v[t]);
+        for (int r = 0; r < R; r++) {
+            const int a = pad(j + r * nb);
+            v[t][r] = {re[a], im[a]};
         }
+        if (Ns > 1) {
+#pragma unroll
+            for (int r = 1; r < R; r++) {
+                const int a = 2 * ((r - 1) * Ns + k);
+                v[t][r] = mul(v[t][r], Cx<T>{tw[a], tw[a + 1]});
+            }
+        }
+        dft<R>(v[t]);
     }
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < NB; t++) {
-        if (int(threadIdx.x + t * blockDim.x) < nb) {
+        if (int(tid + t * blockDim.x) < nb) {
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 const int a = pad(dst[t] + r * Ns);
@@ -216,54 +221,80 @@ __device__ inline void stage_any(T *re, T *im, int N, int Ns, int R, const T *tw
     __syncthreads();
 }
 
+// The twiddles that the transform reads from LDS (RowPlan::tw): loaded with the
+// rows, so that their latency is paid once and not in every stage.
 template <typename T>
-__device__ inline void fft(const RowPlan &P, T *re, T *im, const T *__restrict__ tw, T *twl) {
-    const int N = P.N;
-    const T *tws = tw;
-    if (P.tw_lds) {
-        for (int t = threadIdx.x; t < 2 * N; t += blockDim.x) twl[t] = tw[t];
-        tws = twl;
+struct Twiddles {
+    Cx<T> v[8];
+    __device__ inline void load(const RowPlan &P, const T *__restrict__ tw) {
+        if (P.tw == RowPlan::TW_GLOBAL) return;
+        const Cx<T> *src = reinterpret_cast<const Cx<T> *>(tw) + (P.tw == RowPlan::TW_STAGES ? P.N : 0);
+#pragma unroll
+        for (int t = 0; t < 8; t++) v[t] = src[min(int(threadIdx.x + t * blockDim.x), P.N - 1)];
     }
-    __syncthreads();
+    __device__ inline void store(const RowPlan &P, T *twl) const {
+        if (P.tw == RowPlan::TW_GLOBAL) return;
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            const int i = threadIdx.x + t * blockDim.x;
+            if (i < P.N) {
+                twl[2 * i] = v[t].x;
+                twl[2 * i + 1] = v[t].y;
+            }
+        }
+    }
+};
+
+template <bool LDS, typename T>
+__device__ inline void fft_stages(const RowPlan &P, T *re, T *im, const T *tw, const T *twl) {
+    const int N = P.N;
     int Ns = 1;
     for (int s = 0; s < P.nst; s++) {
         const int R = P.radix[s];
         // the stages' tables follow the table of all N roots; those before
         // hold sum (R - 1) Ns = Ns - 1 values
-        const T *ts = tw + 2 * (N + Ns - 1);
+        const T *ts = LDS ? twl + 2 * (Ns - 1) : tw + 2 * (N + Ns - 1);
         switch (R) {
             case 8: stage<8>(re, im, N, Ns, ts); break;
             case 4: stage<4>(re, im, N, Ns, ts); break;
             case 2: stage<2>(re, im, N, Ns, ts); break;
             case 3: stage<3>(re, im, N, Ns, ts); break;
             case 5: stage<5>(re, im, N, Ns, ts); break;
-            default: stage_any(re, im, N, Ns, R, tws); break;
+            default:
+                if constexpr (!LDS) stage_any(re, im, N, Ns, R, P.tw == RowPlan::TW_ROOTS ? twl : tw);
         }
         Ns *= R;
     }
 }
+template <typename T>
+__device__ inline void fft(const RowPlan &P, T *re, T *im, const T *__restrict__ tw, const T *twl) {
+    __syncthreads();
+    if (P.tw == RowPlan::TW_STAGES) fft_stages<true>(P, re, im, tw, twl);
+    else fft_stages<false>(P, re, im, tw, twl);
+}
 
-// Hartley values (Re - Im) of the two rows at frequency q, from the complex
+// Hartley values (Re - Im) of the two rows at frequency q, times 2 h, from the complex
 // spectrum Z of row a + i row b: A(q) = (Z(q) + Z*(N-q)) / 2,
 // B(q) = (Z(q) - Z*(N-q)) / 2i.
 template <typename T>
-__device__ inline void hartley_pair(const T *re, const T *im, int N, int q, T &ha, T &hb) {
+__device__ inline void hartley_pair(const T *re, const T *im, int N, int q, T h, T &ha, T &hb) {
     const int a = pad(q), c = pad(q == 0 ? 0 : N - q);
     const T zr = re[a], zi = im[a], cr = re[c], ci = im[c];
-    ha = T(0.5) * ((zr + cr) - (zi - ci));
-    hb = T(0.5) * ((zi + ci) + (zr - cr));
+    ha = h * ((zr + cr) - (zi - ci));
+    hb = h * ((zi + ci) + (zr - cr));
 }
 
 // Forward: rows j, j+1 of r (RHS false), or cal_w's right-hand side
 // f = -b / rhow, b = rhow^2 (zetap[i+1] - zetap[i]) dx
 // (src/PoissonSolver.cpp:444-450), formed from zetap and stored (RHS true).
+// Times 1/N, the inverse transform's.
 // With RHS and a step the last workgroup does pubarTop_pt instead: it reads u, w and K as
 // the solve finds them, and alone it was a launch of 5 to 8 us.
 template <typename T, bool RHS>
 __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restrict__ tw, const double *__restrict__ r,
                                                    T *__restrict__ spec, Grid G, StepPtrs S, int step,
                                                    double *__restrict__ f) {
-    extern __shared__ unsigned char lds_raw[];
+    extern __shared__ __align__(16) unsigned char lds_raw[];
     if (RHS && step >= 0 && blockIdx.x == gridDim.x - 1) {
         pubartop_block(G, S, step);
         return;
@@ -273,34 +304,53 @@ __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restric
     T *re = reinterpret_cast<T *>(lds_raw), *im = re + LN, *twl = im + LN;
     const int j = 1 + 2 * blockIdx.x;
     const bool two = j + 1 <= M;
-    auto value = [&](int row, int i) -> double {
-        if constexpr (!RHS) return r[size_t(row) * N + i];
-        const int k = row + 1;
-        const double rw = rhow[k];
-        double v;
-        {
-#pragma clang fp contract(off)
-            const double b = rw * rw * (zetap[ix(G, i + 2, k)] - zetap[ix(G, i + 1, k)]) * G.dx;
-            v = -b / rw;
+    const int j1 = two ? j + 1 : j;
+    Twiddles<T> W;
+    W.load(P, tw);
+    // all loads in flight at once: past the last column it is read again, and
+    // nothing is waited for in a branch (a guarded load was 0.7 us, eight times)
+    double va[8], vb[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {  // threads >= N / 8
+        const int i = min(int(threadIdx.x + t * blockDim.x), N - 1);
+        if constexpr (RHS) {
+            va[t] = at(zetap, G, i + 2, j + 1) - at(zetap, G, i + 1, j + 1);
+            vb[t] = at(zetap, G, i + 2, j1 + 1) - at(zetap, G, i + 1, j1 + 1);
+        } else {
+            va[t] = r[size_t(j) * N + i];
+            vb[t] = r[size_t(j1) * N + i];
         }
-        f[size_t(row) * N + i] = v;
-        return v;
+    }
+    W.store(P, twl);
+    auto rhs = [&](double d, double rw) {
+#pragma clang fp contract(off)
+        const double b = rw * rw * d * G.dx;
+        return -b / rw;
     };
 #pragma unroll
-    for (int t = 0; t < 8; t++) {  // threads >= N / 8; unrolled, all loads in flight at once
+    for (int t = 0; t < 8; t++) {
         const int i = threadIdx.x + t * blockDim.x;
+        if constexpr (RHS) {
+            va[t] = rhs(va[t], rhow[j + 1]);
+            vb[t] = rhs(vb[t], rhow[j1 + 1]);
+        }
         if (i < N) {
-            re[pad(i)] = T(value(j, i));
-            im[pad(i)] = two ? T(value(j + 1, i)) : T(0);
+            if constexpr (RHS) {
+                f[size_t(j) * N + i] = va[t];
+                if (two) f[size_t(j + 1) * N + i] = vb[t];
+            }
+            re[pad(i)] = T(va[t]);
+            im[pad(i)] = two ? T(vb[t]) : T(0);
         }
     }
     fft(P, re, im, tw, twl);
+    const T h = T(0.5 / N);
 #pragma unroll
     for (int t = 0; t < 8; t++) {
         const int q = threadIdx.x + t * blockDim.x;
+        T ha, hb;
+        hartley_pair(re, im, N, min(q, N - 1), h, ha, hb);
         if (q < N) {
-            T ha, hb;
-            hartley_pair(re, im, N, q, ha, hb);
             spec[size_t(j - 1) * N + q] = ha;
             if (two) spec[size_t(j) * N + q] = hb;
         }
@@ -314,17 +364,28 @@ template <typename T, bool ADD, bool W>
 __global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restrict__ tw, const T *__restrict__ spec,
                                                    const double *x0, double *x, Grid G, double *__restrict__ w,
                                                    const double *__restrict__ rhow) {
-    extern __shared__ unsigned char lds_raw[];
+    extern __shared__ __align__(16) unsigned char lds_raw[];
     const int N = P.N, M = P.M, LN = pad(N - 1) + 1;
     T *re = reinterpret_cast<T *>(lds_raw), *im = re + LN, *twl = im + LN;
     const int j = 1 + 2 * blockIdx.x;
     const bool two = j + 1 <= M;
+    const int j1 = two ? j + 1 : j;
+    Twiddles<T> Tw;
+    Tw.load(P, tw);
+    T va[8], vb[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const int i = min(int(threadIdx.x + t * blockDim.x), N - 1);
+        va[t] = spec[size_t(j - 1) * N + i];
+        vb[t] = spec[size_t(j1 - 1) * N + i];
+    }
+    Tw.store(P, twl);
 #pragma unroll
     for (int t = 0; t < 8; t++) {
         const int i = threadIdx.x + t * blockDim.x;
         if (i < N) {
-            re[pad(i)] = spec[size_t(j - 1) * N + i];
-            im[pad(i)] = two ? spec[size_t(j) * N + i] : T(0);
+            re[pad(i)] = va[t];
+            im[pad(i)] = two ? vb[t] : T(0);
         }
     }
     if constexpr (W) {  // the zero rows of w
@@ -334,20 +395,36 @@ __global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restric
         }
     }
     fft(P, re, im, tw, twl);
-    auto put = [&](int row, int i, T e) {
-        const size_t a = size_t(row) * N + i;
-        const double v = ADD ? x0[a] + double(e) : double(e);
-        x[a] = v;
-        if constexpr (W) store_westdown(w, G, i + 1, row + 1, v / rhow[row + 1]);
-    };
+    double xa[8], xb[8];
+    if constexpr (ADD) {
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            const int i = min(int(threadIdx.x + t * blockDim.x), N - 1);
+            xa[t] = x0[size_t(j) * N + i];
+            xb[t] = x0[size_t(j1) * N + i];
+        }
+    }
 #pragma unroll
     for (int t = 0; t < 8; t++) {
         const int q = threadIdx.x + t * blockDim.x;
+        T ha, hb;
+        hartley_pair(re, im, N, min(q, N - 1), T(0.5), ha, hb);
+        double da = double(ha), db = double(hb), wa = 0., wb = 0.;
+        if constexpr (ADD) {
+            da += xa[t];
+            db += xb[t];
+        }
+        if constexpr (W) {
+            wa = da / rhow[j + 1];
+            wb = db / rhow[j1 + 1];
+        }
         if (q < N) {
-            T ha, hb;
-            hartley_pair(re, im, N, q, ha, hb);
-            put(j, q, ha);
-            if (two) put(j + 1, q, hb);
+            x[size_t(j) * N + q] = da;
+            if constexpr (W) store_westdown(w, G, q + 1, j + 1, wa);
+            if (two) {
+                x[size_t(j + 1) * N + q] = db;
+                if constexpr (W) store_westdown(w, G, q + 1, j + 2, wb);
+            }
         }
     }
 }
@@ -356,16 +433,16 @@ __global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restric
 //
 // Row j (1-based) of frequency q: d_j x_j - cu_j x_{j+1} - cu_{j-1} x_{j-1} =
 // F_j.  Eliminated from both ends towards row mid = (M+1)/2 at once, which
-// halves the serial chain:
-//   downwards (j < mid): g_j = cu_j / p_j, y_{j+1} = F_{j+1} + g_j y_j,
-//   upwards   (j > mid): g_j = cu_{j-1} / p_j, y_{j-1} = F_{j-1} + g_j y_j,
-// x_mid = y_mid / p_mid, and back x_j = y_j / p_j + g_j x_{j+-1}.
-// The factors g and 1 / (N p) (the inverse transform's 1/N folded in) are
-// formed once, for q = 0..N/2 (lambda_q = lambda_{N-q}).
+// halves the serial chain; with the pivots p and F' = F / p,
+//   downwards (j < mid): z_j = F'_j + (cu_{j-1} / p_j) z_{j-1},
+//   upwards   (j > mid): z_j = F'_j + (cu_j / p_j) z_{j+1},
+// at mid both, x_mid = z_mid, and back x_j = z_j + (cu_j / p_j) x_{j+1} or
+// z_j + (cu_{j-1} / p_j) x_{j-1}.  Only 1 / p_j is kept, formed once, for
+// q = 0..N/2 (lambda_q = lambda_{N-q}).
 
 template <typename T>
 __global__ void __launch_bounds__(64) k_factor(int N, int M, const double *__restrict__ cx,
-                                               const double *__restrict__ cu, T *__restrict__ g, T *__restrict__ di) {
+                                               const double *__restrict__ cu, T *__restrict__ di) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x, Nq = N / 2 + 1;
     if (q >= Nq) return;
     const double s = sinpi(double(q) / N), lam = 4. * s * s;
@@ -373,160 +450,165 @@ __global__ void __launch_bounds__(64) k_factor(int N, int M, const double *__res
     auto diag = [&](int j) { return cx[j] * lam + cu[j] + cu[j - 1]; };
     double top = 0., bot = 0.;  // what the rows above and below take off p_mid
     for (int j = 1; j < mid; j++) {
-        const double p = diag(j) - top, gj = cu[j] / p;
-        g[size_t(j - 1) * Nq + q] = T(gj);
-        di[size_t(j - 1) * Nq + q] = T(1. / (p * N));
-        top = cu[j] * gj;
+        const double p = diag(j) - top;
+        di[size_t(j - 1) * Nq + q] = T(1. / p);
+        top = cu[j] * (cu[j] / p);
     }
     for (int j = M; j > mid; j--) {
-        const double p = diag(j) - bot, gj = cu[j - 1] / p;
-        g[size_t(j - 1) * Nq + q] = T(gj);
-        di[size_t(j - 1) * Nq + q] = T(1. / (p * N));
-        bot = cu[j - 1] * gj;
+        const double p = diag(j) - bot;
+        di[size_t(j - 1) * Nq + q] = T(1. / p);
+        bot = cu[j - 1] * (cu[j - 1] / p);
     }
-    g[size_t(mid - 1) * Nq + q] = T(0);
-    di[size_t(mid - 1) * Nq + q] = T(1. / ((diag(mid) - top - bot) * N));
+    di[size_t(mid - 1) * Nq + q] = T(1. / (diag(mid) - top - bot));
 }
 
-// Eight columns a workgroup.  Every thread moves them and their factors to LDS
-// in the order of the elimination's steps (all loads in flight at once): slot s
-// of a direction holds its s-th row, after enough empty slots to make the
-// number of steps a multiple of eight.  Then 16 lanes, 8 columns x 2
-// directions, run all steps without a branch, the next eight steps' values in
-// registers; an empty slot leaves y = 0 and x is not read after it.
-// At 2048 x 255: 15 us; with the rows in place and the two directions'
-// last steps under a mask 27 us.
+// Eight columns a workgroup.  Every thread scales them and forms their factors
+// on the way to LDS (all loads in flight at once), in the order of the
+// elimination's steps: slot s of a direction holds its s-th row, after enough
+// empty slots to make the number of steps a multiple of eight.  Then 16 lanes,
+// 8 columns x 2 directions, run all steps without a branch, the next eight
+// steps' values in registers: one 16-byte LDS read, one multiply-add and one
+// write a step, which is the serial chain that bounds the kernel (1.4 us down,
+// 2 us back for 64 steps at 1024 x 127; with three reads, a multiply and a
+// kept factor more 2.4 and 1.7).  An empty slot leaves z = 0, and x is not
+// read after it.  At 2048 x 255: 12.7 us, 15.5 before.
+// Neighbouring workgroups share a cache line of every row, and the columns q
+// and N - q their pivots: an XCD gets neighbours and their mirror images.
 constexpr int KC = 8, KSTEP = 8, KL = 2 * KC;
+template <typename T>
+struct alignas(2 * sizeof(T)) Elim {
+    T z, f;  // F', then z, then x; the elimination's factor
+};
+template <typename T>
+struct ColStep {
+    Elim<T> e[KL];
+    T b[KL];  // the back substitution's factor
+};
+template <typename T>
+struct ColMid {
+    T z[KC], dn[KC], up[KC];
+};
 struct ColSteps {
     int mid, steps, pad_dn, pad_up;
 };
 __host__ __device__ inline ColSteps col_steps(int M) {
     ColSteps c;
     c.mid = (M + 1) / 2 - 1;  // 0-based
-    const int dn = c.mid, up = M - 1 - c.mid;
-    c.steps = ((dn > up ? dn : up) + KSTEP - 1) / KSTEP * KSTEP;
+    const int dn = c.mid, up = M - 1 - c.mid, n = dn > up ? dn : up;
+    c.steps = ((n > 1 ? n : 1) + KSTEP - 1) / KSTEP * KSTEP;
     c.pad_dn = c.steps - dn;
     c.pad_up = c.steps - up;
     return c;
 }
-// LDS elements: [steps][F, g, 1/p][KL], then the middle row's F and 1/p
-inline size_t col_lds_elems(int M) { return size_t(col_steps(M).steps) * 3 * KL + 2 * KC; }
+template <typename T>
+size_t col_lds_bytes(int M) {
+    return size_t(col_steps(M).steps) * sizeof(ColStep<T>) + sizeof(ColMid<T>);
+}
 
 template <typename T>
-__global__ void __launch_bounds__(256) k_columns(int N, int M, T *__restrict__ spec, const T *__restrict__ g,
-                                                 const T *__restrict__ di) {
-    extern __shared__ unsigned char lds_raw[];
-    T *L = reinterpret_cast<T *>(lds_raw);
+__global__ void __launch_bounds__(256) k_columns(int N, int M, T *__restrict__ spec, const T *__restrict__ di,
+                                                 const double *__restrict__ cu) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    ColStep<T> *L = reinterpret_cast<ColStep<T> *>(lds_raw);
     const ColSteps cs = col_steps(M);
-    T *Mid = L + size_t(cs.steps) * 3 * KL;
-    const int Nq = N / 2 + 1;
+    ColMid<T> &Mid = *reinterpret_cast<ColMid<T> *>(L + cs.steps);
+    const int Nq = N / 2 + 1, nt = (N + KC - 1) / KC, tile = xcd_tile(nt);
+    if (tile >= nt) return;
+    const int b = tile % 2 ? nt - 1 - tile / 2 : tile / 2;
     // columns past the last repeat it (never stored)
-    const int c = threadIdx.x % KC, q = min(int(blockIdx.x) * KC + c, N - 1), qq = min(q, N - q);
+    const int c = threadIdx.x % KC, q = min(b * KC + c, N - 1), qq = min(q, N - q);
     const int rstep = blockDim.x / KC;
-    // element of row j (0-based, not mid) in L
-    auto slot = [&](int j) {
-        return j < cs.mid ? (cs.pad_dn + j) * 3 * KL + c : (cs.pad_up + M - 1 - j) * 3 * KL + KC + c;
-    };
+    // step and lane of row j (0-based, not mid)
+    auto step = [&](int j) { return j < cs.mid ? cs.pad_dn + j : cs.pad_up + M - 1 - j; };
+    auto lane = [&](int j) { return j < cs.mid ? c : KC + c; };
     for (int j0 = threadIdx.x / KC; j0 < M; j0 += 8 * rstep) {
-        T vf[8], vg[8], vd[8];
+        T vf[8], vd[8];
+        double c0[8], c1[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const int j = min(j0 + u * rstep, M - 1);
             vf[u] = spec[size_t(j) * N + q];
-            vg[u] = g[size_t(j) * Nq + qq];
             vd[u] = di[size_t(j) * Nq + qq];
+            c0[u] = cu[j];
+            c1[u] = cu[j + 1];
         }
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const int j = j0 + u * rstep;
+            const T z = vf[u] * vd[u], lo = T(c0[u]) * vd[u], hi = T(c1[u]) * vd[u];
             if (j < M && j != cs.mid) {
-                T *p = L + slot(j);
-                p[0] = vf[u];
-                p[KL] = vg[u];
-                p[2 * KL] = vd[u];
+                ColStep<T> &l = L[step(j)];
+                l.e[lane(j)] = {z, j < cs.mid ? lo : hi};
+                l.b[lane(j)] = j < cs.mid ? hi : lo;
             } else if (j == cs.mid) {
-                Mid[c] = vf[u];
-                Mid[KC + c] = vd[u];
+                Mid.z[c] = z;
+                Mid.dn[c] = lo;
+                Mid.up[c] = hi;
             }
         }
     }
-    for (int t = threadIdx.x; t < cs.pad_dn * 3 * KL; t += blockDim.x)
-        if (t % KL < KC) L[t] = T(0);
-    for (int t = threadIdx.x; t < cs.pad_up * 3 * KL; t += blockDim.x)
-        if (t % KL >= KC) L[t] = T(0);
+    for (int t = threadIdx.x; t < cs.pad_dn * KC; t += blockDim.x) L[t / KC].e[t % KC] = {T(0), T(0)};
+    for (int t = threadIdx.x; t < cs.pad_up * KC; t += blockDim.x) L[t / KC].e[KC + t % KC] = {T(0), T(0)};
     __syncthreads();
     if (threadIdx.x < KL) {
-        T *p = L + threadIdx.x;
-        T y = T(0), gp = T(0);
-        T nf[KSTEP], ng[KSTEP], nd[KSTEP];
+        __builtin_amdgcn_s_setprio(3);  // the second stream's kernels share the CU
+        const int l = threadIdx.x;
+        ColStep<T> *p = L;
+        T z = T(0);
+        Elim<T> ne[KSTEP];
 #pragma unroll
-        for (int u = 0; u < KSTEP; u++) {
-            nf[u] = p[u * 3 * KL];
-            ng[u] = p[u * 3 * KL + KL];
-            nd[u] = p[u * 3 * KL + 2 * KL];
-        }
-        for (int s = 0; s < cs.steps; s += KSTEP, p += KSTEP * 3 * KL) {
-            T vf[KSTEP], vg[KSTEP], vd[KSTEP];
+        for (int u = 0; u < KSTEP; u++) ne[u] = p[u].e[l];
+        for (int s = 0; s < cs.steps; s += KSTEP, p += KSTEP) {
+            Elim<T> e[KSTEP];
 #pragma unroll
-            for (int u = 0; u < KSTEP; u++) {
-                vf[u] = nf[u];
-                vg[u] = ng[u];
-                vd[u] = nd[u];
-            }
+            for (int u = 0; u < KSTEP; u++) e[u] = ne[u];
             // past the last step this reads the same eight again
-            const T *nx = s + KSTEP < cs.steps ? p + KSTEP * 3 * KL : p;
+            const ColStep<T> *nx = s + KSTEP < cs.steps ? p + KSTEP : p;
+#pragma unroll
+            for (int u = 0; u < KSTEP; u++) ne[u] = nx[u].e[l];
 #pragma unroll
             for (int u = 0; u < KSTEP; u++) {
-                nf[u] = nx[u * 3 * KL];
-                ng[u] = nx[u * 3 * KL + KL];
-                nd[u] = nx[u * 3 * KL + 2 * KL];
+                z = e[u].z + e[u].f * z;
+                p[u].e[l].z = z;
             }
-#pragma unroll
-            for (int u = 0; u < KSTEP; u++) {
-                y = vf[u] + gp * y;
-                gp = vg[u];
-                vf[u] = y * vd[u];
-            }
-#pragma unroll
-            for (int u = 0; u < KSTEP; u++) p[u * 3 * KL] = vf[u];
         }
-        const int col = threadIdx.x % KC;
-        const bool up = threadIdx.x >= KC;
-        const T off = gp * y, other = __shfl_xor(off, KC, kWave);
+        const bool up = l >= KC;
+        const T other = __shfl_xor(z, KC, kWave);
         // the same order of terms in both directions' lanes
-        T x = (Mid[col] + (up ? other : off) + (up ? off : other)) * Mid[KC + col];
-        if (!up) Mid[col] = x;
-        p -= KSTEP * 3 * KL;
+        const int col = l % KC;
+        T x = Mid.z[col] + Mid.dn[col] * (up ? other : z) + Mid.up[col] * (up ? z : other);
+        if (!up) Mid.z[col] = x;
+        p -= KSTEP;
+        T nz[KSTEP], nb[KSTEP];
 #pragma unroll
         for (int u = 0; u < KSTEP; u++) {
-            nf[u] = p[u * 3 * KL];
-            ng[u] = p[u * 3 * KL + KL];
+            nz[u] = p[u].e[l].z;
+            nb[u] = p[u].b[l];
         }
-        for (int s = cs.steps; s > 0; s -= KSTEP, p -= KSTEP * 3 * KL) {
-            T vf[KSTEP], vg[KSTEP];
+        for (int s = cs.steps; s > 0; s -= KSTEP, p -= KSTEP) {
+            T vz[KSTEP], vb[KSTEP];
 #pragma unroll
             for (int u = 0; u < KSTEP; u++) {
-                vf[u] = nf[u];
-                vg[u] = ng[u];
+                vz[u] = nz[u];
+                vb[u] = nb[u];
             }
-            const T *nx = s > KSTEP ? p - KSTEP * 3 * KL : p;
+            const ColStep<T> *nx = s > KSTEP ? p - KSTEP : p;
 #pragma unroll
             for (int u = 0; u < KSTEP; u++) {
-                nf[u] = nx[u * 3 * KL];
-                ng[u] = nx[u * 3 * KL + KL];
+                nz[u] = nx[u].e[l].z;
+                nb[u] = nx[u].b[l];
             }
 #pragma unroll
             for (int u = KSTEP - 1; u >= 0; u--) {
-                x = vf[u] + vg[u] * x;
-                vf[u] = x;
+                x = vz[u] + vb[u] * x;
+                p[u].e[l].z = x;
             }
-#pragma unroll
-            for (int u = 0; u < KSTEP; u++) p[u * 3 * KL] = vf[u];
         }
     }
     __syncthreads();
-    if (int(blockIdx.x) * KC + c >= N) return;
-    for (int j = threadIdx.x / KC; j < M; j += rstep) spec[size_t(j) * N + q] = j == cs.mid ? Mid[c] : L[slot(j)];
+    if (b * KC + c >= N) return;
+    for (int j = threadIdx.x / KC; j < M; j += rstep)
+        spec[size_t(j) * N + q] = j == cs.mid ? Mid.z[c] : L[step(j)].e[lane(j)].z;
 }
 
 constexpr size_t kLdsMax = 160 * 1024;
@@ -571,11 +653,11 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
     plan.threads = std::min(1024, std::max(64, ((N + 7) / 8 + 63) / 64 * 64));
     const size_t LN = size_t(N - 1) + size_t((N - 1) >> 5) + 1;
     row_lds = 2 * LN * sizeof(T);
-    if (other && row_lds + 2 * size_t(N) * sizeof(T) <= kLdsMax) {
-        plan.tw_lds = 1;
+    if (row_lds + 2 * size_t(N) * sizeof(T) <= kLdsMax) {
+        plan.tw = other ? RowPlan::TW_ROOTS : RowPlan::TW_STAGES;
         row_lds += 2 * size_t(N) * sizeof(T);
     }
-    col_lds = col_lds_elems(M) * sizeof(T);
+    col_lds = col_lds_bytes<T>(M);
     if (row_lds > kLdsMax || col_lds > kLdsMax) return VVM_ERR_SIZE;
     if (!allow_lds(k_rows_fwd<T, false>, row_lds) || !allow_lds(k_rows_fwd<T, true>, row_lds) ||
         !allow_lds(k_rows_inv<T, false, false>, row_lds) || !allow_lds(k_rows_inv<T, true, false>, row_lds) ||
@@ -583,10 +665,9 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
         return VVM_ERR_HIP;
     const size_t Nq = size_t(N) / 2 + 1;
     tw = dalloc<T>(4 * size_t(N));
-    g = dalloc<T>(Nq * M);
     di = dalloc<T>(Nq * M);
     spec = dalloc<T>(size_t(N) * M);
-    if (!tw || !g || !di || !spec) {
+    if (!tw || !di || !spec) {
         destroy();
         return VVM_ERR_NOMEM;
     }
@@ -607,21 +688,22 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
             }
     }
     if (hipMemcpy(tw, t.data(), t.size() * sizeof(T), hipMemcpyHostToDevice) != hipSuccess) return VVM_ERR_HIP;
-    hipLaunchKernelGGL(k_factor<T>, dim3(unsigned((Nq + 63) / 64)), dim3(64), 0, nullptr, N, M, cx, cu, g, di);
+    hipLaunchKernelGGL(k_factor<T>, dim3(unsigned((Nq + 63) / 64)), dim3(64), 0, nullptr, N, M, cx, cu, di);
+    cu_dev = cu;
     return hipStreamSynchronize(nullptr) == hipSuccess ? VVM_OK : VVM_ERR_HIP;
 }
 
 template <typename T>
 void Direct<T>::destroy() {
-    for (T *p : {tw, g, di, spec})
+    for (T *p : {tw, di, spec})
         if (p) (void)hipFree(p);
-    tw = g = di = spec = nullptr;
+    tw = di = spec = nullptr;
 }
 
 template <typename T>
 void Direct<T>::columns(hipStream_t st) {
-    hipLaunchKernelGGL(k_columns<T>, dim3((plan.N + KC - 1) / KC), dim3(256), col_lds, st, plan.N, plan.M, spec, g,
-                       di);
+    hipLaunchKernelGGL(k_columns<T>, xcd_grid((plan.N + KC - 1) / KC), dim3(256), col_lds, st, plan.N, plan.M, spec,
+                       di, cu_dev);
 }
 
 template <typename T>

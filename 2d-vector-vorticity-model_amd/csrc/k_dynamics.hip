@@ -543,18 +543,18 @@ void launch_bc_one(const Grid &G, double *a, bool westdown, hipStream_t st) {
 Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
     const int n = t4_tiles_x(G) * t4_tiles_z(G);
     hipLaunchKernelGGL(k_thermo4, xcd_grid(n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
-    return negval_partials(S, rs, n, st);
+    return {rs, n};
 }
 // The ratios of NegativeValueProcess from nblk workgroups' partials: by
 // k_finalize (nblk 0 is returned), or, up to kFoldBlocks, by the workgroups of
 // the second pass themselves (nblk).  The launch costs 4 to 5 us
 // whatever it does; every workgroup's own sum costs the traffic of all partials
 // for each of them, which at 2048 x 256 (1089 and 2145 partials) is no gain.
-Negval negval_partials(const StepPtrs &S, const RedSlot &rs, int nblk, hipStream_t st) {
+Negval negval_partials(const StepPtrs &S, const Negval &nv, hipStream_t st) {
     constexpr int kFoldBlocks = 640;
-    if (nblk <= kFoldBlocks) return {rs, nblk};
-    finalize<6>(rs, nblk, S.s, RED_NEGVAL, S_NEG_RATIO, st);
-    return {rs, 0};
+    if (nv.nblk <= kFoldBlocks) return nv;
+    finalize<6>(nv.rs, nv.nblk, S.s, RED_NEGVAL, S_NEG_RATIO, st);
+    return {nv.rs, 0};
 }
 void launch_scale_forcing(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, hipStream_t st,
                           bool halos) {

@@ -267,12 +267,12 @@ __global__ void __launch_bounds__(256) k_update_mean(Grid G, StepPtrs S, int shi
 
 Negval launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipStream_t st) {
     hipLaunchKernelGGL(k_kessler<KP_ALL>, interior_grid(G), dim3(BX, BY), 0, st, G, S, Negval{}, Forcing{}, rs);
-    return negval_partials(S, rs, nblocks(interior_grid(G)), st);
+    return {rs, nblocks(interior_grid(G))};
 }
 Negval launch_kessler(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, const RedSlot &rs,
                       hipStream_t st) {
     hipLaunchKernelGGL((k_kessler<KP_ALL | KP_PRE>), interior_grid(G), dim3(BX, BY), 0, st, G, S, nv, F, rs);
-    return negval_partials(S, rs, nblocks(interior_grid(G)), st);
+    return {rs, nblocks(interior_grid(G))};
 }
 void launch_kessler_process(const Grid &G, const StepPtrs &S, int process, hipStream_t st) {
     const RedSlot none{nullptr, 0};

@@ -846,7 +846,7 @@ int step_begin(vvm_dev *h, int timer, bool last) {
     }
     if (h->mp_fn) {
         KTimer t(h, VVM_KT_SCALE);
-        launch_scale_forcing(G, S, nv, F, h->st);
+        launch_scale_forcing(G, S, negval_partials(S, nv, h->st), F, h->st);
     }
     if (h->ghosts_dirty) {
         launch_bc_uw(G, S, h->st);
@@ -867,11 +867,11 @@ int step_begin(vvm_dev *h, int timer, bool last) {
         mark(h, 6, cs);
         {
             KTimer t(h, VVM_KT_KESSLER, cs);
-            nv = launch_kessler(G, S, nv, F, h->red.misc, cs);
+            nv = launch_kessler(G, S, negval_partials(S, nv, cs), F, h->red.misc, cs);
         }
         {
             KTimer t(h, VVM_KT_SCALE, cs);
-            launch_scale_forcing(G, S, nv, Forcing{}, cs);
+            launch_scale_forcing(G, S, negval_partials(S, nv, cs), Forcing{}, cs);
         }
         mark(h, 7, cs);
     }
@@ -1020,7 +1020,8 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             launch_pzeta(G, S, h->step, h->st);
             break;
         case VVM_OP_PSCALARS:
-            launch_scale_forcing(G, S, launch_thermo4(G, S, h->step, h->red.negval, h->st), Forcing{}, h->st);
+            launch_scale_forcing(G, S, negval_partials(S, launch_thermo4(G, S, h->step, h->red.negval, h->st), h->st),
+                                 Forcing{}, h->st);
             break;
         case VVM_OP_FORCING_BC: {
             const double none[3] = {-1., -1., -1.};
@@ -1052,7 +1053,8 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             launch_cal_u(G, S, h->st);
             break;
         case VVM_OP_MICROPHYSICS:
-            launch_scale_forcing(G, S, launch_kessler(G, S, h->red.negval, h->st), Forcing{}, h->st);
+            launch_scale_forcing(G, S, negval_partials(S, launch_kessler(G, S, h->red.negval, h->st), h->st), Forcing{},
+                                 h->st);
             launch_bc_all_prog(G, S, h->st);
             break;
         case VVM_OP_TURBULENCE:

@@ -72,8 +72,9 @@ struct Reductions {
 // Dynamics (k_dynamics.hip)
 void launch_pzeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st);
 // launch_thermo4 and launch_kessler leave NegativeValueProcess's first pass in
-// rs; what they return (negval_partials) goes, with rs, to the second pass:
-// launch_scale_forcing, or the launch_kessler behind launch_thermo4.
+// rs; what they return goes through negval_partials, on the second pass's
+// stream, to that pass: launch_scale_forcing, or the launch_kessler behind
+// launch_thermo4.
 struct Negval {
     RedSlot rs;
     int nblk;
@@ -82,7 +83,7 @@ struct Forcing {
     int on, tropical, random_kick;
 };
 Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);
-Negval negval_partials(const StepPtrs &S, const RedSlot &rs, int nblk, hipStream_t st);
+Negval negval_partials(const StepPtrs &S, const Negval &nv, hipStream_t st);
 void launch_scale_forcing(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, hipStream_t st,
                           bool halos = true);
 void launch_bc_uw(const Grid &G, const StepPtrs &S, hipStream_t st);
