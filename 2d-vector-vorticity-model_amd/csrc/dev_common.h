@@ -72,15 +72,57 @@ __device__ inline void store_westdown(double *a, const Grid &G, int i, int k, do
 
 constexpr int kWave = 64;
 
-template <typename T>
-__device__ inline T wave_sum(T v) {
+// The value CTRL (a DPP control) brings from another lane, 0 where there is
+// none or the row of 16 lanes is not in ROWS: a register move, where a shuffle
+// is a round trip through LDS.
+enum { DPP_ROW_SHR = 0x110, DPP_WAVE_SHR1 = 0x138, DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143 };
+template <int CTRL, int ROWS = 0xf, typename T>
+__device__ inline T dpp(T v) {
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "32 or 64 bits");
+    int w[sizeof(T) / 4];
+    __builtin_memcpy(w, &v, sizeof(T));
 #pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+    for (int &x : w) x = __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, true);
+    __builtin_memcpy(&v, w, sizeof(T));
+    return v;
+}
+// lane l's value, l uniform
+template <typename T>
+__device__ inline T from_lane(T v, int l) {
+    int w[sizeof(T) / 4];
+    __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+    for (int &x : w) x = __builtin_amdgcn_readlane(x, l);
+    __builtin_memcpy(&v, w, sizeof(T));
     return v;
 }
 
+// Inclusive prefix sums over each row of 16 lanes, and over the wavefront.
+template <typename T>
+__device__ inline T row_scan(T v) {
+    v += dpp<DPP_ROW_SHR + 1>(v);
+    v += dpp<DPP_ROW_SHR + 2>(v);
+    v += dpp<DPP_ROW_SHR + 4>(v);
+    v += dpp<DPP_ROW_SHR + 8>(v);
+    return v;
+}
+template <typename T>
+__device__ inline T wave_scan(T v) {
+    v = row_scan(v);
+    v += dpp<DPP_ROW_BCAST15, 0xa>(v);
+    v += dpp<DPP_ROW_BCAST31, 0xc>(v);
+    return v;
+}
+template <typename T>
+__device__ inline T wave_sum(T v) {
+    return from_lane(wave_scan(v), kWave - 1);
+}
+
 // Block-wide sums of NV values; the totals are returned to every thread.
-// blockDim must be a multiple of 64 and at most 1024.
+// blockDim must be a multiple of 64 and at most 1024, so that the wavefronts'
+// sums of a value fit a row of lanes: a wavefront adds up to four values' at
+// once.  With shuffles and a loop over the wavefronts, two values over 1024
+// threads took 2 us.
 template <int NV, typename T>
 __device__ inline void block_sum(T (&v)[NV]) {
     __shared__ T sh[NV][16];
@@ -95,10 +137,12 @@ __device__ inline void block_sum(T (&v)[NV]) {
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < NV; j++) {
-        T s = 0;
-        for (int w = 0; w < nw; w++) s += sh[j][w];
-        v[j] = s;
+    for (int j0 = 0; j0 < NV; j0 += 4) {
+        const int j = j0 + lane / 16;
+        const T s = row_scan(j < NV && lane % 16 < nw ? sh[min(j, NV - 1)][lane % 16] : T(0));
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (j0 + q < NV) v[j0 + q] = from_lane(s, 16 * q + 15);
     }
     __syncthreads();
 }

@@ -197,13 +197,15 @@ __global__ void __launch_bounds__(BX *TBY) k_turb_coeffs(Grid G, StepPtrs S, dou
         const double v = turb_point(G, S, i, k);
         m = max_or_nan(m, v);
     }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-        const double o = __shfl_xor(m, off, kWave);
-        m = max_or_nan(m, o);
-    }
+    // m >= 0 or NaN, so that a lane without a partner takes 0 (dpp)
+    m = max_or_nan(m, dpp<DPP_ROW_SHR + 1>(m));
+    m = max_or_nan(m, dpp<DPP_ROW_SHR + 2>(m));
+    m = max_or_nan(m, dpp<DPP_ROW_SHR + 4>(m));
+    m = max_or_nan(m, dpp<DPP_ROW_SHR + 8>(m));
+    m = max_or_nan(m, dpp<DPP_ROW_BCAST15, 0xa>(m));
+    m = max_or_nan(m, dpp<DPP_ROW_BCAST31, 0xc>(m));
     __shared__ double sh[TBY];
-    if (threadIdx.x == 0) sh[threadIdx.y] = m;
+    if (threadIdx.x == kWave - 1) sh[threadIdx.y] = m;
     __syncthreads();
     if (threadIdx.x == 0 && threadIdx.y == 0) {
         for (int w = 1; w < TBY; w++) m = max_or_nan(m, sh[w]);

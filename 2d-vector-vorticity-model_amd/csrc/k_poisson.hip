@@ -195,43 +195,52 @@ __global__ void k_extrapolate(size_t n, double *x, const double *x1, const doubl
 
 // ------------------------------------------------------------------ cal_u
 
-// Sums over 1024 threads of per-thread element runs: exclusive prefix of the
-// thread totals (LDS scratch for 16 waves).
-__device__ inline double block_excl_sum(double v, double *total) {
-    __shared__ double ws[16];
-    const int tid = threadIdx.x, lane = tid % kWave, wid = tid / kWave, nw = blockDim.x / kWave;
-    double inc = v;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const double o = __shfl_up(inc, off, kWave);
-        if (lane >= off) inc += o;
-    }
-    const double below = __shfl_up(inc, 1, kWave);
-    if (lane == kWave - 1) ws[wid] = inc;
-    __syncthreads();
-    double wpre = 0., all = 0.;
-    for (int w2 = 0; w2 < nw; w2++) {
-        if (w2 < wid) wpre += ws[w2];
-        all += ws[w2];
+// Over 1024 threads (16 wavefronts): the exclusive prefix sum of v, its total
+// and that of t.
+__device__ inline double block_excl_sum(double v, double t, double *total, double *ttotal) {
+    __shared__ double ws[2][16];
+    const int lane = threadIdx.x % kWave, wid = uniform(threadIdx.x / kWave);
+    const double inc = wave_scan(v), below = dpp<DPP_WAVE_SHR1>(inc), tw = wave_scan(t);
+    if (lane == kWave - 1) {
+        ws[0][wid] = inc;
+        ws[1][wid] = tw;
     }
     __syncthreads();
-    *total = all;
-    return (lane == 0) ? wpre : wpre + below;
+    const double s = row_scan(ws[lane / 16 % 2][lane % 16]);
+    __syncthreads();
+    *total = from_lane(s, 15);
+    *ttotal = from_lane(s, 31);
+    return wid > 0 ? from_lane(s, wid - 1) + below : below;
 }
 
 // The residual's norms, one pair of partial sums per workgroup: block of nblk
-// 1024-thread workgroups, each walking 64 x 16 tiles.
+// 1024-thread workgroups, each walking 64 x 16 tiles, four tiles' loads in
+// flight (a thread outside the grid reads its edge).
 __device__ inline void residual_norms(const Residual &R, int block, int nblk) {
-    constexpr int RX = 64, RY = 16;
+    constexpr int RX = 64, RY = 16, U = 4;
     const int N = R.N, M = R.M, tx = (N + RX - 1) / RX, nt = tx * ((M + RY - 1) / RY);
     double part[2] = {0., 0.};
-    for (int t = block; t < nt; t += nblk) {
-        const int i = (t % tx) * RX + threadIdx.x % RX, j = 1 + (t / tx) * RY + threadIdx.x / RX;
-        if (i < N && j <= M) {
-            const double fv = R.f[size_t(j) * N + i];
-            const double wr = R.wD[j] * (fv - applyL(R.x, N, i, j, R.cx[j], R.cu[j], R.cu[j - 1])), wb = R.wD[j] * fv;
-            part[0] += wr * wr;
-            part[1] += wb * wb;
+    for (int t0 = block; t0 < nt; t0 += U * nblk) {
+        double fv[U], lv[U], wd[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (u > 0 && t0 + u * nblk >= nt) break;
+            const int t = t0 + u * nblk;
+            const int i = min((t % tx) * RX + int(threadIdx.x % RX), N - 1);
+            const int j = min(1 + (t / tx) * RY + uniform(threadIdx.x / RX), M);
+            fv[u] = R.f[size_t(j) * N + i];
+            lv[u] = applyL(R.x, N, i, j, R.cx[j], R.cu[j], R.cu[j - 1]);
+            wd[u] = R.wD[j];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int t = t0 + u * nblk;
+            const int i = (t % tx) * RX + threadIdx.x % RX, j = 1 + (t / tx) * RY + threadIdx.x / RX;
+            if (t < nt && i < N && j <= M) {
+                const double wr = wd[u] * (fv[u] - lv[u]), wb = wd[u] * fv[u];
+                part[0] += wr * wr;
+                part[1] += wb * wb;
+            }
         }
     }
     block_sum<2>(part);
@@ -246,7 +255,8 @@ __device__ inline void residual_norms(const Residual &R, int block, int nblk) {
 // D_{r+1} - D_r = h_r and sum_r D_r = 0, so D_r = S_r - mean(S) with S the
 // exclusive prefix sum of h.  uxi = D rdx (mean removed as in the
 // reference), u[i][nz-2] = uxi + ubarTopp, and xi = the mean-free y.  With P
-// the prefix sum of h as it is, S_r = P_r - r mean(h).
+// the prefix sum of h as it is, S_r = P_r - r mean(h), and sum_r S_r =
+// sum_r ((N-1)/2 - r) h_r, which the scan of h brings along.
 //
 // Then the downward integration u[i][k] = u[i][nz-2] - dz sum_{k'=k}^{nz-3}
 // ((w[i][k'+1]-w[i-1][k'+1]) rdx - rhow[k'+1] zetap[i][k'+1]) (:643-650):
@@ -254,57 +264,82 @@ __device__ inline void residual_norms(const Residual &R, int block, int nblk) {
 // enough workgroups for every CU), chunk sums scanned in LDS.
 //
 // Every workgroup forms the whole top row's prefix sums for its own 16
-// columns, three block scans of about half a microsecond: cheaper than a
-// kernel of one workgroup before this one (13 us at 2048 columns, 11 at 128).
+// columns, two block scans that take 1.6 us at 1024 columns (three, through LDS
+// shuffles, 4.5): cheaper than a kernel of one workgroup before this one (13
+// us at 2048 columns, 11 at 128).  The rest is the latency of the first loads,
+// 3 us there; a chunk's levels, up to UT, are read once and kept.  64 registers
+// at most, so that a CU holds two workgroups and 4096 columns run in one round.
 // The workgroups from ncol on form the residual norms of the solve that left
 // w, which would be a launch of 4 to 5 us.
-constexpr int UW = 16, UC = 64;
-__global__ void __launch_bounds__(UW *UC) k_calu(Grid G, StepPtrs S, int ncol, Residual R) {
+constexpr int UW = 16, UC = 64, UT = 4;
+__global__ void __launch_bounds__(UW *UC) __attribute__((amdgpu_waves_per_eu(8))) k_calu(Grid G, StepPtrs S, int ncol, Residual R) {
     extern __shared__ double sh[];  // N doubles: P
-    __shared__ double cs[UC][UW], top[UW];
+    __shared__ double cs[UW * UC / kWave][UW], top[UW];
     if (int(blockIdx.x) >= ncol) {
         residual_norms(R, blockIdx.x - ncol, gridDim.x - ncol);
         return;
     }
     const int N = G.nx - 2, nz = G.nz, tid = threadIdx.x;
     const double *w = S.w, *zp = S.fut[F_ZETA], *rhow = S.P.rhow, *rhou = S.P.rhou;
-    const int i = 1 + blockIdx.x * UW + tid % UW, c = tid / UW;
+    const int i = 1 + blockIdx.x * UW + tid % UW, c = tid / UW, ic = min(i, N);
     const int K = nz - 3;  // levels nz-3 .. 1
     const int C = (K + UC - 1) / UC;
     const bool col = (i <= N);
+    const int E = (N + UW * UC - 1) / (UW * UC), r0 = min(tid * E, N), r1 = min(r0 + E, N);
+    // every load before the first wait: the top row, and up to UT levels of
+    // the thread's chunk
+    double hv[8], tv[UT];
+#pragma unroll
+    for (int e = 0; e < 8; e++)  // N <= 8 UW UC
+        if (e < E) hv[e] = w[ix(G, 1 + min(tid + e * UW * UC, N - 1), nz - 2)];
     auto term = [&](int k) {  // level k's part of the integral
-        return ((w[ix(G, i, k + 1)] - w[ix(G, i - 1, k + 1)]) * G.rdx - rhow[k + 1] * zp[ix(G, i, k + 1)]) * -G.dz;
+        return ((w[ix(G, ic, k + 1)] - w[ix(G, ic - 1, k + 1)]) * G.rdx - rhow[k + 1] * zp[ix(G, ic, k + 1)]) * -G.dz;
     };
+    const int kk0 = min(c * C, K), kk1 = min(kk0 + C, K);
+#pragma unroll
+    for (int u = 0; u < UT; u++)
+        if (u < C) tv[u] = term(max(nz - 3 - (kk0 + u), 1));
+    const double ubp = S.s[S_UBARTOPP];
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        if (e < E && tid + e * UW * UC < N)  // src/PoissonSolver.cpp:585-594
+            sh[tid + e * UW * UC] = -(0. - rhow[nz - 2] * hv[e]) / rhou[nz - 2] * G.dx;
+    // the chunk's sum; the sums of the wavefront's chunks above it (four, 16
+    // lanes apart), and the wavefront's to LDS
     double loc = 0.;
-    if (col)
-        for (int kk = c * C; kk < min((c + 1) * C, K); kk++) loc += term(nz - 3 - kk);
-    cs[c][tid % UW] = loc;
-
-    const int E = (N + UW * UC - 1) / (UW * UC), r0 = tid * E, r1 = min(r0 + E, N);
-    loc = 0.;
-    for (int r = r0; r < r1; r++) {  // src/PoissonSolver.cpp:585-594
-        const double h = -(0. - rhow[nz - 2] * w[ix(G, r + 1, nz - 2)]) / rhou[nz - 2] * G.dx;
-        sh[r] = h;
-        loc += h;
+#pragma unroll
+    for (int u = 0; u < UT; u++)
+        if (kk0 + u < kk1) loc += tv[u];
+    for (int kk = kk0 + UT; kk < kk1; kk++) loc += term(nz - 3 - kk);
+    double above = 0.;
+#pragma unroll
+    for (int d = 1; d < kWave / UW; d++) {
+        const double o = __shfl_up(loc, d * UW, kWave);
+        if (tid % kWave >= d * UW) above += o;
     }
-    double tot;
-    double p = block_excl_sum(loc, &tot);
+    if (tid % kWave >= kWave - UW) cs[tid / kWave][tid % UW] = above + loc;
+    __syncthreads();
+
+    loc = 0.;
+    double mom = 0.;  // sum over r of S_r
+    for (int r = r0; r < r1; r++) {
+        loc += sh[r];
+        mom += (0.5 * (N - 1) - r) * sh[r];
+    }
+    double tot, sm;
+    double p = block_excl_sum(loc, mom, &tot, &sm);
     const double hm = tot / N;
-    double sp = 0.;
+    sm /= N;
     for (int r = r0; r < r1; r++) {
         const double h = sh[r];
         sh[r] = p;
-        sp += p;
         p += h;
     }
-    block_excl_sum(sp, &tot);
-    const double sm = tot / N - hm * (0.5 * (N - 1));
     auto D = [&](int r) { return sh[r] - r * hm - sm; };
-    double sd = 0.;
+    double sd = 0., none;
     for (int r = r0; r < r1; r++) sd += D(r);
-    double y = block_excl_sum(sd, &tot);
+    double y = block_excl_sum(sd, 0., &tot, &none);
     const double um = tot * G.rdx / N;  // :621-634
-    const double ubp = S.s[S_UBARTOPP];
     const int b0 = blockIdx.x * UW;
     for (int r = max(r0, b0); r < min(r1, b0 + UW); r++) {
         const double uxi = D(r) * G.rdx - um;
@@ -315,17 +350,20 @@ __global__ void __launch_bounds__(UW *UC) k_calu(Grid G, StepPtrs S, int ncol, R
         store_center(S.u, G, r + 1, nz - 2, uxi + ubp);
     }
     if (blockIdx.x == 0) {
-        // xi: y_r = sum_{j<=r} D_j minus its mean (min-norm solution)
+        // xi: y_r = sum_{j<=r} D_j minus its mean (min-norm solution); what
+        // rounding left of D's own mean would grow with r
+        const double dm = tot / N;
+        y -= r0 * dm;
         double sy = 0., yr = y;
         for (int r = r0; r < r1; r++) {
-            yr += D(r);
+            yr += D(r) - dm;
             sy += yr;
         }
-        block_excl_sum(sy, &tot);
+        block_excl_sum(sy, 0., &tot, &none);
         const double ym = tot / N;
         yr = y;
         for (int r = r0; r < r1; r++) {
-            yr += D(r);
+            yr += D(r) - dm;
             const double xi = yr - ym;
             S.xi[r + 1] = xi;
             if (r + 1 == N) S.xi[0] = xi;
@@ -335,12 +373,18 @@ __global__ void __launch_bounds__(UW *UC) k_calu(Grid G, StepPtrs S, int ncol, R
     __syncthreads();  // top
     if (!col) return;
     double area = 0.;
-    for (int c2 = 0; c2 < c; c2++) area += cs[c2][tid % UW];
+    for (int w2 = 0; w2 < tid / kWave; w2++) area += cs[w2][tid % UW];
+    area += above;
     const double utop = top[tid % UW];
-    for (int kk = c * C; kk < min((c + 1) * C, K); kk++) {
-        const int k = nz - 3 - kk;
-        area += term(k);
-        store_center(S.u, G, i, k, area + utop);
+#pragma unroll
+    for (int u = 0; u < UT; u++)
+        if (kk0 + u < kk1) {
+            area += tv[u];
+            store_center(S.u, G, i, nz - 3 - (kk0 + u), area + utop);
+        }
+    for (int kk = kk0 + UT; kk < kk1; kk++) {
+        area += term(nz - 3 - kk);
+        store_center(S.u, G, i, nz - 3 - kk, area + utop);
     }
 }
 

@@ -47,7 +47,7 @@ struct SolveResult {
 
 // ||wD (f - L x)||^2 and ||wD f||^2: a pair of partial sums per workgroup into
 // hres (host-mapped memory, at most kResidualBlocks pairs).
-constexpr int kResidualBlocks = 512;
+constexpr int kResidualBlocks = 256;
 struct Residual {
     int N, M;
     const double *f, *x, *cx, *cu, *wD;
