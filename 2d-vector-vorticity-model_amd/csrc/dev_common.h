@@ -118,10 +118,24 @@ __device__ inline T wave_sum(T v) {
     return from_lane(wave_scan(v), kWave - 1);
 }
 
+// v[j] = sh[j][0] + .. + sh[j][n - 1], n <= W <= 16, in every lane: a row of
+// lanes a value, four values at once.
+template <int W, int NV, typename T>
+__device__ inline void sum_rows(const T (&sh)[NV][W], int n, T (&v)[NV]) {
+    const int lane = (threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z)) % kWave;
+#pragma unroll
+    for (int j0 = 0; j0 < NV; j0 += 4) {
+        const int j = j0 + lane / 16;
+        const T s = row_scan(j < NV && lane % 16 < n ? sh[min(j, NV - 1)][min(lane % 16, W - 1)] : T(0));
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (j0 + q < NV) v[j0 + q] = from_lane(s, 16 * q + 15);
+    }
+}
+
 // Block-wide sums of NV values; the totals are returned to every thread.
 // blockDim must be a multiple of 64 and at most 1024, so that the wavefronts'
-// sums of a value fit a row of lanes: a wavefront adds up to four values' at
-// once.  With shuffles and a loop over the wavefronts, two values over 1024
+// sums of a value fit a row of lanes.  With shuffles and a loop over the wavefronts, two values over 1024
 // threads took 2 us.
 template <int NV, typename T>
 __device__ inline void block_sum(T (&v)[NV]) {
@@ -136,14 +150,7 @@ __device__ inline void block_sum(T (&v)[NV]) {
         for (int j = 0; j < NV; j++) sh[j][wid] = v[j];
     }
     __syncthreads();
-#pragma unroll
-    for (int j0 = 0; j0 < NV; j0 += 4) {
-        const int j = j0 + lane / 16;
-        const T s = row_scan(j < NV && lane % 16 < nw ? sh[min(j, NV - 1)][lane % 16] : T(0));
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            if (j0 + q < NV) v[j0 + q] = from_lane(s, 16 * q + 15);
-    }
+    sum_rows<16>(sh, nw, v);
     __syncthreads();
 }
 
@@ -208,19 +215,30 @@ __device__ inline double negval_ratio(double P, double N) {
 }
 
 // The totals of nblk workgroups' partials, in every thread of a workgroup.
-// The partials are added by a fixed 256 threads in a fixed order, so that all
-// callers agree bit for bit; blockDim is 256.
+// They are added as by 256 threads, in a fixed order, whatever the workgroup's
+// size: all callers agree bit for bit.
 template <int NV>
 __device__ inline void sum_partials(const RedSlot &rs, int nblk, double (&acc)[NV]) {
-    const int tid = threadIdx.x + blockDim.x * threadIdx.y;
+    __shared__ double sh[NV][4];
+    const int tid = threadIdx.x + blockDim.x * threadIdx.y, nw = blockDim.x * blockDim.y / kWave;
+    const int lane = tid % kWave, wid = tid / kWave;
+    for (int vw = wid; vw < 4; vw += nw) {
 #pragma unroll
-    for (int j = 0; j < NV; j++) acc[j] = 0.;
+        for (int j = 0; j < NV; j++) acc[j] = 0.;
 #pragma unroll 4
-    for (int b = tid; b < nblk; b += 256) {
+        for (int b = vw * kWave + lane; b < nblk; b += 256) {
 #pragma unroll
-        for (int j = 0; j < NV; j++) acc[j] += rs.partial[size_t(j) * rs.max_blocks + b];
+            for (int j = 0; j < NV; j++) acc[j] += rs.partial[size_t(j) * rs.max_blocks + b];
+        }
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            const double t = wave_sum(acc[j]);
+            if (lane == 0) sh[j][vw] = t;
+        }
     }
-    block_sum<NV>(acc);
+    __syncthreads();
+    sum_rows<4>(sh, 4, acc);
+    __syncthreads();
 }
 
 namespace {

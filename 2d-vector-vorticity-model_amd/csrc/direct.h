@@ -12,6 +12,8 @@
 
 namespace vvmd {
 
+struct Micro;
+
 constexpr int kMaxStages = 16;
 
 // The factors of N and the launch shape of the row transforms.
@@ -39,8 +41,10 @@ class Direct {
     void solve(const double *r, const double *x0, double *x, hipStream_t st);
     // cal_w whole: f = -b / rhow from zetap (f is written, for the residual),
     // x = L^-1 f, w = x / rhow with its halos; pubarTop_pt beside the first
-    // kernel's row transforms (step < 0: not).
-    void solve_step(const Grid &G, const StepPtrs &S, int step, double *f, double *x, hipStream_t st);
+    // kernel's row transforms (step < 0: not), and the microphysics (if set)
+    // beside the first two kernels.
+    void solve_step(const Grid &G, const StepPtrs &S, int step, const Micro *micro, double *f, double *x,
+                    hipStream_t st);
 
    private:
     RowPlan plan;
@@ -49,7 +53,8 @@ class Direct {
     T *di = nullptr;    // [M][N/2+1] 1 / pivot
     const double *cu_dev = nullptr;
     T *spec = nullptr;  // [M][N] transformed rows
-    void columns(hipStream_t st);
+    template <typename Mic>
+    void columns(const Mic &mic, int nmic, hipStream_t st);
 };
 
 }  // namespace vvmd

@@ -7,9 +7,11 @@
 // kernel), four LDS round trips of 1 us, the elimination's serial chain.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "direct.h"
+#include "micro.h"
 #include "pubartop.h"
 
 namespace vvmd {
@@ -288,16 +290,21 @@ __device__ inline void hartley_pair(const T *re, const T *im, int N, int q, T h,
 // f = -b / rhow, b = rhow^2 (zetap[i+1] - zetap[i]) dx
 // (src/PoissonSolver.cpp:444-450), formed from zetap and stored (RHS true).
 // Times 1/N, the inverse transform's.
-// With RHS and a step the last workgroup does pubarTop_pt instead: it reads u, w and K as
-// the solve finds them, and alone it was a launch of 5 to 8 us.
+// With RHS the workgroups behind the rows' do what else has to follow the
+// advection: with a step one pubarTop_pt, which reads u, w and K as the solve
+// finds them (alone it was a launch of 5 to 8 us), and m.nblk Kessler.
 template <typename T, bool RHS>
 __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restrict__ tw, const double *__restrict__ r,
                                                    T *__restrict__ spec, Grid G, StepPtrs S, int step,
-                                                   double *__restrict__ f) {
+                                                   double *__restrict__ f, Micro m) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    if (RHS && step >= 0 && blockIdx.x == gridDim.x - 1) {
-        pubartop_block(G, S, step);
-        return;
+    if constexpr (RHS) {
+        const int extra = int(blockIdx.x) - (P.M + 1) / 2, first = step >= 0 ? 1 : 0;
+        if (extra >= 0) {
+            if (extra < first) pubartop_block(G, S, step);
+            else kessler_block(G, S, m, extra - first);
+            return;
+        }
     }
     const double *zetap = S.fut[F_ZETA], *rhow = S.P.rhow;
     const int N = P.N, M = P.M, LN = pad(N - 1) + 1;
@@ -505,14 +512,30 @@ size_t col_lds_bytes(int M) {
     return size_t(col_steps(M).steps) * sizeof(ColStep<T>) + sizeof(ColMid<T>);
 }
 
-template <typename T>
+// With Mic the workgroups behind those of the columns do the second pass of
+// the microphysics that rode in k_rows_fwd.
+struct NoMicro {};
+struct MicroPass {
+    Grid G;
+    StepPtrs S;
+    Negval nv;
+    int nblk;
+};
+template <typename T, typename Mic>
 __global__ void __launch_bounds__(256) k_columns(int N, int M, T *__restrict__ spec, const T *__restrict__ di,
-                                                 const double *__restrict__ cu) {
+                                                 const double *__restrict__ cu, Mic mic) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ColStep<T> *L = reinterpret_cast<ColStep<T> *>(lds_raw);
     const ColSteps cs = col_steps(M);
     ColMid<T> &Mid = *reinterpret_cast<ColMid<T> *>(L + cs.steps);
     const int Nq = N / 2 + 1, nt = (N + KC - 1) / KC, tile = xcd_tile(nt);
+    if constexpr (std::is_same<Mic, MicroPass>::value) {
+        const int extra = int(blockIdx.x) - kXcds * xcd_run(nt);
+        if (extra >= 0) {
+            scale_block(mic.G, mic.S, mic.nv, extra, mic.nblk);
+            return;
+        }
+    }
     if (tile >= nt) return;
     const int b = tile % 2 ? nt - 1 - tile / 2 : tile / 2;
     // columns past the last repeat it (never stored)
@@ -611,7 +634,7 @@ __global__ void __launch_bounds__(256) k_columns(int N, int M, T *__restrict__ s
         spec[size_t(j) * N + q] = j == cs.mid ? Mid.z[c] : L[step(j)].e[lane(j)].z;
 }
 
-constexpr size_t kLdsMax = 160 * 1024;
+constexpr size_t kLdsMax = 160 * 1024, kLdsStatic = 4 * 1024;  // the sums' arrays
 
 template <typename T>
 T *dalloc(size_t n) {
@@ -653,7 +676,7 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
     plan.threads = std::min(1024, std::max(64, ((N + 7) / 8 + 63) / 64 * 64));
     const size_t LN = size_t(N - 1) + size_t((N - 1) >> 5) + 1;
     row_lds = 2 * LN * sizeof(T);
-    if (row_lds + 2 * size_t(N) * sizeof(T) <= kLdsMax) {
+    if (row_lds + 2 * size_t(N) * sizeof(T) <= kLdsMax - kLdsStatic) {
         plan.tw = other ? RowPlan::TW_ROOTS : RowPlan::TW_STAGES;
         row_lds += 2 * size_t(N) * sizeof(T);
     }
@@ -661,7 +684,8 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
     if (row_lds > kLdsMax || col_lds > kLdsMax) return VVM_ERR_SIZE;
     if (!allow_lds(k_rows_fwd<T, false>, row_lds) || !allow_lds(k_rows_fwd<T, true>, row_lds) ||
         !allow_lds(k_rows_inv<T, false, false>, row_lds) || !allow_lds(k_rows_inv<T, true, false>, row_lds) ||
-        !allow_lds(k_rows_inv<T, false, true>, row_lds) || !allow_lds(k_columns<T>, col_lds))
+        !allow_lds(k_rows_inv<T, false, true>, row_lds) || !allow_lds(k_columns<T, NoMicro>, col_lds) ||
+        !allow_lds(k_columns<T, MicroPass>, col_lds))
         return VVM_ERR_HIP;
     const size_t Nq = size_t(N) / 2 + 1;
     tw = dalloc<T>(4 * size_t(N));
@@ -701,17 +725,18 @@ void Direct<T>::destroy() {
 }
 
 template <typename T>
-void Direct<T>::columns(hipStream_t st) {
-    hipLaunchKernelGGL(k_columns<T>, xcd_grid((plan.N + KC - 1) / KC), dim3(256), col_lds, st, plan.N, plan.M, spec,
-                       di, cu_dev);
+template <typename Mic>
+void Direct<T>::columns(const Mic &mic, int nmic, hipStream_t st) {
+    const dim3 gr(xcd_grid((plan.N + KC - 1) / KC).x + nmic);
+    hipLaunchKernelGGL((k_columns<T, Mic>), gr, dim3(256), col_lds, st, plan.N, plan.M, spec, di, cu_dev, mic);
 }
 
 template <typename T>
 void Direct<T>::solve(const double *r, const double *x0, double *x, hipStream_t st) {
     const dim3 gr((plan.M + 1) / 2), b(plan.threads);
-    hipLaunchKernelGGL((k_rows_fwd<T, false>), gr, b, row_lds, st, plan, tw, r, spec, Grid{}, StepPtrs{}, 0,
-                       nullptr);
-    columns(st);
+    hipLaunchKernelGGL((k_rows_fwd<T, false>), gr, b, row_lds, st, plan, tw, r, spec, Grid{}, StepPtrs{}, 0, nullptr,
+                       Micro{});
+    columns(NoMicro{}, 0, st);
     if (x0)
         hipLaunchKernelGGL((k_rows_inv<T, true, false>), gr, b, row_lds, st, plan, tw, spec, x0, x, Grid{}, nullptr,
                            nullptr);
@@ -721,10 +746,22 @@ void Direct<T>::solve(const double *r, const double *x0, double *x, hipStream_t 
 }
 
 template <typename T>
-void Direct<T>::solve_step(const Grid &G, const StepPtrs &S, int step, double *f, double *x, hipStream_t st) {
+void Direct<T>::solve_step(const Grid &G, const StepPtrs &S, int step, const Micro *micro, double *f, double *x,
+                           hipStream_t st) {
     const dim3 gr((plan.M + 1) / 2), b(plan.threads);
-    hipLaunchKernelGGL((k_rows_fwd<T, true>), dim3(gr.x + (step >= 0 ? 1 : 0)), b, row_lds, st, plan, tw, nullptr, spec, G, S, step, f);
-    columns(st);
+    Micro m;
+    if (micro) {
+        m = *micro;
+        m.nblk = std::min(kMicroBlocks, micro_tiles(G, plan.threads));
+    }
+    hipLaunchKernelGGL((k_rows_fwd<T, true>), dim3(gr.x + (step >= 0 ? 1 : 0) + m.nblk), b, row_lds, st, plan, tw,
+                       nullptr, spec, G, S, step, f, m);
+    if (micro) {
+        const int n = std::min(kMicroBlocks, micro_tiles(G, 256));
+        columns(MicroPass{G, S, Negval{m.rs, m.nblk}, n}, n, st);
+    } else {
+        columns(NoMicro{}, 0, st);
+    }
     hipLaunchKernelGGL((k_rows_inv<T, false, true>), gr, b, row_lds, st, plan, tw, spec, nullptr, x, G, S.w,
                        S.P.rhow);
 }

@@ -10,7 +10,7 @@
 #pragma clang fp contract(off)
 
 #include "pubartop.h"
-#include "scale_forcing.h"
+#include "micro.h"
 #include "vvm_internal.h"
 
 namespace vvmd {
@@ -393,26 +393,11 @@ __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8
     block_partials<6>(part, rs, tile);
 }
 
-// Second pass of NegativeValueProcess for qv, qc, qr (MicroPhysics.cpp:
-// 129-137), AddForcing (F.on), and the center halos of thp, qvp, qcp, qrp.
-// halos == 0 is AddForcing alone (ratios < 0): interior thp and qvp only.
 __global__ void __launch_bounds__(BX *BY) k_scale_forcing(Grid G, StepPtrs S, Negval nv, Forcing F, int halos) {
     const int i = 1 + blockIdx.x * BX + threadIdx.x, k = 1 + blockIdx.y * BY + uniform(threadIdx.y);
     double ratios[3];
     negval_ratios(S, nv.rs, nv.nblk, ratios);
-    if (i > G.nx - 2 || k > G.nz - 2) return;
-#pragma unroll
-    for (int q = 0; q < 3; q++) {
-        const int f = F_QV + q;
-        double v = rescaled(at(S.fut[f], G, i, k), ratios[q]);
-        if (F.on && f == F_QV) v = forced_qv(G, S, F, k, v);
-        if (halos) store_center(S.fut[f], G, i, k, v);
-        else if (f == F_QV) at(S.fut[f], G, i, k) = v;
-    }
-    double th = at(S.fut[F_TH], G, i, k);
-    if (F.on) th = forced_th(G, S, F, i, k, th);
-    if (halos) store_center(S.fut[F_TH], G, i, k, th);
-    else at(S.fut[F_TH], G, i, k) = th;
+    if (i <= G.nx - 2 && k <= G.nz - 2) scale_point(G, S, F, ratios, halos != 0, i, k);
 }
 
 // Halo value of BoundaryProcess2D_center at a perimeter cell.
@@ -543,7 +528,6 @@ Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot 
 // whatever it does; every workgroup's own sum costs the traffic of all partials
 // for each of them, which at 2048 x 256 (1089 and 2145 partials) is no gain.
 Negval negval_partials(const StepPtrs &S, const Negval &nv, hipStream_t st) {
-    constexpr int kFoldBlocks = 640;
     if (nv.nblk <= kFoldBlocks) return nv;
     finalize<6>(nv.rs, nv.nblk, S.s, RED_NEGVAL, S_NEG_RATIO, st);
     return {nv.rs, 0};

@@ -7,7 +7,7 @@
 // (b<a)?b:a.
 #pragma clang fp contract(off)
 
-#include "scale_forcing.h"
+#include "micro.h"
 #include "vvm_internal.h"
 
 #include <cstdio>
@@ -20,110 +20,19 @@ namespace {
 constexpr int BX = 64, BY = 4;
 
 __device__ inline double max_or_nan(double a, double b) { return (a != a || a > b) ? a : b; }
-__device__ inline double maxs(double a, double b) { return (a < b) ? b : a; }
-__device__ inline double mins(double a, double b) { return (b < a) ? b : a; }
 
 inline dim3 grid2d(const Grid &G) { return dim3((G.nx + BX - 1) / BX, (G.nz + BY - 1) / BY); }
 // from the first interior point on: one tile less where the grid's columns and
 // rows are multiples of the tile, and with it the last, nearly empty round
 inline dim3 interior_grid(const Grid &G) { return dim3((G.nx - 2 + BX - 1) / BX, (G.nz - 2 + BY - 1) / BY); }
 
-// MicroPhysics::autoconversion, accretion, evaporation, condensation
-// (MicroPhysics.cpp:29-51, 54-77, 80-114, 7-26).  Each is pointwise, so
-// running the four in call order per point equals the reference's four
-// sweeps.  Then the first pass of NegativeValueProcess on qvp, qcp, qrp
-// (src/Iteration.cpp:309-311); k_finalize computes the three ratios.
-// PROC selects the processes (KP_*); the timestep runs them all with the
-// negative-value pass (KP_ALL).  One process alone (the reference's
-// MicroPhysics statics) writes only the fields and the rate it changes.
-// KP_PRE: the fields are read as thermo4 left them, and its negative-value
-// rescale and AddForcing are applied on the way.  In the timestep that is one
-// launch and one pass over four fields less, 9 us at 2048 x 256 between the
-// advection and the solve: 20 steps there go 4948 -> 4806 us,
-// 4096 x 256 8177 -> 7850.
-enum { KP_AUTO = 1, KP_ACCR = 2, KP_EVAP = 4, KP_COND = 8, KP_NEG = 16, KP_ALL = 31, KP_PRE = 32 };
-
 template <int PROC>
 __global__ void __launch_bounds__(BX *BY) k_kessler(Grid G, StepPtrs S, Negval nv, Forcing F, RedSlot rs) {
     const int i = 1 + blockIdx.x * BX + threadIdx.x, k = 1 + blockIdx.y * BY + uniform(threadIdx.y);
-    const bool inside = (i >= 1 && i <= G.nx - 2 && k >= 1 && k <= G.nz - 2);
     double part[6] = {0., 0., 0., 0., 0., 0.};
     double ratios[3] = {-1., -1., -1.};
     if constexpr ((PROC & KP_PRE) != 0) negval_ratios(S, nv.rs, nv.nblk, ratios);
-    if (inside) {
-        const double dt = G.dt, pib = S.P.pib[k], rhou = S.P.rhou[k], pb = S.P.pb[k], pc = S.P.pcoef[k];
-        double qc = at(S.fut[F_QC], G, i, k), qr = at(S.fut[F_QR], G, i, k), qv = at(S.fut[F_QV], G, i, k), th = at(S.fut[F_TH], G, i, k);
-        if constexpr ((PROC & KP_PRE) != 0) {
-            qv = forced_qv(G, S, F, k, rescaled(qv, ratios[0]));
-            qc = rescaled(qc, ratios[1]);
-            qr = rescaled(qr, ratios[2]);
-            th = forced_th(G, S, F, i, k, th);
-        }
-        if constexpr ((PROC & KP_AUTO) != 0) {  // autoconversion
-            const double qcplus = maxs(0., qc);
-            double ar = 0.001 * (qcplus - 0.001);
-            ar = maxs(0., ar);
-            const double arcrdt = mins(ar * dt, qcplus);
-            qc = qc - arcrdt;
-            qr = qr + arcrdt;
-            at(S.autoc, G, i, k) = arcrdt;
-        }
-        if constexpr ((PROC & KP_ACCR) != 0) {  // accretion
-            const double qcplus = maxs(0., qc), qrplus = maxs(0., qr);
-            // no rain, over most of a domain: the power is zero
-            const double cr = 2.2 * qcplus * (qrplus == 0. ? 0. : pow(qrplus, 0.875));
-            const double arcrdt = mins(cr * dt, qcplus);
-            qc = qc - arcrdt;
-            qr = qr + arcrdt;
-            at(S.accr, G, i, k) = arcrdt;
-        }
-        if constexpr ((PROC & KP_EVAP) != 0) {  // rain evaporation
-            const double qrplus = maxs(0., qr), qvplus = maxs(0., qv);
-            double erdt = 0.;
-            if (qrplus != 0.) {  // otherwise nothing evaporates: erdt = min(0, ..)
-                const double qvs = pc * exp(17.27 * (pib * th - 273.) / (pib * th - 36.));
-                const double deficit = maxs((1. - qvplus / qvs), 0.);
-                const double coef = 1.6 + 124.9 * pow((1E-3 * rhou * qrplus), 0.2046);
-                const double er = coef * deficit * (pow(1E-3 * rhou * qrplus, 0.525)) /
-                                  ((5.4E5 + 2.55E6 / (1E-2 * pb * qvs)) * 1E-3 * rhou);
-                erdt = mins(qrplus, maxs(0., er * dt));
-            }
-            qr = qr - erdt;
-            qv = qv + erdt;
-            th = th - G.Lv * erdt / (G.Cp * pib);
-            at(S.evap, G, i, k) = erdt;
-        }
-        if constexpr ((PROC & KP_COND) != 0) {  // saturation adjustment
-            const double qvs = pc * exp(17.27 * (pib * th - 273.) / (pib * th - 36.));
-            const double tm = th * pib - 36.;
-            const double phi = qvs * (17.27 * 237. * G.Lv) / (G.Cp * (tm * tm));
-            double C = (qv - qvs) / (1 + phi);
-            if (fabs(C) > qc && C < 0) C = -qc;
-            qv = qv - C;
-            qc = qc + C;
-            th = th + G.Lv / (G.Cp * pib) * C;
-            at(S.cond, G, i, k) = C;
-        }
-        double q3[3] = {qv, qc, qr};
-        if constexpr ((PROC & KP_NEG) != 0) {
-#pragma unroll
-            for (int q = 0; q < 3; q++) {
-                if (q3[q] >= 0.) part[2 * q] += q3[q];
-                else {
-                    part[2 * q + 1] += q3[q];
-                    q3[q] = 0.;
-                }
-            }
-        }
-        constexpr bool wv = (PROC & (KP_EVAP | KP_COND | KP_NEG)) != 0;
-        constexpr bool wc = (PROC & (KP_AUTO | KP_ACCR | KP_COND | KP_NEG)) != 0;
-        constexpr bool wr = (PROC & (KP_AUTO | KP_ACCR | KP_EVAP | KP_NEG)) != 0;
-        constexpr bool wt = (PROC & (KP_EVAP | KP_COND)) != 0;
-        if (wv) at(S.fut[F_QV], G, i, k) = q3[0];
-        if (wc) at(S.fut[F_QC], G, i, k) = q3[1];
-        if (wr) at(S.fut[F_QR], G, i, k) = q3[2];
-        if (wt) at(S.fut[F_TH], G, i, k) = th;
-    }
+    if (i <= G.nx - 2 && k <= G.nz - 2) kessler_point<PROC>(G, S, F, ratios, i, k, part);
     if constexpr ((PROC & KP_NEG) != 0) block_partials<6>(part, rs);
 }
 

@@ -941,7 +941,8 @@ SolveResult Poisson::solve_mixed(double tol, int max_sweeps, hipStream_t st) {
     return refine(direct32, tol, false, max_sweeps, st);
 }
 
-void Poisson::queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, hipStream_t st) {
+void Poisson::queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, const Micro *micro,
+                         hipStream_t st) {
     double *w = S.w;
     const double *rhow_dev = S.P.rhow;
     x_pending = XF_NONE;
@@ -962,7 +963,7 @@ void Poisson::queue_step(const Grid &G, const StepPtrs &S, int step, bool f_read
         direct64.solve(f, nullptr, pcg64.x, st);
         back_to_w(G, w, rhow_dev, st);
     } else {
-        direct64.solve_step(G, S, step, f, pcg64.x, st);
+        direct64.solve_step(G, S, step, micro, f, pcg64.x, st);
     }
     bn_pending = 0;
 }

@@ -104,7 +104,7 @@ class Poisson {
     // (the caller has waited for queue_cal_u's or queue_check's work): if the
     // norms miss the stop rule, corrects x further; *redo says that x and w have changed since queue_step, so cal_u and what
     // was queued behind it have to run again.
-    void queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, hipStream_t st);
+    void queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, const Micro *micro, hipStream_t st);
     void queue_cal_u(const Grid &G, const StepPtrs &S, hipStream_t st);
     void queue_check(hipStream_t st);
     SolveResult finish_step(const Grid &G, double *w, const double *rhow_dev, double tol, bool to_floor,

@@ -14,6 +14,7 @@
 
 #include "poisson.h"
 #include "transfer.h"
+#include "micro.h"
 #include "vvm_internal.h"
 
 using namespace vvmd;
@@ -368,10 +369,12 @@ int solve_w_iter(vvm_dev *h, const StepPtrs &S, vvm_solve_stats *ss, bool run_ne
 // pubarTop_pt (not if step < 0) and cal_w by the direct solver: queued first, so that what follows it can be
 // queued behind it, then finished, which waits for the residual's norms.
 // redo: w has changed since, and what was queued behind it has to run again.
-void queue_w(vvm_dev *h, const StepPtrs &S, int step, bool run_net, bool prepared) {
+// micro (if set; only where neither guess nor samples are asked for): the
+// microphysics rides in the solve's launches.
+void queue_w(vvm_dev *h, const StepPtrs &S, int step, bool run_net, bool prepared, const Micro *micro) {
     const bool first = prepared || run_net || h->pois.sample_cap > 0;
     if (first && !prepared) prepare_guess(h, S, run_net, h->st);
-    h->pois.queue_step(h->G, S, step, first, h->st);
+    h->pois.queue_step(h->G, S, step, first, micro, h->st);
 }
 int finish_w(vvm_dev *h, const StepPtrs &S, vvm_solve_stats *ss, bool *redo) {
     const vvm_dev_config &c = h->cfg;
@@ -475,7 +478,7 @@ int vvm_dev_create(const vvm_dev_config *cfg, int device, vvm_dev_t **out) {
                        &h->P.rate_th, &h->P.rate_z};
     for (double **p : prof) *p = A(G.nz);
     // reduction scratch: enough partials for the largest launch grid
-    const int maxb = ((G.nx + 63) / 64 + 1) * ((G.nz + 3) / 4 + 1);
+    const int maxb = std::max(kMicroBlocks, ((G.nx + 63) / 64 + 1) * ((G.nz + 3) / 4 + 1));
     RedSlot *slots[] = {&h->red.negval, &h->red.solver, &h->red.misc};
     for (RedSlot *rs : slots) {
         rs->max_blocks = maxb;
@@ -798,6 +801,19 @@ bool finish_solve(vvm_dev *h, bool wait) {
     return redo;
 }
 
+// Whether the step's microphysics rides in the solve's launches: up to 640 of
+// thermo4's tiles.  That saves the host two launches and the two streams'
+// events, whose waits alone take it 24 us; above, the solve's LDS leaves too
+// few of these workgroups on a CU.  A step in us, riding against the second
+// stream: 128 x 64 68 / 85, 1024 x 128 84 / 101, 2048 x 128 106 / 111, 2048 x
+// 256 (1024 tiles) 141 / 143, 4096 x 256 261 / 247.  640 is also where the
+// ratios still come from the partial sums, without a k_finalize between.
+bool ride_along(const vvm_dev *h, const Negval &nv, bool run_net) {
+    if (!uses_direct(h->cfg) || h->mp_fn || run_net || h->pois.sample_cap > 0) return false;
+    if (h->kt_kernel == VVM_KT_KESSLER || h->kt_kernel == VVM_KT_SCALE) return false;  // timed alone
+    return nv.nblk <= kFoldBlocks;
+}
+
 // Queues the loop body of TimeMarching up to the diffusion sweep.  The direct
 // solve's residual is read as late as what follows can still be run again:
 // with the tiled sweep, which leaves its inputs alone, that is after the sweep
@@ -818,9 +834,8 @@ int step_begin(vvm_dev *h, int timer, bool last) {
     r.timer = timer;
     r.last = last;
     const StepPtrs &S = r.S;
-    if (h->overlap_c && !h->mp_fn && !h->side)
-        HIPCHK(h, hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking));
     const bool overlap = h->overlap_c && !h->mp_fn;
+    if (overlap && !h->side) HIPCHK(h, hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking));
     // the learned guess's network is the longest serial chain before the
     // solve; it needs only pzeta's zetap and the past solutions
     const bool run_net = net_due(h);
@@ -854,17 +869,20 @@ int step_begin(vvm_dev *h, int timer, bool last) {
     }
     mark(h, 1, h->st);
     // C: Kessler (with the scalars' negative-value rescale and forcing) and its
-    // NegativeValueProcess x3 + halos (:303-311, 404), on the side stream while
-    // B runs; the main stream waits for it before D (with host microphysics, C
-    // runs after B on the host instead).  Its partial sums go to another slot
-    // than thermo4's, which it may still be reading.
-    hipStream_t cs = overlap ? h->side : h->st;
-    if (overlap) {
+    // NegativeValueProcess x3 + halos (:303-311, 404): as further workgroups of
+    // the solve's launches (ride), or on the side stream while B runs; the main
+    // stream waits for it before D (with host microphysics, C runs after B on
+    // the host instead).  Its partial sums go to another slot than thermo4's,
+    // which it may still be reading.
+    const bool ride = ride_along(h, nv, run_net);
+    const bool aside = overlap && !ride;
+    hipStream_t cs = aside ? h->side : h->st;
+    if (aside) {
         hipEventRecord(h->ev_fork, h->st);
         hipStreamWaitEvent(h->side, h->ev_fork, 0);
     }
-    if (!h->mp_fn) {
-        mark(h, 6, cs);
+    if (!h->mp_fn) mark(h, 6, cs);
+    if (!h->mp_fn && !ride) {
         {
             KTimer t(h, VVM_KT_KESSLER, cs);
             nv = launch_kessler(G, S, negval_partials(S, nv, cs), F, h->red.misc, cs);
@@ -875,15 +893,17 @@ int step_begin(vvm_dev *h, int timer, bool last) {
         }
         mark(h, 7, cs);
     }
-    if (overlap) hipEventRecord(h->ev_join, h->side);
+    if (aside) hipEventRecord(h->ev_join, h->side);
     // B: pubarTop_pt, cal_w, cal_u (:292-296)
     if (!direct) launch_pubartop(G, S, h->step, h->st);
     {
         KTimer t(h, VVM_KT_SOLVE);
         if (early_guess) hipStreamWaitEvent(h->st, h->ev_guess, 0);
-        if (direct) queue_w(h, S, h->step, run_net, early_guess);
+        const Micro micro{nv, F, h->red.misc};
+        if (direct) queue_w(h, S, h->step, run_net, early_guess, ride ? &micro : nullptr);
         else r.rc = solve_w_iter(h, S, &r.ss, run_net, early_guess);
     }
+    if (ride) mark(h, 7, h->st);  // the launches it shared
     {
         KTimer t(h, VVM_KT_CALU);
         if (direct) h->pois.queue_cal_u(G, S, h->st);
@@ -893,7 +913,7 @@ int step_begin(vvm_dev *h, int timer, bool last) {
     r.solved = !direct;
     if (h->mp_fn || r.halo == 0) finish_solve(h, true);
     mark(h, 2, h->st);
-    if (overlap) hipStreamWaitEvent(h->st, h->ev_join, 0);
+    if (aside) hipStreamWaitEvent(h->st, h->ev_join, 0);
     if (h->mp_fn) {
         mark(h, 6, h->st);
         const int mrc = host_microphysics(h, S);
@@ -1039,7 +1059,7 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             h->cfg.guess_mode = VVM_GUESS_ZERO;
             if (uses_direct(h->cfg)) {
                 bool redo = false;
-                queue_w(h, S, -1, false, false);
+                queue_w(h, S, -1, false, false, nullptr);
                 h->pois.queue_check(h->st);
                 HIPCHK(h, hipStreamSynchronize(h->st));
                 rc = finish_w(h, S, nullptr, &redo);

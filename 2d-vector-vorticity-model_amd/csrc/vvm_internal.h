@@ -75,6 +75,7 @@ void launch_pzeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st);
 // rs; what they return goes through negval_partials, on the second pass's
 // stream, to that pass: launch_scale_forcing, or the launch_kessler behind
 // launch_thermo4.
+constexpr int kFoldBlocks = 640;  // up to which the second pass adds the partials itself
 struct Negval {
     RedSlot rs;
     int nblk;

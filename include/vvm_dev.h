@@ -130,6 +130,8 @@ typedef struct vvm_step_stats {
     int32_t not_converged;     /* solves that hit max_iter                   */
     double rel_residual_last;  /* ||b-Ax||/||b|| of the last solve          */
     double t_advection, t_poisson, t_microphysics, t_diffusion, t_all; /* s */
+    /* t_microphysics is the time on the second stream or, where the microphysics
+     * shares the solve's launches (up to 640 tiles of 64 x 8 points), theirs */
     int32_t guess_fallbacks;   /* solves whose learned guess started worse
                                   than the extrapolation (or not finite) and
                                   were dropped                             */
