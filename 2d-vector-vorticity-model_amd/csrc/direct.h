@@ -5,7 +5,7 @@
 // system along z for each of the N frequencies: diagonal
 // cx_j lambda_q + cu_j + cu_{j-1}, lambda_q = 4 sin^2(pi q / N), off-diagonal
 // -cu_j.  Any N and M: the transform is a mixed-radix FFT (8, 4, 2, 3, 5, and
-// a direct sum for any other prime factor).
+// direct sums for small other prime factors); with large ones a convolution.
 #pragma once
 
 #include "vvm_internal.h"
@@ -16,11 +16,13 @@ struct Micro;
 
 constexpr int kMaxStages = 16;
 
-// The factors of N and the launch shape of the row transforms.
+// The factors of L and the launch shape of the row transforms.
 struct RowPlan {
     int N = 0, M = 0;
+    int L = 0;            // the FFT's length: N, or the convolution's (chirp)
+    int chirp = 0;        // large prime factors: the transform as a convolution
     int nst = 0, radix[kMaxStages] = {};
-    int threads = 0;      // at least N / 8: a thread holds at most 8 outputs of a stage
+    int threads = 0;      // at least L / 8: a thread holds at most 8 outputs of a stage
     // in LDS: nothing, the table of all roots (a prime factor above 5 reads it),
     // or the stages' twiddles; nothing where that would pass the LDS size
     enum { TW_GLOBAL, TW_ROOTS, TW_STAGES };
@@ -49,10 +51,16 @@ class Direct {
    private:
     RowPlan plan;
     size_t row_lds = 0, col_lds = 0;
-    T *tw = nullptr;    // [N][2]: cos, -sin of 2 pi k / N; then the stages' twiddles, [N-1][2]
+    T *tw = nullptr;    // [L][2]: cos, -sin of 2 pi k / L; then the stages' twiddles, [L-1][2]
+    T *chirp = nullptr; // [N][2] the chirp, [L][2] the transform of its inverse, over L
     T *di = nullptr;    // [M][N/2+1] 1 / pivot
     const double *cu_dev = nullptr;
     T *spec = nullptr;  // [M][N] transformed rows
+    template <bool C>
+    void rows_solve(const double *r, const double *x0, double *x, hipStream_t st);
+    template <bool C>
+    void rows_solve_step(const Grid &G, const StepPtrs &S, int step, const Micro *micro, double *f, double *x,
+                         hipStream_t st);
     template <typename Mic>
     void columns(const Mic &mic, int nmic, hipStream_t st);
 };

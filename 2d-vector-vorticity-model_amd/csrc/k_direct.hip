@@ -7,6 +7,7 @@
 // kernel), four LDS round trips of 1 us, the elimination's serial chain.
 #include <algorithm>
 #include <cmath>
+#include <complex>
 #include <type_traits>
 #include <vector>
 
@@ -230,16 +231,16 @@ struct Twiddles {
     Cx<T> v[8];
     __device__ inline void load(const RowPlan &P, const T *__restrict__ tw) {
         if (P.tw == RowPlan::TW_GLOBAL) return;
-        const Cx<T> *src = reinterpret_cast<const Cx<T> *>(tw) + (P.tw == RowPlan::TW_STAGES ? P.N : 0);
+        const Cx<T> *src = reinterpret_cast<const Cx<T> *>(tw) + (P.tw == RowPlan::TW_STAGES ? P.L : 0);
 #pragma unroll
-        for (int t = 0; t < 8; t++) v[t] = src[min(int(threadIdx.x + t * blockDim.x), P.N - 1)];
+        for (int t = 0; t < 8; t++) v[t] = src[min(int(threadIdx.x + t * blockDim.x), P.L - 1)];
     }
     __device__ inline void store(const RowPlan &P, T *twl) const {
         if (P.tw == RowPlan::TW_GLOBAL) return;
 #pragma unroll
         for (int t = 0; t < 8; t++) {
             const int i = threadIdx.x + t * blockDim.x;
-            if (i < P.N) {
+            if (i < P.L) {
                 twl[2 * i] = v[t].x;
                 twl[2 * i + 1] = v[t].y;
             }
@@ -247,32 +248,89 @@ struct Twiddles {
     }
 };
 
-template <bool LDS, typename T>
+template <bool LDS, bool ANY, typename T>
 __device__ inline void fft_stages(const RowPlan &P, T *re, T *im, const T *tw, const T *twl) {
-    const int N = P.N;
+    const int L = P.L;
     int Ns = 1;
     for (int s = 0; s < P.nst; s++) {
         const int R = P.radix[s];
-        // the stages' tables follow the table of all N roots; those before
+        // the stages' tables follow the table of all L roots; those before
         // hold sum (R - 1) Ns = Ns - 1 values
-        const T *ts = LDS ? twl + 2 * (Ns - 1) : tw + 2 * (N + Ns - 1);
+        const T *ts = LDS ? twl + 2 * (Ns - 1) : tw + 2 * (L + Ns - 1);
         switch (R) {
-            case 8: stage<8>(re, im, N, Ns, ts); break;
-            case 4: stage<4>(re, im, N, Ns, ts); break;
-            case 2: stage<2>(re, im, N, Ns, ts); break;
-            case 3: stage<3>(re, im, N, Ns, ts); break;
-            case 5: stage<5>(re, im, N, Ns, ts); break;
+            case 8: stage<8>(re, im, L, Ns, ts); break;
+            case 4: stage<4>(re, im, L, Ns, ts); break;
+            case 2: stage<2>(re, im, L, Ns, ts); break;
+            case 3: if constexpr (ANY) stage<3>(re, im, L, Ns, ts); break;
+            case 5: if constexpr (ANY) stage<5>(re, im, L, Ns, ts); break;
             default:
-                if constexpr (!LDS) stage_any(re, im, N, Ns, R, P.tw == RowPlan::TW_ROOTS ? twl : tw);
+                if constexpr (ANY && !LDS) stage_any(re, im, L, Ns, R, P.tw == RowPlan::TW_ROOTS ? twl : tw);
         }
         Ns *= R;
     }
 }
-template <typename T>
-__device__ inline void fft(const RowPlan &P, T *re, T *im, const T *__restrict__ tw, const T *twl) {
+
+// The transform of the N values in re, im (after a barrier).
+//
+// CHIRP, for large prime factors: n k = (n^2 + k^2 - (k - n)^2) / 2 makes it a
+// convolution with a chirp (Bluestein's algorithm), by two transforms of length
+// L = 2^j >= 2 N - 1.  The values come multiplied by the chirp c_n = exp(-i pi
+// n^2 / N) and padded with zeros; bhat is the transform of 1 / c over L.  The
+// inverse transform is the forward one with real and imaginary parts swapped.
+// 317 columns: an isolated solve 75 us, 383 with the direct sums of 317 terms.
+template <bool CHIRP, typename T>
+__device__ inline void fft(const RowPlan &P, T *re, T *im, const T *__restrict__ tw, const T *twl,
+                           const T *__restrict__ chirp) {
     __syncthreads();
-    if (P.tw == RowPlan::TW_STAGES) fft_stages<true>(P, re, im, tw, twl);
-    else fft_stages<false>(P, re, im, tw, twl);
+    if constexpr (!CHIRP) {
+        if (P.tw == RowPlan::TW_STAGES) fft_stages<true, true>(P, re, im, tw, twl);
+        else fft_stages<false, true>(P, re, im, tw, twl);
+    } else {
+        auto times = [&](const T *by, int n) {
+            const Cx<T> *c = reinterpret_cast<const Cx<T> *>(by);
+            Cx<T> v[8];
+#pragma unroll
+            for (int t = 0; t < 8; t++) v[t] = c[min(int(threadIdx.x + t * blockDim.x), n - 1)];
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                const int i = threadIdx.x + t * blockDim.x;
+                if (i < n) {
+                    const Cx<T> z = mul(Cx<T>{re[pad(i)], im[pad(i)]}, v[t]);
+                    re[pad(i)] = z.x;
+                    im[pad(i)] = z.y;
+                }
+            }
+            __syncthreads();
+        };
+        for (int pass = 0; pass < 2; pass++) {
+            T *a = pass ? im : re, *b = pass ? re : im;
+            if (P.tw == RowPlan::TW_STAGES) fft_stages<true, false>(P, a, b, tw, twl);
+            else fft_stages<false, false>(P, a, b, tw, twl);
+            if (pass == 0) times(chirp + 2 * P.N, P.L);
+            else times(chirp, P.N);
+        }
+    }
+}
+// The rows' values to LDS, past the last column zeros.
+template <bool CHIRP, typename T, typename V>
+__device__ inline void fill_rows(const RowPlan &P, T *re, T *im, const V (&va)[8], const V (&vb)[8], bool two,
+                                 const T *__restrict__ chirp) {
+    const Cx<T> *c = reinterpret_cast<const Cx<T> *>(chirp);
+    Cx<T> cv[8];
+    if constexpr (CHIRP) {
+#pragma unroll
+        for (int t = 0; t < 8; t++) cv[t] = c[min(int(threadIdx.x + t * blockDim.x), P.N - 1)];
+    }
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const int i = threadIdx.x + t * blockDim.x;
+        Cx<T> z{T(va[t]), two ? T(vb[t]) : T(0)};
+        if constexpr (CHIRP) z = i < P.N ? mul(z, cv[t]) : Cx<T>{T(0), T(0)};
+        if (i < (CHIRP ? P.L : P.N)) {
+            re[pad(i)] = z.x;
+            im[pad(i)] = z.y;
+        }
+    }
 }
 
 // Hartley values (Re - Im) of the two rows at frequency q, times 2 h, from the complex
@@ -293,8 +351,9 @@ __device__ inline void hartley_pair(const T *re, const T *im, int N, int q, T h,
 // With RHS the workgroups behind the rows' do what else has to follow the
 // advection: with a step one pubarTop_pt, which reads u, w and K as the solve
 // finds them (alone it was a launch of 5 to 8 us), and m.nblk Kessler.
-template <typename T, bool RHS>
-__global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restrict__ tw, const double *__restrict__ r,
+template <typename T, bool RHS, bool CHIRP>
+__global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restrict__ tw, const T *__restrict__ chirp,
+                                                   const double *__restrict__ r,
                                                    T *__restrict__ spec, Grid G, StepPtrs S, int step,
                                                    double *__restrict__ f, Micro m) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -307,7 +366,7 @@ __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restric
         }
     }
     const double *zetap = S.fut[F_ZETA], *rhow = S.P.rhow;
-    const int N = P.N, M = P.M, LN = pad(N - 1) + 1;
+    const int N = P.N, M = P.M, LN = pad(P.L - 1) + 1;
     T *re = reinterpret_cast<T *>(lds_raw), *im = re + LN, *twl = im + LN;
     const int j = 1 + 2 * blockIdx.x;
     const bool two = j + 1 <= M;
@@ -334,23 +393,20 @@ __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restric
         const double b = rw * rw * d * G.dx;
         return -b / rw;
     };
+    if constexpr (RHS) {
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-        const int i = threadIdx.x + t * blockDim.x;
-        if constexpr (RHS) {
+        for (int t = 0; t < 8; t++) {
+            const int i = threadIdx.x + t * blockDim.x;
             va[t] = rhs(va[t], rhow[j + 1]);
             vb[t] = rhs(vb[t], rhow[j1 + 1]);
-        }
-        if (i < N) {
-            if constexpr (RHS) {
+            if (i < N) {
                 f[size_t(j) * N + i] = va[t];
                 if (two) f[size_t(j + 1) * N + i] = vb[t];
             }
-            re[pad(i)] = T(va[t]);
-            im[pad(i)] = two ? T(vb[t]) : T(0);
         }
     }
-    fft(P, re, im, tw, twl);
+    fill_rows<CHIRP>(P, re, im, va, vb, two, chirp);
+    fft<CHIRP>(P, re, im, tw, twl, chirp);
     const T h = T(0.5 / N);
 #pragma unroll
     for (int t = 0; t < 8; t++) {
@@ -367,12 +423,12 @@ __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restric
 // Inverse: x = the transform of rows j, j+1 of spec (ADD: x0 + it); with w also
 // w[i][k] = x / rhow[k] and BoundaryProcess2D_westdown(w)
 // (src/PoissonSolver.cpp:469-476).
-template <typename T, bool ADD, bool W>
-__global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restrict__ tw, const T *__restrict__ spec,
-                                                   const double *x0, double *x, Grid G, double *__restrict__ w,
+template <typename T, bool ADD, bool W, bool CHIRP>
+__global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restrict__ tw, const T *__restrict__ chirp,
+                                                   const T *__restrict__ spec, const double *x0, double *x, Grid G, double *__restrict__ w,
                                                    const double *__restrict__ rhow) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    const int N = P.N, M = P.M, LN = pad(N - 1) + 1;
+    const int N = P.N, M = P.M, LN = pad(P.L - 1) + 1;
     T *re = reinterpret_cast<T *>(lds_raw), *im = re + LN, *twl = im + LN;
     const int j = 1 + 2 * blockIdx.x;
     const bool two = j + 1 <= M;
@@ -387,21 +443,14 @@ __global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restric
         vb[t] = spec[size_t(j1 - 1) * N + i];
     }
     Tw.store(P, twl);
-#pragma unroll
-    for (int t = 0; t < 8; t++) {
-        const int i = threadIdx.x + t * blockDim.x;
-        if (i < N) {
-            re[pad(i)] = va[t];
-            im[pad(i)] = two ? vb[t] : T(0);
-        }
-    }
+    fill_rows<CHIRP>(P, re, im, va, vb, two, chirp);
     if constexpr (W) {  // the zero rows of w
         for (int i = threadIdx.x; i < G.nx; i += blockDim.x) {
             if (blockIdx.x == 0) w[ix(G, i, 0)] = w[ix(G, i, 1)] = 0.;
             if (blockIdx.x == gridDim.x - 1) w[ix(G, i, G.nz - 1)] = 0.;
         }
     }
-    fft(P, re, im, tw, twl);
+    fft<CHIRP>(P, re, im, tw, twl, chirp);
     double xa[8], xb[8];
     if constexpr (ADD) {
 #pragma unroll
@@ -650,66 +699,131 @@ bool allow_lds(K kernel, size_t bytes) {
                                                      int(bytes)) == hipSuccess;
 }
 
+// exp(-2 pi i k / n)
+inline std::complex<long double> root(long long k, long long n) {
+    const long double a = 2.0L * 3.14159265358979323846264338327950288L * (k % n) / n;
+    return {std::cos(a), -std::sin(a)};
+}
+// in place, forward, n a power of two
+void host_fft(std::vector<std::complex<long double>> &v) {
+    const size_t n = v.size();
+    for (size_t i = 1, j = 0; i < n; i++) {
+        size_t bit = n >> 1;
+        for (; j & bit; bit >>= 1) j ^= bit;
+        j ^= bit;
+        if (i < j) std::swap(v[i], v[j]);
+    }
+    std::vector<std::complex<long double>> w(n / 2 + 1);
+    for (size_t k = 0; k < w.size(); k++) w[k] = root((long long)k, (long long)n);
+    for (size_t len = 2; len <= n; len *= 2)
+        for (size_t i = 0; i < n; i += len)
+            for (size_t k = 0; k < len / 2; k++) {
+                const auto a = v[i + k], b = v[i + k + len / 2] * w[k * (n / len)];
+                v[i + k] = a + b;
+                v[i + k + len / 2] = a - b;
+            }
+}
+
+// Up to this sum of the prime factors above 5 the direct sums are used, where
+// they cost no more than the chirp's second transform and longer rows.  A whole
+// isolated solve with 64 rows in us, sums / chirp: 28 columns (sum 7) 72 / 69,
+// 176 (11) 75 / 70, 208 (13) 76 / 68, 437 (42) 106 / 75; 1100 (11) 81 / 87, 1472
+// (23) 90 / 86, 1184 (37) 103 / 87, 2128 (26) 106 / 113, 3712 (29) 115 / 116, 3059
+// (49) 138 / 115; and the primes 317 383 / 75, 1021 1141 / 78, 4093 5316 / 116.
+inline int max_sums(int N) { return N <= 1024 ? 10 : 28; }
+
 }  // namespace
 
 template <typename T>
 int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
     plan = RowPlan();
-    plan.N = N;
+    plan.N = plan.L = N;
     plan.M = M;
     int n = N;
-    for (int r : {8, 4, 2, 3, 5})
+    auto take = [&](int r) {
         while (n % r == 0 && plan.nst < kMaxStages) {
             plan.radix[plan.nst++] = r;
             n /= r;
         }
-    bool other = false;
+    };
+    for (int r : {8, 4, 2, 3, 5}) take(r);
+    const int small = plan.nst;
+    int sums = 0;
     for (int r = 7; n > 1 && plan.nst < kMaxStages; r += 2) {
         if (r * r > n) r = n;
-        while (n % r == 0 && plan.nst < kMaxStages) {
-            plan.radix[plan.nst++] = r;
-            n /= r;
-            other = true;
-        }
+        take(r);
     }
+    for (int s = small; s < plan.nst; s++) sums += plan.radix[s];
     if (n != 1 || N > 8192) return VVM_ERR_SIZE;
-    plan.threads = std::min(1024, std::max(64, ((N + 7) / 8 + 63) / 64 * 64));
-    const size_t LN = size_t(N - 1) + size_t((N - 1) >> 5) + 1;
+    if (sums > max_sums(N) && 2 * N - 1 <= 8192) {
+        plan.chirp = 1;
+        plan.L = 1;
+        while (plan.L < 2 * N - 1) plan.L *= 2;
+        plan.nst = 0;
+        n = plan.L;
+        for (int r : {8, 4, 2}) take(r);
+    }
+    const int L = plan.L;
+    plan.threads = std::min(1024, std::max(64, ((L + 7) / 8 + 63) / 64 * 64));
+    const size_t LN = size_t(L - 1) + size_t((L - 1) >> 5) + 1;
     row_lds = 2 * LN * sizeof(T);
-    if (row_lds + 2 * size_t(N) * sizeof(T) <= kLdsMax - kLdsStatic) {
-        plan.tw = other ? RowPlan::TW_ROOTS : RowPlan::TW_STAGES;
-        row_lds += 2 * size_t(N) * sizeof(T);
+    if (row_lds + 2 * size_t(L) * sizeof(T) <= kLdsMax - kLdsStatic) {
+        plan.tw = sums && !plan.chirp ? RowPlan::TW_ROOTS : RowPlan::TW_STAGES;
+        row_lds += 2 * size_t(L) * sizeof(T);
     }
     col_lds = col_lds_bytes<T>(M);
     if (row_lds > kLdsMax || col_lds > kLdsMax) return VVM_ERR_SIZE;
-    if (!allow_lds(k_rows_fwd<T, false>, row_lds) || !allow_lds(k_rows_fwd<T, true>, row_lds) ||
-        !allow_lds(k_rows_inv<T, false, false>, row_lds) || !allow_lds(k_rows_inv<T, true, false>, row_lds) ||
-        !allow_lds(k_rows_inv<T, false, true>, row_lds) || !allow_lds(k_columns<T, NoMicro>, col_lds) ||
-        !allow_lds(k_columns<T, MicroPass>, col_lds))
-        return VVM_ERR_HIP;
+    bool ok = allow_lds(k_columns<T, NoMicro>, col_lds) && allow_lds(k_columns<T, MicroPass>, col_lds);
+    auto allow_rows = [&](auto chirp) {
+        constexpr bool C = decltype(chirp)::value;
+        ok = ok && allow_lds(k_rows_fwd<T, false, C>, row_lds) && allow_lds(k_rows_fwd<T, true, C>, row_lds) &&
+             allow_lds(k_rows_inv<T, false, false, C>, row_lds) && allow_lds(k_rows_inv<T, true, false, C>, row_lds) &&
+             allow_lds(k_rows_inv<T, false, true, C>, row_lds);
+    };
+    if (plan.chirp) allow_rows(std::true_type());
+    else allow_rows(std::false_type());
+    if (!ok) return VVM_ERR_HIP;
     const size_t Nq = size_t(N) / 2 + 1;
-    tw = dalloc<T>(4 * size_t(N));
+    tw = dalloc<T>(4 * size_t(L));
+    if (plan.chirp) chirp = dalloc<T>(2 * size_t(N + L));
     di = dalloc<T>(Nq * M);
     spec = dalloc<T>(size_t(N) * M);
-    if (!tw || !di || !spec) {
+    if (!tw || !di || !spec || (plan.chirp && !chirp)) {
         destroy();
         return VVM_ERR_NOMEM;
     }
-    std::vector<T> t(4 * size_t(N), T(0));
-    for (int k = 0; k < N; k++) {
-        const long double a = 2.0L * 3.14159265358979323846264338327950288L * k / N;
-        t[2 * k] = T(std::cos(a));
-        t[2 * k + 1] = T(-std::sin(a));
+    std::vector<T> t(4 * size_t(L), T(0));
+    for (int k = 0; k < L; k++) {
+        const auto c = root(k, L);
+        t[2 * k] = T(c.real());
+        t[2 * k + 1] = T(c.imag());
     }
-    // the stages' twiddles, picked from those (r k < Ns R, so r k N / (Ns R) < N)
+    // the stages' twiddles, picked from those (r k < Ns R, so r k L / (Ns R) < L)
     for (int s = 0, Ns = 1; s < plan.nst; Ns *= plan.radix[s++]) {
-        const int R = plan.radix[s], m = N / (Ns * R);
+        const int R = plan.radix[s], m = L / (Ns * R);
         for (int r = 1; r < R; r++)
             for (int k = 0; k < Ns; k++) {
-                const size_t a = 2 * (size_t(N) + Ns - 1 + size_t(r - 1) * Ns + k), b = 2 * size_t(r) * k * m;
+                const size_t a = 2 * (size_t(L) + Ns - 1 + size_t(r - 1) * Ns + k), b = 2 * size_t(r) * k * m;
                 t[a] = t[b];
                 t[a + 1] = t[b + 1];
             }
+    }
+    if (plan.chirp) {
+        std::vector<T> ch(2 * size_t(N + L));
+        std::vector<std::complex<long double>> b(L, 0.0L);
+        for (long long k = 0; k < N; k++) {
+            const auto c = root(k * k, 2LL * N);
+            ch[2 * k] = T(c.real());
+            ch[2 * k + 1] = T(c.imag());
+            b[k] = b[(L - k) % L] = std::conj(c);
+        }
+        host_fft(b);
+        for (int k = 0; k < L; k++) {
+            ch[2 * size_t(N + k)] = T(b[k].real() / L);
+            ch[2 * size_t(N + k) + 1] = T(b[k].imag() / L);
+        }
+        if (hipMemcpy(chirp, ch.data(), ch.size() * sizeof(T), hipMemcpyHostToDevice) != hipSuccess)
+            return VVM_ERR_HIP;
     }
     if (hipMemcpy(tw, t.data(), t.size() * sizeof(T), hipMemcpyHostToDevice) != hipSuccess) return VVM_ERR_HIP;
     hipLaunchKernelGGL(k_factor<T>, dim3(unsigned((Nq + 63) / 64)), dim3(64), 0, nullptr, N, M, cx, cu, di);
@@ -719,9 +833,9 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
 
 template <typename T>
 void Direct<T>::destroy() {
-    for (T *p : {tw, di, spec})
+    for (T *p : {tw, chirp, di, spec})
         if (p) (void)hipFree(p);
-    tw = di = spec = nullptr;
+    tw = chirp = di = spec = nullptr;
 }
 
 template <typename T>
@@ -732,38 +846,51 @@ void Direct<T>::columns(const Mic &mic, int nmic, hipStream_t st) {
 }
 
 template <typename T>
-void Direct<T>::solve(const double *r, const double *x0, double *x, hipStream_t st) {
+template <bool C>
+void Direct<T>::rows_solve(const double *r, const double *x0, double *x, hipStream_t st) {
     const dim3 gr((plan.M + 1) / 2), b(plan.threads);
-    hipLaunchKernelGGL((k_rows_fwd<T, false>), gr, b, row_lds, st, plan, tw, r, spec, Grid{}, StepPtrs{}, 0, nullptr,
-                       Micro{});
+    hipLaunchKernelGGL((k_rows_fwd<T, false, C>), gr, b, row_lds, st, plan, tw, chirp, r, spec, Grid{}, StepPtrs{}, 0,
+                       nullptr, Micro{});
     columns(NoMicro{}, 0, st);
     if (x0)
-        hipLaunchKernelGGL((k_rows_inv<T, true, false>), gr, b, row_lds, st, plan, tw, spec, x0, x, Grid{}, nullptr,
-                           nullptr);
+        hipLaunchKernelGGL((k_rows_inv<T, true, false, C>), gr, b, row_lds, st, plan, tw, chirp, spec, x0, x, Grid{},
+                           nullptr, nullptr);
     else
-        hipLaunchKernelGGL((k_rows_inv<T, false, false>), gr, b, row_lds, st, plan, tw, spec, x0, x, Grid{}, nullptr,
-                           nullptr);
+        hipLaunchKernelGGL((k_rows_inv<T, false, false, C>), gr, b, row_lds, st, plan, tw, chirp, spec, x0, x, Grid{},
+                           nullptr, nullptr);
+}
+template <typename T>
+void Direct<T>::solve(const double *r, const double *x0, double *x, hipStream_t st) {
+    if (plan.chirp) rows_solve<true>(r, x0, x, st);
+    else rows_solve<false>(r, x0, x, st);
 }
 
 template <typename T>
-void Direct<T>::solve_step(const Grid &G, const StepPtrs &S, int step, const Micro *micro, double *f, double *x,
-                           hipStream_t st) {
+template <bool C>
+void Direct<T>::rows_solve_step(const Grid &G, const StepPtrs &S, int step, const Micro *micro, double *f, double *x,
+                                hipStream_t st) {
     const dim3 gr((plan.M + 1) / 2), b(plan.threads);
     Micro m;
     if (micro) {
         m = *micro;
         m.nblk = std::min(kMicroBlocks, micro_tiles(G, plan.threads));
     }
-    hipLaunchKernelGGL((k_rows_fwd<T, true>), dim3(gr.x + (step >= 0 ? 1 : 0) + m.nblk), b, row_lds, st, plan, tw,
-                       nullptr, spec, G, S, step, f, m);
+    hipLaunchKernelGGL((k_rows_fwd<T, true, C>), dim3(gr.x + (step >= 0 ? 1 : 0) + m.nblk), b, row_lds, st, plan, tw,
+                       chirp, nullptr, spec, G, S, step, f, m);
     if (micro) {
         const int n = std::min(kMicroBlocks, micro_tiles(G, 256));
         columns(MicroPass{G, S, Negval{m.rs, m.nblk}, n}, n, st);
     } else {
         columns(NoMicro{}, 0, st);
     }
-    hipLaunchKernelGGL((k_rows_inv<T, false, true>), gr, b, row_lds, st, plan, tw, spec, nullptr, x, G, S.w,
+    hipLaunchKernelGGL((k_rows_inv<T, false, true, C>), gr, b, row_lds, st, plan, tw, chirp, spec, nullptr, x, G, S.w,
                        S.P.rhow);
+}
+template <typename T>
+void Direct<T>::solve_step(const Grid &G, const StepPtrs &S, int step, const Micro *micro, double *f, double *x,
+                           hipStream_t st) {
+    if (plan.chirp) rows_solve_step<true>(G, S, step, micro, f, x, st);
+    else rows_solve_step<false>(G, S, step, micro, f, x, st);
 }
 
 template class Direct<double>;
