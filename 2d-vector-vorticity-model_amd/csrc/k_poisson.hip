@@ -250,6 +250,55 @@ __device__ inline void residual_norms(const Residual &R, int block, int nblk) {
     }
 }
 
+// r = f - L x and the norms, before a correction.  FIRST: the right-hand side
+// and the guess in the reference's order (bref, xref), f and x formed on the
+// way: four passes in one.
+template <bool FIRST>
+__global__ void __launch_bounds__(1024) k_solve_residual(Residual R, const double *__restrict__ bref,
+                                                         const double *__restrict__ xref, double *__restrict__ f,
+                                                         double *__restrict__ x, double *__restrict__ r) {
+    constexpr int RX = 64, RY = 16;
+    const int N = R.N, M = R.M, tx = (N + RX - 1) / RX, nt = tx * ((M + RY - 1) / RY);
+    double part[2] = {0., 0.};
+#pragma unroll 2
+    for (int t = blockIdx.x; t < nt; t += gridDim.x) {
+        const int i = (t % tx) * RX + threadIdx.x % RX, j = 1 + (t / tx) * RY + uniform(threadIdx.x / RX);
+        if (j > M) continue;
+        const int ic = min(i, N - 1), im = ic == 0 ? N - 1 : ic - 1, ip = ic == N - 1 ? 0 : ic + 1;
+        const size_t c = size_t(j) * N + ic;
+        double xc, xw, xe, xu, xd, fv, wb;
+        if constexpr (FIRST) {
+            const double *row = xref + size_t(j - 1) * N;  // rows 0 and M + 1 are zero
+            xc = row[ic], xw = row[im], xe = row[ip];
+            xu = j < M ? row[N + ic] : 0.;
+            xd = j > 1 ? row[ic - N] : 0.;
+            wb = bref[size_t(j - 1) * N + ic];
+            fv = -wb / R.wD[j];
+        } else {
+            const double *row = R.x + size_t(j) * N;
+            xc = row[ic], xw = row[im], xe = row[ip], xu = row[N + ic], xd = row[ic - N];
+            fv = R.f[c];
+            wb = R.wD[j] * fv;
+        }
+        const double rv = fv - (R.cx[j] * (2. * xc - xw - xe) + R.cu[j] * (xc - xu) + R.cu[j - 1] * (xc - xd));
+        const double wr = R.wD[j] * rv;
+        if (i < N) {
+            r[c] = rv;
+            if constexpr (FIRST) {
+                f[c] = fv;
+                x[c] = xc;
+            }
+            part[0] += wr * wr;
+            part[1] += wb * wb;
+        }
+    }
+    block_sum<2>(part);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(R.hres + 2 * blockIdx.x, part[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(R.hres + 2 * blockIdx.x + 1, part[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // cal_u.  Top row: h (mean removed), the periodic 1-D problem G y = h solved
 // in closed form through its first differences D_r = y_r - y_{r-1}:
 // D_{r+1} - D_r = h_r and sum_r D_r = 0, so D_r = S_r - mean(S) with S the
@@ -673,7 +722,7 @@ int Poisson::init(const Grid &G, const double *rhou, const double *rhow, const R
                       hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
         return VVM_ERR_NOMEM;
     if (hipHostGetDevicePointer(reinterpret_cast<void **>(&hscal_dev), hscal, 0) != hipSuccess) return VVM_ERR_HIP;
-    if (hipHostMalloc(reinterpret_cast<void **>(&hres), 2 * kResidualBlocks * sizeof(double),
+    if (hipHostMalloc(reinterpret_cast<void **>(&hres), 4 * kResidualBlocks * sizeof(double),
                       hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
         return VVM_ERR_NOMEM;
     if (hipHostGetDevicePointer(reinterpret_cast<void **>(&hres_dev), hres, 0) != hipSuccess) return VVM_ERR_HIP;
@@ -899,46 +948,88 @@ SolveResult Poisson::solve_fp64(double tol, int max_iter, hipStream_t st) {
 // sides; the bound is the condition number's worth above that.
 constexpr double kRoundOff = 1e-12;
 
-// Each sweep: the FP64 residual, then x += L^-1 r by a direct solve, formed in
-// another buffer so that the first one can be queued before the host has read
-// the residual of the guess (which may already meet the stop rule).
-template <typename T>
-SolveResult Poisson::refine(Direct<T> &D, double tol, bool to_floor, int max_sweeps, hipStream_t st) {
-    SolveResult R;
-    double prev = -1.;
-    for (int sweep = 0;; sweep++) {
-        first_residual(pcg64.r, st);
-        hipEventRecord(ev_res, st);
-        if (sweep == 0) D.solve(pcg64.r, pcg64.x, x64B, st);
-        hipEventSynchronize(ev_res);
-        const double bn2 = hscal[P_BNORM2], rn2 = hscal[P_RNORM2];
-        const bool finite = std::isfinite(bn2) && std::isfinite(rn2);  // else: a bad right-hand side or guess
-        if (finite && bn2 == 0.) {
-            hipMemsetAsync(pcg64.x, 0, size_t(M + 2) * N * sizeof(double), st);
-            R.converged = true;
-            return R;
-        }
-        R.rel = std::sqrt(rn2 / bn2);
-        if (sweep == 0) R.rel0 = R.rel;
-        R.iters = R.refine = sweep;
-        if (!finite) return R;
-        const bool stalled = prev >= 0. && R.rel > 0.5 * prev;
-        R.converged = R.rel <= tol || (to_floor && stalled && R.rel <= kRoundOff);
-        if (R.converged || stalled || sweep == max_sweeps) return R;
-        prev = R.rel;
-        if (sweep > 0) D.solve(pcg64.r, pcg64.x, x64B, st);
-        std::swap(pcg64.x, x64B);
+// Norms of the residual kernel's slot (the caller has waited for it).
+void Poisson::norms(int slot, double *rn2, double *bn2) const {
+    const volatile double *p = hres + slot * 2 * kResidualBlocks;
+    *rn2 = *bn2 = 0.;
+    for (int b = 0; b < res_blocks; b++) {  // fixed order: deterministic
+        *rn2 += p[2 * b];
+        *bn2 += p[2 * b + 1];
     }
 }
 
-SolveResult Poisson::solve_direct(double tol, bool to_floor, int max_sweeps, hipStream_t st) {
-    SolveResult R = refine(direct64, tol, to_floor, max_sweeps, st);
+// r of x (with ref: of the given right-hand side and guess), norms into slot.
+void Poisson::queue_r(const RefArrays *ref, int slot, hipStream_t st) {
+    res_blocks = residual_blocks();
+    const Residual R{N, M, f, pcg64.x, cx0, cu0, pcg64.wD, hres_dev + slot * 2 * kResidualBlocks};
+    if (ref)
+        hipLaunchKernelGGL(k_solve_residual<true>, dim3(res_blocks), dim3(1024), 0, st, R, ref->b, ref->x, f,
+                           pcg64.x, pcg64.r);
+    else
+        hipLaunchKernelGGL(k_solve_residual<false>, dim3(res_blocks), dim3(1024), 0, st, R, nullptr, nullptr, nullptr,
+                           nullptr, pcg64.r);
+}
+
+// Each sweep: x += L^-1 r by a direct solve, formed in another buffer, the FP64
+// residual and (ref) the solution in the reference's order, all queued before
+// the host reads the norms; the first sweep also before it has read those of
+// the guess, which may already meet the stop rule.  2048 x 255 in FP64: 138 us, 6
+// launches and one wait, where 10 and three took 170.
+template <typename T>
+SolveResult Poisson::refine(Direct<T> &D, const RefArrays *ref, double tol, bool to_floor, int max_sweeps,
+                            hipStream_t st) {
+    SolveResult R;
+    double rn2 = 0., bn2 = 0.;
+    auto out = [&] {
+        if (!ref) return;
+        hipEventRecord(ref->done, st);
+        x_to_ref(ref->x, st);
+    };
+    auto correct = [&] {
+        D.solve(pcg64.r, pcg64.x, x64B, st);
+        std::swap(pcg64.x, x64B);
+        queue_r(nullptr, 1, st);
+        out();
+        hipStreamSynchronize(st);
+    };
+    x_pending = XF_NONE;
+    queue_r(ref, 0, st);
+    correct();
+    norms(0, &rn2, &bn2);
+    const bool finite = std::isfinite(bn2) && std::isfinite(rn2);  // else: a bad right-hand side or guess
+    R.rel = R.rel0 = std::sqrt(rn2 / bn2);
+    R.converged = finite && (bn2 == 0. || R.rel <= tol);
+    if (R.converged || !finite || max_sweeps < 1) {  // the guess stays
+        if (finite && bn2 == 0.) {
+            R = SolveResult();
+            R.converged = true;
+            hipMemsetAsync(x64B, 0, size_t(M + 2) * N * sizeof(double), st);
+        }
+        std::swap(pcg64.x, x64B);
+        out();
+        return R;
+    }
+    for (int sweep = 1;; sweep++) {
+        const double prev = R.rel;
+        norms(1, &rn2, &bn2);
+        R.rel = std::sqrt(rn2 / bn2);
+        R.iters = R.refine = sweep;
+        if (!std::isfinite(bn2) || !std::isfinite(rn2)) return R;
+        const bool stalled = R.rel > 0.5 * prev;
+        R.converged = R.rel <= tol || (to_floor && stalled && R.rel <= kRoundOff);
+        if (R.converged || stalled || sweep == max_sweeps) return R;
+        correct();
+    }
+}
+
+SolveResult Poisson::solve_direct(const RefArrays &ref, double tol, bool to_floor, int max_sweeps, hipStream_t st) {
+    SolveResult R = refine(direct64, &ref, tol, to_floor, max_sweeps, st);
     R.refine = 0;
     return R;
 }
 
-SolveResult Poisson::solve_mixed(double tol, int max_sweeps, hipStream_t st) {
-    return refine(direct32, tol, false, max_sweeps, st);
+SolveResult Poisson::solve_mixed(const RefArrays &ref, double tol, int max_sweeps, hipStream_t st) {
+    return refine(direct32, &ref, tol, false, max_sweeps, st);
 }
 
 void Poisson::queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, const Micro *micro,
@@ -973,19 +1064,14 @@ SolveResult Poisson::finish_step(const Grid &G, double *w, const double *rhow_de
     SolveResult R;
     *redo = false;
     double rn2 = 0., bn2 = 0.;
-    const volatile double *p = hres;
-    for (int b = 0; b < res_blocks; b++) {  // fixed order: deterministic
-        rn2 += p[2 * b];
-        bn2 += p[2 * b + 1];
-    }
+    norms(0, &rn2, &bn2);
     R.iters = 1;
     R.rel0 = 1.;
     R.rel = bn2 > 0. ? std::sqrt(rn2 / bn2) : std::sqrt(rn2);
     R.converged = std::isfinite(bn2) && R.rel <= tol;
     if (R.converged || !std::isfinite(R.rel) || max_sweeps <= 1) return R;
     // beyond what one solve gives: corrected further
-    hscal[P_BNORM2] = bn2;
-    SolveResult C = refine(direct64, tol, to_floor, max_sweeps - 1, st);
+    SolveResult C = refine(direct64, nullptr, tol, to_floor, max_sweeps - 1, st);
     C.iters++;
     C.rel0 = 1.;
     back_to_w(G, w, rhow_dev, st);
@@ -1011,7 +1097,7 @@ void Poisson::queue_check(hipStream_t st) { queue_residual(Grid{}, StepPtrs{}, 0
 
 // k_calu's residual workgroups, behind ncol workgroups of cal_u
 void Poisson::queue_residual(const Grid &G, const StepPtrs &S, int ncol, hipStream_t st) {
-    res_blocks = std::min(kResidualBlocks, ((N + 63) / 64) * ((M + 15) / 16));
+    res_blocks = residual_blocks();
     hipLaunchKernelGGL(k_calu, dim3(ncol + res_blocks), dim3(UW * UC), ncol ? size_t(N) * sizeof(double) : 0, st, G,
                        S, ncol, Residual{N, M, f, pcg64.x, cx0, cu0, pcg64.wD, hres_dev});
 }

@@ -18,6 +18,8 @@
 // BiCGSTAB is a comparison mode.
 #pragma once
 
+#include <algorithm>
+
 #include "direct.h"
 #include "mg.h"
 #include "net.h"
@@ -46,12 +48,19 @@ struct SolveResult {
 };
 
 // ||wD (f - L x)||^2 and ||wD f||^2: a pair of partial sums per workgroup into
-// hres (host-mapped memory, at most kResidualBlocks pairs).
+// hres (host-mapped memory, at most kResidualBlocks pairs a slot).
 constexpr int kResidualBlocks = 256;
 struct Residual {
     int N, M;
     const double *f, *x, *cx, *cu, *wD;
     double *hres;
+};
+// An isolated solve's arrays in the reference's order: right-hand side, guess
+// and solution; done is recorded when the solve is.
+struct RefArrays {
+    const double *b;
+    double *x;
+    hipEvent_t done;
 };
 
 class Poisson {
@@ -94,8 +103,8 @@ class Poisson {
     // until ||b-Ax||/||b|| <= tol: by FP64 ones (solve_direct) or FP32 ones
     // (solve_mixed).  to_floor: also done when the residual has stopped
     // decreasing at FP64's round-off (kRoundOff).
-    SolveResult solve_direct(double tol, bool to_floor, int max_sweeps, hipStream_t st);
-    SolveResult solve_mixed(double tol, int max_sweeps, hipStream_t st);
+    SolveResult solve_direct(const RefArrays &ref, double tol, bool to_floor, int max_sweeps, hipStream_t st);
+    SolveResult solve_mixed(const RefArrays &ref, double tol, int max_sweeps, hipStream_t st);
     // The step's pubarTop_pt (not if step < 0), cal_w and cal_u in two halves.
     // queue_step: mean flow at the top, right-hand side (formed already if f_ready), solve and
     // w; queue_cal_u: u, and the residual's norms on their way to the host
@@ -160,11 +169,14 @@ class Poisson {
     Direct<double> direct64;
     Direct<float> direct32;
     double *cx0 = nullptr, *cu0 = nullptr;  // coefficients of L
-    double *hres = nullptr, *hres_dev = nullptr;  // k_calu's residual norms (mapped host memory)
+    double *hres = nullptr, *hres_dev = nullptr;  // residual norms, two slots (mapped host memory)
     void queue_residual(const Grid &G, const StepPtrs &S, int ncol, hipStream_t st);
     int res_blocks = 0;
     template <typename T>
-    SolveResult refine(Direct<T> &D, double tol, bool to_floor, int max_sweeps, hipStream_t st);
+    SolveResult refine(Direct<T> &D, const RefArrays *ref, double tol, bool to_floor, int max_sweeps, hipStream_t st);
+    void queue_r(const RefArrays *ref, int slot, hipStream_t st);
+    void norms(int slot, double *rn2, double *bn2) const;
+    int residual_blocks() const { return std::min(kResidualBlocks, ((N + 63) / 64) * ((M + 15) / 16)); }
     bool keep_guess(double rn2);
     double *f = nullptr;       // rhs of L x = f, (M+2)*N
     double *xprev = nullptr;   // previous solution (for extrapolation)

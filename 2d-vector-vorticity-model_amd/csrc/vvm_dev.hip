@@ -1190,21 +1190,27 @@ int vvm_dev_op_field(vvm_dev_t *h, int op, int field) {
 
 static int poisson_common(vvm_dev *h, const double *d_b, double *d_x, vvm_solve_stats *stats) {
     const vvm_dev_config &c = h->cfg;
-    h->pois.rhs_from_b(d_b, h->st);
-    h->pois.x_from_ref(d_x, h->st);
+    const bool direct = c.solver_mode == VVM_SOLVER_MIXED || (c.solver_mode != VVM_SOLVER_BICGSTAB && !uses_pcg(c));
+    if (!direct) {
+        h->pois.rhs_from_b(d_b, h->st);
+        h->pois.x_from_ref(d_x, h->st);
+    }
     hipEventRecord(h->ev[6], h->st);
     SolveResult R;
     const int maxit = max_iterations(c), sweeps = std::min(kMaxSweeps, maxit);
-    if (c.solver_mode == VVM_SOLVER_BICGSTAB)
+    const RefArrays ref{d_b, d_x, h->ev[7]};
+    if (c.solver_mode == VVM_SOLVER_MIXED)
+        R = h->pois.solve_mixed(ref, stop_tol(c), sweeps, h->st);
+    else if (direct)
+        R = h->pois.solve_direct(ref, stop_tol(c), true, sweeps, h->st);
+    else if (c.solver_mode == VVM_SOLVER_BICGSTAB)
         R = h->pois.solve_bicgstab(stop_tol(c), c.stop_mode == VVM_STOP_ABS, maxit, h->st);
-    else if (c.solver_mode == VVM_SOLVER_MIXED)
-        R = h->pois.solve_mixed(stop_tol(c), sweeps, h->st);
-    else if (uses_pcg(c))
-        R = h->pois.solve_fp64(c.stop_mode == VVM_STOP_PARITY ? 0. : c.tol_rel, maxit, h->st);
     else
-        R = h->pois.solve_direct(stop_tol(c), true, sweeps, h->st);
-    hipEventRecord(h->ev[7], h->st);
-    h->pois.x_to_ref(d_x, h->st);
+        R = h->pois.solve_fp64(c.stop_mode == VVM_STOP_PARITY ? 0. : c.tol_rel, maxit, h->st);
+    if (!direct) {
+        hipEventRecord(h->ev[7], h->st);
+        h->pois.x_to_ref(d_x, h->st);
+    }
     HIPCHK(h, hipStreamSynchronize(h->st));
     float ms = 0.f;
     hipEventElapsedTime(&ms, h->ev[6], h->ev[7]);
