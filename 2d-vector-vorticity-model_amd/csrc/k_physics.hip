@@ -134,7 +134,7 @@ __global__ void __launch_bounds__(BX *BY) k_nudge_qv(Grid G, StepPtrs S, double 
 // Iteration::updateMean (src/Iteration.cpp:42-86) as called by
 // nextTimeStep: one block per level.  thb_zeta is not read by the step and
 // is formed on download.
-__global__ void __launch_bounds__(256) k_update_mean(Grid G, StepPtrs S, int shift_ubar) {
+__global__ void __launch_bounds__(256) k_update_mean(Grid G, StepPtrs S, MeanMode mode) {
     const int k = blockIdx.x + 1;
     const double *thp = S.fut[F_TH], *qvp = S.fut[F_QV];
     double acc[2] = {0., 0.};
@@ -147,26 +147,27 @@ __global__ void __launch_bounds__(256) k_update_mean(Grid G, StepPtrs S, int shi
         double *thb = S.P.thb, *qvb = S.P.qvb, *thvb = S.P.thvb;
         const double tb = acc[0] / (double)(G.nx - 2.), qb = acc[1] / (double)(G.nx - 2.);
         const double tv = tb * (1 + 0.608 * qb);
-        S.P.thbm[k] = thb[k];
-        S.P.thvbm[k] = thvb[k];
+        const bool shift = mode != MEAN_AGAIN;
+        if (shift) S.P.thbm[k] = thb[k];
+        if (shift) S.P.thvbm[k] = thvb[k];
         thb[k] = tb;
         qvb[k] = qb;
         thvb[k] = tv;
         if (k == 1) {
-            S.P.thbm[0] = thb[0];
-            S.P.thvbm[0] = thvb[0];
+            if (shift) S.P.thbm[0] = thb[0];
+            if (shift) S.P.thvbm[0] = thvb[0];
             thb[0] = tb;
             qvb[0] = qb;
             thvb[0] = tv;
-            if (shift_ubar) {
+            if (mode == MEAN_STEP) {
                 // nextTimeStep's copy loop (src/Iteration.cpp:166-167)
                 S.s[S_UBARTOPM] = S.s[S_UBARTOPP];
                 S.s[S_UBARTOP] = S.s[S_UBARTOPP];
             }
         }
         if (k == G.nz - 2) {
-            S.P.thbm[k + 1] = thb[k + 1];
-            S.P.thvbm[k + 1] = thvb[k + 1];
+            if (shift) S.P.thbm[k + 1] = thb[k + 1];
+            if (shift) S.P.thvbm[k + 1] = thvb[k + 1];
             thb[k + 1] = tb;
             qvb[k + 1] = qb;
             thvb[k + 1] = tv;
@@ -223,8 +224,8 @@ void launch_nudge(const Grid &G, const StepPtrs &S, int nudge, hipStream_t st) {
 void launch_nudge_qv(const Grid &G, const StepPtrs &S, double tau, hipStream_t st) {
     hipLaunchKernelGGL(k_nudge_qv, grid2d(G), dim3(BX, BY), 0, st, G, S, tau);
 }
-void launch_update_mean(const Grid &G, const StepPtrs &S, bool shift_ubar, hipStream_t st) {
-    hipLaunchKernelGGL(k_update_mean, dim3(G.nz - 2), dim3(256), 0, st, G, S, int(shift_ubar));
+void launch_update_mean(const Grid &G, const StepPtrs &S, MeanMode mode, hipStream_t st) {
+    hipLaunchKernelGGL(k_update_mean, dim3(G.nz - 2), dim3(256), 0, st, G, S, mode);
 }
 
 }  // namespace vvmd

@@ -1064,6 +1064,7 @@ SolveResult Poisson::finish_step(const Grid &G, double *w, const double *rhow_de
     SolveResult R;
     *redo = false;
     double rn2 = 0., bn2 = 0.;
+    await_set(hres, 2 * res_blocks, st);
     norms(0, &rn2, &bn2);
     R.iters = 1;
     R.rel0 = 1.;
@@ -1098,6 +1099,7 @@ void Poisson::queue_check(hipStream_t st) { queue_residual(Grid{}, StepPtrs{}, 0
 // k_calu's residual workgroups, behind ncol workgroups of cal_u
 void Poisson::queue_residual(const Grid &G, const StepPtrs &S, int ncol, hipStream_t st) {
     res_blocks = residual_blocks();
+    mark_unset(hres, 2 * res_blocks);
     hipLaunchKernelGGL(k_calu, dim3(ncol + res_blocks), dim3(UW * UC), ncol ? size_t(N) * sizeof(double) : 0, st, G,
                        S, ncol, Residual{N, M, f, pcg64.x, cx0, cu0, pcg64.wD, hres_dev});
 }

@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "poisson.h"
@@ -40,12 +41,11 @@ struct vvm_dev {
     int dstrip_cw = 0;              // diffusion strip width in wavefronts (0: default)
     // The diffusion sweep's warm-up (diffusion_halo; 0: in order), guessed from
     // the last step's coefficients and checked against this step's, which
-    // k_turb_coeffs leaves in kmax (host-mapped) before ev_turb.
+    // k_turb_coeffs leaves in kmax (host-mapped; mark_unset, await_set).
     int diff_halo = 0;
     double *kmax = nullptr, *kmax_dev = nullptr;  // [kTurbBlocks], then the sweep's error flag
     int kmax_blocks = 0;
     double rho_per_k = 0.;          // largest a + d of the sweep per unit of K
-    hipEvent_t ev_turb = nullptr;
     GuessNet *guess_net = nullptr;  // attached learned guess (not owned)
     int guess_net_device = -1;
     Profiles P{};
@@ -201,13 +201,13 @@ StepPtrs ptrs(vvm_dev *h) {
 
 // Turbulence coefficients, and the largest of them on its way to the host.
 void queue_turbulence(vvm_dev *h, const StepPtrs &S) {
+    mark_unset(h->kmax, kTurbBlocks);
     h->kmax_blocks = launch_turbulence_coeffs(h->G, S, h->kmax_dev, h->st);
-    hipEventRecord(h->ev_turb, h->st);
 }
 
-// The sweep's largest weight sum, once ev_turb has passed.
+// The sweep's largest weight sum, once it is there.
 double diffusion_rho(vvm_dev *h) {
-    hipEventSynchronize(h->ev_turb);
+    await_set(h->kmax, h->kmax_blocks, h->st);
     const volatile double *p = h->kmax;
     double m = 0.;
     for (int b = 0; b < h->kmax_blocks; b++) {
@@ -227,18 +227,21 @@ void take_tiles(vvm_dev *h, StepPtrs &S) {
     }
 }
 
-// Mparam and Hparam of the five fields.  queued: the halo of the tiled sweep
-// that is in the stream already (0: none); it is redone where the
-// coefficients ask for a longer one.
-void finish_diffusion(vvm_dev *h, StepPtrs &S, int nudge, int queued) {
+// The warm-up the coefficients ask for (0: the sweep in order); the next step is
+// queued with some reserve.
+int sweep_halo(vvm_dev *h) {
     const double rho = diffusion_rho(h);
-    const int need = diffusion_halo(rho);
     h->diff_halo = diffusion_halo(1.25 * rho);
-    if (need == 0) {
+    return diffusion_halo(rho);
+}
+
+// Mparam and Hparam of the five fields.
+void diffuse(vvm_dev *h, StepPtrs &S, int nudge, int halo) {
+    if (halo == 0) {
         launch_diffusion(h->G, S, nudge, h->st);
         return;
     }
-    if (need > queued) launch_diffusion_tiles(h->G, S, nudge, need, h->st);
+    launch_diffusion_tiles(h->G, S, nudge, halo, h->st);
     take_tiles(h, S);
 }
 
@@ -487,8 +490,7 @@ int vvm_dev_create(const vvm_dev_config *cfg, int device, vvm_dev_t **out) {
     ok = ok &&
          hipHostMalloc(reinterpret_cast<void **>(&h->kmax), (kTurbBlocks + 1) * sizeof(double),
                        hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess &&
-         hipHostGetDevicePointer(reinterpret_cast<void **>(&h->kmax_dev), h->kmax, 0) == hipSuccess &&
-         hipEventCreateWithFlags(&h->ev_turb, hipEventDisableTiming) == hipSuccess;
+         hipHostGetDevicePointer(reinterpret_cast<void **>(&h->kmax_dev), h->kmax, 0) == hipSuccess;
     if (h->kmax) h->kmax[kTurbBlocks] = 0.;
     for (auto &e : h->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
     for (auto &e : h->ev_mp) ok = ok && hipEventCreate(&e) == hipSuccess;
@@ -523,7 +525,7 @@ void vvm_dev_destroy(vvm_dev_t *h) {
         if (e) hipEventDestroy(e);
     for (auto &e : h->kt_ev)
         if (e) hipEventDestroy(e);
-    for (hipEvent_t e : {h->ev_turb, h->ev_fork0, h->ev_guess, h->ev_fork, h->ev_join, h->ev_mp[0], h->ev_mp[1]})
+    for (hipEvent_t e : {h->ev_fork0, h->ev_guess, h->ev_fork, h->ev_join, h->ev_mp[0], h->ev_mp[1]})
         if (e) hipEventDestroy(e);
     for (hipEvent_t e : h->tev)
         if (e) hipEventDestroy(e);
@@ -801,6 +803,21 @@ bool finish_solve(vvm_dev *h, bool wait) {
     return redo;
 }
 
+// Nudge_qv and nextTimeStep's updateMean (:153-204).  again: after the
+// diffusion has been redone, when the means of the step before have moved on
+// already.
+void queue_end(vvm_dev *h, bool again) {
+    const StepPtrs &S = h->run.S;
+    const double tau = h->cfg.moisture_nudge_time;
+    if (tau != 0) launch_nudge_qv(h->G, S, tau, h->st);
+    mark(h, 4, h->st);
+    {
+        KTimer t(h, VVM_KT_MEAN);
+        launch_update_mean(h->G, S, again ? MEAN_AGAIN : MEAN_STEP, h->st);
+    }
+    mark(h, 5, h->st);
+}
+
 // Whether the step's microphysics rides in the solve's launches: up to 640 of
 // thermo4's tiles.  That saves the host two launches and the two streams'
 // events, whose waits alone take it 24 us; above, the solve's LDS leaves too
@@ -928,39 +945,39 @@ int step_begin(vvm_dev *h, int timer, bool last) {
         queue_turbulence(h, S);
     }
     if (r.halo) {
-        KTimer t(h, VVM_KT_DIFFUSION);
-        launch_diffusion_tiles(G, S, step_nudge(c), r.halo, h->st);
+        {
+            KTimer t(h, VVM_KT_DIFFUSION);
+            launch_diffusion_tiles(G, S, step_nudge(c), r.halo, h->st);
+        }
+        take_tiles(h, r.S);
+        queue_end(h, false);
     }
     return check_launch(h);
 }
 
-// The rest of the step: the checks, updateMean, the rotation of the levels.
-// Adds the solve to acc.
+// The rest of the step: the checks and what they ask for again, the rotation of
+// the levels.  Adds the solve to acc.
 int step_finish(vvm_dev *h, vvm_step_stats *acc) {
     const Grid &G = h->G;
     const vvm_dev_config &c = h->cfg;
     vvm_dev::Run &r = h->run;
     StepPtrs &S = r.S;
-    hipEventSynchronize(h->ev_turb);  // the residual's norms and the coefficients' maximum are in
-    if (finish_solve(h, false)) {
-        queue_turbulence(h, S);
-        if (r.halo) launch_diffusion_tiles(G, S, step_nudge(c), r.halo, h->st);
+    if (r.halo) take_tiles(h, S);  // back to what the sweep started from, which a correction needs
+    const bool redo = finish_solve(h, false);
+    if (redo) queue_turbulence(h, S);
+    const int need = sweep_halo(h);
+    if (!redo && need && need <= r.halo) {
+        take_tiles(h, S);
+    } else {
+        diffuse(h, S, step_nudge(c), need);
+        queue_end(h, r.halo != 0);
     }
-    finish_diffusion(h, S, step_nudge(c), r.halo);
     if (r.rc == VVM_WARN_NOT_CONVERGED) acc->not_converged++;
     acc->solve_iters_total += r.ss.iters;
     acc->solve_iters_last = r.ss.iters;
     acc->refine_last = r.ss.refine;
     acc->rel_residual_last = r.ss.rel_residual;
-    if (c.moisture_nudge_time != 0) launch_nudge_qv(G, S, c.moisture_nudge_time, h->st);
-    mark(h, 4, h->st);
-    // E: nextTimeStep (:153-204)
-    {
-        KTimer t(h, VVM_KT_MEAN);
-        launch_update_mean(G, S, true, h->st);
-    }
     rotate(h);
-    mark(h, 5, h->st);
     h->stepped = true;
     return check_launch(h);
 }
@@ -1079,14 +1096,14 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             break;
         case VVM_OP_TURBULENCE:
             queue_turbulence(h, S);
-            finish_diffusion(h, S, 0, 0);
+            diffuse(h, S, 0, sweep_halo(h));
             break;
         case VVM_OP_NUDGE:
             launch_nudge(G, S, 1 | (c.CASE != 2 ? 2 : 0), h->st);
             if (c.moisture_nudge_time != 0) launch_nudge_qv(G, S, c.moisture_nudge_time, h->st);
             break;
         case VVM_OP_NEXT:
-            launch_update_mean(G, S, true, h->st);
+            launch_update_mean(G, S, MEAN_STEP, h->st);
             rotate(h);
             h->stepped = true;
             break;
@@ -1151,7 +1168,7 @@ int vvm_dev_op_field(vvm_dev_t *h, int op, int field) {
             launch_precip(G, S, h->st);
             launch_bc_one(G, S.fut[F_QR], false, h->st);
             break;
-        case VVM_OP_UPDATE_MEAN: launch_update_mean(G, S, false, h->st); break;
+        case VVM_OP_UPDATE_MEAN: launch_update_mean(G, S, MEAN_ONLY, h->st); break;
         case VVM_OP_AUTOCONVERSION: launch_kessler_process(G, S, 0, h->st); break;
         case VVM_OP_ACCRETION: launch_kessler_process(G, S, 1, h->st); break;
         case VVM_OP_EVAPORATION: launch_kessler_process(G, S, 2, h->st); break;
@@ -1441,6 +1458,28 @@ int vvm_dev_tune(vvm_dev_t *h, int steps, vvm_tune_result *out) {
 }  // extern "C"
 
 namespace vvmd {
+static constexpr uint64_t kUnset = 0x7ff85a5ac3c30f0full;
+
+void mark_unset(double *p, int n) {
+    volatile uint64_t *q = reinterpret_cast<volatile uint64_t *>(p);
+    for (int i = 0; i < n; i++) q[i] = kUnset;
+}
+
+void await_set(const double *p, int n, hipStream_t st) {
+    const volatile uint64_t *q = reinterpret_cast<const volatile uint64_t *>(p);
+    bool ended = false;
+    for (int i = 0; i < n; i++) {
+        for (int spins = 1; q[i] == kUnset && !ended; spins++) {
+            if (spins % 64 == 0) std::this_thread::yield();
+            if (spins % 8192 == 0) {
+                const hipError_t e = hipStreamQuery(st);
+                if (e == hipErrorNotReady) (void)hipGetLastError();  // not an error
+                else ended = true;
+            }
+        }
+    }
+}
+
 void dev_set_phase_overlap(vvm_dev_t *h, bool on) {
     if (h) h->overlap_c = on;
 }

@@ -89,6 +89,14 @@ void launch_scale_forcing(const Grid &G, const StepPtrs &S, const Negval &nv, co
                           bool halos = true);
 void launch_bc_uw(const Grid &G, const StepPtrs &S, hipStream_t st);
 void launch_bc_all_prog(const Grid &G, const StepPtrs &S, hipStream_t st);
+// Sums that kernels leave in mapped host memory for the host to read while the
+// stream runs on: marked before the launch, and waited for by reading them.  An
+// event behind the kernel held the next one back by 3 us and cost the host 2 us
+// to record and a wake-up.  The mark is a NaN that no arithmetic gives; should
+// the stream end (or fail) without the sums, the wait ends and they stay NaN.
+void mark_unset(double *p, int n);
+void await_set(const double *p, int n, hipStream_t st);
+
 // Whether a handle runs the microphysics phase on its second stream beside
 // the elliptic solve (default on).  The ensemble turns it off: with one
 // stream pair per member on a few hardware queues, the cross-stream waits
@@ -135,7 +143,10 @@ void diffusion_slots_release(unsigned long long *p);
 bool diffusion_strip_waves_ok(int cw);
 void launch_nudge(const Grid &G, const StepPtrs &S, int nudge, hipStream_t st);
 void launch_nudge_qv(const Grid &G, const StepPtrs &S, double tau, hipStream_t st);
-void launch_update_mean(const Grid &G, const StepPtrs &S, bool shift_ubar, hipStream_t st);
+// MEAN_ONLY: updateMean; MEAN_STEP: with nextTimeStep's shift of ubarTop;
+// MEAN_AGAIN: the means alone, thbm and thvbm as a first pass has left them.
+enum MeanMode { MEAN_ONLY, MEAN_STEP, MEAN_AGAIN };
+void launch_update_mean(const Grid &G, const StepPtrs &S, MeanMode mode, hipStream_t st);
 
 // Elliptic (k_poisson.hip): see poisson.h
 }  // namespace vvmd
