@@ -133,13 +133,16 @@ __host__ __device__ inline int pz_tiles_z(const Grid &G) { return (G.nz - 3 + PZ
 // advection, zetap += ... for the buoyancy) and its AB2 history.
 enum { PZ_ADV = 1, PZ_BUOY = 2, PZ_BOTH = 3 };
 
+struct PzLds {
+    double Fx[PZY][PZX + 1];  // slot c: x-flux east of column i0 + c - 1
+    double Fz[PZY + 1][PZX];  // slot r: z-flux above row k0 + r - 1
+};
 template <int PARTS>
-__global__ void __launch_bounds__(PZX *PZY) k_pzeta(Grid G, StepPtrs S, int step) {
-    __shared__ double Fx[PZY][PZX + 1];  // slot c: x-flux east of column i0 + c - 1
-    __shared__ double Fz[PZY + 1][PZX];  // slot r: z-flux above row k0 + r - 1
+__device__ inline void pzeta_tile(const Grid &G, const StepPtrs &S, int step, int tile, PzLds &lds) {
+    auto &Fx = lds.Fx;
+    auto &Fz = lds.Fz;
     const int tx = threadIdx.x, ty = uniform(threadIdx.y);  // PZX = T4X = 64: one row a wavefront
-    const int tiles_x = pz_tiles_x(G), tiles_z = pz_tiles_z(G), tile = xcd_tile(tiles_x * tiles_z);
-    if (tile >= tiles_x * tiles_z) return;
+    const int tiles_x = pz_tiles_x(G);
     const int i0 = 1 + (tile % tiles_x) * PZX, k0 = 2 + (tile / tiles_x) * PZY;
     const int i = i0 + tx, k = k0 + ty;
     const int nx = G.nx, nz = G.nz;
@@ -207,6 +210,12 @@ __global__ void __launch_bounds__(PZX *PZY) k_pzeta(Grid G, StepPtrs S, int step
     zeta_new += (1.5 * G.dt * db) - (0.5 * G.dt * bold);
     if constexpr (PARTS == PZ_BOTH) store_westdown(zp, G, i, k, zeta_new);
     else at(zp, G, i, k) = zeta_new;
+}
+template <int PARTS>
+__global__ void __launch_bounds__(PZX *PZY) k_pzeta(Grid G, StepPtrs S, int step) {
+    __shared__ PzLds lds;
+    const int nt = pz_tiles_x(G) * pz_tiles_z(G), tile = xcd_tile(nt);
+    if (tile < nt) pzeta_tile<PARTS>(G, S, step, tile, lds);
 }
 
 // ----------------------------------------------------------- scalars
@@ -298,14 +307,15 @@ constexpr int T4X = 64, T4Y = 8;
 __host__ __device__ inline int t4_tiles_x(const Grid &G) { return (G.nx - 2 + T4X - 1) / T4X; }
 __host__ __device__ inline int t4_tiles_z(const Grid &G) { return (G.nz - 2 + T4Y - 1) / T4Y; }
 
-// Four workgroups a CU (the LDS allows four), so that 1024 of them cover
-// 2048 x 256 in one round: eight waves a SIMD, at most 64 VGPRs.
-__global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8))) k_thermo4(Grid G, StepPtrs S, int step, RedSlot rs) {
-    __shared__ double Fx[4][T4Y][T4X + 1];  // x-face flux at faces i0 .. i0+T4X (west faces)
-    __shared__ double Fz[5][T4Y + 1][T4X];  // z-face flux (4 fields, rain fall) at faces k0 .. k0+T4Y
+struct T4Lds {
+    double Fx[4][T4Y][T4X + 1];  // x-face flux at faces i0 .. i0+T4X (west faces)
+    double Fz[5][T4Y + 1][T4X];  // z-face flux (4 fields, rain fall) at faces k0 .. k0+T4Y
+};
+__device__ inline void thermo4_tile(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, int tile, T4Lds &lds) {
+    auto &Fx = lds.Fx;
+    auto &Fz = lds.Fz;
     const int tx = threadIdx.x, ty = uniform(threadIdx.y);  // PZX = T4X = 64: one row a wavefront
-    const int tiles_x = t4_tiles_x(G), ntiles = tiles_x * t4_tiles_z(G), tile = xcd_tile(ntiles);
-    if (tile >= ntiles) return;
+    const int tiles_x = t4_tiles_x(G);
     const int i0 = 1 + (tile % tiles_x) * T4X, k0 = 1 + (tile / tiles_x) * T4Y;
     const int i = i0 + tx, k = k0 + ty;
     const int nx = G.nx, nz = G.nz;
@@ -391,6 +401,29 @@ __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8
         }
     }
     block_partials<6>(part, rs, tile);
+}
+// Four workgroups a CU (the LDS allows four), so that 1024 of them cover
+// 2048 x 256 in one round: eight waves a SIMD, at most 64 VGPRs.
+__global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8)))
+k_thermo4(Grid G, StepPtrs S, int step, RedSlot rs) {
+    __shared__ T4Lds lds;
+    const int nt = t4_tiles_x(G) * t4_tiles_z(G), tile = xcd_tile(nt);
+    if (tile < nt) thermo4_tile(G, S, step, rs, tile, lds);
+}
+
+// Both in one launch, a tile of each in turn: neither reads what the other
+// writes, and the second of a pair finds the winds and scalars in its XCD's L2.
+static_assert(T4X == PZX && T4Y == PZY, "one block shape");
+__global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8)))
+k_advect(Grid G, StepPtrs S, int step, RedSlot rs) {
+    __shared__ union Lds {
+        T4Lds t4;
+        PzLds pz;
+    } lds;
+    const int nt = t4_tiles_x(G) * t4_tiles_z(G), slot = xcd_tile(2 * nt), tile = slot / 2;
+    if (slot >= 2 * nt) return;
+    if (slot % 2 == 0) thermo4_tile(G, S, step, rs, tile, lds.t4);
+    else if (tile < pz_tiles_x(G) * pz_tiles_z(G)) pzeta_tile<PZ_BOTH>(G, S, step, tile, lds.pz);
 }
 
 __global__ void __launch_bounds__(BX *BY) k_scale_forcing(Grid G, StepPtrs S, Negval nv, Forcing F, int halos) {
@@ -520,6 +553,17 @@ void launch_bc_one(const Grid &G, double *a, bool westdown, hipStream_t st) {
 Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
     const int n = t4_tiles_x(G) * t4_tiles_z(G);
     hipLaunchKernelGGL(k_thermo4, xcd_grid(n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
+    return {rs, n};
+}
+// Up to 1024 tiles of each, four to a CU: there the two shorten each other's
+// last round and save a launch.  Above, the launch is nothing and thermo4's
+// LDS keeps CUs from filling up with pzeta's tiles.  A step in us, together /
+// apart: 128 x 64 55.7 / 63.5, 1024 x 128 78.9 / 83.1, 2048 x 128 104.4 / 106.5,
+// 2048 x 256 (1024 tiles) 142.9 / 146.4, 4096 x 256 257.7 / 254.2.
+bool advect_together(const Grid &G) { return t4_tiles_x(G) * t4_tiles_z(G) <= 1024; }
+Negval launch_advect(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
+    const int n = t4_tiles_x(G) * t4_tiles_z(G);  // no fewer than pzeta's
+    hipLaunchKernelGGL(k_advect, xcd_grid(2 * n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
     return {rs, n};
 }
 // The ratios of NegativeValueProcess from nblk workgroups' partials: by

@@ -861,18 +861,20 @@ int step_begin(vvm_dev *h, int timer, bool last) {
     const bool direct = uses_direct(c);
     mark(h, 0, h->st);
     // A: advection, buoyancy, forcing, halos (src/Iteration.cpp:263-285)
-    {
-        KTimer t(h, VVM_KT_PZETA);
-        launch_pzeta(G, S, h->step, h->st);
-    }
-    if (early_guess) {
-        hipEventRecord(h->ev_fork0, h->st);
-        hipStreamWaitEvent(h->side, h->ev_fork0, 0);
-        prepare_guess(h, S, true, h->side);
-        hipEventRecord(h->ev_guess, h->side);
-    }
     Negval nv;
-    {
+    if (!early_guess && advect_together(G) && h->kt_kernel != VVM_KT_PZETA && h->kt_kernel != VVM_KT_THERMO4) {
+        nv = launch_advect(G, S, h->step, h->red.negval, h->st);
+    } else {
+        {
+            KTimer t(h, VVM_KT_PZETA);
+            launch_pzeta(G, S, h->step, h->st);
+        }
+        if (early_guess) {
+            hipEventRecord(h->ev_fork0, h->st);
+            hipStreamWaitEvent(h->side, h->ev_fork0, 0);
+            prepare_guess(h, S, true, h->side);
+            hipEventRecord(h->ev_guess, h->side);
+        }
         KTimer t(h, VVM_KT_THERMO4);
         nv = launch_thermo4(G, S, h->step, h->red.negval, h->st);
     }

@@ -84,6 +84,9 @@ struct Forcing {
     int on, tropical, random_kick;
 };
 Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);
+// launch_pzeta and launch_thermo4 in one launch; whether that is the faster way
+bool advect_together(const Grid &G);
+Negval launch_advect(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);
 Negval negval_partials(const StepPtrs &S, const Negval &nv, hipStream_t st);
 void launch_scale_forcing(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, hipStream_t st,
                           bool halos = true);

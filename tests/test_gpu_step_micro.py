@@ -3,7 +3,9 @@ left them and applies the negative-value rescale and AddForcing on the way.
 
 Grids whose 64 x 4 tiles (Kessler) and 64 x 8 tiles (advection) are full, have
 one column and row more, and are both, one, or none at most 640, up to which
-the ratios come from the producer's partial sums instead of k_finalize.  One
+the ratios come from the producer's partial sums instead of k_finalize; and one
+row and column past 1024 of the latter, up to which the vorticity's advection
+shares their launch (the operators have one each).  One
 step with every kind of forcing, negative cloud and a few points of negative
 rain (whose fall speed is NaN), against the same phases as separate operators.
 The microphysics' rates come straight from that kernel and have to be the same
@@ -23,7 +25,8 @@ PHASES = ["pzeta_pt", "pscalars", "forcing_bc", "pubarTop_pt", "cal_w", "cal_u",
 RATES = ["evaporation", "accretion", "autoconversion", "condensation", "precip"]
 
 
-@pytest.mark.parametrize("nx,nz", [(64, 8), (65, 9), (66, 10), (67, 11), (63, 19), (1100, 150), (2100, 170)])
+@pytest.mark.parametrize("nx,nz", [(64, 8), (65, 9), (66, 10), (67, 11), (63, 19), (1100, 150), (2100, 170), (2048, 256),
+                                   (2049, 257)])
 @pytest.mark.parametrize("forced", [False, True])
 def test_step_forcing_and_kessler(nx, nz, forced):
     kw = dict(tropical_forcing=1, addforcingtime=10.0) if forced else {}
