@@ -68,6 +68,19 @@ __device__ inline void store_westdown(double *a, const Grid &G, int i, int k, do
     if (i == 1) at(a, G, G.nx - 1, k) = v;
 }
 
+// Notes the time in slot of clock, if there is one: the first workgroup's first
+// thread as the kernel starts, or the last one's as it ends.
+__device__ inline void note_time(long long *clock, int slot) {
+    if (threadIdx.x == 0 && threadIdx.y == 0)
+        __hip_atomic_store(clock + slot, (long long)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ inline void note_start(long long *clock, int slot) {
+    if (clock && blockIdx.x == 0 && blockIdx.y == 0) note_time(clock, slot);
+}
+__device__ inline void note_end(long long *clock, int slot) {
+    if (clock && blockIdx.x == gridDim.x - 1 && blockIdx.y == gridDim.y - 1) note_time(clock, slot);
+}
+
 // ---------------------------------------------------------------- sums
 
 constexpr int kWave = 64;

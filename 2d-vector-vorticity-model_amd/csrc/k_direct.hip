@@ -358,6 +358,8 @@ __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restric
                                                    double *__restrict__ f, Micro m) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     if constexpr (RHS) {
+        note_start(S.clock, CLK_SOLVE);
+        if (m.nblk) note_start(S.clock, CLK_MICRO);
         const int extra = int(blockIdx.x) - (P.M + 1) / 2, first = step >= 0 ? 1 : 0;
         if (extra >= 0) {
             if (extra < first) pubartop_block(G, S, step);
@@ -426,7 +428,7 @@ __global__ void __launch_bounds__(1024) k_rows_fwd(RowPlan P, const T *__restric
 template <typename T, bool ADD, bool W, bool CHIRP>
 __global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restrict__ tw, const T *__restrict__ chirp,
                                                    const T *__restrict__ spec, const double *x0, double *x, Grid G, double *__restrict__ w,
-                                                   const double *__restrict__ rhow) {
+                                                   const double *__restrict__ rhow, long long *micro_clock) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int N = P.N, M = P.M, LN = pad(P.L - 1) + 1;
     T *re = reinterpret_cast<T *>(lds_raw), *im = re + LN, *twl = im + LN;
@@ -445,6 +447,7 @@ __global__ void __launch_bounds__(1024) k_rows_inv(RowPlan P, const T *__restric
     Tw.store(P, twl);
     fill_rows<CHIRP>(P, re, im, va, vb, two, chirp);
     if constexpr (W) {  // the zero rows of w
+        note_start(micro_clock, CLK_MICRO_END);
         for (int i = threadIdx.x; i < G.nx; i += blockDim.x) {
             if (blockIdx.x == 0) w[ix(G, i, 0)] = w[ix(G, i, 1)] = 0.;
             if (blockIdx.x == gridDim.x - 1) w[ix(G, i, G.nz - 1)] = 0.;
@@ -854,10 +857,10 @@ void Direct<T>::rows_solve(const double *r, const double *x0, double *x, hipStre
     columns(NoMicro{}, 0, st);
     if (x0)
         hipLaunchKernelGGL((k_rows_inv<T, true, false, C>), gr, b, row_lds, st, plan, tw, chirp, spec, x0, x, Grid{},
-                           nullptr, nullptr);
+                           nullptr, nullptr, nullptr);
     else
         hipLaunchKernelGGL((k_rows_inv<T, false, false, C>), gr, b, row_lds, st, plan, tw, chirp, spec, x0, x, Grid{},
-                           nullptr, nullptr);
+                           nullptr, nullptr, nullptr);
 }
 template <typename T>
 void Direct<T>::solve(const double *r, const double *x0, double *x, hipStream_t st) {
@@ -884,7 +887,7 @@ void Direct<T>::rows_solve_step(const Grid &G, const StepPtrs &S, int step, cons
         columns(NoMicro{}, 0, st);
     }
     hipLaunchKernelGGL((k_rows_inv<T, false, true, C>), gr, b, row_lds, st, plan, tw, chirp, spec, nullptr, x, G, S.w,
-                       S.P.rhow);
+                       S.P.rhow, micro ? S.clock : nullptr);
 }
 template <typename T>
 void Direct<T>::solve_step(const Grid &G, const StepPtrs &S, int step, const Micro *micro, double *f, double *x,

@@ -213,6 +213,7 @@ __device__ inline void pzeta_tile(const Grid &G, const StepPtrs &S, int step, in
 }
 template <int PARTS>
 __global__ void __launch_bounds__(PZX *PZY) k_pzeta(Grid G, StepPtrs S, int step) {
+    note_start(S.clock, CLK_ADVECT);
     __shared__ PzLds lds;
     const int nt = pz_tiles_x(G) * pz_tiles_z(G), tile = xcd_tile(nt);
     if (tile < nt) pzeta_tile<PARTS>(G, S, step, tile, lds);
@@ -420,6 +421,7 @@ k_advect(Grid G, StepPtrs S, int step, RedSlot rs) {
         T4Lds t4;
         PzLds pz;
     } lds;
+    note_start(S.clock, CLK_ADVECT);
     const int nt = t4_tiles_x(G) * t4_tiles_z(G), slot = xcd_tile(2 * nt), tile = slot / 2;
     if (slot >= 2 * nt) return;
     if (slot % 2 == 0) thermo4_tile(G, S, step, rs, tile, lds.t4);
@@ -431,6 +433,7 @@ __global__ void __launch_bounds__(BX *BY) k_scale_forcing(Grid G, StepPtrs S, Ne
     double ratios[3];
     negval_ratios(S, nv.rs, nv.nblk, ratios);
     if (i <= G.nx - 2 && k <= G.nz - 2) scale_point(G, S, F, ratios, halos != 0, i, k);
+    note_end(S.clock, CLK_MICRO_END);
 }
 
 // Halo value of BoundaryProcess2D_center at a perimeter cell.
@@ -551,18 +554,19 @@ void launch_bc_one(const Grid &G, double *a, bool westdown, hipStream_t st) {
     hipLaunchKernelGGL(k_bc_one, grid2d(G), dim3(BX, BY), 0, st, G, a, int(westdown));
 }
 Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
-    const int n = t4_tiles_x(G) * t4_tiles_z(G);
+    const int n = advect_tiles(G);
     hipLaunchKernelGGL(k_thermo4, xcd_grid(n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
     return {rs, n};
 }
+int advect_tiles(const Grid &G) { return t4_tiles_x(G) * t4_tiles_z(G); }
 // Up to 1024 tiles of each, four to a CU: there the two shorten each other's
 // last round and save a launch.  Above, the launch is nothing and thermo4's
 // LDS keeps CUs from filling up with pzeta's tiles.  A step in us, together /
 // apart: 128 x 64 55.7 / 63.5, 1024 x 128 78.9 / 83.1, 2048 x 128 104.4 / 106.5,
 // 2048 x 256 (1024 tiles) 142.9 / 146.4, 4096 x 256 257.7 / 254.2.
-bool advect_together(const Grid &G) { return t4_tiles_x(G) * t4_tiles_z(G) <= 1024; }
+bool advect_together(const Grid &G) { return advect_tiles(G) <= 1024; }
 Negval launch_advect(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
-    const int n = t4_tiles_x(G) * t4_tiles_z(G);  // no fewer than pzeta's
+    const int n = advect_tiles(G);  // no fewer than pzeta's
     hipLaunchKernelGGL(k_advect, xcd_grid(2 * n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
     return {rs, n};
 }

@@ -31,7 +31,10 @@ __global__ void __launch_bounds__(BX *BY) k_kessler(Grid G, StepPtrs S, Negval n
     const int i = 1 + blockIdx.x * BX + threadIdx.x, k = 1 + blockIdx.y * BY + uniform(threadIdx.y);
     double part[6] = {0., 0., 0., 0., 0., 0.};
     double ratios[3] = {-1., -1., -1.};
-    if constexpr ((PROC & KP_PRE) != 0) negval_ratios(S, nv.rs, nv.nblk, ratios);
+    if constexpr ((PROC & KP_PRE) != 0) {
+        note_start(S.clock, CLK_MICRO);
+        negval_ratios(S, nv.rs, nv.nblk, ratios);
+    }
     if (i <= G.nx - 2 && k <= G.nz - 2) kessler_point<PROC>(G, S, F, ratios, i, k, part);
     if constexpr ((PROC & KP_NEG) != 0) block_partials<6>(part, rs);
 }
@@ -98,6 +101,7 @@ constexpr int TBY = 16;
 // coefficient it formed in kmax, from which the host chooses the diffusion
 // sweep.  A NaN (unstable stratification at rest: Ri = -inf) stays one.
 __global__ void __launch_bounds__(BX *TBY) k_turb_coeffs(Grid G, StepPtrs S, double *kmax) {
+    note_start(S.clock, CLK_TURB);
     const int tx = (G.nx - 2 + BX - 1) / BX, nt = tx * ((G.nz - 2 + TBY - 1) / TBY);
     double m = 0.;
     for (int t = blockIdx.x; t < nt; t += gridDim.x) {
@@ -135,6 +139,7 @@ __global__ void __launch_bounds__(BX *BY) k_nudge_qv(Grid G, StepPtrs S, double 
 // nextTimeStep: one block per level.  thb_zeta is not read by the step and
 // is formed on download.
 __global__ void __launch_bounds__(256) k_update_mean(Grid G, StepPtrs S, MeanMode mode) {
+    note_start(S.clock, CLK_MEAN);
     const int k = blockIdx.x + 1;
     const double *thp = S.fut[F_TH], *qvp = S.fut[F_QV];
     double acc[2] = {0., 0.};

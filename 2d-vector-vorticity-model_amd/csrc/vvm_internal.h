@@ -60,7 +60,12 @@ struct StepPtrs {
     unsigned long long *dslots;
     int dstrip_cw;  // compute wavefronts per strip of that sweep (0: default)
     double *sweep_err;  // host-mapped: set to 1 if one of its waves gave up waiting
+    long long *clock;   // host-mapped, [CLK_N]: where kernels note the time; nullptr: nowhere
 };
+
+// The phase boundaries of a step whose kernels note them (StepPtrs::clock).
+enum { CLK_ADVECT = 0, CLK_SOLVE, CLK_MICRO, CLK_MICRO_END, CLK_TURB, CLK_MEAN, CLK_N };
+
 
 struct Reductions {
     RedSlot negval;  // 6 sums: P,N for qv, qc, qr
@@ -87,6 +92,7 @@ Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot 
 // launch_pzeta and launch_thermo4 in one launch; whether that is the faster way
 bool advect_together(const Grid &G);
 Negval launch_advect(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);
+int advect_tiles(const Grid &G);  // thermo4's, and its partials
 Negval negval_partials(const StepPtrs &S, const Negval &nv, hipStream_t st);
 void launch_scale_forcing(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, hipStream_t st,
                           bool halos = true);
