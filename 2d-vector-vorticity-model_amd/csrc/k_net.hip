@@ -92,10 +92,14 @@ __device__ inline long halo_src(const NetGeo &g, int b, int y0, int x0, int ry, 
 // (66 x FTH+2)-pixel haloed input staged in LDS; a tile holds 2 FTH MFMA
 // output blocks of 32 channels x 32 pixels, FTH / 2 per wavefront, and a
 // wavefront applies each weight fragment to all of its blocks.  The
-// workgroups stay resident and walk the tiles with a stride of the grid:
-// a lane loads its 18 weight fragments once, and the next tile's input is
+// workgroups stay resident and walk the tiles with a stride of the grid: the
+// 18 weight fragments are loaded once, and the next tile's input is
 // fetched into registers while the current tile's products run, so neither
 // the weights' nor the input's memory latency sits between two tiles.
+// Two-row tiles (FTH 2) are bound by latency, and their one block a wavefront
+// uses a fragment once a tile: they keep the weights in LDS, which leaves
+// registers for four workgroups a CU, where with the weights in registers there
+// were two.  A hidden layer at 1024 x 127: 8.6 us, 10.2 before.
 template <int MODE, int IN = 0, int FTH = 4>
 __global__ void __launch_bounds__(256) k_conv(NetGeo g, const __bf16 *__restrict__ in,
                                               const bf16x8 *__restrict__ wpk, const float *__restrict__ bias,
@@ -113,10 +117,18 @@ __global__ void __launch_bounds__(256) k_conv(NetGeo g, const __bf16 *__restrict
     const int i = lane & 31, gk = lane >> 5;
     // IN 1: channels 3..31 of the input are zero, so the steps over input
     // channels 16..31 (odd s) add nothing and are skipped
-    bf16x8 wr[18];
+    constexpr bool WLDS = FTH == 2;
+    __shared__ bf16x8 wl[WLDS ? 18 * 64 : 1];
+    bf16x8 wr[18];  // WLDS: this thread's part of wl on its way there
+    constexpr int NW = (18 * 64 + 255) / 256;
+    if constexpr (WLDS) {
 #pragma unroll
-    for (int s = 0; s < 18; s++)
-        if (IN == 0 || (s & 1) == 0) wr[s] = wpk[s * 64 + lane];
+        for (int k = 0; k < NW; k++) wr[k] = wpk[min(int(threadIdx.x) + 256 * k, 18 * 64 - 1)];
+    } else {
+#pragma unroll
+        for (int s = 0; s < 18; s++)
+            if (IN == 0 || (s & 1) == 0) wr[s] = wpk[s * 64 + lane];
+    }
     float bv[16];
     if (MODE == 0) {
 #pragma unroll
@@ -170,6 +182,11 @@ __global__ void __launch_bounds__(256) k_conv(NetGeo g, const __bf16 *__restrict
     };
     int t = blockIdx.x;
     if (t < ntile) fetch(t);
+    if constexpr (WLDS) {
+#pragma unroll
+        for (int k = 0; k < NW; k++)
+            if (int(threadIdx.x) + 256 * k < 18 * 64) wl[threadIdx.x + 256 * k] = wr[k];
+    }
     for (; t < ntile; t += gridDim.x) {
         const int b = t / (gx * gy), y0 = (t / gx) % gy * FTH, x0 = t % gx * FTW;
         __syncthreads();  // the previous tile's reads of the LDS tile are done
@@ -187,7 +204,8 @@ __global__ void __launch_bounds__(256) k_conv(NetGeo g, const __bf16 *__restrict
                 const int gq = BPW * wv + q, ty = gq >> 1, cb = (gq & 1) * 32;
                 const int px = (ty + 1 + dy) * FHW + (cb + i + 1 + dx);
                 const bf16x8 a = *reinterpret_cast<const bf16x8 *>(tile + px * PXS + hh * 16 + gk * 8);
-                acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wr[s], a, acc[q], 0, 0, 0);
+                const bf16x8 wv8 = WLDS ? wl[s * 64 + lane] : wr[s];
+                acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv8, a, acc[q], 0, 0, 0);
             }
         }
         // weights as the A operand, pixels as B: D[m][n] with n = lane % 32
