@@ -558,7 +558,7 @@ __global__ void __launch_bounds__((CW + 1) * kWave) k_diff_strips(Grid G, StepPt
 // scalars in one wavefront, which the instruction count bound) and leave twice
 // the wavefronts of four.
 //
-// 2048 x 256, FP64: 20 us (H = 8) against 122 us for k_diff_coeffs and
+// 2048 x 256, FP64: 18 to 20 us (H = 8) against 122 us for k_diff_coeffs and
 // k_diff_strips, whose time is 256 rows one after another.
 constexpr int TROWS = 8;
 constexpr int TWAVES = 4;

@@ -5,7 +5,7 @@
 // zeros at k = 1 and k = nz-1.  Row (i,k) of A divided by rhow[k] is
 //   -L x = cx_k (x_{i-1} - 2 x_i + x_{i+1}) + cu_k (x_{k+1} - x_k) - cu_{k-1} (x_k - x_{k-1})
 // with cx_k = 1/rhow[k] and cu_k = 1/rhou[k]: L is symmetric positive
-// definite, so the solve is preconditioned CG on L x = f, f = -b / rhow.
+// definite; the solve is of L x = f, f = -b / rhow.
 // The true residual of the reference system is ||b - A x|| = ||rhow r||.
 //
 // Unknown arrays are (M+2) rows x N columns, x-contiguous, rows 0 and M+1

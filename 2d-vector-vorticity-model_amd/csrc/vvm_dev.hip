@@ -303,7 +303,7 @@ LevelConstants level_constants(vvm_dev *h, const vvm_host_view *v) {
 
 // FP64 from a guess: MG-PCG, whose iteration count tells what the guess is
 // worth.  Everything else but BiCGSTAB is solved directly, which takes no
-// guess.  A step's cal_w and cal_u at 2048 x 256: 95 us, against 870 us with
+// guess.  A step's cal_w and cal_u at 2048 x 256: 60 us, against 870 us with
 // FP64 MG-PCG from zero and 480 us with FP32 MG-PCG in FP64 refinement from
 // the quadratic extrapolation; columns that cannot be halved (317 x 61): 0.1
 // against 13 ms.

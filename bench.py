@@ -7,13 +7,14 @@ over the config-2 grid (2048 x 256 interior, dx = dz = 100 m, dt = 1 s,
 Gaussian theta noise, 100 W/m^2 surface heat flux, qv surface ramp), state
 resident in HBM.  The solve stops at ||b - A x|| / ||b|| <= 1e-10.
 
-Three paths are timed:
-  fp64_plain     -- FP64 MG-PCG from a zero guess (the reference's guess);
-  mixed          -- FP32 MG-PCG inside FP64 refinement from the linear
-                    extrapolation of the last two solutions;
-  mixed_quadratic -- the same solver from the quadratic extrapolation of
-                    the last three solutions;
-  mixed_learned  -- the same solver from the conv-net correction of the
+Four solver settings are timed.  A step's solve is an FP64 direct one in all of
+them, so that they differ only in the network's work (solve_iters counts direct
+solves, one a step):
+  fp64_plain     -- VVM_SOLVER_FP64;
+  mixed          -- VVM_SOLVER_MIXED with the linear extrapolation;
+  mixed_quadratic -- the same with the quadratic extrapolation of the last
+                    three solutions;
+  mixed_learned  -- the same with the conv-net correction of the
                     quadratic extrapolation, whose weights come from --net or
                     are trained here first (untimed) on samples the model
                     records from 1024x128 runs; a guess that starts worse
@@ -55,28 +56,25 @@ KERNEL_BYTES_PER_POINT = {
 
 
 # Algorithmic bytes of a whole step (the same rule): the non-solver kernels
-# above plus the solve, per PCG iteration and unknown ~220 B in FP64 (CG
-# vectors 88 B + a V(2,2) cycle ~4/3 x 100 B) and ~110 B in FP32, plus
-# ~100 B per unknown for each FP64 refinement (residual, conversion,
-# correction).
-STEP_NONSOLVER_BYTES_PER_POINT = sum(KERNEL_BYTES_PER_POINT.values()) + 64.0  # the second scale pass
-SOLVER_BYTES_PER_ITER = {"f64": 220.0, "f32": 110.0}
-REFINE_BYTES = 100.0
+# above plus, per direct solve and unknown in FP64, the transforms (zetap read, f
+# and spectrum written; spectrum read, x and w written), the elimination
+# (spectrum and pivots read, spectrum written) and the residual (f, x read).
+STEP_NONSOLVER_BYTES_PER_POINT = sum(KERNEL_BYTES_PER_POINT.values())
+SOLVE_BYTES = 88.0
 
 
-def step_roofline(ms_per_step: float, iters: float, refine: float, fp32: bool, pts: int, unknowns: int) -> dict:
+def step_roofline(ms_per_step: float, iters: float, pts: int, unknowns: int) -> dict:
     """The whole step as a fraction of HBM peak, from algorithmic bytes."""
-    per_iter = SOLVER_BYTES_PER_ITER["f32" if fp32 else "f64"]
-    b = STEP_NONSOLVER_BYTES_PER_POINT * pts + (iters * per_iter + refine * REFINE_BYTES) * unknowns
+    b = STEP_NONSOLVER_BYTES_PER_POINT * pts + iters * SOLVE_BYTES * unknowns
     gbs = b / (ms_per_step * 1e-3) / 1e9
     return {"bytes_per_step": b, "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS}
 
 
 # kernels behind each timed phase (rows of the committed traffic table)
 KERNEL_NAMES = {
-    "diffusion": ["k_diff_coeffs", "k_diff_strips"], "thermo4": ["k_thermo4"], "pzeta": ["k_pzeta"],
+    "diffusion": ["k_diff_tiles"], "thermo4": ["k_thermo4"], "pzeta": ["k_pzeta"],
     "kessler": ["k_kessler"], "scale": ["k_scale_forcing"], "turb": ["k_turb_coeffs"], "mean": ["k_update_mean"],
-    "calu": ["k_calu_top", "k_calu_cols"],
+    "calu": ["k_calu"],
 }
 TRAFFIC_TABLE = os.path.join(ROOT, "profiles", "hbm_traffic_2048x256.md")
 
@@ -224,9 +222,8 @@ def calw_rhs(cfg, rhow: np.ndarray, zeta: np.ndarray) -> np.ndarray:
 def solve_bench(nfields: int = 3) -> dict:
     """The isolated elliptic solve on seeded k^-3 vorticity fields at
     2048x256: iterations and device time to ||b - A x|| / ||b|| <= 1e-10 of
-    FP64 MG-PCG and of FP32 MG-PCG in FP64 refinement (both from a zero
-    guess: a lone solve has no previous solutions to extrapolate or feed the
-    network), the mixed solution's error against the FP64 solution iterated
+    the FP64 direct solve and of FP32 direct solves in FP64 refinement (both
+    from a zero guess), the mixed solution's error against the FP64 solution iterated
     until its residual stops falling, and the reference's Eigen BiCGSTAB +
     ILUT iterations at the same 1e-10 (oracle/_ref, one thread) where that
     binary is present."""
@@ -341,7 +338,7 @@ def ensemble_bench(steps: int, net_path: str | None, seed: int = 4) -> dict:
     return {
         "metric": "ensemble grid-point-steps/s (64 uneven members, mixed precision)",
         "value": out["mixed"]["value"], "unit": "grid-point-steps/s", "n_gpus": 1, "steps": steps,
-        "higher_is_better": True, "dtype": "f64+f32", "data": "synthetic",
+        "higher_is_better": True, "dtype": "f64", "data": "synthetic",
         "config": {"workload": "config 4: 64 members, nx in {256,512,1024,2048}, nz in {64,128,256}, "
                                "dx=dz=100 m", "grid_points_total": pts,
                    "guess": "learned" if net_path else "quadratic extrapolation"},
@@ -412,8 +409,8 @@ def main():
             "kernel_avg_us": 1e6 * kavg, "kernel_launches": kn,
         }
         results[name]["step_roofline"] = step_roofline(
-            results[name]["ms_per_step"], results[name]["solve_iters_per_step"], float(stats.refine_last),
-            paths[name]["solver_mode"] == V.VVM_SOLVER_MIXED, pts, (base.cfg.nx - 2) * (base.cfg.nz - 3))
+            results[name]["ms_per_step"], results[name]["solve_iters_per_step"], pts,
+            (base.cfg.nx - 2) * (base.cfg.nz - 3))
         log(f"[bench] {name}: {results[name]['value']:.4g} grid-point-steps/s, "
             f"{results[name]['ms_per_step']:.3f} ms/step, {results[name]['solve_iters_per_step']:.2f} iters/step")
 
@@ -425,7 +422,7 @@ def main():
         "metric": "grid-point-steps/s at 2048x256, FP64 plain vs mixed+learned; Poisson iters to 1e-10",
         "value": R["value"], "unit": "grid-point-steps/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": R["ms_per_step"], "higher_is_better": True, "scaling": "weak",
-        "vs_baseline": None, "dtype": "f64+f32", "data": "synthetic",
+        "vs_baseline": None, "dtype": "f64", "data": "synthetic",
         "config": {"workload": "config 2: 2048x256 interior, dx=dz=100 m, dt=1 s, Kessler, sigma=0.1 K theta "
                                "noise < 500 m, 100 W/m^2 surface heat flux, qv surface ramp; solve to 1e-10",
                    "grid_points": pts, "path": head},

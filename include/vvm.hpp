@@ -170,7 +170,7 @@ class vvm {
     // step's fields in the [i][k] layout (see vvm_dev_set_host_microphysics)
     // and takes back thp, qvp, qcp, qrp and the process rates; it returns 0.
     std::function<int(vvm_host_view &)> host_microphysics;
-    long long solve_iters_total = 0;   // PCG iterations over the run
+    long long solve_iters_total = 0;   // direct solves (or PCG iterations) over the run
     vvm_host_view host_view();          // pointers into this model's arrays
     void sync_to_device();              // upload when dev_stale
     void sync_to_host();                // download when host_stale

@@ -33,7 +33,7 @@ typedef struct vvm_ens_member {
 typedef struct vvm_ens_stats {
     double seconds;             /* wall time of the call                   */
     double grid_point_steps;    /* sum over members of interior points x steps */
-    int64_t solve_iters_total;  /* PCG iterations over all members         */
+    int64_t solve_iters_total;  /* direct solves (or PCG iterations), all  */
     int32_t not_converged;      /* solves that missed their stop rule      */
     int32_t members;
 } vvm_ens_stats;

@@ -9,9 +9,9 @@
  * from three features of the unknown grid: the residual of the extrapolated
  * guess, the last solution increment x_{t-1} - x_{t-2}, and the
  * extrapolated guess itself, each scaled by its RMS.  The output is scaled
- * by RMS(x_{t-1} - x_{t-2}).  The solver still iterates to its stop rule
- * from that guess, so the network changes the iteration count, never the
- * stopping criterion.
+ * by RMS(x_{t-1} - x_{t-2}).  A step corrects that guess by a direct solve of
+ * its residual; the FP64 solver with a guess mode iterates from it.  Either
+ * meets its stop rule, whatever the guess.
  *
  * Parameters are one fp32 array of vvm_net_param_count() values: for each
  * layer l = 1..6, W_l[co][ci][t] (32 x 32 x 9, tap t = 3 (dz+1) + (dx+1))
