@@ -707,8 +707,8 @@ inline std::complex<long double> root(long long k, long long n) {
     const long double a = 2.0L * 3.14159265358979323846264338327950288L * (k % n) / n;
     return {std::cos(a), -std::sin(a)};
 }
-// in place, forward, n a power of two
-void host_fft(std::vector<std::complex<long double>> &v) {
+// in place, forward, n a power of two; w: the n roots
+void host_fft(std::vector<std::complex<long double>> &v, const std::vector<std::complex<long double>> &w) {
     const size_t n = v.size();
     for (size_t i = 1, j = 0; i < n; i++) {
         size_t bit = n >> 1;
@@ -716,12 +716,13 @@ void host_fft(std::vector<std::complex<long double>> &v) {
         j ^= bit;
         if (i < j) std::swap(v[i], v[j]);
     }
-    std::vector<std::complex<long double>> w(n / 2 + 1);
-    for (size_t k = 0; k < w.size(); k++) w[k] = root((long long)k, (long long)n);
     for (size_t len = 2; len <= n; len *= 2)
         for (size_t i = 0; i < n; i += len)
             for (size_t k = 0; k < len / 2; k++) {
-                const auto a = v[i + k], b = v[i + k + len / 2] * w[k * (n / len)];
+                const auto a = v[i + k], c = v[i + k + len / 2], r = w[k * (n / len)];
+                // spelled out: std::complex's product checks for infinities
+                const std::complex<long double> b(c.real() * r.real() - c.imag() * r.imag(),
+                                                  c.real() * r.imag() + c.imag() * r.real());
                 v[i + k] = a + b;
                 v[i + k + len / 2] = a - b;
             }
@@ -796,10 +797,11 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
         return VVM_ERR_NOMEM;
     }
     std::vector<T> t(4 * size_t(L), T(0));
+    std::vector<std::complex<long double>> roots(L);
     for (int k = 0; k < L; k++) {
-        const auto c = root(k, L);
-        t[2 * k] = T(c.real());
-        t[2 * k + 1] = T(c.imag());
+        roots[k] = root(k, L);
+        t[2 * k] = T(roots[k].real());
+        t[2 * k + 1] = T(roots[k].imag());
     }
     // the stages' twiddles, picked from those (r k < Ns R, so r k L / (Ns R) < L)
     for (int s = 0, Ns = 1; s < plan.nst; Ns *= plan.radix[s++]) {
@@ -820,7 +822,7 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
             ch[2 * k + 1] = T(c.imag());
             b[k] = b[(L - k) % L] = std::conj(c);
         }
-        host_fft(b);
+        host_fft(b, roots);
         for (int k = 0; k < L; k++) {
             ch[2 * size_t(N + k)] = T(b[k].real() / L);
             ch[2 * size_t(N + k) + 1] = T(b[k].imag() / L);
