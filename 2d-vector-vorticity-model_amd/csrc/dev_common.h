@@ -81,6 +81,18 @@ __device__ inline void note_end(long long *clock, int slot) {
     if (clock && blockIdx.x == gridDim.x - 1 && blockIdx.y == gridDim.y - 1) note_time(clock, slot);
 }
 
+// A plane's value that the step does not touch again, past the caches if PAST.
+template <bool PAST>
+__device__ inline double load_once(const double &a) {
+    if constexpr (PAST) return __builtin_nontemporal_load(&a);
+    else return a;
+}
+template <bool PAST>
+__device__ inline void store_once(double &a, double v) {
+    if constexpr (PAST) __builtin_nontemporal_store(v, &a);
+    else a = v;
+}
+
 // ---------------------------------------------------------------- sums
 
 constexpr int kWave = 64;

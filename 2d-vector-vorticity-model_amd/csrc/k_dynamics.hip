@@ -103,15 +103,16 @@ __device__ inline double thv(const Grid &G, const double *th, const double *qv, 
 
 // AB2 update of one history slot: writes d to slot sn (and to slot 0 on the
 // reference's step-0 start, Advection.cpp:70) and returns the old slot.
+template <bool PAST = false>
 __device__ inline double ab2_hist(double *const (&h)[2], const Grid &G, int i, int k, int step, double d) {
     // the slot pointers are picked by selects, not by a run-time index into
     // the kernel-argument array (which would read them through generic
     // memory accesses)
     const bool odd = (step & 1) != 0;
     double *const hn = odd ? h[0] : h[1], *const ho = odd ? h[1] : h[0];
-    at(hn, G, i, k) = d;
+    store_once<PAST>(at(hn, G, i, k), d);
     if (step == 0) at(h[0], G, i, k) = d;
-    return at(ho, G, i, k);
+    return load_once<PAST>(at(ho, G, i, k));
 }
 
 // ------------------------------------------------------------------ zeta
@@ -137,7 +138,7 @@ struct PzLds {
     double Fx[PZY][PZX + 1];  // slot c: x-flux east of column i0 + c - 1
     double Fz[PZY + 1][PZX];  // slot r: z-flux above row k0 + r - 1
 };
-template <int PARTS>
+template <int PARTS, bool PAST>
 __device__ inline void pzeta_tile(const Grid &G, const StepPtrs &S, int step, int tile, PzLds &lds) {
     auto &Fx = lds.Fx;
     auto &Fz = lds.Fz;
@@ -183,7 +184,7 @@ __device__ inline void pzeta_tile(const Grid &G, const StepPtrs &S, int step, in
         const double px = (fu0 - fum) * G.r2dx / rhow[k];
         const double pz = (fw0 - fwm) * G.r2dz / rhow[k];
         const double dadv = -px - pz;
-        const double dold = ab2_hist(S.hist[H_ZETA_ADV], G, i, k, step, dadv);
+        const double dold = ab2_hist<PAST>(S.hist[H_ZETA_ADV], G, i, k, step, dadv);
         zeta_new = at(z, G, i, k) + 1.5 * G.dt * dadv - 0.5 * G.dt * dold;
         if constexpr (PARTS == PZ_ADV) {
             at(zp, G, i, k) = zeta_new;
@@ -206,17 +207,17 @@ __device__ inline void pzeta_tile(const Grid &G, const StepPtrs &S, int step, in
                        G.rdx;
     double db = gth;
     db += -gqc - gqr;
-    const double bold = ab2_hist(S.hist[H_TH_BUOY], G, i, k, step, db);
+    const double bold = ab2_hist<PAST>(S.hist[H_TH_BUOY], G, i, k, step, db);
     zeta_new += (1.5 * G.dt * db) - (0.5 * G.dt * bold);
     if constexpr (PARTS == PZ_BOTH) store_westdown(zp, G, i, k, zeta_new);
     else at(zp, G, i, k) = zeta_new;
 }
-template <int PARTS>
+template <int PARTS, bool PAST = false>
 __global__ void __launch_bounds__(PZX *PZY) k_pzeta(Grid G, StepPtrs S, int step) {
     note_start(S.clock, CLK_ADVECT);
     __shared__ PzLds lds;
     const int nt = pz_tiles_x(G) * pz_tiles_z(G), tile = xcd_tile(nt);
-    if (tile < nt) pzeta_tile<PARTS>(G, S, step, tile, lds);
+    if (tile < nt) pzeta_tile<PARTS, PAST>(G, S, step, tile, lds);
 }
 
 // ----------------------------------------------------------- scalars
@@ -312,6 +313,7 @@ struct T4Lds {
     double Fx[4][T4Y][T4X + 1];  // x-face flux at faces i0 .. i0+T4X (west faces)
     double Fz[5][T4Y + 1][T4X];  // z-face flux (4 fields, rain fall) at faces k0 .. k0+T4Y
 };
+template <bool PAST>
 __device__ inline void thermo4_tile(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, int tile, T4Lds &lds) {
     auto &Fx = lds.Fx;
     auto &Fz = lds.Fz;
@@ -372,7 +374,7 @@ __device__ inline void thermo4_tile(const Grid &G, const StepPtrs &S, int step, 
             const double px = (fu1 - fu0) * G.r2dx / rhou[k];
             const double pz = (fw1 - fw0) * G.r2dz / rhou[k];
             const double d = -px - pz;
-            const double dold = ab2_hist(S.hist[hid[q]], G, i, k, step, d);
+            const double dold = ab2_hist<PAST>(S.hist[hid[q]], G, i, k, step, d);
             double v = at(fl[q], G, i, k) + 1.5 * G.dt * d - 0.5 * G.dt * dold;
             if (q == 0) {
                 at(S.fut[F_TH], G, i, k) = v;
@@ -382,7 +384,7 @@ __device__ inline void thermo4_tile(const Grid &G, const StepPtrs &S, int step, 
                 const double f1 = top ? 0. : Fz[4][ty + 1][tx];
                 const double f0 = Fz[4][ty][tx];
                 const double dvt = (f1 - f0) * G.r2dz / rhou[k];
-                const double vold = ab2_hist(S.hist[H_QR_VT], G, i, k, step, dvt);
+                const double vold = ab2_hist<PAST>(S.hist[H_QR_VT], G, i, k, step, dvt);
                 v += 1.5 * G.dt * dvt - 0.5 * G.dt * vold;
             }
             if (v >= 0.) part[2 * (q - 1)] += v;
@@ -405,11 +407,12 @@ __device__ inline void thermo4_tile(const Grid &G, const StepPtrs &S, int step, 
 }
 // Four workgroups a CU (the LDS allows four), so that 1024 of them cover
 // 2048 x 256 in one round: eight waves a SIMD, at most 64 VGPRs.
+template <bool PAST>
 __global__ void __launch_bounds__(T4X *T4Y) __attribute__((amdgpu_waves_per_eu(8)))
 k_thermo4(Grid G, StepPtrs S, int step, RedSlot rs) {
     __shared__ T4Lds lds;
     const int nt = t4_tiles_x(G) * t4_tiles_z(G), tile = xcd_tile(nt);
-    if (tile < nt) thermo4_tile(G, S, step, rs, tile, lds);
+    if (tile < nt) thermo4_tile<PAST>(G, S, step, rs, tile, lds);
 }
 
 // Both in one launch, a tile of each in turn: neither reads what the other
@@ -424,8 +427,8 @@ k_advect(Grid G, StepPtrs S, int step, RedSlot rs) {
     note_start(S.clock, CLK_ADVECT);
     const int nt = t4_tiles_x(G) * t4_tiles_z(G), slot = xcd_tile(2 * nt), tile = slot / 2;
     if (slot >= 2 * nt) return;
-    if (slot % 2 == 0) thermo4_tile(G, S, step, rs, tile, lds.t4);
-    else if (tile < pz_tiles_x(G) * pz_tiles_z(G)) pzeta_tile<PZ_BOTH>(G, S, step, tile, lds.pz);
+    if (slot % 2 == 0) thermo4_tile<false>(G, S, step, rs, tile, lds.t4);
+    else if (tile < pz_tiles_x(G) * pz_tiles_z(G)) pzeta_tile<PZ_BOTH, false>(G, S, step, tile, lds.pz);
 }
 
 __global__ void __launch_bounds__(BX *BY) k_scale_forcing(Grid G, StepPtrs S, Negval nv, Forcing F, int halos) {
@@ -531,7 +534,8 @@ inline dim3 interior_grid(const Grid &G) { return dim3((G.nx - 2 + BX - 1) / BX,
 
 void launch_pzeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st) {
     const dim3 g = xcd_grid(pz_tiles_x(G) * pz_tiles_z(G));
-    hipLaunchKernelGGL(k_pzeta<PZ_BOTH>, g, dim3(PZX, PZY), 0, st, G, S, step);
+    if (past_caches(G)) hipLaunchKernelGGL((k_pzeta<PZ_BOTH, true>), g, dim3(PZX, PZY), 0, st, G, S, step);
+    else hipLaunchKernelGGL((k_pzeta<PZ_BOTH, false>), g, dim3(PZX, PZY), 0, st, G, S, step);
 }
 void launch_advection_zeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st) {
     const dim3 g = xcd_grid(pz_tiles_x(G) * pz_tiles_z(G));
@@ -555,7 +559,8 @@ void launch_bc_one(const Grid &G, double *a, bool westdown, hipStream_t st) {
 }
 Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
     const int n = advect_tiles(G);
-    hipLaunchKernelGGL(k_thermo4, xcd_grid(n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
+    if (past_caches(G)) hipLaunchKernelGGL(k_thermo4<true>, xcd_grid(n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
+    else hipLaunchKernelGGL(k_thermo4<false>, xcd_grid(n), dim3(T4X, T4Y), 0, st, G, S, step, rs);
     return {rs, n};
 }
 int advect_tiles(const Grid &G) { return t4_tiles_x(G) * t4_tiles_z(G); }

@@ -188,7 +188,10 @@ Negval launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipSt
 }
 Negval launch_kessler(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, const RedSlot &rs,
                       hipStream_t st) {
-    hipLaunchKernelGGL((k_kessler<KP_ALL | KP_PRE>), interior_grid(G), dim3(BX, BY), 0, st, G, S, nv, F, rs);
+    if (past_caches(G))
+        hipLaunchKernelGGL((k_kessler<KP_ALL | KP_PRE | KP_PAST>), interior_grid(G), dim3(BX, BY), 0, st, G, S, nv, F, rs);
+    else
+        hipLaunchKernelGGL((k_kessler<KP_ALL | KP_PRE>), interior_grid(G), dim3(BX, BY), 0, st, G, S, nv, F, rs);
     return {rs, nblocks(interior_grid(G))};
 }
 void launch_kessler_process(const Grid &G, const StepPtrs &S, int process, hipStream_t st) {

@@ -59,7 +59,8 @@ __device__ inline double mins(double a, double b) { return (b < a) ? b : a; }
 // launch and one pass over four fields less, 9 us at 2048 x 256 between the
 // advection and the solve: 20 steps there go 4948 -> 4806 us,
 // 4096 x 256 8177 -> 7850.
-enum { KP_AUTO = 1, KP_ACCR = 2, KP_EVAP = 4, KP_COND = 8, KP_NEG = 16, KP_ALL = 31, KP_PRE = 32 };
+// KP_PAST: the rates are written past the caches (past_caches).
+enum { KP_AUTO = 1, KP_ACCR = 2, KP_EVAP = 4, KP_COND = 8, KP_NEG = 16, KP_ALL = 31, KP_PRE = 32, KP_PAST = 64 };
 
 template <int PROC>
 __device__ inline void kessler_point(const Grid &G, const StepPtrs &S, const Forcing &F, const double (&ratios)[3],
@@ -80,7 +81,7 @@ __device__ inline void kessler_point(const Grid &G, const StepPtrs &S, const For
                 const double arcrdt = mins(ar * dt, qcplus);
                 qc = qc - arcrdt;
                 qr = qr + arcrdt;
-                at(S.autoc, G, i, k) = arcrdt;
+                store_once<(PROC & KP_PAST) != 0>(at(S.autoc, G, i, k), arcrdt);
             }
             if constexpr ((PROC & KP_ACCR) != 0) {  // accretion
                 const double qcplus = maxs(0., qc), qrplus = maxs(0., qr);
@@ -89,7 +90,7 @@ __device__ inline void kessler_point(const Grid &G, const StepPtrs &S, const For
                 const double arcrdt = mins(cr * dt, qcplus);
                 qc = qc - arcrdt;
                 qr = qr + arcrdt;
-                at(S.accr, G, i, k) = arcrdt;
+                store_once<(PROC & KP_PAST) != 0>(at(S.accr, G, i, k), arcrdt);
             }
             if constexpr ((PROC & KP_EVAP) != 0) {  // rain evaporation
                 const double qrplus = maxs(0., qr), qvplus = maxs(0., qv);
@@ -105,7 +106,7 @@ __device__ inline void kessler_point(const Grid &G, const StepPtrs &S, const For
                 qr = qr - erdt;
                 qv = qv + erdt;
                 th = th - G.Lv * erdt / (G.Cp * pib);
-                at(S.evap, G, i, k) = erdt;
+                store_once<(PROC & KP_PAST) != 0>(at(S.evap, G, i, k), erdt);
             }
             if constexpr ((PROC & KP_COND) != 0) {  // saturation adjustment
                 const double qvs = pc * exp(17.27 * (pib * th - 273.) / (pib * th - 36.));
@@ -116,7 +117,7 @@ __device__ inline void kessler_point(const Grid &G, const StepPtrs &S, const For
                 qv = qv - C;
                 qc = qc + C;
                 th = th + G.Lv / (G.Cp * pib) * C;
-                at(S.cond, G, i, k) = C;
+                store_once<(PROC & KP_PAST) != 0>(at(S.cond, G, i, k), C);
             }
             double q3[3] = {qv, qc, qr};
             if constexpr ((PROC & KP_NEG) != 0) {

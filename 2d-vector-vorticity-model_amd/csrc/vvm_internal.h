@@ -89,6 +89,14 @@ struct Forcing {
     int on, tropical, random_kick;
 };
 Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);
+// Whether the planes that a step touches once (the old and new tendencies, the
+// microphysics' rates) are read and written past the caches: where the 42
+// planes of the state (15 time levels, 14 tendencies, u, w, K, the rates, the
+// sweep's) are more than the 256 MB last-level cache, which they would push the
+// rest out of.  A step in us, past / through them: 2816 x 256 (250 MB) 209 / 208,
+// 3072 x 256 (273) 198 / 204, 4096 x 256 234 / 251, 8192 x 256 454 / 481; through
+// a shared launch at 2048 x 256 (the tendencies alone) 153 / 141.
+inline bool past_caches(const Grid &G) { return 42. * sizeof(double) * G.pitch * G.nz > 256. * 1048576; }
 // launch_pzeta and launch_thermo4 in one launch; whether that is the faster way
 bool advect_together(const Grid &G);
 Negval launch_advect(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st);

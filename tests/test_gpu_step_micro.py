@@ -5,7 +5,8 @@ Grids whose 64 x 4 tiles (Kessler) and 64 x 8 tiles (advection) are full, have
 one column and row more, and are both, one, or none at most 640, up to which
 the ratios come from the producer's partial sums instead of k_finalize; and one
 row and column past 1024 of the latter, up to which the vorticity's advection
-shares their launch (the operators have one each).  One
+shares their launch (the operators have one each); and 4096 x 200, whose rates
+are written past the caches.  One
 step with every kind of forcing, negative cloud and a few points of negative
 rain (whose fall speed is NaN), against the same phases as separate operators.
 The microphysics' rates come straight from that kernel and have to be the same
@@ -26,7 +27,7 @@ RATES = ["evaporation", "accretion", "autoconversion", "condensation", "precip"]
 
 
 @pytest.mark.parametrize("nx,nz", [(64, 8), (65, 9), (66, 10), (67, 11), (63, 19), (1100, 150), (2100, 170), (2048, 256),
-                                   (2049, 257)])
+                                   (2049, 257), (4096, 200)])
 @pytest.mark.parametrize("forced", [False, True])
 def test_step_forcing_and_kessler(nx, nz, forced):
     kw = dict(tropical_forcing=1, addforcingtime=10.0) if forced else {}
