@@ -943,10 +943,12 @@ SolveResult Poisson::solve_fp64(double tol, int max_iter, hipStream_t st) {
     return R;
 }
 
-// Relative residual below which one that no longer decreases counts as FP64's
-// round-off.  A direct solve leaves 1e-16 to 1e-14 on the model's right-hand
-// sides; the bound is the condition number's worth above that.
-constexpr double kRoundOff = 1e-12;
+// Relative residual up to which one that no longer decreases counts as FP64's
+// round-off: 2^-53 times the largest condition number, 8 (M + 1)^2 / pi^2 times
+// the density's range over the column, 4e-10 at 480 levels.  The round-off of
+// L x itself is 1e-16 of ||b|| where b is rough, 3e-14 on k^-3 vorticity and
+// 1e-12 on the lowest mode (2048 x 256).
+constexpr double kRoundOff = 1e-9;
 
 // Norms of the residual kernel's slot (the caller has waited for it).
 void Poisson::norms(int slot, double *rn2, double *bn2) const {
