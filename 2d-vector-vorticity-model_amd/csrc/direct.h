@@ -41,6 +41,9 @@ class Direct {
     // x = L^-1 r on rows 1..M of (M+2) x N arrays, or x0 + L^-1 r if x0 is set
     // (which may be x).
     void solve(const double *r, const double *x0, double *x, hipStream_t st);
+    // x = x0 + L^-1 r, and w = x / rhow with its halos.
+    void solve_w(const double *r, const double *x0, double *x, const Grid &G, double *w, const double *rhow,
+                 hipStream_t st);
     // cal_w whole: f = -b / rhow from zetap (f is written, for the residual),
     // x = L^-1 f, w = x / rhow with its halos; pubarTop_pt beside the first
     // kernel's row transforms (step < 0: not), and the microphysics (if set)
@@ -57,7 +60,8 @@ class Direct {
     const double *cu_dev = nullptr;
     T *spec = nullptr;  // [M][N] transformed rows
     template <bool C>
-    void rows_solve(const double *r, const double *x0, double *x, hipStream_t st);
+    void rows_solve(const double *r, const double *x0, double *x, const Grid &G, double *w, const double *rhow,
+                    hipStream_t st);
     template <bool C>
     void rows_solve_step(const Grid &G, const StepPtrs &S, int step, const Micro *micro, double *f, double *x,
                          hipStream_t st);

@@ -782,7 +782,7 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
         constexpr bool C = decltype(chirp)::value;
         ok = ok && allow_lds(k_rows_fwd<T, false, C>, row_lds) && allow_lds(k_rows_fwd<T, true, C>, row_lds) &&
              allow_lds(k_rows_inv<T, false, false, C>, row_lds) && allow_lds(k_rows_inv<T, true, false, C>, row_lds) &&
-             allow_lds(k_rows_inv<T, false, true, C>, row_lds);
+             allow_lds(k_rows_inv<T, false, true, C>, row_lds) && allow_lds(k_rows_inv<T, true, true, C>, row_lds);
     };
     if (plan.chirp) allow_rows(std::true_type());
     else allow_rows(std::false_type());
@@ -852,22 +852,31 @@ void Direct<T>::columns(const Mic &mic, int nmic, hipStream_t st) {
 
 template <typename T>
 template <bool C>
-void Direct<T>::rows_solve(const double *r, const double *x0, double *x, hipStream_t st) {
+void Direct<T>::rows_solve(const double *r, const double *x0, double *x, const Grid &G, double *w, const double *rhow,
+                           hipStream_t st) {
     const dim3 gr((plan.M + 1) / 2), b(plan.threads);
     hipLaunchKernelGGL((k_rows_fwd<T, false, C>), gr, b, row_lds, st, plan, tw, chirp, r, spec, Grid{}, StepPtrs{}, 0,
                        nullptr, Micro{});
     columns(NoMicro{}, 0, st);
-    if (x0)
-        hipLaunchKernelGGL((k_rows_inv<T, true, false, C>), gr, b, row_lds, st, plan, tw, chirp, spec, x0, x, Grid{},
+    if (w)
+        hipLaunchKernelGGL((k_rows_inv<T, true, true, C>), gr, b, row_lds, st, plan, tw, chirp, spec, x0, x, G, w,
+                           rhow, nullptr);
+    else if (x0)
+        hipLaunchKernelGGL((k_rows_inv<T, true, false, C>), gr, b, row_lds, st, plan, tw, chirp, spec, x0, x, G,
                            nullptr, nullptr, nullptr);
     else
-        hipLaunchKernelGGL((k_rows_inv<T, false, false, C>), gr, b, row_lds, st, plan, tw, chirp, spec, x0, x, Grid{},
+        hipLaunchKernelGGL((k_rows_inv<T, false, false, C>), gr, b, row_lds, st, plan, tw, chirp, spec, x0, x, G,
                            nullptr, nullptr, nullptr);
 }
 template <typename T>
 void Direct<T>::solve(const double *r, const double *x0, double *x, hipStream_t st) {
-    if (plan.chirp) rows_solve<true>(r, x0, x, st);
-    else rows_solve<false>(r, x0, x, st);
+    solve_w(r, x0, x, Grid{}, nullptr, nullptr, st);
+}
+template <typename T>
+void Direct<T>::solve_w(const double *r, const double *x0, double *x, const Grid &G, double *w, const double *rhow,
+                        hipStream_t st) {
+    if (plan.chirp) rows_solve<true>(r, x0, x, G, w, rhow, st);
+    else rows_solve<false>(r, x0, x, G, w, rhow, st);
 }
 
 template <typename T>

@@ -945,14 +945,18 @@ SolveResult Poisson::solve_fp64(double tol, int max_iter, hipStream_t st) {
 
 // Relative residual up to which one that no longer decreases counts as FP64's
 // round-off: 2^-53 times the largest condition number, 8 (M + 1)^2 / pi^2 times
-// the density's range over the column, 4e-10 at 480 levels.  The round-off of
-// L x itself is 1e-16 of ||b|| where b is rough, 3e-14 on k^-3 vorticity and
-// 1e-12 on the lowest mode (2048 x 256).
+// the density's range over the column, 4e-10 at 480 levels.  2^-53 of ||L|| ||x|| is 1e-16 of
+// ||b|| where b is rough, 3e-14 on k^-3 vorticity and 1e-12 on the lowest mode
+// (2048 x 256).  One solve leaves three to five times that and an error of up
+// to 3e-14, and a correction cuts an error by at least 1e-9, so that the
+// second solve always reaches the floor: 512 x 64, k^-3 vorticity, one / two /
+// three solves leave residuals of 4.6e-14 / 1.1e-14 / 1.1e-14 and errors of
+// 1.2e-14 / 9e-17 / 9e-17.
 constexpr double kRoundOff = 1e-9;
 
 // Norms of the residual kernel's slot (the caller has waited for it).
 void Poisson::norms(int slot, double *rn2, double *bn2) const {
-    const volatile double *p = hres + slot * 2 * kResidualBlocks;
+    const volatile double *p = slot_host(slot);
     *rn2 = *bn2 = 0.;
     for (int b = 0; b < res_blocks; b++) {  // fixed order: deterministic
         *rn2 += p[2 * b];
@@ -963,7 +967,7 @@ void Poisson::norms(int slot, double *rn2, double *bn2) const {
 // r of x (with ref: of the given right-hand side and guess), norms into slot.
 void Poisson::queue_r(const RefArrays *ref, int slot, hipStream_t st) {
     res_blocks = residual_blocks();
-    const Residual R{N, M, f, pcg64.x, cx0, cu0, pcg64.wD, hres_dev + slot * 2 * kResidualBlocks};
+    const Residual R{N, M, f, pcg64.x, cx0, cu0, pcg64.wD, slot_dev(slot)};
     if (ref)
         hipLaunchKernelGGL(k_solve_residual<true>, dim3(res_blocks), dim3(1024), 0, st, R, ref->b, ref->x, f,
                            pcg64.x, pcg64.r);
@@ -972,13 +976,22 @@ void Poisson::queue_r(const RefArrays *ref, int slot, hipStream_t st) {
                            nullptr, pcg64.r);
 }
 
+// Whether a correction that took the relative residual from prev to R.rel was
+// the last, and (R.converged) met the stop rule.
+static bool at_end(SolveResult &R, double prev, double tol, Floor floor) {
+    const bool stalled = R.rel > 0.5 * prev;
+    R.converged = R.rel <= tol || (floor != Floor::NONE && stalled && R.rel <= kRoundOff) ||
+                  (floor == Floor::PARITY && prev <= kRoundOff);
+    return R.converged || stalled;
+}
+
 // Each sweep: x += L^-1 r by a direct solve, formed in another buffer, the FP64
 // residual and (ref) the solution in the reference's order, all queued before
 // the host reads the norms; the first sweep also before it has read those of
 // the guess, which may already meet the stop rule.  2048 x 255 in FP64: 138 us, 6
 // launches and one wait, where 10 and three took 170.
 template <typename T>
-SolveResult Poisson::refine(Direct<T> &D, const RefArrays *ref, double tol, bool to_floor, int max_sweeps,
+SolveResult Poisson::refine(Direct<T> &D, const RefArrays *ref, double tol, Floor floor, int max_sweeps,
                             hipStream_t st) {
     SolveResult R;
     double rn2 = 0., bn2 = 0.;
@@ -1017,21 +1030,19 @@ SolveResult Poisson::refine(Direct<T> &D, const RefArrays *ref, double tol, bool
         R.rel = std::sqrt(rn2 / bn2);
         R.iters = R.refine = sweep;
         if (!std::isfinite(bn2) || !std::isfinite(rn2)) return R;
-        const bool stalled = R.rel > 0.5 * prev;
-        R.converged = R.rel <= tol || (to_floor && stalled && R.rel <= kRoundOff);
-        if (R.converged || stalled || sweep == max_sweeps) return R;
+        if (at_end(R, prev, tol, floor) || sweep == max_sweeps) return R;
         correct();
     }
 }
 
-SolveResult Poisson::solve_direct(const RefArrays &ref, double tol, bool to_floor, int max_sweeps, hipStream_t st) {
-    SolveResult R = refine(direct64, &ref, tol, to_floor, max_sweeps, st);
+SolveResult Poisson::solve_direct(const RefArrays &ref, double tol, Floor floor, int max_sweeps, hipStream_t st) {
+    SolveResult R = refine(direct64, &ref, tol, floor, max_sweeps, st);
     R.refine = 0;
     return R;
 }
 
 SolveResult Poisson::solve_mixed(const RefArrays &ref, double tol, int max_sweeps, hipStream_t st) {
-    return refine(direct32, &ref, tol, false, max_sweeps, st);
+    return refine(direct32, &ref, tol, Floor::NONE, max_sweeps, st);
 }
 
 void Poisson::queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, const Micro *micro,
@@ -1059,23 +1070,51 @@ void Poisson::queue_step(const Grid &G, const StepPtrs &S, int step, bool f_read
         direct64.solve_step(G, S, step, micro, f, pcg64.x, st);
     }
     bn_pending = 0;
+    corrected = expect_more;
+    if (corrected) {
+        mark_unset(slot_host(0), 2 * residual_blocks());
+        queue_r(nullptr, 0, st);
+        direct64.solve_w(pcg64.r, pcg64.x, x64B, G, w, rhow_dev, st);
+        std::swap(pcg64.x, x64B);
+    }
 }
 
-SolveResult Poisson::finish_step(const Grid &G, double *w, const double *rhow_dev, double tol, bool to_floor,
+SolveResult Poisson::finish_step(const Grid &G, double *w, const double *rhow_dev, double tol, Floor floor,
                                  int max_sweeps, bool *redo, hipStream_t st) {
     SolveResult R;
     *redo = false;
     double rn2 = 0., bn2 = 0.;
-    await_set(hres, 2 * res_blocks, st);
+    const bool more = corrected;
+    corrected = expect_more = false;
+    await_set(slot_host(0), 2 * res_blocks, st);
+    if (more) await_set(slot_host(1), 2 * res_blocks, st);
     norms(0, &rn2, &bn2);
     R.iters = 1;
     R.rel0 = 1.;
     R.rel = bn2 > 0. ? std::sqrt(rn2 / bn2) : std::sqrt(rn2);
     R.converged = std::isfinite(bn2) && R.rel <= tol;
-    if (R.converged || !std::isfinite(R.rel) || max_sweeps <= 1) return R;
+    if (R.converged || !std::isfinite(R.rel) || max_sweeps <= 1) {
+        if (more) {
+            hipStreamSynchronize(st);  // what is queued again marks its sums unset
+            std::swap(pcg64.x, x64B);
+            back_to_w(G, w, rhow_dev, st);
+            *redo = true;
+        }
+        return R;
+    }
     // beyond what one solve gives: corrected further
-    SolveResult C = refine(direct64, nullptr, tol, to_floor, max_sweeps - 1, st);
-    C.iters++;
+    expect_more = true;
+    if (more) {
+        const double prev = R.rel;
+        norms(1, &rn2, &bn2);
+        R.rel = std::sqrt(rn2 / bn2);
+        R.iters = 2;
+        R.refine = 1;
+        if (!std::isfinite(R.rel) || at_end(R, prev, tol, floor) || max_sweeps <= 2) return R;
+    }
+    SolveResult C = refine(direct64, nullptr, tol, floor, max_sweeps - R.iters, st);
+    C.iters += R.iters;
+    C.refine += R.refine;
     C.rel0 = 1.;
     back_to_w(G, w, rhow_dev, st);
     *redo = true;
@@ -1101,9 +1140,10 @@ void Poisson::queue_check(hipStream_t st) { queue_residual(Grid{}, StepPtrs{}, 0
 // k_calu's residual workgroups, behind ncol workgroups of cal_u
 void Poisson::queue_residual(const Grid &G, const StepPtrs &S, int ncol, hipStream_t st) {
     res_blocks = residual_blocks();
-    mark_unset(hres, 2 * res_blocks);
+    const int slot = corrected ? 1 : 0;
+    mark_unset(slot_host(slot), 2 * res_blocks);
     hipLaunchKernelGGL(k_calu, dim3(ncol + res_blocks), dim3(UW * UC), ncol ? size_t(N) * sizeof(double) : 0, st, G,
-                       S, ncol, Residual{N, M, f, pcg64.x, cx0, cu0, pcg64.wD, hres_dev});
+                       S, ncol, Residual{N, M, f, pcg64.x, cx0, cu0, pcg64.wD, slot_dev(slot)});
 }
 
 }  // namespace vvmd

@@ -63,6 +63,12 @@ struct RefArrays {
     hipEvent_t done;
 };
 
+// What ends a refinement, as converged, besides its tolerance: nothing; a
+// residual that has stopped decreasing, for a tolerance below round-off; or
+// that, and every correction of a residual that was no more than kRoundOff
+// already (VVM_STOP_PARITY in FP64).
+enum class Floor { NONE, STALL, PARITY };
+
 class Poisson {
    public:
     // rhou/rhow are the host profiles (nz long).  Allocates with hipMalloc.
@@ -101,22 +107,24 @@ class Poisson {
     SolveResult solve_fp64(double tol, int max_iter, hipStream_t st);
     // x as the guess, corrected by direct solves of the FP64 residual's system
     // until ||b-Ax||/||b|| <= tol: by FP64 ones (solve_direct) or FP32 ones
-    // (solve_mixed).  to_floor: also done when the residual has stopped
-    // decreasing at FP64's round-off (kRoundOff).
-    SolveResult solve_direct(const RefArrays &ref, double tol, bool to_floor, int max_sweeps, hipStream_t st);
+    // (solve_mixed).
+    SolveResult solve_direct(const RefArrays &ref, double tol, Floor floor, int max_sweeps, hipStream_t st);
     SolveResult solve_mixed(const RefArrays &ref, double tol, int max_sweeps, hipStream_t st);
     // The step's pubarTop_pt (not if step < 0), cal_w and cal_u in two halves.
     // queue_step: mean flow at the top, right-hand side (formed already if f_ready), solve and
     // w; queue_cal_u: u, and the residual's norms on their way to the host
     // (queue_check: the norms alone).  Nothing is waited for, but the network's
     // guess (if learned_guess wrote one) is judged in queue_step.  finish_step
-    // (the caller has waited for queue_cal_u's or queue_check's work): if the
-    // norms miss the stop rule, corrects x further; *redo says that x and w have changed since queue_step, so cal_u and what
-    // was queued behind it have to run again.
+    // waits for the norms: if they miss the stop rule, corrects x further;
+    // *redo says that x and w have changed since queue_step, so cal_u and what
+    // was queued behind it have to run again.  After a step that needed a
+    // correction the next one queues its own ahead of cal_u (it is taken back
+    // should the norms say that it was not due: what a step gives does not
+    // depend on the steps before).
     void queue_step(const Grid &G, const StepPtrs &S, int step, bool f_ready, const Micro *micro, hipStream_t st);
     void queue_cal_u(const Grid &G, const StepPtrs &S, hipStream_t st);
     void queue_check(hipStream_t st);
-    SolveResult finish_step(const Grid &G, double *w, const double *rhow_dev, double tol, bool to_floor,
+    SolveResult finish_step(const Grid &G, double *w, const double *rhow_dev, double tol, Floor floor,
                             int max_sweeps, bool *redo, hipStream_t st);
     // The reference GPU back-end's solver (k_bicgstab.hip): BiCGSTAB with a
     // red-black ILU0 preconditioner; stops at ||b - A x||_2 <= tol
@@ -172,10 +180,14 @@ class Poisson {
     double *hres = nullptr, *hres_dev = nullptr;  // residual norms, two slots (mapped host memory)
     void queue_residual(const Grid &G, const StepPtrs &S, int ncol, hipStream_t st);
     int res_blocks = 0;
+    bool expect_more = false;  // the last step's solve had to be corrected
+    bool corrected = false;    // this one's has been; x64B: as it was, slot 0: its norms
     template <typename T>
-    SolveResult refine(Direct<T> &D, const RefArrays *ref, double tol, bool to_floor, int max_sweeps, hipStream_t st);
+    SolveResult refine(Direct<T> &D, const RefArrays *ref, double tol, Floor floor, int max_sweeps, hipStream_t st);
     void queue_r(const RefArrays *ref, int slot, hipStream_t st);
     void norms(int slot, double *rn2, double *bn2) const;
+    double *slot_host(int slot) const { return hres + slot * 2 * kResidualBlocks; }
+    double *slot_dev(int slot) const { return hres_dev + slot * 2 * kResidualBlocks; }
     int residual_blocks() const { return std::min(kResidualBlocks, ((N + 63) / 64) * ((M + 15) / 16)); }
     bool keep_guess(double rn2);
     double *f = nullptr;       // rhs of L x = f, (M+2)*N

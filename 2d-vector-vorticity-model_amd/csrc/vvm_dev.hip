@@ -311,9 +311,19 @@ bool uses_pcg(const vvm_dev_config &c) {
     return c.solver_mode == VVM_SOLVER_FP64 && c.guess_mode != VVM_GUESS_ZERO;
 }
 bool uses_direct(const vvm_dev_config &c) { return c.solver_mode != VVM_SOLVER_BICGSTAB && !uses_pcg(c); }
-constexpr double kParityTol = 1e-13;  // VVM_STOP_PARITY where the residual is formed anew each sweep
+// VVM_STOP_PARITY: in FP64 until the residual no longer decreases, which one
+// below kParityTol64 counts as (solve_fp64 stops there too); the others meet
+// kParityTol.
+constexpr double kParityTol64 = 1e-15, kParityTol = 1e-13;
 constexpr int kMaxSweeps = 8;
-double stop_tol(const vvm_dev_config &c) { return c.stop_mode == VVM_STOP_PARITY ? kParityTol : c.tol_rel; }
+double stop_tol(const vvm_dev_config &c) {
+    if (c.stop_mode != VVM_STOP_PARITY) return c.tol_rel;
+    return c.solver_mode == VVM_SOLVER_FP64 ? kParityTol64 : kParityTol;
+}
+Floor stop_floor(const vvm_dev_config &c) {
+    if (c.solver_mode != VVM_SOLVER_FP64) return Floor::NONE;
+    return c.stop_mode == VVM_STOP_PARITY ? Floor::PARITY : Floor::STALL;
+}
 int max_iterations(const vvm_dev_config &c) { return c.max_iter > 0 ? c.max_iter : 200; }
 
 int ensure_poisson(vvm_dev *h, const double *rhou, const double *rhow) {
@@ -386,7 +396,7 @@ void queue_w(vvm_dev *h, const StepPtrs &S, int step, bool run_net, bool prepare
 int finish_w(vvm_dev *h, const StepPtrs &S, vvm_solve_stats *ss, bool *redo) {
     const vvm_dev_config &c = h->cfg;
     const bool fp64 = c.solver_mode == VVM_SOLVER_FP64;
-    SolveResult R = h->pois.finish_step(h->G, S.w, h->P.rhow, stop_tol(c), fp64,
+    SolveResult R = h->pois.finish_step(h->G, S.w, h->P.rhow, stop_tol(c), stop_floor(c),
                                         std::min(kMaxSweeps, max_iterations(c)), redo, h->st);
     if (!fp64) R.refine = R.iters;
     h->pois.collect_target(h->st);
@@ -1245,7 +1255,7 @@ static int poisson_common(vvm_dev *h, const double *d_b, double *d_x, vvm_solve_
     if (c.solver_mode == VVM_SOLVER_MIXED)
         R = h->pois.solve_mixed(ref, stop_tol(c), sweeps, h->st);
     else if (direct)
-        R = h->pois.solve_direct(ref, stop_tol(c), true, sweeps, h->st);
+        R = h->pois.solve_direct(ref, stop_tol(c), stop_floor(c), sweeps, h->st);
     else if (c.solver_mode == VVM_SOLVER_BICGSTAB)
         R = h->pois.solve_bicgstab(stop_tol(c), c.stop_mode == VVM_STOP_ABS, maxit, h->st);
     else

@@ -66,7 +66,8 @@ extern "C" {
                                 form until three solutions exist             */
 
 /* Stop rules of the elliptic solve. */
-#define VVM_STOP_PARITY 0  /* iterate until the residual stops decreasing   */
+#define VVM_STOP_PARITY 0  /* FP64: until the residual stops decreasing (or is
+                              1e-15 of ||b||); else 1e-13 of ||b||          */
 #define VVM_STOP_REL 1     /* ||b - A x||_2 / ||b||_2 <= tol_rel            */
 #define VVM_STOP_ABS 2     /* ||b - A x||_2 <= tol_rel (BiCGSTAB only)       */
 
