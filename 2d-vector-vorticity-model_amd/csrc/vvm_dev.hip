@@ -817,7 +817,10 @@ bool finish_solve(vvm_dev *h, bool wait) {
         r.rc = finish_w(h, r.S, &r.ss, &redo);
     }
     r.solved = true;
-    if (redo) launch_cal_u(h->G, r.S, h->st);
+    if (redo) {
+        KTimer t(h, VVM_KT_CALU);
+        launch_cal_u(h->G, r.S, h->st);
+    }
     return redo;
 }
 
@@ -991,12 +994,18 @@ int step_finish(vvm_dev *h, vvm_step_stats *acc) {
     StepPtrs &S = r.S;
     if (r.halo) take_tiles(h, S);  // back to what the sweep started from, which a correction needs
     const bool redo = finish_solve(h, false);
-    if (redo) queue_turbulence(h, S);
+    if (redo) {
+        KTimer t(h, VVM_KT_TURB);
+        queue_turbulence(h, S);
+    }
     const int need = sweep_halo(h);
     if (!redo && need && need <= r.halo) {
         take_tiles(h, S);
     } else {
-        diffuse(h, S, step_nudge(c), need);
+        {
+            KTimer t(h, VVM_KT_DIFFUSION);
+            diffuse(h, S, step_nudge(c), need);
+        }
         queue_end(h, r.halo != 0);
     }
     if (r.rc == VVM_WARN_NOT_CONVERGED) acc->not_converged++;
