@@ -1018,6 +1018,25 @@ int step_finish(vvm_dev *h, vvm_step_stats *acc) {
     return check_launch(h);
 }
 
+double event_seconds(hipEvent_t a, hipEvent_t b) {
+    float ms = 0.f;
+    return hipEventElapsedTime(&ms, a, b) == hipSuccess ? double(ms) * 1e-3 : 0.;
+}
+
+// The phase times of the first n timed steps, as the reference fills t_*[step]
+// every step (after a synchronisation).
+void read_step_timers(vvm_dev *h, int n) {
+    for (int q = 0; q < n; q++) {
+        const hipEvent_t *E = &h->tev[size_t(q) * 8];
+        double *o = h->tout + size_t(q) * 5;
+        o[0] = event_seconds(E[0], E[1]);  // advection (phase A)
+        o[1] = event_seconds(E[1], E[2]);  // poisson (phase B)
+        o[2] = event_seconds(E[6], E[7]);  // microphysics (phase C, on its own stream)
+        o[3] = event_seconds(E[3], E[4]);  // turbulence and diffusion (phase D)
+        o[4] = event_seconds(E[0], E[5]);  // the whole step
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -1041,20 +1060,7 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
     const double wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     kt_collect(h);
     if (const int erc = check_sweep(h)) return erc;
-    // per-step phase times, as the reference fills t_*[step] every step
-    auto span = [&](hipEvent_t a, hipEvent_t b) {
-        float ms = 0.f;
-        return hipEventElapsedTime(&ms, a, b) == hipSuccess ? double(ms) * 1e-3 : 0.;
-    };
-    for (int n = 0; n < std::min(nsteps, h->tcap); n++) {
-        const hipEvent_t *E = &h->tev[size_t(n) * 8];
-        double *o = h->tout + size_t(n) * 5;
-        o[0] = span(E[0], E[1]);  // advection (phase A)
-        o[1] = span(E[1], E[2]);  // poisson (phase B)
-        o[2] = span(E[6], E[7]);  // microphysics (phase C, possibly on the second stream)
-        o[3] = span(E[3], E[4]);  // diffusion and nudging (phase E)
-        o[4] = span(E[0], E[5]);  // the whole step on the device
-    }
+    read_step_timers(h, std::min(nsteps, h->tcap));
     if (stats) {
         *stats = acc;
         stats->steps = nsteps;
@@ -1071,11 +1077,11 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
                 return warn;
             }
             const hipEvent_t *E = row ? &h->tev[size_t(nsteps - 1) * 8] : h->ev, *mp = row ? E + 6 : h->ev_mp;
-            stats->t_advection = span(E[0], E[1]);
-            stats->t_poisson = span(E[1], E[2]);
+            stats->t_advection = event_seconds(E[0], E[1]);
+            stats->t_poisson = event_seconds(E[1], E[2]);
             // phase C ran on the side stream (E[2] -> E[3] is only the wait for it)
-            stats->t_microphysics = span(mp[0], mp[1]);
-            stats->t_diffusion = span(E[3], E[4]);
+            stats->t_microphysics = event_seconds(mp[0], mp[1]);
+            stats->t_diffusion = event_seconds(E[3], E[4]);
             stats->t_all = wall / nsteps;
         }
     }
@@ -1531,11 +1537,17 @@ void dev_set_phase_overlap(vvm_dev_t *h, bool on) {
 int dev_step_begin(vvm_dev_t *h) {
     if (!h->uploaded) return fail(h, VVM_ERR_STATE, "step before upload");
     HIPCHK(h, hipSetDevice(h->device));
-    return step_begin(h, -1, false);
+    if (h->kt_used) {  // a kernel is being timed: every launch counts, whatever their number
+        HIPCHK(h, hipStreamSynchronize(h->st));
+        kt_collect(h);
+    }
+    return step_begin(h, h->tcap > 0 ? 0 : -1, false);
 }
 int dev_step_finish(vvm_dev_t *h, vvm_step_stats *acc) { return step_finish(h, acc); }
-int dev_steps_end(vvm_dev_t *h) {
+int dev_steps_end(vvm_dev_t *h, bool stepped) {
     HIPCHK(h, hipStreamSynchronize(h->st));
+    kt_collect(h);
+    if (stepped) read_step_timers(h, std::min(1, h->tcap));
     return check_sweep(h);
 }
 }  // namespace vvmd

@@ -16,7 +16,7 @@ void dev_set_phase_overlap(vvm_dev_t *h, bool on);
 // a step in two halves, and the wait for the last of them
 int dev_step_begin(vvm_dev_t *h);
 int dev_step_finish(vvm_dev_t *h, vvm_step_stats *acc);
-int dev_steps_end(vvm_dev_t *h);
+int dev_steps_end(vvm_dev_t *h, bool stepped);
 }  // namespace vvmd
 
 struct vvm_ens {
@@ -156,7 +156,7 @@ int vvm_ens_step(vvm_ens_t *e, int nsteps, vvm_ens_stats *stats) {
         // before the first one's checks are waited for, so all their streams
         // have work meanwhile
         vvm_step_stats st{};
-        bool ok = true;
+        bool ok = true, stepped = false;
         for (int s = 0; s < nsteps && ok && first_err.load() == 0; s++) {
             size_t begun = 0;
             for (int i : e->work[w]) {
@@ -168,8 +168,9 @@ int vvm_ens_step(vvm_ens_t *e, int nsteps, vvm_ens_stats *stats) {
                 const int i = e->work[w][k];
                 if (failed(i, vvmd::dev_step_finish(e->dev[i], &st))) ok = false;
             }
+            stepped = stepped || ok;
         }
-        for (int i : e->work[w]) failed(i, vvmd::dev_steps_end(e->dev[i]));
+        for (int i : e->work[w]) failed(i, vvmd::dev_steps_end(e->dev[i], stepped));
         iters += st.solve_iters_total;
         notconv += st.not_converged;
     };

@@ -121,10 +121,12 @@ void await_set(const double *p, int n, hipStream_t st);
 void dev_set_phase_overlap(vvm_dev_t *h, bool on);
 // A step in two halves, for callers that drive several handles: dev_step_begin
 // queues it, dev_step_finish waits for its checks (and adds the solve to acc)
-// and queues its end, dev_steps_end waits for all of it.  No phase times.
+// and queues its end, dev_steps_end waits for all of it.  Each counts as a call
+// of one step for the handle's timers: the kernel timer sees every launch, and
+// row 0 of the step timers holds the last step (if stepped).
 int dev_step_begin(vvm_dev_t *h);
 int dev_step_finish(vvm_dev_t *h, vvm_step_stats *acc);
-int dev_steps_end(vvm_dev_t *h);
+int dev_steps_end(vvm_dev_t *h, bool stepped);
 void launch_pubartop(const Grid &G, const StepPtrs &S, int step, hipStream_t st);
 // The reference operators one at a time (vvm_dev_op_field).
 void launch_advection_zeta(const Grid &G, const StepPtrs &S, int step, hipStream_t st);

@@ -2,6 +2,7 @@
 selected kernel, also where the sweep runs in order or a step's end runs twice.
 The inputs that lead there are those of test_gpu_redo and
 test_gpu_diffusion_order."""
+import numpy as np
 import pytest
 
 import vvm_amd as V
@@ -39,3 +40,21 @@ def test_repeated_launches_are_timed(kernel):
         s = dev.step(1)
         _, n = dev.kernel_time()
     assert s.solve_iters_last > 1 and n == 2
+
+
+def test_ensemble_members_are_timed():
+    """A member's timers count the ensemble's steps as calls of one step."""
+    cases = [V.grid_case(64, 32, seed=k) for k in range(3)]
+    steps = 300  # more than the kernel timer holds between two readings
+    times = np.zeros((2, 5))
+    with V.Ensemble(cases, threads=2) as ens:
+        a, b = ens.member(0), ens.member(1)
+        a.kernel_timer(KT_CALU)
+        b._check(b.lib.vvm_dev_set_step_timers(b.h, times.ctypes.data_as(V.PTR), 2), "set_step_timers")
+        ens.step(0)
+        assert not times.any()
+        ens.step(steps)
+        avg, n = a.kernel_time()
+        assert n == steps and avg > 0.0
+        assert (times[0] > 0.0).all() and not times[1].any()
+        assert times[0, :4].max() <= times[0, 4]
