@@ -326,6 +326,7 @@ __global__ void __launch_bounds__(UW *UC) __attribute__((amdgpu_waves_per_eu(8))
     __shared__ double cs[UW * UC / kWave][UW], top[UW];
     if (int(blockIdx.x) >= ncol) {
         residual_norms(R, blockIdx.x - ncol, gridDim.x - ncol);
+        note_end(S.clock, CLK_SOLVE_END);
         return;
     }
     const int N = G.nx - 2, nz = G.nz, tid = threadIdx.x;

@@ -996,7 +996,9 @@ int step_finish(vvm_dev *h, vvm_step_stats *acc) {
     const bool redo = finish_solve(h, false);
     if (redo) {
         KTimer t(h, VVM_KT_TURB);
-        queue_turbulence(h, S);
+        StepPtrs again = S;
+        again.clock = nullptr;  // the phase began with the first pass, as it does with events
+        queue_turbulence(h, again);
     }
     const int need = sweep_halo(h);
     if (!redo && need && need <= r.halo) {
@@ -1070,7 +1072,7 @@ int vvm_dev_step(vvm_dev_t *h, int nsteps, vvm_step_stats *stats) {
             if (h->run.clocked) {
                 const volatile long long *k = reinterpret_cast<long long *>(h->kmax + kTurbBlocks + 1);
                 stats->t_advection = double(k[CLK_SOLVE] - k[CLK_ADVECT]) * h->clock_s;
-                stats->t_poisson = double(k[CLK_TURB] - k[CLK_SOLVE]) * h->clock_s;
+                stats->t_poisson = double(k[CLK_SOLVE_END] - k[CLK_SOLVE]) * h->clock_s;
                 stats->t_microphysics = double(k[CLK_MICRO_END] - k[CLK_MICRO]) * h->clock_s;
                 stats->t_diffusion = double(k[CLK_MEAN] - k[CLK_TURB]) * h->clock_s;
                 stats->t_all = wall / nsteps;

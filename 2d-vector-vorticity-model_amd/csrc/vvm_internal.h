@@ -64,7 +64,7 @@ struct StepPtrs {
 };
 
 // The phase boundaries of a step whose kernels note them (StepPtrs::clock).
-enum { CLK_ADVECT = 0, CLK_SOLVE, CLK_MICRO, CLK_MICRO_END, CLK_TURB, CLK_MEAN, CLK_N };
+enum { CLK_ADVECT = 0, CLK_SOLVE, CLK_SOLVE_END, CLK_MICRO, CLK_MICRO_END, CLK_TURB, CLK_MEAN, CLK_N };
 
 
 struct Reductions {

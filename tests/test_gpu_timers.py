@@ -58,3 +58,18 @@ def test_ensemble_members_are_timed():
         assert n == steps and avg > 0.0
         assert (times[0] > 0.0).all() and not times[1].any()
         assert times[0, :4].max() <= times[0, 4]
+
+
+def test_phases_of_a_repeated_end():
+    """What a correction repeats belongs to the phase of turbulence and
+    diffusion, with the kernels' clocks as with events."""
+    c = V.grid_case(128, 64, stop_mode=V.VVM_STOP_REL, tol_rel=1e-18)
+    st = V.init_state(c)
+    for timed in (False, True):
+        with V.Device(c.cfg) as dev:
+            dev.upload(st)
+            s = dev.step_timed(1)[0] if timed else dev.step(1)
+        print(f"events {timed}: poisson {s.t_poisson * 1e6:.0f} us, diffusion {s.t_diffusion * 1e6:.0f} us", flush=True)
+        assert s.solve_iters_last > 1
+        assert 0.0 < s.t_poisson < s.t_diffusion
+        assert s.t_advection > 0.0 and s.t_microphysics > 0.0
