@@ -1402,17 +1402,40 @@ int vvm_dev_set_shape(vvm_dev_t *h, int cw, int kib) {
     return VVM_OK;
 }
 
+// Whether the state's coefficients (at least 10, the closure's smallest) ask for
+// the diffusion sweep in order.
+static int sweeps_in_order(vvm_dev *h, bool *in_order) {
+    std::vector<double> k[2];
+    h->link.clear();
+    for (int q = 0; q < 2; q++) {
+        k[q].resize(size_t(h->G.nx) * h->G.nz);
+        h->link.field(k[q].data(), q ? h->RKH : h->RKM);
+    }
+    if (const int rc = receive(h)) return rc;
+    double m = 10.;
+    for (const auto &f : k)
+        for (double v : f)
+            if (!(v <= m)) m = v;
+    *in_order = diffusion_halo(m * h->rho_per_k) == 0;
+    return VVM_OK;
+}
+
 // Launch-shape tuner: times whole steps for each candidate (diffusion strip
 // width x multigrid coarse-kernel LDS budget) on the live state, keeps the
-// fastest, and restores the state.  Results are cached per device, grid and
-// solver mode for the life of the process.
+// fastest, and restores the state.  A width is a candidate only where the sweep
+// runs in order, a budget only where MG-PCG solves: elsewhere they change no
+// launch, the times differ by noise alone, and the default stays.  Results are
+// cached per device, grid, solver and these two for the life of the process.
 int vvm_dev_tune(vvm_dev_t *h, int steps, vvm_tune_result *out) {
     if (!h || steps <= 0) return VVM_ERR_ARG;
     if (!h->uploaded || !h->pois_ready) return fail(h, VVM_ERR_STATE, "tune before upload");
     HIPCHK(h, hipSetDevice(h->device));
     static std::mutex mu;
-    static std::vector<std::pair<std::array<int, 4>, vvm_tune_result>> cache;
-    const std::array<int, 4> key{h->device, h->cfg.nx, h->cfg.nz, h->cfg.solver_mode};
+    static std::vector<std::pair<std::array<int, 6>, vvm_tune_result>> cache;
+    const bool pcg = uses_pcg(h->cfg);
+    bool in_order = false;
+    if (const int rc = sweeps_in_order(h, &in_order)) return rc;
+    const std::array<int, 6> key{h->device, h->cfg.nx, h->cfg.nz, h->cfg.solver_mode, pcg, in_order};
     {
         std::lock_guard<std::mutex> lk(mu);
         for (auto &e : cache)
@@ -1463,9 +1486,10 @@ int vvm_dev_tune(vvm_dev_t *h, int steps, vvm_tune_result *out) {
     best.ms_per_step = 1e300;
     double ms_default = 0.;
     for (int cw : cws) {
-        if (!h->dslots && cw != 4) continue;  // one-workgroup sweep: nothing to choose
+        if (!(h->dslots && in_order) && cw != 4) continue;  // tiles or the one-workgroup sweep: nothing to choose
         if (h->dslots && (G.nx - 2 + cw * 64 - 1) / (cw * 64) > 64) continue;
         for (int kb : kib) {
+            if (!pcg && kb != 64) continue;
             h->dstrip_cw = cw;
             if ((rc = h->pois.replan(size_t(kb) * 1024)) != VVM_OK) break;
             if ((rc = vvm_dev_step(h, 1, nullptr)) < 0) break;  // warm-up

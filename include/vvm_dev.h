@@ -277,10 +277,12 @@ int vvm_dev_kernel_time(vvm_dev_t *h, double *avg_seconds, int *launches);
 /* Launch-shape autotuner (no counterpart in the reference): times `steps`
  * whole steps for each candidate launch shape on the live state and keeps
  * the fastest; the model state is restored afterwards.  Candidates: the
- * diffusion sweep's strip width (2, 4 or 8 wavefronts of 64 columns) and
- * the LDS budget (16, 32, 64 KiB) that decides which multigrid levels run in
- * the one-workgroup coarse kernel.  Results are cached per device, grid and
- * solver mode for the life of the process. */
+ * diffusion sweep's strip width (2, 4 or 8 wavefronts of 64 columns), where
+ * the state's coefficients are so large that the sweep runs in order, and the
+ * LDS budget (16, 32, 64 KiB) that decides which multigrid levels run in the
+ * one-workgroup coarse kernel, where the solver is MG-PCG; otherwise the
+ * default shape is timed and kept.  Results are cached per device, grid, solver
+ * and candidates for the life of the process. */
 typedef struct vvm_tune_result {
     int32_t diffusion_strip_waves;
     int32_t mg_coarse_lds_kib;
