@@ -686,7 +686,7 @@ __global__ void __launch_bounds__(256) k_columns(int N, int M, T *__restrict__ s
         spec[size_t(j) * N + q] = j == cs.mid ? Mid.z[c] : L[step(j)].e[lane(j)].z;
 }
 
-constexpr size_t kLdsMax = 160 * 1024, kLdsStatic = 4 * 1024;  // the sums' arrays
+constexpr size_t kLdsMax = 156 * 1024;  // of a CU's 160 KiB; the sums' arrays take the rest
 
 template <typename T>
 T *dalloc(size_t n) {
@@ -695,11 +695,13 @@ T *dalloc(size_t n) {
     return static_cast<T *>(p);
 }
 
+// The attribute belongs to the kernel, not to this plan: always the most that
+// any plan may ask for, so that no handle lowers it under another.
 template <typename K>
 bool allow_lds(K kernel, size_t bytes) {
     return bytes <= 64 * 1024 || hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                     int(bytes)) == hipSuccess;
+                                                     int(kLdsMax)) == hipSuccess;
 }
 
 // exp(-2 pi i k / n)
@@ -771,7 +773,7 @@ int Direct<T>::init(int N, int M, const double *cx, const double *cu) {
     plan.threads = std::min(1024, std::max(64, ((L + 7) / 8 + 63) / 64 * 64));
     const size_t LN = size_t(L - 1) + size_t((L - 1) >> 5) + 1;
     row_lds = 2 * LN * sizeof(T);
-    if (row_lds + 2 * size_t(L) * sizeof(T) <= kLdsMax - kLdsStatic) {
+    if (row_lds + 2 * size_t(L) * sizeof(T) <= kLdsMax) {
         plan.tw = sums && !plan.chirp ? RowPlan::TW_ROOTS : RowPlan::TW_STAGES;
         row_lds += 2 * size_t(L) * sizeof(T);
     }
