@@ -3,6 +3,7 @@
 #include <atomic>
 #include <cstring>
 #include <thread>
+#include <utility>
 
 #include "transfer.h"
 
@@ -110,6 +111,16 @@ int HostLink::reserve(int n, size_t doubles) {
     return VVM_OK;
 }
 
+bool HostLink::host_arrays_overlap(const Grid &G) const {
+    std::vector<std::pair<const double *, const double *>> r;
+    for (const Item &it : items)
+        r.emplace_back(it.host, it.host + (it.n > 0 ? size_t(it.n) : size_t(G.nx) * G.nz * (it.dev2 ? 2 : 1)));
+    std::sort(r.begin(), r.end());
+    for (size_t q = 1; q < r.size(); q++)
+        if (r[q].first < r[q - 1].second) return true;
+    return false;
+}
+
 // Chunks of at most a slot; small states go as one, by this thread alone.
 // Otherwise up to kThreads threads each keep two slots going: while the GPU
 // moves one, the thread copies the other (one thread copies at 10 to 18 GB/s,
@@ -163,7 +174,10 @@ int HostLink::move(bool up, const Grid &G, int device, hipStream_t st) {
             i += n;
         }
     }
-    const int nc = int(chunks.size()), nt = std::min(kThreads, (nc + 1) / 2), per_thread = std::min(2, nc);
+    // arrays of a download that share memory: one thread, whose copies follow the
+    // list, so that the array listed last is the one that stays
+    const bool shared = !up && host_arrays_overlap(G);
+    const int nc = int(chunks.size()), nt = shared ? 1 : std::min(kThreads, (nc + 1) / 2), per_thread = std::min(2, nc);
     if (const int rc = reserve(nt * per_thread, cap)) return rc;
     const size_t lds = size_t(kCols) * (G.nz + 1) * sizeof(double);
     auto copy = [&](int c, double *s) {

@@ -39,6 +39,7 @@ class HostLink {
     size_t slot_doubles = 0;
     int nslots = 0;
     int reserve(int n, size_t doubles);
+    bool host_arrays_overlap(const Grid &G) const;
     int move(bool up, const Grid &G, int device, hipStream_t st);
 };
 
