@@ -121,6 +121,7 @@ __global__ void __launch_bounds__(BX *TBY) k_turb_coeffs(Grid G, StepPtrs S, dou
     if (threadIdx.x == kWave - 1) sh[threadIdx.y] = m;
     __syncthreads();
     if (threadIdx.x == 0 && threadIdx.y == 0) {
+        m = sh[0];
         for (int w = 1; w < TBY; w++) m = max_or_nan(m, sh[w]);
         __hip_atomic_store(kmax + blockIdx.x, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }

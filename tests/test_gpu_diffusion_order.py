@@ -87,3 +87,44 @@ def test_tiles_at_row_edges(oracle, rows, want_halo):
 def test_tiles_of_more_rows(oracle, nx, nz):
     """More than a workgroup a CU at 8 rows a wavefront: 16 and 24 of them."""
     check_sweep(oracle, nx, nz, 8)
+
+
+def unstable_row(row, cols):
+    """Coefficients that are large in some columns of one row alone: stable
+    stratification (K at its smallest, 10) but for a layer turned over there."""
+    c = V.grid_case(300, 60, dx=100.0, dt=4.0)
+    st = perturbed_state(c, seed=row, step=5)
+    for f in ("u", "w", "RKM", "RKH"):
+        st[f][:] *= 1e-6
+    st["th"][:] = (300.0 + 0.4 * np.arange(st.nz))[None, :]
+    st["th"][cols, row - 1] += 60.0
+    st["th"][cols, row + 1] -= 60.0
+    for f in ("zeta", "th", "qv", "qc", "qr"):
+        st[f + "p"][:] = st[f]
+    return c, st
+
+
+# whole rows, single columns, and all columns of the coefficients' 64-wide tiles
+# but their first
+COLUMNS = {"all": list(range(302)), "inner": [i for i in range(1, 301) if i % 64 != 1], "second": list(range(66, 129)),
+           "1": [1], "65": [65], "128": [128], "300": [300]}
+
+
+@pytest.mark.parametrize("cols", list(COLUMNS))
+@pytest.mark.parametrize("row", [1, 2, 16, 17, 18, 33, 49, 60])
+def test_warm_up_sees_every_coefficient(oracle, row, cols):
+    """The largest coefficient decides, whichever row and columns it is in."""
+    cols = COLUMNS[cols]
+    c, st = unstable_row(row, cols)
+    want = st.copy()
+    oracle.op("turbulence", c.cfg, want)
+    k = want["RKH"].copy()
+    k[cols, row] = 0.0
+    k = k[1:-1, 1:-1]  # the ghost cells repeat it
+    small = halo(c, {"rhou": want["rhou"], "rhow": want["rhow"], "RKM": k, "RKH": k})
+    need = halo(c, want)
+    print(f"turned over at row {row}, {len(cols)} columns: warm-up {need}, {small} without it", flush=True)
+    assert small == 8 and need != 8
+    with V.Device(c.cfg) as dev:
+        got = gpu_run_op(dev, st, "turbulence")
+    assert_fields_close(got, want, FIELDS, 1e-12, where=f"row {row}, {len(cols)} columns")
