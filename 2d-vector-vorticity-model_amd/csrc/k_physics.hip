@@ -63,7 +63,13 @@ __global__ void __launch_bounds__(BX *BY) k_negval_scale(Grid G, double *a, cons
 }
 
 // Turbulence::RKM_RKH coefficient part (Turbulent.cpp:13-45), with the
-// center halos of RKM and RKH.  Returns the larger of the two.
+// center halos of RKM and RKH.  Returns the larger of the two, and NaN where th
+// is not finite (ALL: any field that is diffused, or a neighbour of it): such a
+// value reaches every point to its east and above, so the sweep has to run in
+// order.  The coefficients do not tell: a Richardson number that is NaN gives
+// the smallest.  In a step without host microphysics th is enough: zeta shows in the solve's residual, and
+// the microphysics' negative-value pass leaves no such qv, qc or qr.
+template <bool ALL>
 __device__ inline double turb_point(const Grid &G, const StepPtrs &S, int i, int k) {
     const double *u = S.u, *w = S.w, *thp = S.fut[F_TH];
     const double Rz =
@@ -92,14 +98,24 @@ __device__ inline double turb_point(const Grid &G, const StepPtrs &S, int i, int
     kh = mins(kh, kmax);
     store_center(S.RKM, G, i, k, km);
     store_center(S.RKH, G, i, k, kh);
-    return max_or_nan(km, kh);
+    const double t = at(thp, G, i, k);
+    double bad = t - t;  // 0, or NaN
+    if constexpr (ALL) {
+        for (const double *f : S.fut)
+            for (double v : {at(f, G, i, k), at(f, G, i - 1, k), at(f, G, i + 1, k), at(f, G, i, k - 1),
+                             at(f, G, i, k + 1)})
+                bad += v - v;
+    }
+    return max_or_nan(max_or_nan(km, kh), bad);
 }
 
 constexpr int TBY = 16;
 // At most kTurbBlocks workgroups walk the tiles (few and large: every one ends
 // with a store to host memory, and 1089 of them made the kernel 2 us longer); each leaves the largest
 // coefficient it formed in kmax, from which the host chooses the diffusion
-// sweep.  A NaN (unstable stratification at rest: Ri = -inf) stays one.
+// sweep.  A NaN (unstable stratification at rest: Ri = -inf; fields that are not
+// finite) stays one.
+template <bool ALL>
 __global__ void __launch_bounds__(BX *TBY) k_turb_coeffs(Grid G, StepPtrs S, double *kmax) {
     note_start(S.clock, CLK_TURB);
     const int tx = (G.nx - 2 + BX - 1) / BX, nt = tx * ((G.nz - 2 + TBY - 1) / TBY);
@@ -107,7 +123,7 @@ __global__ void __launch_bounds__(BX *TBY) k_turb_coeffs(Grid G, StepPtrs S, dou
     for (int t = blockIdx.x; t < nt; t += gridDim.x) {
         const int i = 1 + (t % tx) * BX + threadIdx.x, k = 1 + (t / tx) * TBY + uniform(threadIdx.y);
         if (i < 1 || i > G.nx - 2 || k < 1 || k > G.nz - 2) continue;
-        const double v = turb_point(G, S, i, k);
+        const double v = turb_point<ALL>(G, S, i, k);
         m = max_or_nan(m, v);
     }
     // m >= 0 or NaN, so that a lane without a partner takes 0 (dpp)
@@ -209,10 +225,11 @@ void launch_negative_value(const Grid &G, const StepPtrs &S, double *a, const Re
     finalize<2>(rs, nblocks(grid2d(G)), S.s, RED_NEGVAL, S_NEG_RATIO, st);
     hipLaunchKernelGGL(k_negval_scale, grid2d(G), dim3(BX, BY), 0, st, G, a, S.s + S_NEG_RATIO);
 }
-int launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, double *kmax, hipStream_t st) {
+int launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, double *kmax, bool all, hipStream_t st) {
     const int nt = ((G.nx - 2 + BX - 1) / BX) * ((G.nz - 2 + TBY - 1) / TBY), turns = (nt + kTurbBlocks - 1) / kTurbBlocks,
               nb = (nt + turns - 1) / turns;
-    hipLaunchKernelGGL(k_turb_coeffs, dim3(nb), dim3(BX, TBY), 0, st, G, S, kmax);
+    if (all) hipLaunchKernelGGL(k_turb_coeffs<true>, dim3(nb), dim3(BX, TBY), 0, st, G, S, kmax);
+    else hipLaunchKernelGGL(k_turb_coeffs<false>, dim3(nb), dim3(BX, TBY), 0, st, G, S, kmax);
     return nb;
 }
 

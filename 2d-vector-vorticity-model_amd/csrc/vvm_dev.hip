@@ -203,10 +203,11 @@ StepPtrs ptrs(vvm_dev *h) {
     return S;
 }
 
-// Turbulence coefficients, and the largest of them on its way to the host.
-void queue_turbulence(vvm_dev *h, const StepPtrs &S) {
+// Turbulence coefficients, and the largest of them on its way to the host (all:
+// NaN if any field that the sweep takes is not finite).
+void queue_turbulence(vvm_dev *h, const StepPtrs &S, bool all) {
     mark_unset(h->kmax, kTurbBlocks);
-    h->kmax_blocks = launch_turbulence_coeffs(h->G, S, h->kmax_dev, h->st);
+    h->kmax_blocks = launch_turbulence_coeffs(h->G, S, h->kmax_dev, all, h->st);
 }
 
 // The sweep's largest weight sum, once it is there.
@@ -231,10 +232,11 @@ void take_tiles(vvm_dev *h, StepPtrs &S) {
     }
 }
 
-// The warm-up the coefficients ask for (0: the sweep in order); the next step is
-// queued with some reserve.
-int sweep_halo(vvm_dev *h) {
-    const double rho = diffusion_rho(h);
+// The warm-up the coefficients ask for (0: the sweep in order, also for fields
+// that are not finite); the next step is queued with some reserve.
+int sweep_halo(vvm_dev *h, bool finite) {
+    double rho = diffusion_rho(h);
+    if (!finite) rho = NAN;
     h->diff_halo = diffusion_halo(1.25 * rho);
     return diffusion_halo(rho);
 }
@@ -972,7 +974,7 @@ int step_begin(vvm_dev *h, int timer, bool last) {
     // updateMean (:408) is overwritten by nextTimeStep's before any read.
     {
         KTimer t(h, VVM_KT_TURB);
-        queue_turbulence(h, S);
+        queue_turbulence(h, S, h->mp_fn != nullptr);
     }
     if (r.halo) {
         {
@@ -998,9 +1000,10 @@ int step_finish(vvm_dev *h, vvm_step_stats *acc) {
         KTimer t(h, VVM_KT_TURB);
         StepPtrs again = S;
         again.clock = nullptr;  // the phase began with the first pass, as it does with events
-        queue_turbulence(h, again);
+        queue_turbulence(h, again, h->mp_fn != nullptr);
     }
-    const int need = sweep_halo(h);
+    // a zeta that is not finite leaves no finite residual
+    const int need = sweep_halo(h, std::isfinite(r.ss.rel_residual));
     if (!redo && need && need <= r.halo) {
         take_tiles(h, S);
     } else {
@@ -1148,8 +1151,8 @@ int vvm_dev_op(vvm_dev_t *h, int op) {
             launch_bc_all_prog(G, S, h->st);
             break;
         case VVM_OP_TURBULENCE:
-            queue_turbulence(h, S);
-            diffuse(h, S, 0, sweep_halo(h));
+            queue_turbulence(h, S, true);
+            diffuse(h, S, 0, sweep_halo(h, true));
             break;
         case VVM_OP_NUDGE:
             launch_nudge(G, S, 1 | (c.CASE != 2 ? 2 : 0), h->st);

@@ -145,9 +145,10 @@ Negval launch_kessler(const Grid &G, const StepPtrs &S, const RedSlot &rs, hipSt
 Negval launch_kessler(const Grid &G, const StepPtrs &S, const Negval &nv, const Forcing &F, const RedSlot &rs,
                       hipStream_t st);
 // kmax (host-mapped, kTurbBlocks doubles): the largest RKM or RKH each
-// workgroup formed; returns their count.
+// workgroup formed, NaN where th (all: any of the fields) is not finite;
+// returns their count.
 constexpr int kTurbBlocks = 640;
-int launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, double *kmax, hipStream_t st);
+int launch_turbulence_coeffs(const Grid &G, const StepPtrs &S, double *kmax, bool all, hipStream_t st);
 bool diffusion_supported(const Grid &G);  // nx - 2 <= 8192
 // nudge bit 0 fuses Nudge_theta, bit 1 Nudge_zeta into the sweep's store;
 // only_field >= 0 sweeps that one field (Mparam or one Hparam) alone.
