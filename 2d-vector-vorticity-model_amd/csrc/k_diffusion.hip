@@ -12,6 +12,8 @@
 // columns or rows away falls as (a + d)^m and is below FP64's rounding after a
 // few.  Where that holds (diffusion_halo), k_diff_tiles cuts the fields into
 // independent tiles, each of which starts that many columns and rows early.
+// Finite values, that is: a NaN or an infinity does not decay, and fields that
+// hold one are swept in order (k_turb_coeffs).
 //
 // Otherwise the sweep runs in order, in two kernels.  k_diff_coeffs forms
 // a, c, d for every point of the five fields in parallel over the whole GPU (a

@@ -731,11 +731,17 @@ void host_fft(std::vector<std::complex<long double>> &v, const std::vector<std::
 }
 
 // Up to this sum of the prime factors above 5 the direct sums are used, where
-// they cost no more than the chirp's second transform and longer rows.  A whole
-// isolated solve with 64 rows in us, sums / chirp: 28 columns (sum 7) 72 / 69,
-// 176 (11) 75 / 70, 208 (13) 76 / 68, 437 (42) 106 / 75; 1100 (11) 81 / 87, 1472
-// (23) 90 / 86, 1184 (37) 103 / 87, 2128 (26) 106 / 113, 3712 (29) 115 / 116, 3059
-// (49) 138 / 115; and the primes 317 383 / 75, 1021 1141 / 78, 4093 5316 / 116.
+// they cost no more, to 3%, than the chirp's second transform and longer rows: at
+// such a tie their residual is the smaller one (28 columns 3.7e-15 against
+// 4.7e-15, 1472 8.2e-15 against 9.8e-15).  A whole isolated solve with 64 rows in
+// us, sums / chirp: 28 columns (sum 7) 49.6 / 48.0, 56 49.6 / 49.9, 448 54.2 /
+// 60.0, 896 57.4 / 62.2, 176 (11) 56.9 / 52.8, 208 (13) 58.8 / 52.6; for more than
+// 1024 columns 1792 (7) 59.2 / 72.0, 1100 (11) 62.7 / 70.6, 1216 (19) 68.6 / 70.6,
+// 1472 (23) 73.2 / 71.1, 2128 (26) 92.8 / 103.9, 2401 (28) 102.0 / 104.7, 1856
+// (29) 85.3 / 72.6, 1184 (37) 89.6 / 75.3, 3059 (49) 127.6 / 106.6.  Above 1024
+// the lines of 2048 and 4096 columns' chirps are not told apart (3712 (29) 101.2
+// / 104.7), nor below it those of 11 and 13 (704 58.8 / 61.4, 832 61.9 / 62.1).
+// With sums a prime of 317 columns took 383 us, 4093 5316.
 inline int max_sums(int N) { return N <= 1024 ? 10 : 28; }
 
 }  // namespace

@@ -564,11 +564,14 @@ Negval launch_thermo4(const Grid &G, const StepPtrs &S, int step, const RedSlot 
     return {rs, n};
 }
 int advect_tiles(const Grid &G) { return t4_tiles_x(G) * t4_tiles_z(G); }
-// Up to 1024 tiles of each, four to a CU: there the two shorten each other's
-// last round and save a launch.  Above, the launch is nothing and thermo4's
-// LDS keeps CUs from filling up with pzeta's tiles.  A step in us, together /
-// apart: 128 x 64 55.7 / 63.5, 1024 x 128 78.9 / 83.1, 2048 x 128 104.4 / 106.5,
-// 2048 x 256 (1024 tiles) 142.9 / 146.4, 4096 x 256 257.7 / 254.2.
+// Up to 1024 tiles of each, four to a CU and one round: there the two shorten
+// each other's last round and save a launch.  On large grids the launch is
+// nothing and thermo4's LDS keeps CUs from filling up with pzeta's tiles.  A
+// step in us, together / apart: 128 x 64 55.7 / 63.5, 1024 x 128 78.9 / 83.1,
+// 1536 x 256 128.0 / 132.2, 2048 x 256 (1024 tiles) 142.2 / 143.4; past the line
+// the last round decides, 1152 tiles 163.4 / 168.1, 1280 171.5 / 172.8, 1536
+// 193.5 / 199.1, 1792 236.5 / 226.7, 2048 (4096 x 256) 252.4 / 235.6: the line is
+// the last whole round, not the last grid that gains.
 bool advect_together(const Grid &G) { return advect_tiles(G) <= 1024; }
 Negval launch_advect(const Grid &G, const StepPtrs &S, int step, const RedSlot &rs, hipStream_t st) {
     const int n = advect_tiles(G);  // no fewer than pzeta's
@@ -579,7 +582,8 @@ Negval launch_advect(const Grid &G, const StepPtrs &S, int step, const RedSlot &
 // k_finalize (nblk 0 is returned), or, up to kFoldBlocks, by the workgroups of
 // the second pass themselves (nblk).  The launch costs 4 to 5 us
 // whatever it does; every workgroup's own sum costs the traffic of all partials
-// for each of them, which at 2048 x 256 (1089 and 2145 partials) is no gain.
+// for each of them, which at 2048 x 256 (1024 partials of thermo4, 2048 of
+// k_kessler) is no gain.
 Negval negval_partials(const StepPtrs &S, const Negval &nv, hipStream_t st) {
     if (nv.nblk <= kFoldBlocks) return nv;
     finalize<6>(nv.rs, nv.nblk, S.s, RED_NEGVAL, S_NEG_RATIO, st);

@@ -842,12 +842,14 @@ void queue_end(vvm_dev *h, bool again) {
 }
 
 // Whether the step's microphysics rides in the solve's launches: up to 640 of
-// thermo4's tiles.  That saves the host two launches and the two streams'
-// events, whose waits alone take it 24 us; above, the solve's LDS leaves too
-// few of these workgroups on a CU.  A step in us, riding against the second
-// stream: 128 x 64 68 / 85, 1024 x 128 84 / 101, 2048 x 128 106 / 111, 2048 x
-// 256 (1024 tiles) 141 / 143, 4096 x 256 261 / 247.  640 is also where the
-// ratios still come from the partial sums, without a k_finalize between.
+// thermo4's tiles, where the ratios still come from the partial sums, without a
+// k_finalize between.  That saves the host two launches and the two streams'
+// events, whose waits alone take it 24 us; on large grids the solve's LDS leaves
+// too few of these workgroups on a CU.  A step in us, riding against the second
+// stream: 128 x 64 68 / 85, 1024 x 128 84 / 101, 1024 x 256 103 / 106, 1280 x 256
+// (640 tiles) 114 / 115; past the line, every workgroup adding up to 1024
+// partials, 704 tiles 128 / 136, 800 132 / 132, 896 142 / 146, 1024 (2048 x 256)
+// 141 / 143, 2048 (4096 x 256) 261 / 247.
 bool ride_along(const vvm_dev *h, bool run_net) {
     if (!uses_direct(h->cfg) || h->mp_fn || run_net || h->pois.sample_cap > 0) return false;
     if (h->kt_kernel == VVM_KT_KESSLER || h->kt_kernel == VVM_KT_SCALE) return false;  // timed alone

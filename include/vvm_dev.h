@@ -269,8 +269,9 @@ int vvm_negative_value_noalloc(double *d_var, int nx, int nz, int pitch, void *s
 #define VVM_KT_TURB 5        /* RKM/RKH                                       */
 #define VVM_KT_DIFFUSION 6   /* in-place K-diffusion sweep (5 fields) + nudge */
 #define VVM_KT_MEAN 7        /* horizontal means (updateMean)                 */
-#define VVM_KT_CALU 8        /* cal_u (both kernels)                          */
-#define VVM_KT_SOLVE 9       /* the whole elliptic solve (many kernels)       */
+#define VVM_KT_CALU 8        /* cal_u (and the residual of a direct solve)   */
+#define VVM_KT_SOLVE 9       /* the elliptic solve (many kernels), without a
+                                direct solve's corrections after the fact    */
 int vvm_dev_kernel_timer(vvm_dev_t *h, int kernel);
 int vvm_dev_kernel_time(vvm_dev_t *h, double *avg_seconds, int *launches);
 
