@@ -98,15 +98,14 @@ __device__ inline double turb_point(const Grid &G, const StepPtrs &S, int i, int
     kh = mins(kh, kmax);
     store_center(S.RKM, G, i, k, km);
     store_center(S.RKH, G, i, k, kh);
-    const double t = at(thp, G, i, k);
-    double bad = t - t;  // 0, or NaN
+    bool finite = __builtin_isfinite(at(thp, G, i, k));
     if constexpr (ALL) {
         for (const double *f : S.fut)
             for (double v : {at(f, G, i, k), at(f, G, i - 1, k), at(f, G, i + 1, k), at(f, G, i, k - 1),
                              at(f, G, i, k + 1)})
-                bad += v - v;
+                finite = finite && __builtin_isfinite(v);
     }
-    return max_or_nan(max_or_nan(km, kh), bad);
+    return finite ? max_or_nan(km, kh) : __builtin_nan("");
 }
 
 constexpr int TBY = 16;
